@@ -1,0 +1,285 @@
+// out[M, N] = a[M, K] . w[N, K]^T (+ bias[N]), all float32, every product and sum in 32 bits: the
+// matrix product of the float32 engine, on v_mfma_f32_16x16x4f32.  That instruction is a chain of
+// four fused multiply-adds in ascending slot order, one rounding each (checked bit by bit against
+// fmaf, denormals too), so nothing is rounded more than by plain FMAs at twice their rate.
+//
+// Every output element is summed in one order, whatever the kernel and the step's row count:
+//   part: 16 consecutive k, chained from 0 in the order k = e + 4 g, e = 0..3 outside, g = 0..3
+//         inside (slot g of MFMA e holds element e of the four values at 4 g, so that a lane's
+//         operands for four MFMAs are one 16-byte load);
+//   mid:  the parts of 256 consecutive k, added in ascending order;
+//   total: the mids in ascending order.
+// So a row's result is the same bits alone and in any batch, and the rounding error of a sum over
+// thousands of k grows with its blocks (16 + 16 + K / 256 additions deep) and not with K.
+//
+// Few rows (gemm_f32_rows_kernel): bound by reading w once.  A block owns 16 or 32 rows of w and
+// all of k; its waves take 256 k in turn straight from memory, a mid each, and LDS adds the mids
+// in order.  Many rows (gemm_f32_tiles_kernel): bound by the matrix cores (157 TFLOP/s); tiles of
+// 128 x 64, 64 x 64 or 64 x 32 through two LDS buffers of 32 k.
+// Measured (us; before: plain FMAs in tiles of 64 x 64, up to 32 rows a wave for a few columns).  705 rows of the 1B
+// sizes: gate/up [16384, 2048] 1,507 -> 477 (99 TFLOP/s), o [2048, 2048] about 390 -> 81, down [2048, 8192] about
+// 1,510 -> 300, q/k/v [3072, 2048] 448 -> 123.  2 rows: gate/up 28.3 -> 28.6 (4.7 TB/s), head [128256, 2048] 209 -> 180
+// (5.8 TB/s).  Distance from 64 bits at k = 8192: 1.5e-7 of the result.
+#include "common.h"
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// values k .. k + 3 of a row, zeros from K on; VEC: rows start at multiples of 16 bytes and K % 4 == 0
+template <bool VEC>
+__device__ __forceinline__ f32x4 load4(const float* __restrict__ row, int k, int K) {
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    if (VEC) {
+        if (k < K) v = *reinterpret_cast<const f32x4*>(row + k);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) if (k + e < K) v[e] = row[k + e];
+    }
+    return v;
+}
+
+// four neighbouring columns of one row of the result
+__device__ __forceinline__ void store4(float* __restrict__ out, const float* __restrict__ bias, f32x4 v, int m, int n, int N, int ldo, bool vec) {
+    if (vec && n + 3 < N) {
+        if (bias) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] += bias[n + r];
+        }
+        *reinterpret_cast<f32x4*>(out + (size_t)m * ldo + n) = v;
+        return;
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+        if (n + r < N) out[(size_t)m * ldo + n + r] = bias ? v[r] + bias[n + r] : v[r];
+}
+
+// part = the chain over one block of 16 k: lane (i = lane & 15, g = lane >> 4) holds k = 4 g .. 4 g + 3 of row i of either operand
+__device__ __forceinline__ f32x4 chain16(f32x4 w, f32x4 a) {
+    f32x4 p = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) p = __builtin_amdgcn_mfma_f32_16x16x4f32(w[e], a[e], p, 0, 0, 0);
+    return p;
+}
+
+// WAVES waves a block; MT tiles of 16 rows of a and NS strips of 16 rows of w.  PL blocks of 16 k are asked for at once (8 KB of w a
+// wave at MT = NS = 1): in flight enough to stream w from memory with 16 waves a compute unit.
+template <int WAVES, int MT, int NS, bool VEC>
+__global__ __launch_bounds__(WAVES * 64) void gemm_f32_rows_kernel(
+        float* __restrict__ out, const float* __restrict__ a, const float* __restrict__ w,
+        const float* __restrict__ bias, int M, int N, int K, int lda, int ldo, int vec_out) {
+    constexpr int TILES = MT * NS, PL = TILES == 1 ? 8 : 4, OWN = (TILES + WAVES - 1) / WAVES;
+    __shared__ f32x4 mids[WAVES][TILES][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = lane & 15, g = lane >> 4;
+    const int n0 = blockIdx.x * 16 * NS, m0 = blockIdx.y * 16 * MT;
+    const float* wrow[NS];
+    const float* arow[MT];
+#pragma unroll
+    for (int s = 0; s < NS; ++s) wrow[s] = w + (size_t)min(n0 + 16 * s + i, N - 1) * K;
+#pragma unroll
+    for (int t = 0; t < MT; ++t) arow[t] = a + (size_t)min(m0 + 16 * t + i, M - 1) * lda;
+    f32x4 total[OWN];
+#pragma unroll
+    for (int o = 0; o < OWN; ++o) total[o] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int groups = (K + 255) / 256;
+    for (int g0 = 0; g0 < groups; g0 += WAVES) {                 // the same trips for every wave: the barriers match
+        const int grp = g0 + wave;
+        f32x4 mid[NS][MT];
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+#pragma unroll
+            for (int t = 0; t < MT; ++t) mid[s][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (grp < groups) {
+#pragma unroll 1
+            for (int p0 = 0; p0 < 16; p0 += PL) {
+                const int k0 = grp * 256 + p0 * 16;
+                if (k0 >= K) break;
+                f32x4 wv[PL][NS], av[PL][MT];
+#pragma unroll
+                for (int p = 0; p < PL; ++p) {
+#pragma unroll
+                    for (int s = 0; s < NS; ++s) wv[p][s] = load4<VEC>(wrow[s], k0 + 16 * p + 4 * g, K);
+#pragma unroll
+                    for (int t = 0; t < MT; ++t) av[p][t] = load4<VEC>(arow[t], k0 + 16 * p + 4 * g, K);
+                }
+#pragma unroll
+                for (int p = 0; p < PL; ++p)
+                    if (k0 + 16 * p < K) {
+#pragma unroll
+                        for (int s = 0; s < NS; ++s)
+#pragma unroll
+                            for (int t = 0; t < MT; ++t) mid[s][t] += chain16(wv[p][s], av[p][t]);
+                    }
+            }
+        }
+        if (g0 > 0) __syncthreads();                             // the mids of the trip before have been read
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+#pragma unroll
+            for (int t = 0; t < MT; ++t) mids[wave][s * MT + t][lane] = mid[s][t];
+        __syncthreads();
+        const int here = min(WAVES, groups - g0);
+#pragma unroll
+        for (int o = 0; o < OWN; ++o) {
+            const int tile = wave + o * WAVES;
+            if (tile < TILES)
+                for (int j = 0; j < here; ++j) total[o] += mids[j][tile][lane];
+        }
+    }
+#pragma unroll
+    for (int o = 0; o < OWN; ++o) {
+        const int tile = wave + o * WAVES;
+        if (tile >= TILES) continue;
+        const int m = m0 + 16 * (tile % MT) + i, n = n0 + 16 * (tile / MT) + 4 * g;
+        if (m < M) store4(out, bias, total[o], m, n, N, ldo, vec_out != 0);
+    }
+}
+
+// Tiles of TM rows of a x TN rows of w, four waves in two rows and two columns.  Rows of 32 k lie in LDS at a stride of 40 words:
+// 16 rows x 4 columns of 16 bytes are then read without bank conflicts.
+template <int TM, int TN, bool VEC>
+__global__ __launch_bounds__(256, 2) void gemm_f32_tiles_kernel(
+        float* __restrict__ out, const float* __restrict__ a, const float* __restrict__ w,
+        const float* __restrict__ bias, int M, int N, int K, int lda, int ldo, int vec_out, int m_tiles, int n_tiles) {
+    constexpr int KS = 32, LD = 40, MT = TM / 32, NT = TN / 32, COPIES = (TM + TN) * (KS / 4) / 256;
+    __shared__ __align__(16) float lds[2][(TM + TN) * LD];
+    // an XCD (every eighth block) takes neighbouring tiles, the rows of a fastest: its L2 keeps the rows of w
+    const int blocks = m_tiles * n_tiles, per = blocks / 8, more = blocks % 8, xcd = blockIdx.x & 7;
+    const int tile = xcd * per + min(xcd, more) + (blockIdx.x >> 3);
+    const int m0 = (tile % m_tiles) * TM, n0 = (tile / m_tiles) * TN;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, i = lane & 15, g = lane >> 4;
+    const int wm = (wave & 1) * (TM / 2), wn = (wave >> 1) * (TN / 2);
+
+    const float* src[COPIES];
+    int dst[COPIES];
+#pragma unroll
+    for (int c = 0; c < COPIES; ++c) {
+        const int piece = tid + 256 * c, row = piece >> 3, col = (piece & 7) * 4;
+        src[c] = row < TM ? a + (size_t)min(m0 + row, M - 1) * lda : w + (size_t)min(n0 + row - TM, N - 1) * K;
+        dst[c] = row * LD + col;
+    }
+    const int col = (tid & 7) * 4;
+    f32x4 next[COPIES];
+#pragma unroll
+    for (int c = 0; c < COPIES; ++c) next[c] = load4<VEC>(src[c], col, K);
+#pragma unroll
+    for (int c = 0; c < COPIES; ++c) *reinterpret_cast<f32x4*>(&lds[0][dst[c]]) = next[c];
+    __syncthreads();
+
+    f32x4 mid[NT][MT], total[NT][MT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) mid[n][m] = total[n][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int k0 = 0, s = 0; k0 < K; k0 += KS, ++s) {
+        const bool another = k0 + KS < K;
+        if (another) {
+#pragma unroll
+            for (int c = 0; c < COPIES; ++c) next[c] = load4<VEC>(src[c], k0 + KS + col, K);
+        }
+        const float* buf = lds[s & 1];
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            if (k0 + 16 * p >= K) break;
+            f32x4 av[MT], wv[NT];
+#pragma unroll
+            for (int m = 0; m < MT; ++m) av[m] = *reinterpret_cast<const f32x4*>(buf + (wm + 16 * m + i) * LD + 16 * p + 4 * g);
+#pragma unroll
+            for (int n = 0; n < NT; ++n) wv[n] = *reinterpret_cast<const f32x4*>(buf + (TM + wn + 16 * n + i) * LD + 16 * p + 4 * g);
+            f32x4 part[NT][MT];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int n = 0; n < NT; ++n)
+#pragma unroll
+                    for (int m = 0; m < MT; ++m)
+                        part[n][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[n][e], av[m][e], e ? part[n][m] : f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+            const bool fold = ((k0 / 16 + p) & 15) == 15;
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+#pragma unroll
+                for (int m = 0; m < MT; ++m) mid[n][m] += part[n][m];
+            if (fold) {
+#pragma unroll
+                for (int n = 0; n < NT; ++n)
+#pragma unroll
+                    for (int m = 0; m < MT; ++m) { total[n][m] += mid[n][m]; mid[n][m] = f32x4{0.f, 0.f, 0.f, 0.f}; }
+            }
+        }
+        if (another) {                                           // the other buffer was last read before the barrier behind it
+#pragma unroll
+            for (int c = 0; c < COPIES; ++c) *reinterpret_cast<f32x4*>(&lds[(s + 1) & 1][dst[c]]) = next[c];
+        }
+        __syncthreads();
+    }
+    const bool open = (((K + 15) / 16) & 15) != 0;              // parts since the last fold
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            f32x4 v = total[n][m];
+            if (open) v += mid[n][m];
+            const int row = m0 + wm + 16 * m + i;
+            if (row < M) store4(out, bias, v, row, n0 + wn + 16 * n + 4 * g, N, ldo, vec_out != 0);
+        }
+}
+
+namespace {
+
+constexpr double kUnits = 256, kUnitFlops = 157.3e12 / 256;
+
+// Seconds that the two kernels take, fitted to sweeps of 1 to 2,048 rows over eight matrices.  Tiles: a stage of 32 k takes a block that is
+// alone on its compute unit 0.35 us beside its products; blocks that share a unit hide that, and share the matrix cores, which the
+// kernel keeps busy 70 % of the time.
+double tiles_cost(double M, double N, double K, int tm, int tn) {
+    const double blocks = ceil(M / tm) * ceil(N / tn), tile = tm * (double)tn * 2 / kUnitFlops * (tn == 32 ? 1.6 : 1.4);
+    const double together = tn == 32 ? 4 : tm == 64 ? 3 : 2;
+    const double busy = ceil(blocks / kUnits) * tile * K, waits = ceil(blocks / (kUnits * together)) * (tile * K + K / 32 * 0.35e-6);
+    return (busy > waits ? busy : waits) + 3e-6;
+}
+
+// 17 rows and more by the few-row kernel: what its blocks ask of the caches (their strips of w and the rows of a, once a block), at the rates
+// that the three forms were measured at, with compute units idle while a last round of blocks runs.
+double rows_cost(double M, double N, double K, int mt, int ns) {
+    const double blocks = ceil(N / (16 * ns)) * ceil(M / (16 * mt));
+    const double spread = blocks < kUnits ? blocks / kUnits : blocks / kUnits / ceil(blocks / kUnits);
+    return blocks * (ns + mt) * 64 * K / (ns == 2 ? 5.3e12 : mt == 4 ? 6.7e12 : 9.5e12) / spread + 4e-6;
+}
+
+}  // namespace
+
+#define ROWS(W, MT, NS) do { \
+        const dim3 grid((N + 16 * NS - 1) / (16 * NS), (M + 16 * MT - 1) / (16 * MT)); \
+        if (vec) gemm_f32_rows_kernel<W, MT, NS, true><<<grid, W * 64, 0, stream>>>(out, a, w, bias, M, N, K, lda, ldo, vec_out); \
+        else gemm_f32_rows_kernel<W, MT, NS, false><<<grid, W * 64, 0, stream>>>(out, a, w, bias, M, N, K, lda, ldo, vec_out); \
+    } while (0)
+#define TILES(TM, TN) do { \
+        const int mt = (M + TM - 1) / TM, nt = (N + TN - 1) / TN; \
+        if (vec) gemm_f32_tiles_kernel<TM, TN, true><<<mt * nt, 256, 0, stream>>>(out, a, w, bias, M, N, K, lda, ldo, vec_out, mt, nt); \
+        else gemm_f32_tiles_kernel<TM, TN, false><<<mt * nt, 256, 0, stream>>>(out, a, w, bias, M, N, K, lda, ldo, vec_out, mt, nt); \
+    } while (0)
+
+// form: 0 chosen by the costs above; 1 to 4 the few-row kernel with 16, 32, 64 rows of a or 64 rows of a and 32 of w a block; 5 to 7 tiles of
+// 64 x 32, 64 x 64, 128 x 64
+LLOGOS_EXPORT int llogos_gemm_f32(float* out, const float* a, const float* w, const float* bias,
+                                  int M, int N, int K, int lda, int ldo, int form, hipStream_t stream) {
+    if (M <= 0 || N <= 0 || K <= 0 || lda < K || ldo < N || form < 0 || form > 7) return LLOGOS_BAD_ARGUMENT;
+    const bool vec = (K & 3) == 0 && (lda & 3) == 0 && (((uintptr_t)a | (uintptr_t)w) & 15) == 0;
+    const int vec_out = (ldo & 3) == 0 && ((uintptr_t)out & 15) == 0;
+    if (form == 0) {
+        const double cost[8] = {0, 0, rows_cost(M, N, K, 2, 1), rows_cost(M, N, K, 4, 1), rows_cost(M, N, K, 4, 2),
+                                tiles_cost(M, N, K, 64, 32), tiles_cost(M, N, K, 64, 64), tiles_cost(M, N, K, 128, 64)};
+        form = M <= 16 ? 1 : 2;
+        for (int f = 3; form > 1 && f <= 7; ++f) if (cost[f] < cost[form]) form = f;
+    }
+    // 16 waves a block where a matrix has few blocks and enough of k for all of them
+    const bool wide = K >= 16 * 256 && (N + 15) / 16 * ((M + 15) / 16) <= 512;
+    switch (form) {
+        case 1: if (wide) ROWS(16, 1, 1); else ROWS(8, 1, 1); break;
+        case 2: if (wide) ROWS(16, 2, 1); else ROWS(8, 2, 1); break;
+        case 3: ROWS(8, 4, 1); break;
+        case 4: ROWS(8, 4, 2); break;
+        case 5: TILES(64, 32); break;
+        case 6: TILES(64, 64); break;
+        default: TILES(128, 64); break;
+    }
+    return LLOGOS_LAUNCH_CHECK();
+}

@@ -211,9 +211,13 @@ def concat_rows(a: torch.Tensor, b: torch.Tensor, out_dtype: torch.dtype, delta:
     return out
 
 
+F32_FORM = 0                 # 0: chosen by the sizes; 1 to 7 force a form of the float32 product (tests)
+
+
 def gemm_generic(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out_dtype: torch.dtype,
                  out: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """a [M, K] . w [N, K]^T (+ bias) with plain 32-bit FMAs."""
+    """a [M, K] . w [N, K]^T (+ bias) with every product and sum in 32 bits; float32 throughout: on the matrix
+    cores' 32-bit instruction, a row's result the same bits whatever the other rows are."""
     _dev(w, bias)
     _need(a.is_cuda and a.dim() == 2 and a.stride(1) == 1, "gemm: a must be [M, K] with unit inner stride")
     M, K = a.shape
@@ -226,6 +230,9 @@ def gemm_generic(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor],
     else:
         _need(out.shape == (M, N) and out.dtype == out_dtype and out.stride(1) == 1, "gemm: bad out")
     if M == 0:
+        return out
+    if a.dtype == w.dtype == out_dtype == torch.float32:
+        _check(_lib().llogos_gemm_f32(_p(out), _p(a), _p(w), _p(bias), M, N, K, a.stride(0), out.stride(0), F32_FORM, _stream()), "gemm_f32")
         return out
     _check(_lib().llogos_gemm_generic(_p(out), _dt(out), _p(a), _dt(a), _p(w), _dt(w), _p(bias),
                                       M, N, K, a.stride(0), out.stride(0), _stream()), "gemm_generic")

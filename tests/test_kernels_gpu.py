@@ -281,6 +281,23 @@ def test_float32_product_of_few_rows_is_the_tiled_product_bit_for_bit(N, K_):
     assert torch.equal(few, many[:5])
 
 
+@pytest.mark.parametrize("M,N,K_", [(1, 16, 16), (17, 33, 40), (33, 70, 272), (64, 129, 4112), (65, 31, 255), (130, 66, 2049), (200, 250, 513)])
+def test_float32_product_gives_the_same_bits_in_every_form(M, N, K_, monkeypatch):
+    """The forms of the float32 product (few rows in three heights of blocks, tiles in three sizes) at remainders of
+    tiles, of blocks of 16 and of 256 k and of 16 bytes: one result, and right (a sum is at most 16 + 16 + K / 256
+    additions deep)."""
+    rng = np.random.default_rng(M)
+    a, w, b = _t(rng.standard_normal((M, K_))), _t(rng.standard_normal((N, K_)) * 0.05), _t(rng.standard_normal(N))
+    chosen = K.gemm_generic(a, w, b, torch.float32)
+    bound = 2.0 ** -24 * (34 + K_ / 256) * (_np(a.abs()) @ _np(w.abs()).T + np.abs(_np(b)))
+    assert (np.abs(_np(chosen) - pm.linear(_np(a), _np(w), _np(b))) <= bound).all()
+    for form in range(1, 8):
+        monkeypatch.setattr(K, "F32_FORM", form)
+        out = torch.full((M, N + 3), 7.0, device=DEV)
+        assert torch.equal(K.gemm_generic(a, w, b, torch.float32, out=out[:, :N]), chosen), form
+        assert (out[:, N:] == 7.0).all()
+
+
 def test_rope_table_is_double_precision():
     pos = _t([0, 1, 4095, 100000], torch.int32)
     f = pm.rope_frequencies(64, 5e5)
