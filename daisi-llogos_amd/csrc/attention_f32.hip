@@ -1,0 +1,211 @@
+// Attention of the float32 engine over the paged cache on the matrix cores' 32-bit instruction
+// (v_mfma_f32_16x16x4f32: a chain of four fused multiply-adds, nothing is rounded to fewer bits),
+// for heads of 64 and 128 dimensions; a window and sinks as in the kernel for any shape.
+//
+// A block takes 16 query rows of one sequence and kv head: rows are (token, head of the group)
+// pairs in order, so that the heads that share keys share a tile whatever the group's size.  Its
+// waves take the sequence's pages in turn.  A page is worked on by itself: scores of its 64 keys,
+// their maximum and sum, the weighted sum of its values from zero; the pages' results go through
+// LDS and are added in ascending order with the running maximum.  The order of every addition so
+// depends on the query's position alone, not on how many waves share the pages, on how the tokens
+// were cut into steps or on what else is in the batch: single tokens and prompts run this kernel
+// with the same bits.  (A page of which a row sees no key leaves the row as it was: factors 1 and
+// 0.)
+//
+// Bound by the latency of a page's loads in single-token steps and by the matrix cores in prompts
+// (a page of 16 rows of 64 dimensions: 128 instructions, 4,096 clocks).  The kernel for any shape
+// gave a block to every (token, head), whose threads walk keys and values with scalar loads.
+// Measured (us, before -> now): heads of 64, 32 to 8 kv heads, prompts of 515 and 190 tokens 1,019 -> 47, one of 2,048
+// tokens 14,731 -> 288; single tokens behind 515 and 190: 158 -> 17, behind 8,192: 2,625 -> 142.  Heads of 128: 1,496 -> 90,
+// 19,143 -> 536, 180 -> 27, 2,721 -> 259.
+#include "common.h"
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x8 __attribute__((ext_vector_type(8), aligned(16)));
+
+// cu: token offsets of the sequences [batch + 1]; null: every sequence brings one token
+template <int HD, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void attn_f32_kernel(
+        float* __restrict__ out, const float* __restrict__ q, int q_stride, const float* __restrict__ k_pool,
+        const float* __restrict__ v_pool, PagedKV cache, const int* __restrict__ cu, int batch,
+        const int* __restrict__ tok_pos, int n_heads, int group, float scale, int window, int sinks) {
+    constexpr int DB = HD / 16, OWN = (DB + WAVES - 1) / WAVES;
+    __shared__ f32x4 sums[WAVES][DB][64];
+    __shared__ float tops[WAVES][16], dens[WAVES][16];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = lane & 15, g = lane >> 4;
+    const int kvh = blockIdx.y;
+
+    // which sequence this tile of rows belongs to; the tiles of late tokens, which have most pages, go first
+    int seq = 0, first = 0, tokens = 1, tile = gridDim.x - 1 - blockIdx.x;
+    if (cu) {
+        for (;; ++seq) {
+            first = cu[seq];
+            tokens = cu[seq + 1] - first;
+            const int tiles = (tokens * group + 15) / 16;
+            if (tile < tiles || seq + 1 >= batch) break;
+            tile -= tiles;
+        }
+    } else {
+        const int tiles = (group + 15) / 16;
+        seq = tile / tiles;
+        tile -= seq * tiles;
+        first = seq;
+    }
+    const int rows = tokens * group, row = tile * 16 + i;        // this lane's query row (columns of the products)
+    const bool real = row < rows;
+    const int tok = first + min(row, rows - 1) / group, head = kvh * group + min(row, rows - 1) % group;
+    const int pos = real ? tok_pos[tok] : -1;
+    const int last = tok_pos[first + min(tile * 16 + 15, rows - 1) / group];       // the tile's latest position ...
+    const int early = tok_pos[first + tile * 16 / group];                          // ... and its earliest
+
+    f32x8 qv[HD / 32];
+#pragma unroll
+    for (int d = 0; d < HD / 32; ++d)
+        qv[d] = *reinterpret_cast<const f32x8*>(q + (size_t)tok * q_stride + (size_t)head * HD + 32 * d + 8 * g);
+
+    f32x4 acc[OWN];
+    float top = -INFINITY, den = 0.f;
+#pragma unroll
+    for (int o = 0; o < OWN; ++o) acc[o] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    const int pages = last / kPageTokens + 1;
+    for (int p0 = 0; p0 < pages; p0 += WAVES) {                  // the same trips for every wave: the barriers match
+        // pages that no row of the tile sees may have been given back: nothing of them is read
+        if (window > 0 && p0 * kPageTokens >= sinks && (p0 + WAVES) * kPageTokens - 1 <= early - window) continue;
+        const int page = p0 + wave, t0 = page * kPageTokens;
+        const bool seen = page < pages && !(window > 0 && t0 >= sinks && t0 + kPageTokens - 1 <= early - window);
+        float m = -INFINITY, l = 0.f;
+        f32x4 o[DB];
+#pragma unroll
+        for (int d = 0; d < DB; ++d) o[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (seen) {
+            const size_t base = paged_base(cache, seq, kvh, t0);
+            const float* kp = k_pool + base;
+            const float* vp = v_pool + base;
+            // S^T = K . Q^T: block rb of four tokens gives lane (i, g) the scores of row i with tokens 16 g + 4 rb .. + 3
+            f32x4 s[4];
+#pragma unroll
+            for (int rb = 0; rb < 4; ++rb) {
+                f32x8 kv[HD / 32];
+#pragma unroll
+                for (int d = 0; d < HD / 32; ++d)
+                    kv[d] = *reinterpret_cast<const f32x8*>(kp + ((rb * (HD / 8) + 4 * d + g) * 16 + i) * 8);
+                s[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int d = 0; d < HD / 32; ++d)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) s[rb] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[d][e], qv[d][e], s[rb], 0, 0, 0);
+            }
+#pragma unroll
+            for (int rb = 0; rb < 4; ++rb)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int t = t0 + 16 * g + 4 * rb + r;
+                    s[rb][r] = key_visible(pos, t, window, sinks) ? s[rb][r] * scale : -INFINITY;
+                    m = fmaxf(m, s[rb][r]);
+                }
+            m = fmaxf(m, __shfl_xor(m, 16, kWave));
+            m = fmaxf(m, __shfl_xor(m, 32, kWave));
+#pragma unroll
+            for (int rb = 0; rb < 4; ++rb)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    s[rb][r] = m == -INFINITY ? 0.f : expf(s[rb][r] - m);
+                    l += s[rb][r];
+                }
+            l += __shfl_xor(l, 16, kWave);
+            l += __shfl_xor(l, 32, kWave);
+            // O^T = V^T . P^T; values behind the tile's latest position were never written
+            const bool edge = t0 + kPageTokens - 1 > early || (window > 0 && t0 < max(sinks, last - window + 1));
+            bool odd = false;                                    // a value that is no number, of a token that some row does not see
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int d = 0; d < DB; ++d) {
+                    f32x8 vv = *reinterpret_cast<const f32x8*>(vp + (((d * 2 + h) * 4 + g) * 16 + i) * 8);
+                    if (t0 + kPageTokens - 1 > last) {
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) if (t0 + 16 * g + 8 * h + e > last) vv[e] = 0.f;
+                    }
+                    if (edge) {
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) odd |= !isfinite(vv[e]);
+                    }
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) o[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[e], s[2 * h + (e >> 2)][e & 3], o[d], 0, 0, 0);
+                }
+            if (edge && __any(odd)) {                            // a weight of 0 must not meet it: token by token, seen ones alone
+#pragma unroll
+                for (int d = 0; d < DB; ++d) o[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+                for (int u = 0; u < 4; ++u)
+#pragma unroll
+                    for (int rb = 0; rb < 4; ++rb)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            const int t = 16 * u + 4 * rb + r;
+                            const float p = __shfl(s[rb][r], 16 * u + i, kWave);
+                            if (!key_visible(pos, t0 + t, window, sinks)) continue;
+#pragma unroll
+                            for (int d = 0; d < DB; ++d)
+#pragma unroll
+                                for (int c = 0; c < 4; ++c) o[d][c] = fmaf(p, vp[page_value_offset(t, 16 * d + 4 * g + c)], o[d][c]);
+                        }
+            }
+        }
+#pragma unroll
+        for (int d = 0; d < DB; ++d) sums[wave][d][lane] = o[d];
+        if (g == 0) { tops[wave][i] = m; dens[wave][i] = l; }
+        __syncthreads();
+        const int here = min(WAVES, pages - p0);
+        for (int j = 0; j < here; ++j) {
+            const float mj = tops[j][i];
+            const float high = fmaxf(top, mj);
+            const float keep = top == -INFINITY ? 0.f : expf(top - high), add = mj == -INFINITY ? 0.f : expf(mj - high);
+#pragma unroll
+            for (int w = 0; w < OWN; ++w) {
+                const int d = wave + w * WAVES;
+                if (d < DB) {
+                    const f32x4 v = sums[j][d][lane];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) acc[w][r] = fmaf(v[r], add, acc[w][r] * keep);
+                }
+            }
+            den = fmaf(dens[j][i], add, den * keep);
+            top = high;
+        }
+        __syncthreads();
+    }
+    const float inv = den > 0.f ? 1.0f / den : 0.f;
+    if (!real) return;
+#pragma unroll
+    for (int w = 0; w < OWN; ++w) {
+        const int d = wave + w * WAVES;
+        if (d < DB) {
+            f32x4 v = acc[w];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] *= inv;
+            *reinterpret_cast<f32x4*>(out + ((size_t)tok * n_heads + head) * HD + 16 * d + 4 * g) = v;
+        }
+    }
+}
+
+// n_tiles: tiles of 16 (token, head of the group) rows over all sequences; cu null: every sequence brings one token
+LLOGOS_EXPORT int llogos_attention_f32(float* out, const float* q, int q_stride, const float* k_pool, const float* v_pool,
+                                       const int* table, int table_stride, const int* cu, const int* tok_pos, int batch, int n_tiles,
+                                       int n_heads, int n_kv_heads, int head_dim, float scale, int window, int sinks, hipStream_t stream) {
+    if (batch <= 0 || n_tiles <= 0 || n_kv_heads <= 0 || n_heads <= 0 || n_heads % n_kv_heads != 0 || window < 0 || sinks < 0) return LLOGOS_BAD_ARGUMENT;
+    if ((head_dim != 64 && head_dim != 128) || (q_stride & 3) || (((uintptr_t)q | (uintptr_t)out) & 15)) return LLOGOS_UNSUPPORTED;
+    const int group = n_heads / n_kv_heads;
+    PagedKV cache{table, table_stride, n_kv_heads, head_dim};
+    const dim3 grid(n_tiles, n_kv_heads);
+    // Waves that share a tile's pages: many where there are few tiles (a single-token step: as many as LDS holds results of), few where
+    // the tiles alone fill the GPU.
+    const bool few = (long long)n_tiles * n_kv_heads < 1024;
+#define ATTN(HD, W) attn_f32_kernel<HD, W><<<grid, W * 64, 0, stream>>>(out, q, q_stride, k_pool, v_pool, cache, cu, batch, tok_pos, \
+                                                                        n_heads, group, scale, window, sinks)
+    if (head_dim == 64) { if (few) ATTN(64, 16); else ATTN(64, 4); }
+    else { if (few) ATTN(128, 8); else ATTN(128, 4); }
+#undef ATTN
+    return LLOGOS_LAUNCH_CHECK();
+}

@@ -2248,6 +2248,34 @@ def attention_decode_fused(ctx, qkv: torch.Tensor, bias: Optional[torch.Tensor],
     return out
 
 
+def attention_f32(ctx, q: torch.Tensor, q_stride: int, k_pool: torch.Tensor, v_pool: torch.Tensor, table: torch.Tensor,
+                  n_heads: int, n_kv_heads: int, head_dim: int, scale: float, window: int = 0, sinks: int = 0) -> Optional[torch.Tensor]:
+    """float32 attention on the matrix cores' 32-bit instruction, the same bits for a token whether it comes alone or in a
+    prompt; None for head sizes other than 64 and 128 (and for rows that are not aligned), which the kernel for any shape serves."""
+    if q.dtype != torch.float32 or head_dim not in (64, 128) or q_stride % 4 or q.data_ptr() % 16:
+        return None
+    _dev(k_pool, v_pool, table, ctx.tok_pos)
+    _i32(table, "table"); _i32(ctx.tok_pos, "tok_pos")
+    _check_pools(k_pool, v_pool, n_kv_heads, head_dim, "attention")
+    _need(k_pool.dtype == torch.float32 and v_pool.dtype == torch.float32, "attention: q and cache types differ")
+    _need(n_heads % n_kv_heads == 0, "attention: heads must be a multiple of kv heads")
+    T, group = ctx.n_tokens, n_heads // n_kv_heads
+    _need(q.numel() >= (T - 1) * q_stride + n_heads * head_dim and q_stride >= n_heads * head_dim, "attention: q too small")
+    _need(table.dim() == 2 and table.shape[0] == ctx.batch and ctx.tok_pos.numel() == T, "attention: one table row a sequence, one position a token")
+    if ctx.is_decode:
+        _need(T == ctx.batch, "attention: one token a sequence")
+        cu, tiles = None, T * -(-group // 16)
+    else:
+        cu = ctx.cu_dev
+        _need(cu is not None and cu.numel() == ctx.batch + 1, "attention: the step's token offsets are missing")
+        tiles = sum(-(-(b - a) * group // 16) for a, b in zip(ctx.cu_seqlens, ctx.cu_seqlens[1:]))
+    out = torch.empty((T, n_heads * head_dim), dtype=torch.float32, device=q.device)
+    _check(_lib().llogos_attention_f32(_p(out), _p(q), q_stride, _p(k_pool), _p(v_pool), _p(table), table.stride(0), _p(cu), _p(ctx.tok_pos),
+                                       ctx.batch, tiles, n_heads, n_kv_heads, head_dim, ctypes.c_float(scale), window, sinks, _stream()),
+           "attention_f32")
+    return out
+
+
 def attention(ctx, q: torch.Tensor, q_stride: int, k_pool: torch.Tensor, v_pool: torch.Tensor,
               table: torch.Tensor, n_heads: int, n_kv_heads: int, head_dim: int, scale: float,
               window: int = 0, sinks: int = 0) -> torch.Tensor:
@@ -2255,8 +2283,10 @@ def attention(ctx, q: torch.Tensor, q_stride: int, k_pool: torch.Tensor, v_pool:
     if q.dtype == torch.bfloat16:
         out = attention_mfma_bf16(ctx, q, q_stride, k_pool, v_pool, table, n_heads, n_kv_heads, head_dim, scale,
                                   window, sinks)
-        if out is not None:
-            return out
+    else:
+        out = attention_f32(ctx, q, q_stride, k_pool, v_pool, table, n_heads, n_kv_heads, head_dim, scale, window, sinks)
+    if out is not None:
+        return out
     return attention_generic(q, q_stride, k_pool, v_pool, table, ctx.tok_seq, ctx.tok_pos,
                              n_heads, n_kv_heads, head_dim, scale, window, sinks)
 

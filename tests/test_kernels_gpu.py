@@ -429,6 +429,40 @@ def test_attention_whole_prompts_and_single_tokens(dtype, nh, nkv, hd):
         _close(out, _plain_attention(c, nh, nkv, hd), dtype)
 
 
+@pytest.mark.parametrize("window,sinks", [(0, 0), (100, 70)])
+@pytest.mark.parametrize("nh,nkv,hd", [(6, 2, 64), (20, 1, 64), (3, 3, 128), (10, 2, 128)])
+def test_float32_attention_of_a_token_alone_and_in_a_prompt(nh, nkv, hd, window, sinks):
+    """On the matrix cores' 32-bit instruction: a token's result is the same bits alone and in a prompt (groups that fill
+    no tile of 16 rows and more than one), what lies behind a sequence's end and in pages given back is never read, and a
+    value that is no number reaches only the tokens that see it."""
+    lens, new = [300, 65, 5], [300, 30, 1]
+    c = _attention_case("float32", nh, nkv, hd, lens, new)
+    table = c["table"].clone()
+    for b, n in enumerate(lens):                                        # NaN behind the end of a sequence's last page
+        page = int(table[b, (n - 1) // 64])
+        c["kp"][page][:, c["ki"][n - 64 * ((n - 1) // 64):]] = float("nan")
+        c["vp"][page][:, c["vi"][n - 64 * ((n - 1) // 64):]] = float("nan")
+        table[b, (n - 1) // 64 + 1:] = 10 ** 6                           # a page of no pool
+    cu = np.concatenate([[0], np.cumsum(new)])
+    pos = _t(c["tok_pos"], torch.int32)
+    ctx = type("Ctx", (), dict(tok_pos=pos, is_decode=False, batch=3, n_tokens=sum(new), cu_seqlens=cu.tolist(), cu_dev=_t(cu, torch.int32)))()
+    call = lambda x, q, t: K.attention_f32(x, q, c["stride"], c["kp"], c["vp"], t, nh, nkv, hd, 1 / math.sqrt(hd), window, sinks)
+    out = call(ctx, c["q"], table)
+    _close(out, _plain_attention(c, nh, nkv, hd, window, sinks), "float32")
+    for t in (0, 15, 63, 64, 170, 299, 300, 329, 330):
+        one = type("Ctx", (), dict(tok_pos=pos[t:t + 1], is_decode=True, batch=1, n_tokens=1))()
+        row = table[int(c["tok_seq"][t])][None].clone()
+        if window:
+            row[:, max(0, -(-sinks // 64)):max(0, (int(pos[t]) - window + 1) // 64)] = 10 ** 6
+        assert torch.equal(call(one, c["q"][t:t + 1], row)[0], out[t]), t
+    c["vp"][int(table[0, 2])][:, c["vi"][150 - 128]] = float("inf")     # token 150 of the first sequence
+    after = call(ctx, c["q"], table)
+    sees = np.array([s == 0 and p >= 150 and (not window or p - 150 < window) for s, p in zip(c["tok_seq"], c["tok_pos"])])
+    clean = torch.isfinite(after).all(1).cpu().numpy()
+    assert np.array_equal(clean, ~sees)
+    _close(after[_t(~sees, torch.bool)], _np(out)[~sees], "float32")
+
+
 @pytest.mark.parametrize("window,sinks", [(0, 0), (200, 70)])
 @pytest.mark.parametrize("nh,nkv,hd,batch,longest", [(8, 4, 128, 64, 700),      # one block a sequence, three pages a wave
                                                      (8, 4, 64, 70, 1500),       # batches beyond the captured sizes
