@@ -459,11 +459,18 @@ LLOGOS_EXPORT int llogos_moe_combine_weighted(float* out, const float* y, const 
 // second 16 sorted rows of activations, so that a lane ends with four neighbouring outputs of one row:
 // D[n = 4 g + r][m = c] for lane (c = lane & 15, g = lane >> 4).  A lane's share of an operand is 8 values of k,
 // 16 bytes.  Two forms:
-//   few rows  tiles of 16 sorted rows; a block of four waves owns 16 rows of the matrix, its waves take the
-//             steps of 32 k in turn (together whole cache lines), straight from memory into operands, and LDS
-//             adds the four waves' sums in order;
-//   tiles     64 or 128 sorted rows x 128 rows of the matrix with v_mfma_f32_32x32x16_bf16, stages of 64 k
-//             through LDS (swizzled rows of 128 bytes), the next stage's loads in registers meanwhile.
+//   few rows  tiles of 16 sorted rows; a block of four waves owns 16 rows of the matrix, its waves take 64 k
+//             (a cache line of every row) in turn, straight from memory into operands, and LDS adds the four waves'
+//             sums in order.  Bound by reading the matrices of the chosen experts: 16 experts of [7168, 4096] and
+//             [4096, 7168], two a token: 4 tokens (6 and 4 experts) 88 -> 64 us (5.5 TB/s) and 48 -> 43, 64 tokens
+//             (all) 220 -> 178 (5.3 TB/s), against a block that found its tile one segment after the other and
+//             whose loads stood in branches, two in flight a wave;
+//   tiles     64 or 256 sorted rows x 128 rows of the matrix with v_mfma_f32_32x32x16_bf16, stages of 64 k
+//             through LDS (swizzled rows of 128 bytes), the next stage's loads in registers meanwhile.  Bound by
+//             how much of the matrix is in flight and by what the caches give (10 TB/s, matrices and rows
+//             together).  The tall form is taken where experts have 64 rows or more on average: it reads an expert's
+//             matrix once, and waves whose 64 rows a segment does not reach only copy: 1,127 tokens 319 -> 271 us
+//             and 340 -> 246 against tiles of 128 rows, whose second tile a segment of 141 rows barely fills.
 // Sums depend on k's order alone, as above.  K must be a multiple of 8 and N of 4.
 typedef __bf16 moe_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float moe_f32x4 __attribute__((ext_vector_type(4)));
@@ -488,14 +495,27 @@ __device__ __forceinline__ void moe_store2(bf16_t* p, float a, float b) {
     *reinterpret_cast<uint32_t*>(p) = (uint32_t)f32_to_bf16(a) | ((uint32_t)f32_to_bf16(b) << 16);
 }
 
-// which tile of `rows` sorted rows is this block's: expert, first row, end of the expert's segment (expert -1: none)
+// which tile of `rows` sorted rows is this block's: expert, first row, end of the expert's segment (expert -1: none).
+// For one whole wave, whose lanes take the segments side by side: a thread that walks them waits for the cache once
+// a segment, several microseconds before a block asks for its first weights.
 __device__ __forceinline__ void moe_find_tile(const int* __restrict__ seg, int E, int rows, int tile, int& expert, int& first, int& end) {
+    const int lane = threadIdx.x & (kWave - 1);
     expert = -1; first = 0; end = 0;
-    for (int e = 0; e < E; ++e) {
-        const int lo = seg[e], hi = seg[e + 1];
+    for (int e0 = 0; e0 < E; e0 += kWave) {
+        const int e = e0 + lane, lo = seg[min(e, E)], hi = seg[min(e + 1, E)];
         const int tiles = (hi - lo + rows - 1) / rows;
-        if (tile < tiles) { expert = e; first = lo + tile * rows; end = hi; return; }
-        tile -= tiles;
+        int before = tiles;                                  // tiles of this segment and the ones in front of it
+#pragma unroll
+        for (int o = 1; o < kWave; o <<= 1) { const int v = __shfl_up(before, o, kWave); if (lane >= o) before += v; }
+        const unsigned long long mine = __ballot(tile < before);
+        if (mine) {
+            const int at = __ffsll(mine) - 1;
+            expert = e0 + at;
+            end = __shfl(hi, at, kWave);
+            first = __shfl(lo + (tile - (before - tiles)) * rows, at, kWave);
+            return;
+        }
+        tile -= __shfl(before, kWave - 1, kWave);
     }
 }
 
@@ -506,26 +526,46 @@ __global__ __launch_bounds__(256) void moe_few_kernel(TO* __restrict__ out, cons
                                                       const float* __restrict__ row_weight, float limit) {
     __shared__ float red[3][kWave][4];
     __shared__ int s_tile[3];
-    if (threadIdx.x == 0) moe_find_tile(seg, E, 16, blockIdx.y, s_tile[0], s_tile[1], s_tile[2]);
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    if (wave == 0) {
+        int e, first, end;
+        moe_find_tile(seg, E, 16, blockIdx.y, e, first, end);
+        if (lane == 0) { s_tile[0] = e; s_tile[1] = first; s_tile[2] = end; }
+    }
     __syncthreads();
     const int e = s_tile[0], m0 = s_tile[1], m_end = s_tile[2];
     if (e < 0) return;
-    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const int c = lane & 15, g = lane >> 4;
     const int n0 = blockIdx.x * 16;
     const int m = m0 + c;
-    const bf16_t* arow = m < m_end ? a + (size_t)(gather ? order[m] / top : m) * lda + 8 * g : nullptr;
-    const bf16_t* wrow = n0 + c < N ? w + ((size_t)e * N + n0 + c) * K + 8 * g : nullptr;
+    // (rows past the segment's end and past the matrix are read as its last ones: their sums go nowhere)
+    const int src = min(m, m_end - 1);
+    const bf16_t* arow = a + (size_t)(gather ? order[src] / top : src) * lda + 8 * g;
+    const bf16_t* wrow = w + ((size_t)e * N + min(n0 + c, N - 1)) * K + 8 * g;
     moe_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    const int steps = (K + 31) / 32;
-#pragma unroll 4
-    for (int s = wave; s < steps; s += 4) {
-        const int k = 32 * s;
-        const bool in = k + 8 * g < K;
-        const moe_bf16x8 wf = (wrow && in) ? moe_frag(wrow + k) : moe_zero();
-        const moe_bf16x8 af = (arow && in) ? moe_frag(arow + k) : moe_zero();
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, af, acc, 0, 0, 0);
+    // A wave takes 64 k at a time, the two halves of a cache line one behind the other, and asks for 256 k before it
+    // multiplies the first: what bounds the kernel is how much of w is in flight (8 KB a wave).
+    constexpr int AHEAD = 8;
+    const int whole = K / 32;
+    int s = 2 * wave;
+    auto step = [&](int i) { return s + 8 * (i >> 1) + (i & 1); };          // the wave's i-th step of 32 k from here
+    for (; step(AHEAD - 1) < whole; s += 4 * AHEAD) {
+        moe_bf16x8 wf[AHEAD], af[AHEAD];
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) wf[i] = moe_frag(wrow + 32 * step(i));
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) af[i] = moe_frag(arow + 32 * step(i));
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[i], af[i], acc, 0, 0, 0);
     }
+    for (; s * 32 < K; s += 8)
+        for (int half = 0; half < 2; ++half) {
+            const int k = 32 * (s + half);
+            const bool in = k + 8 * g < K;
+            const moe_bf16x8 wf = in ? moe_frag(wrow + k) : moe_zero();
+            const moe_bf16x8 af = in ? moe_frag(arow + k) : moe_zero();
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, af, acc, 0, 0, 0);
+        }
     if (wave > 0) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) red[wave - 1][lane][r] = acc[r];
@@ -559,18 +599,23 @@ __device__ __forceinline__ int moe_lds_at(int row, int oct) { return row * kMoeB
 // rows of the expert's matrix are the first operand and the sorted rows the second, so a lane ends with the sums
 // of one sorted row (l & 31) for 4 x 4 neighbouring columns: entry 4 q + e is column 8 q + 4 (l >> 5) + e.
 template <int BM, int BN, typename TO>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void moe_tiles_kernel(
+__global__ __launch_bounds__(BM == 64 ? 256 : 512) __attribute__((amdgpu_waves_per_eu(BM == 64 ? 3 : 4, BM == 64 ? 3 : 4))) void moe_tiles_kernel(
         TO* __restrict__ out, const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, const int* __restrict__ order,
         const int* __restrict__ seg, int E, int top, int gather, int N, int K, int lda, int act, float scale,
                                                           const float* __restrict__ row_weight, float limit) {
-    constexpr int CA = BM * 8 / 256, CW = BN * 8 / 256;           // 16-byte pieces a thread copies a stage
-    constexpr int WN = BM == 128 ? BN / 2 : BN / 4, NT = WN / 32, MT = 2;     // a wave's part: 64 rows x WN columns of the tile
+    constexpr int THREADS = BM == 64 ? 256 : 512;
+    constexpr int CA = BM * 8 / THREADS, CW = BN * 8 / THREADS;   // 16-byte pieces a thread copies a stage
+    constexpr int WN = BM == 64 ? BN / 4 : BN / 2, NT = WN / 32, MT = 2;      // a wave's part: 64 rows x WN columns of the tile
     __shared__ __attribute__((aligned(16))) bf16_t As[BM * kMoeBK];
     __shared__ __attribute__((aligned(16))) bf16_t Ws[BN * kMoeBK];
     __shared__ int src_row[BM];
     __shared__ int s_tile[3];
     const int tid = threadIdx.x;
-    if (tid == 0) moe_find_tile(seg, E, BM, blockIdx.y, s_tile[0], s_tile[1], s_tile[2]);
+    if (tid < kWave) {
+        int e, first, end;
+        moe_find_tile(seg, E, BM, blockIdx.y, e, first, end);
+        if (tid == 0) { s_tile[0] = e; s_tile[1] = first; s_tile[2] = end; }
+    }
     __syncthreads();
     const int e = s_tile[0], m0 = s_tile[1], m_end = s_tile[2];
     if (e < 0) return;
@@ -581,7 +626,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     __syncthreads();
     const int lane = tid & (kWave - 1), wave = tid / kWave;
     const int r32 = lane & 31, h = lane >> 5;
-    const int wm = BM == 128 ? wave >> 1 : 0, wn = BM == 128 ? wave & 1 : wave;
+    const int wm = BM == 64 ? 0 : wave >> 1, wn = BM == 64 ? wave : wave & 1;
+    const bool busy = m0 + 64 * wm < m_end;                       // (a segment rarely fills all of a tile's rows)
     const int n0 = blockIdx.x * BN;
     const bf16_t* we = w + (size_t)e * N * K;
 
@@ -590,14 +636,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     int ka[CA], kw[CW], la[CA], lw[CW];
 #pragma unroll
     for (int j = 0; j < CA; ++j) {
-        const int q = tid + 256 * j, row = q >> 3;
+        const int q = tid + THREADS * j, row = q >> 3;
         ka[j] = (q & 7) * 8;
         la[j] = moe_lds_at(row, q & 7);
         pa[j] = src_row[row] >= 0 ? a + (size_t)src_row[row] * lda + ka[j] : nullptr;
     }
 #pragma unroll
     for (int j = 0; j < CW; ++j) {
-        const int q = tid + 256 * j, row = q >> 3;
+        const int q = tid + THREADS * j, row = q >> 3;
         kw[j] = (q & 7) * 8;
         lw[j] = moe_lds_at(row, q & 7);
         pw[j] = n0 + row < N ? we + (size_t)(n0 + row) * K + kw[j] : nullptr;
@@ -627,6 +673,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
         for (int j = 0; j < CW; ++j) *reinterpret_cast<uint4*>(Ws + lw[j]) = rw[j];
         __syncthreads();
         if (k0 + kMoeBK < K) fetch(k0 + kMoeBK);
+        if (busy)
 #pragma unroll
         for (int ks = 0; ks < kMoeBK / 16; ++ks) {
             moe_bf16x8 af[MT], wf[NT];
@@ -666,20 +713,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     }
 }
 
-// form 0: few rows (tiles of 16); 1: tiles of 64 rows; 2: tiles of 128 rows.  -2 for shapes these do not take.
+// form 0: few rows (tiles of 16); 1: tiles of 64 rows; 2: tiles of 256 rows.  -2 for shapes these do not take.
 LLOGOS_EXPORT int llogos_moe_product_bf16(void* out, int out_dtype, const void* a, const void* w, const int* order, const int* seg,
                                           int E, int top, int gather, int P, int N, int K, int lda, int act, float scale,
                                           const float* row_weight, float limit, int form, hipStream_t stream) {
     if (P <= 0 || N <= 0 || K <= 0 || E <= 0 || top <= 0 || lda < K || act < 0 || act > 3 || form < 0 || form > 2 || (row_weight && act < 2) || (act == 3 && !(limit >= 0.f))) return LLOGOS_BAD_ARGUMENT;
     if ((K % 8) || (N % 4) || (lda % 8) || ((uintptr_t)a % 16) || ((uintptr_t)w % 16) || ((uintptr_t)out % 16)) return LLOGOS_UNSUPPORTED;
     if (out_dtype != DT_F32 && out_dtype != DT_BF16) return LLOGOS_BAD_ARGUMENT;
-    const int rows = form == 0 ? 16 : (form == 1 ? 64 : 128);
+    const int rows = form == 0 ? 16 : (form == 1 ? 64 : 256);
     const int row_tiles = (P + rows - 1) / rows + E;
-#define MOE_GO(KERNEL, NB, TO) KERNEL<<<dim3((N + NB - 1) / NB, row_tiles), 256, 0, stream>>>((TO*)out, (const bf16_t*)a, (const bf16_t*)w, \
+#define MOE_GO(KERNEL, NB, TO) KERNEL<<<dim3((N + NB - 1) / NB, row_tiles), form == 2 ? 512 : 256, 0, stream>>>((TO*)out, (const bf16_t*)a, (const bf16_t*)w, \
         order, seg, E, top, gather, N, K, lda, act, scale, row_weight, limit)
     if (form == 0) { if (out_dtype == DT_F32) MOE_GO(moe_few_kernel<float>, 16, float); else MOE_GO(moe_few_kernel<bf16_t>, 16, bf16_t); }
     else if (form == 1) { if (out_dtype == DT_F32) MOE_GO((moe_tiles_kernel<64, 128, float>), 128, float); else MOE_GO((moe_tiles_kernel<64, 128, bf16_t>), 128, bf16_t); }
-    else { if (out_dtype == DT_F32) MOE_GO((moe_tiles_kernel<128, 128, float>), 128, float); else MOE_GO((moe_tiles_kernel<128, 128, bf16_t>), 128, bf16_t); }
+    else { if (out_dtype == DT_F32) MOE_GO((moe_tiles_kernel<256, 128, float>), 128, float); else MOE_GO((moe_tiles_kernel<256, 128, bf16_t>), 128, bf16_t); }
 #undef MOE_GO
     return LLOGOS_LAUNCH_CHECK();
 }

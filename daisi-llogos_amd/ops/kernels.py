@@ -621,7 +621,7 @@ def activation(x: torch.Tensor, kind: str, out_dtype: torch.dtype, a: float = 0.
 # ----------------------------------------------------------------------------
 MOE_MAX_EXPERTS = 1024
 MOE_FEW_PAIRS = 256          # up to so many (token, choice) pairs a step the experts' product streams the matrices in tiles of 16 rows
-MOE_PRODUCT = "auto"         # "auto": chosen by the step; "plain", "few", "tiles64", "tiles128" force a form (tests)
+MOE_PRODUCT = "auto"         # "auto": chosen by the step; "plain", "few", "tiles64" (low tiles), "tiles128" (tall ones) force a form (tests)
 
 
 def moe_route(ids: Optional[torch.Tensor], table: torch.Tensor, n_experts: int):
@@ -732,8 +732,13 @@ def moe_product(a: torch.Tensor, w: torch.Tensor, order: torch.Tensor, seg: torc
     out = torch.empty((P, N // 2 if gated else N), dtype=out_dtype, device=a.device)
     if a.dtype == torch.bfloat16 and MOE_PRODUCT != "plain" and a.stride(1) == 1:
         # on the matrix cores: tiles of 16 sorted rows straight from memory for steps of few rows, tiles of 64 or
-        # 128 rows through LDS where an expert's segment is long enough on average to fill them
-        form = 0 if P <= MOE_FEW_PAIRS else (2 if P >= 96 * E else 1)
+        # 256 rows through LDS for more: the tall ones (an expert's matrix is read once) from 64 rows an expert on
+        # average (16 experts of 7168 x 4096: 50 rows 230 us in the low form and 246 in the tall one, 75 rows 260 and 246,
+        # 141 rows 327 and 271)
+        # (and the few-row form ends at 8 rows an expert where tiles give every compute unit two blocks: 16 rows an expert
+        # 275 us against 232, and 276 against 160 for the way down)
+        few = P <= 8 * E or E * -(-N // 128) < 512
+        form = 0 if few and P <= MOE_FEW_PAIRS else (2 if P >= 64 * E else 1)
         if MOE_PRODUCT in ("few", "tiles64", "tiles128"):
             form = ("few", "tiles64", "tiles128").index(MOE_PRODUCT)
         code = _lib().llogos_moe_product_bf16(_p(out), _DT[out_dtype], _p(a), _p(w), _p(order), _p(seg), E, top, 1 if gather else 0,

@@ -949,3 +949,26 @@ def test_long_prompts_take_the_tiled_gate_up_product_by_default():
     assert calls == [(len(toks), True)] * 2                                # the gate/up product of both layers
     want = H.plain_logits(name, toks)[[0, 100, len(toks) - 1]]
     H.close(got, want, "bfloat16", "long prompt, tiled gate/up product", config=name)
+
+
+@pytest.mark.parametrize("form", ["few", "tiles64", "tiles128"])
+@pytest.mark.parametrize("N,K_", [(20, 8), (132, 72), (260, 264), (64, 1320)])
+def test_expert_product_at_the_edges_of_its_tiles(form, N, K_, monkeypatch):
+    """Segments of no row, one, and around 16, 64 and 256 rows (in the order of many experts, more than a wave has lanes),
+    matrices that fill no tile, k of no whole stage, and more of k than the few-row form asks for at once."""
+    monkeypatch.setattr(K, "MOE_PRODUCT", form)
+    rng = np.random.default_rng(N)
+    sizes = [0, 1, 15, 16, 17, 0, 63, 64, 65, 255, 256, 257, 300] + [0, 1] * 40
+    seg = _t(np.concatenate([[0], np.cumsum(sizes)]), torch.int32)
+    P, E = sum(sizes), len(sizes)
+    order = _t(rng.permutation(P), torch.int32)
+    a = _t(rng.standard_normal((P, K_)), torch.bfloat16)
+    w = _t(rng.standard_normal((E, N, K_)) * 0.1, torch.bfloat16)
+    for gather in (True, False):
+        rows = a[order.long()] if gather else a
+        want = torch.cat([rows[int(seg[e]):int(seg[e + 1])].double() @ w[e].double().t() for e in range(E)])
+        got = K.moe_product(a, w, order, seg, 1, gather, torch.float32)
+        # (products of bfloat16 are exact in 32 bits; a sum in any order is off by a few roundings of its partial sums)
+        assert (got.double() - want).abs().max() <= 2.0 ** -23 * K_ ** 0.5 * 4 * max(1.0, want.abs().max().item())
+        half = K.moe_product(a, w, order, seg, 1, gather, torch.bfloat16, relu2=True)
+        _close(half, _np(want.clamp(min=0) ** 2), "bfloat16")
