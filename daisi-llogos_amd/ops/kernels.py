@@ -518,12 +518,23 @@ def wkv_scan(ctx, r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, d: torch.Te
     _need(ctx.cu_dev is not None or ctx.n_tokens == ctx.batch, "wkv_scan: a step of several tokens a sequence needs the token offsets")
     _need(6 * dim * 4 <= 65536, f"wkv_scan: head size {dim} is too large")
     y = torch.empty((ctx.n_tokens, HD), dtype=out_dtype, device=r.device)
-    rows, col_blocks, n_seg = scan_plan(ctx.batch, n_heads, dim, None if ctx.is_decode else
-                                        max(ctx.cu_seqlens[i + 1] - ctx.cu_seqlens[i] for i in range(ctx.batch)))
+    longest = None if ctx.is_decode else max(ctx.cu_seqlens[i + 1] - ctx.cu_seqlens[i] for i in range(ctx.batch))
+    if dim == 64 and state.stride(0) % 4 == 0 and state.data_ptr() % 16 == 0 and not (SCAN_ROWS or SCAN_COLUMN_BLOCKS):
+        n_seg = wave_scan_segments(ctx.batch, n_heads, longest)
+        seg_len, seg_state, seg_decay = 0, None, None
+        if n_seg > 1:
+            seg_len = -(-(-(-longest // n_seg)) // 8) * 8                # whole chunks of the kernel
+            seg_state = torch.empty((ctx.batch, n_seg, n_heads, dim, dim), dtype=torch.float32, device=r.device)
+            seg_decay = torch.empty((ctx.batch, n_seg, n_heads, dim), dtype=torch.float32, device=r.device)
+        _check(_lib().llogos_wkv64(_p(y), _DT[out_dtype], _p(r), _p(k), _p(v), _p(d), _p(gate), HD, parts, ctypes.c_longlong(part_stride),
+                                   d_parts, ctypes.c_longlong(d_part_stride), _p(w0), _p(u), _p(g), ctypes.c_float(eps), _p(state),
+                                   ctypes.c_longlong(state.stride(0)), ctypes.c_longlong(HD * dim), _p(h_in), W, _p(ctx.slots),
+                                   _p(ctx.cu_dev), ctx.batch, n_heads, n_seg, seg_len, _p(seg_state), _p(seg_decay), _stream()), "wkv64")
+        return y
+    rows, col_blocks, n_seg = scan_plan(ctx.batch, n_heads, dim, longest)
     o_raw = torch.empty((ctx.n_tokens, HD), dtype=torch.float32, device=r.device) if col_blocks > 1 else None
     seg_len, seg_state, seg_decay = 0, None, None
     if n_seg > 1:
-        longest = max(ctx.cu_seqlens[i + 1] - ctx.cu_seqlens[i] for i in range(ctx.batch))
         seg_len = -(-(-(-longest // n_seg)) // 16) * 16                  # whole chunks of the kernel
         seg_state = torch.empty((ctx.batch, n_seg, n_heads, dim, dim), dtype=torch.float32, device=r.device)
         seg_decay = torch.empty((ctx.batch, n_seg, n_heads, dim), dtype=torch.float32, device=r.device)
@@ -538,6 +549,18 @@ def wkv_scan(ctx, r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, d: torch.Te
 SCAN_COLUMN_BLOCKS = 0       # 0: chosen by the step; 1, 2, 4, ... force the number of blocks a head (tests)
 SCAN_SEGMENTS = 0            # 0: chosen by the step; 1, 2, 3, ... force the number of segments of a prompt (tests)
 SCAN_ROWS = 0                # 0: chosen by the step; 4 or 16 force the rows of the state a thread (tests)
+
+
+def wave_scan_segments(batch: int, n_heads: int, longest: Optional[int], n_cus: Optional[int] = None) -> int:
+    """Segments that the prompts of a step are cut into by the recurrence with a wave a head: as many as bring the waves
+    to two a SIMD, of at least 16 tokens.  A segment costs more than half of its tokens' time again for its end state, but a
+    wave alone on its SIMD issues at half the rate and waits for every token's chain: 64 heads, one prompt of 127 tokens
+    whole 98 us, in 8 segments 39; of 2,048 1,505 whole, 178 in 16, 158 in 32; eight of 250 to 600 470 whole, 281 in 4."""
+    if longest is None:
+        return 1
+    if SCAN_SEGMENTS:
+        return SCAN_SEGMENTS
+    return max(1, min(32, longest // 16, -(-(8 * (n_cus or compute_units())) // max(1, batch * n_heads))))
 
 
 def scan_plan(batch: int, n_heads: int, dim: int, longest: Optional[int], n_cus: Optional[int] = None) -> Tuple[int, int, int]:
