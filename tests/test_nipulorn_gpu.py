@@ -402,3 +402,98 @@ def test_the_command_line_on_a_model_of_the_design(tmp_path):
     p = run("--model", str(out), "--bench", "--batch", "2", "-n", "8", "--prompt-len", "20", "--max-context", "64")
     assert p.returncode == 0, p.stderr[-2000:]
     assert "decode" in (p.stdout + p.stderr)
+
+
+def _recurrence_case(lens, heads, seed):
+    """Inputs of the recurrence for sequences of `lens` tokens, from a state that is not zero, and what float64 makes of them."""
+    rng = np.random.default_rng(seed)
+    T, HD = sum(lens), heads * 64
+    r, k, v, gate, d = (rng.standard_normal((T, HD)) for _ in range(5))
+    w0, u, g = rng.uniform(-6, -0.5, HD), rng.standard_normal(HD), rng.uniform(0.9, 1.1, HD)
+    state = rng.standard_normal((len(lens) + 1, HD * 64 + 48))
+    t32 = lambda x: torch.tensor(x, dtype=torch.float32, device=DEV)
+    f = dict(r=t32(r), k=t32(k), v=t32(v), d=t32(d), gate=t32(gate), w0=t32(w0), u=t32(u), g=t32(g), h=t32(rng.standard_normal((T, 48))), state=t32(state))
+    x = {n: _np(f[n]) for n in f}
+    want, states, at = [], [], 0
+    for i, n in enumerate(lens):
+        rows = slice(at, at + n)
+        shape = (n, heads, 64)
+        S = x["state"][i + 1, :HD * 64].reshape(heads, 64, 64).transpose(0, 2, 1)
+        o, S = pn.wkv_recurrence(x["r"][rows].reshape(shape), x["k"][rows].reshape(shape), x["v"][rows].reshape(shape),
+                                 np.exp(-np.exp(x["d"][rows] + x["w0"])).reshape(shape), x["u"].reshape(heads, 64), S)
+        want.append(pn.root_mean_square_scale(o, 1e-5).reshape(n, HD) * x["g"] * pn.silu(x["gate"][rows]))
+        states.append(S)
+        at += n
+    return f, np.concatenate(want), states
+
+
+def _scan(f, lens, lo, hi, state, heads):
+    """Tokens lo[i] .. hi[i] of every sequence in one step."""
+    starts = np.concatenate([[0], np.cumsum(lens)])
+    rows = torch.tensor(np.concatenate([np.arange(starts[i] + a, starts[i] + b) for i, (a, b) in enumerate(zip(lo, hi))]), device=DEV)
+    counts = [b - a for a, b in zip(lo, hi)]
+    cu = np.concatenate([[0], np.cumsum(counts)]).tolist()
+    ctx = type("Ctx", (), dict(n_tokens=sum(counts), batch=len(lens), slots=torch.arange(1, len(lens) + 1, dtype=torch.int32, device=DEV), cu_seqlens=cu,
+                               cu_dev=None if max(counts) == 1 else torch.tensor(cu, dtype=torch.int32, device=DEV), is_decode=max(counts) == 1))()
+    take = lambda n: f[n][rows].contiguous()
+    return rows, K.wkv_scan(ctx, take("r"), take("k"), take("v"), take("d"), take("gate"), f["w0"], f["u"], f["g"], 1e-5, state, heads, 64, take("h"),
+                            torch.float32)
+
+
+@pytest.mark.parametrize("segments", [0, 1, 3, 16])
+@pytest.mark.parametrize("heads,lens", [(1, [9]), (3, [40, 17]), (6, [8, 1, 70])])
+def test_recurrence_of_heads_of_64_channels(heads, lens, segments, monkeypatch):
+    """A wave a head: prompts whole and cut into segments (chunks of eight that are not full, segments behind a sequence's
+    end, heads that fill no block of waves), against float64; single tokens give the bits of the whole prompt."""
+    monkeypatch.setattr(K, "SCAN_SEGMENTS", segments)
+    f, want, states = _recurrence_case(lens, heads, 5)
+    state = f["state"].clone()
+    _, y = _scan(f, lens, [0] * len(lens), lens, state, heads)
+    assert np.abs(_np(y) - want).max() <= 2e-5 * np.abs(want).max()
+    for i, S in enumerate(states):
+        kept = _np(state[i + 1][:heads * 4096]).reshape(heads, 64, 64).transpose(0, 2, 1)
+        assert np.abs(kept - S).max() <= 2e-6 * max(1.0, np.abs(S).max()) * 8
+        assert torch.equal(state[i + 1][heads * 4096:], f["h"][sum(lens[:i + 1]) - 1])
+    assert torch.equal(state[0], f["state"][0])
+    if segments == 1:
+        ones = f["state"].clone()
+        for t in range(min(lens)):
+            rows, single = _scan(f, lens, [t] * len(lens), [t + 1] * len(lens), ones, heads)
+            assert torch.equal(single, y[rows]), t
+
+
+@pytest.mark.parametrize("out", ["float32", "bfloat16"])
+@pytest.mark.parametrize("taps", [1, 2, 4, 7, 16])
+def test_long_steps_of_convolution_shift_and_activation(taps, out):
+    """The forms for steps of many tokens, four channels a thread: sequences of one token, of fewer than the taps, of a block of
+    eight and more, new ones and ones that go on from their state; widths that fill no block; an activation of a part of rows."""
+    rng = np.random.default_rng(taps)
+    counts, starts, W = [1, 3, 8, 9, 50, 2], [5, 0, 0, 30, 2, 1], 516
+    T, cu = sum(counts), np.concatenate([[0], np.cumsum(counts)])
+    whole = [rng.standard_normal((s + n, W)).astype(np.float32) for s, n in zip(starts, counts)]
+    state = torch.zeros((7, taps - 1, W), device=DEV)
+    for i, (x, s) in enumerate(zip(whole, starts)):
+        past = np.concatenate([np.zeros((taps - 1, W), np.float32), x[:s]])[s:]
+        state[i + 1] = torch.tensor(past, device=DEV)
+    h = torch.tensor(np.concatenate([x[s:] for x, s in zip(whole, starts)]), device=DEV)
+    w = torch.tensor(rng.uniform(-0.5, 0.5, (W, taps)), dtype=torch.float32, device=DEV)
+    i32 = lambda a: torch.tensor(np.asarray(a), dtype=torch.int32, device=DEV)
+    ctx = type("Ctx", (), dict(n_tokens=T, batch=6, slots=i32(np.arange(1, 7)), tok_seq=i32(np.repeat(np.arange(6), counts)), cu_seqlens=cu.tolist(),
+                               tok_pos=i32(np.concatenate([np.arange(s, s + n) for s, n in zip(starts, counts)])), cu_dev=i32(cu), is_decode=False))()
+    dtype = torch.float32 if out == "float32" else torch.bfloat16
+    tol = 2e-6 if out == "float32" else 8e-3
+    got = _np(K.causal_conv(ctx, h, w, state, dtype)) if taps > 1 else None
+    want = np.concatenate([pn.input_convolution(x, _np(w))[s:] for x, s in zip(whole, starts)])
+    if taps > 1:
+        assert np.abs(got - want).max() <= tol * taps * np.abs(want).max()
+    if taps == 4:
+        mu = torch.tensor(rng.uniform(0, 1, (3, W)), dtype=torch.float32, device=DEV)
+        prev = torch.tensor(np.stack([np.zeros(W, np.float32)] + [x[s - 1] if s else np.zeros(W, np.float32) for x, s in zip(whole, starts)]), device=DEV)
+        shifted = _np(K.token_shift(ctx, h, mu, prev, dtype))
+        for m in range(3):
+            mix = np.concatenate([pn.token_shift(x, _np(mu[m]))[s:] for x, s in zip(whole, starts)])
+            assert np.abs(shifted[m] - mix).max() <= tol * np.abs(mix).max()
+    big = torch.tensor(rng.standard_normal((2, 260, 4113)), dtype=torch.float32, device=DEV)
+    act = _np(K.activation(big, "silu", dtype, cols=4104))
+    z = _np(big.sum(0))[:, :4104]
+    assert act.shape == z.shape and np.abs(act - pn.silu(z)).max() <= tol * 4 * np.abs(pn.silu(z)).max()
