@@ -33,19 +33,20 @@
 //    two paths costs register copies and spills.
 //  * One barrier a stage, in the middle of the last sub-step: before it the stores of the next
 //    stage, after it the first reads of that stage, beside the sub-step's remaining products.
-//  * Blocks are numbered so that an XCD (blocks i, i + 8, ...) works on few row tiles at a time
-//    and walks all token tiles of a row tile before the next: its L2 then serves a row tile's
-//    weights to all the token tiles (hit rate 80 % with 8 x 4 tiles in flight on an XCD).
-//  * When the tiles of 256 tokens leave less than half of a last round of blocks, the row tiles
-//    of that round are taken in tiles of 128 tokens, which fill the round at half its length.
+//  * Blocks are numbered so that the 32 that run on an XCD are about 8 x 4 neighbouring tiles (tiles_place): its L2
+//    serves a row tile's weights to eight token tiles and their activations to four row tiles.
+//  * Tiles of 128 tokens where those of 256 leave compute units idle, for all of a product or for its last round
+//    (tiles_n_full).
 //  * Parts of k (blocks along k, float32 partial sums [parts][M][N] that the consumer adds) for
 //    matrices with few rows, whose tiles do not fill the compute units.
-//  * Epilogues: plain (+ bias) in bfloat16 or float32; SwiGLU for a matrix packed with gate_rows.
-//  * Measured, 2,048 tokens of the 8B layer sizes: gate/up with SwiGLU 395 to 412 us against the
-//    library's 392 + 31 for a SwiGLU pass; down 214 (two parts of k) against 189; qkv 100 against
-//    87; o 80 against 61.  By the counters the matrix pipe is busy 76 % of a tile's time (86 %
-//    with the copies left out, barriers 9 %); the rest of the distance to the library's kernels
-//    on the short matrices is the round of blocks that their tiles do not fill.
+//  * Epilogues: plain (+ bias) in bfloat16 or float32; added to a float32 result in place; SwiGLU for a matrix packed
+//    with gate_rows.
+//  * Measured, 2,048 tokens of the 8B layer sizes: gate/up with SwiGLU 387 us against the library's 385 with a SwiGLU
+//    pass; down 200 (two parts of k) against 212; qkv 102 against 80; o 72 against 63; 5,003 tokens of the 14B sizes:
+//    gate/up 1,414 against 1,524, down 783 against 1,037.  By the counters the matrix pipe is busy 76 % of a tile's
+//    time (86 % with the copies left out, barriers 9 %); the rest of the distance to the library's kernels on the short
+//    matrices is the round of blocks that their tiles do not fill.  (Copies straight into LDS, five stages of 32 k deep,
+//    with a barrier a stage were 8 % slower.)
 #include "common.h"
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
@@ -57,7 +58,7 @@ typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 constexpr int kWavesN = 4, kWavesM = 2, kTileWaves = 8;
 constexpr int kStageK = 64;
 constexpr int kStageW = kWavesN * 64 * kStageK * 2;   // 32 KB
-enum { EPI_PLAIN = 0, EPI_SWIGLU = 1 };
+enum { EPI_PLAIN = 0, EPI_SWIGLU = 1, EPI_ADD = 2 };
 
 __device__ __forceinline__ uint32_t tiles_pack_bf16(float lo, float hi) {
     const f32x2_t v = {lo, hi};
@@ -276,21 +277,39 @@ __device__ __forceinline__ void tile_body(
                         pk.y = tiles_pack_bf16(y[2], y[3]);
                         *reinterpret_cast<uint2*>(orow + n) = pk;
                     } else if (sizeof(TO) == 4 && n + 3 < N && ((ldo & 3) == 0) && ((reinterpret_cast<uintptr_t>(out) & 15) == 0)) {
-                        *reinterpret_cast<float4*>(orow + n) = make_float4(y[0], y[1], y[2], y[3]);
+                        float4 v = make_float4(y[0], y[1], y[2], y[3]);
+                        if (EPI == EPI_ADD) {
+                            const float4 x = *reinterpret_cast<const float4*>(orow + n);
+                            v.x += x.x; v.y += x.y; v.z += x.z; v.w += x.w;
+                        }
+                        *reinterpret_cast<float4*>(orow + n) = v;
                     } else {
 #pragma unroll
                         for (int e = 0; e < 4; ++e)
-                            if (n + e < N) store_f32(orow + n + e, y[e]);
+                            if (n + e < N) store_f32(orow + n + e, EPI == EPI_ADD ? y[e] + load_f32(orow + n + e) : y[e]);
                     }
                 }
         }
     }
 }
 
+// Which tile block j of XCD x takes, of `rows` token tiles x `cols` columns (a part of k and a row tile; the parts outermost):
+// tiles are counted in bands of eight token tiles, a column of the band before the next, and every XCD takes a run of them, as
+// long as the others' to one tile.  The 32 blocks that run on an XCD so are about 8 x 4 tiles of one part of k: they share
+// their weights and their activations in its L2, and no XCD is left with a round of blocks more than the others.  (With
+// whole columns dealt to the XCDs in turn 11 x 20 tiles took two rounds on four of them: 715 us for 2,600 x 5,120 x 17,408,
+// 404 now; 5,003 x 5,120 x 17,408 889 -> 783, 5,003 x 34,816 x 5,120 with SwiGLU 1,485 -> 1,414, 2,048 x 28,672 x 4,096 402 -> 387.)
+__device__ __forceinline__ bool tiles_place(int tiles, int rows, int cols, int xcd, int j, int& row, int& col) {
+    const int per = tiles >> 3, more = tiles & 7;
+    if (j >= per + (xcd < more)) return false;
+    const int id = xcd * per + min(xcd, more) + j, band = id / (8 * cols), at = id - band * 8 * cols, high = min(8, rows - 8 * band);
+    col = at / high;
+    row = 8 * band + at % high;
+    return true;
+}
+
 // Blocks 0 .. blocks4 - 1 take tiles of 256 tokens over the first n_full row tiles, the blocks after them tiles of
-// 128 tokens over the remaining row tiles.  A row tile and a part of k together are one index u = row tile *
-// parts + part, and XCD x takes the u that are x modulo 8, walking all token tiles of one before the next: blocks
-// that run together on an XCD then share their weights (same u) and their activations (same part of k).
+// 128 tokens over the remaining row tiles.
 template <typename TO, int EPI>
 __global__ __launch_bounds__(kTileWaves * kWave) void gemm_tiles_kernel(
         TO* __restrict__ out, const bf16_t* __restrict__ a, int lda, const unsigned char* __restrict__ wp,
@@ -299,12 +318,11 @@ __global__ __launch_bounds__(kTileWaves * kWave) void gemm_tiles_kernel(
     extern __shared__ __attribute__((aligned(1024))) unsigned char tiles_lds[];
     const int stages = K / kStageK;
     const bool big = (int)blockIdx.x < blocks4;
-    const int b = big ? blockIdx.x : blockIdx.x - blocks4;
-    const int m_tiles = big ? m_tiles4 : m_tiles2;
-    const int xcd = b & 7, jb = b >> 3;
-    const int m_tile = jb % m_tiles, u = xcd + 8 * (jb / m_tiles);
-    const int part = u % parts, n_tile = (big ? 0 : n_full) + u / parts;
-    if (n_tile >= (big ? n_full : n_tiles)) return;
+    const int b = big ? blockIdx.x : blockIdx.x - blocks4;                   // (blocks4 is a multiple of 8)
+    const int m_tiles = big ? m_tiles4 : m_tiles2, across = big ? n_full : n_tiles - n_full;
+    int m_tile, u;
+    if (!tiles_place(m_tiles * across * parts, m_tiles, across * parts, b & 7, b >> 3, m_tile, u)) return;
+    const int part = u / across, n_tile = (big ? 0 : n_full) + u % across;
     // the parts divide the stages evenly: part p takes [stages p / parts, stages (p + 1) / parts), none is empty
     // when there are at least as many stages as parts
     const int s0 = (int)((long long)stages * part / parts), s1 = (int)((long long)stages * (part + 1) / parts);
@@ -313,16 +331,32 @@ __global__ __launch_bounds__(kTileWaves * kWave) void gemm_tiles_kernel(
     else tile_body<2, TO, EPI>(tiles_lds, dst, a, lda, wp, bias, M, N, K, ldo, n_row_blocks, m_tile, n_tile, s0, s1, limit);
 }
 
+// Microseconds that `tiles` tiles of TM x 64 tokens and `stages` stages of 64 k take: rounds of one block a compute unit (8
+// XCDs), a stage the longer the more of the units work (they share the power and the caches).  Fitted to sweeps of 130 to 8,192
+// rows over twelve matrices, within 10 %.
+static double tiles_cost(int tm, long long tiles, int stages, int compute_units) {
+    if (tiles <= 0) return 0.0;
+    const double rounds = ceil(ceil(tiles / 8.0) / (compute_units / 8.0)), busy = tiles / (rounds * compute_units);
+    return rounds * (tm == 4 ? 9.0 + stages * (1.05 + 0.55 * busy) : 6.0 + stages * (0.72 + 0.30 * busy));
+}
+
 // How the tiles are cut: row tiles 0 .. n_full - 1 in tiles of 256 tokens, the rest in tiles of 128 tokens.
-// token_tiles 4: all of 256, 2: all of 128, 0: the last round of blocks in tiles of 128 tokens when the tiles of 256
-// would fill less than half of it.
-static int tiles_n_full(int n_tiles, int m_tiles4, int parts, int token_tiles, int compute_units) {
+// token_tiles 4: all of 256, 2: all of 128, 0: the cheapest by tiles_cost of all of 256, all of 128 and the last round of
+// blocks in tiles of 128.  (Few rows leave units idle in tiles of 256: 334 x 4,096 x 14,336 in four parts 82 us, in tiles of
+// 128 62; 2,048 x 28,672 x 4,096, three rounds and a half: 413 all of 256, 470 all of 128, 402 mixed.)
+static int tiles_n_full(int n_tiles, int m_tiles4, int m_tiles2, int parts, int stages, int token_tiles, int compute_units) {
     if (token_tiles == 4) return n_tiles;
     if (token_tiles == 2) return 0;
-    const int per_row_tile = m_tiles4 * parts;
-    const int rest = (n_tiles * per_row_tile) % compute_units;
-    if (rest == 0 || rest > compute_units / 2 || n_tiles * per_row_tile < compute_units) return n_tiles;
-    return n_tiles - (rest + per_row_tile - 1) / per_row_tile;
+    const int per = stages / parts;
+    const int whole = (int)((long long)n_tiles * m_tiles4 * parts / compute_units) * compute_units / (m_tiles4 * parts);   // row tiles in whole rounds
+    int best = n_tiles;
+    double least = 1e30;
+    for (int n : {n_tiles, 0, whole}) {
+        const double c = tiles_cost(4, (long long)n * m_tiles4 * parts, per, compute_units) +
+                         tiles_cost(2, (long long)(n_tiles - n) * m_tiles2 * parts, per, compute_units);
+        if (c < least) { least = c; best = n; }
+    }
+    return best;
 }
 
 template <typename TO, int EPI>
@@ -330,9 +364,8 @@ static int launch_tiles(void* out, const void* a, int lda, const void* wp, const
                         int ldo, long long part_stride, int parts, int token_tiles, int compute_units, float limit, hipStream_t stream) {
     const int n_row_blocks = (N + 63) / 64, n_tiles = (n_row_blocks + kWavesN - 1) / kWavesN;
     const int m4 = (M + 255) / 256, m2 = (M + 127) / 128;
-    const int n_full = tiles_n_full(n_tiles, m4, parts, token_tiles, compute_units);
-    const int u4 = n_full * parts, u2 = (n_tiles - n_full) * parts;
-    const int blocks4 = m4 * ((u4 + 7) / 8) * 8, blocks2 = m2 * ((u2 + 7) / 8) * 8;
+    const int n_full = tiles_n_full(n_tiles, m4, m2, parts, K / kStageK, token_tiles, compute_units);
+    const int blocks4 = (m4 * n_full * parts + 7) / 8 * 8, blocks2 = (m2 * (n_tiles - n_full) * parts + 7) / 8 * 8;
     constexpr size_t smem = (size_t)2 * (kStageW + 256 * kStageK * 2);
     // (the attribute is set once per instance: not per launch, which may be recorded into a graph)
     static bool ready = false;
@@ -350,7 +383,8 @@ static int launch_tiles(void* out, const void* a, int lda, const void* wp, const
 
 // a: bfloat16 [M][lda]; packed_w: llogos_pack_weights of w [N][K]; out [parts][M][ldo] bfloat16 or float32.
 // epilogue 0: out = a . w^T (+ bias [N]); 1: w's 16-row strips alternate gate and up rows, out is
-// [M][N / 2] = silu(gate) * up, or with limit >= 0 the form of tiles_gated (no bias, one part).  parts > 1: float32 partial sums over ranges of k, part_stride
+// [M][N / 2] = silu(gate) * up, or with limit >= 0 the form of tiles_gated (no bias, one part); 2: out (float32) += a . w^T (no bias,
+// one part).  parts > 1: float32 partial sums over ranges of k, part_stride
 // elements apart, no bias.  token_tiles: see tiles_n_full.  compute_units: of the GPU, for that choice.
 // K must be a multiple of 64 and every part must hold at least two stages of 64.
 LLOGOS_EXPORT int llogos_gemm_tiles_bf16(void* out, int out_dtype, const void* a, int lda, const void* packed_w,
@@ -358,10 +392,11 @@ LLOGOS_EXPORT int llogos_gemm_tiles_bf16(void* out, int out_dtype, const void* a
                                          int epilogue, int parts, int token_tiles, int compute_units, float limit, hipStream_t stream) {
     if (M <= 0 || N <= 0 || K <= 0 || out == nullptr || a == nullptr || packed_w == nullptr) return LLOGOS_BAD_ARGUMENT;
     if (out_dtype != DT_BF16 && out_dtype != DT_F32) return LLOGOS_BAD_ARGUMENT;
-    if (epilogue != EPI_PLAIN && epilogue != EPI_SWIGLU) return LLOGOS_BAD_ARGUMENT;
+    if (epilogue < EPI_PLAIN || epilogue > EPI_ADD) return LLOGOS_BAD_ARGUMENT;
+    if (epilogue == EPI_ADD && (out_dtype != DT_F32 || bias != nullptr || parts != 1)) return LLOGOS_BAD_ARGUMENT;
     if ((K % kStageK) || (lda % 8) || lda < K || ((uintptr_t)a % 16) || ((uintptr_t)packed_w % 16)) return LLOGOS_UNSUPPORTED;
     if (epilogue == EPI_SWIGLU && ((N % 32) || bias != nullptr || ldo < N / 2 || parts != 1)) return LLOGOS_BAD_ARGUMENT;
-    if (epilogue == EPI_PLAIN && ldo < N) return LLOGOS_BAD_ARGUMENT;
+    if (epilogue != EPI_SWIGLU && ldo < N) return LLOGOS_BAD_ARGUMENT;
     if (token_tiles != 4 && token_tiles != 2 && token_tiles != 0) return LLOGOS_BAD_ARGUMENT;
     if (parts < 1 || compute_units < 1) return LLOGOS_BAD_ARGUMENT;
     if (parts > 1 && (out_dtype != DT_F32 || bias != nullptr || part_stride < (long long)M * ldo)) return LLOGOS_BAD_ARGUMENT;
@@ -369,6 +404,8 @@ LLOGOS_EXPORT int llogos_gemm_tiles_bf16(void* out, int out_dtype, const void* a
 #define GO(EPI) do { if (out_dtype == DT_BF16) return launch_tiles<bf16_t, EPI>(out, a, lda, packed_w, bias, M, N, K, ldo, part_stride, parts, token_tiles, compute_units, limit, stream); \
                      return launch_tiles<float, EPI>(out, a, lda, packed_w, bias, M, N, K, ldo, part_stride, parts, token_tiles, compute_units, limit, stream); } while (0)
     if (epilogue == EPI_SWIGLU) GO(EPI_SWIGLU);
+    if (epilogue == EPI_ADD)
+        return launch_tiles<float, EPI_ADD>(out, a, lda, packed_w, bias, M, N, K, ldo, part_stride, parts, token_tiles, compute_units, limit, stream);
     GO(EPI_PLAIN);
 #undef GO
 }

@@ -1956,10 +1956,11 @@ def tiles_serve_gated(M: int, K: int = 0) -> bool:
     119 / 120 at 2,048; 8B 225 / 217 and 405 / 391, level inside the model; 14B 343 / 413 and 614 / 630).
     The library gains with the rows and with k (8B: 1.11 PFLOP/s at 1,024 rows, 1.34 from 4,096 on; 70B 1.41
     to 1.47) where the tiled product stays at 1.2: 8B at 4,096 rows 825 / 727, 70B at 2,048 rows 1,516 / 1,363,
-    a 16,384-token prompt of the 8B sizes 278 ms against 268."""
+    a 16,384-token prompt of the 8B sizes 278 ms against 268.  With k beyond 4,096 (14B) it is ahead up to 5,120 rows: 2,500
+    rows 751 / 836, 3,529 1,032 / 1,039, 4,096 1,183 / 1,279, 5,003 1,485 / 1,547, 6,144 1,798 / 1,788)."""
     if PROMPT_PRODUCT == "tiles":
         return True
-    return PROMPT_PRODUCT == "auto" and TILES_MIN_ROWS <= M <= TILES_MAX_ROWS and K <= TILES_MAX_K
+    return PROMPT_PRODUCT == "auto" and TILES_MIN_ROWS <= M <= (TILES_MAX_ROWS if K <= 4096 else 5120) and K <= TILES_MAX_K
 
 
 def tiles_plan(M: int, N: int, K: int) -> Optional[Tuple[int, int]]:
@@ -1967,8 +1968,14 @@ def tiles_plan(M: int, N: int, K: int) -> Optional[Tuple[int, int]]:
     the library's does.  Measured on the MI355X at the layer sizes of 8B, 14B and 70B models: a matrix that
     is much longer than high (a feed-forward's down projection) with 129 to 1,024 rows of activations is where
     the library is furthest from its best (14B, 256 rows: 119 us against 65; 70B: 291 against 143; 8B, 512 rows:
-    88 against 68), and blocks along k fill the compute units that its few row tiles leave idle.  Elsewhere
-    the library's product was level or ahead (by 10 to 25 % from 2,048 rows on)."""
+    88 against 68), and blocks along k fill the compute units that its few row tiles leave idle.  With k of 16,384
+    and more the library's kernels are far from their best at many sizes beyond that, too, by what they choose for a size:
+    where tiles of 256 x 256 fill at most half of the compute units the product in two parts is ahead at all sizes
+    measured (4,096 x 21,504: 1,100 rows 267 us against 225, 1,700 399 / 280, 2,048 441 / 306; 5,120 x 17,408:
+    1,400 rows 330 / 227), and where they fill between 78 and 92 % of their rounds the product in one part at most
+    (4,096 x 21,504: 3,400 rows 739 / 523, 7,000 1,348 / 1,081; 5,120 x 17,408: 2,400 519 / 422, 5,003 1,033 / 880;
+    8,192 x 28,672: 1,700 937 / 692, 5,003 2,355 / 2,167; behind at 6,400 rows of the first, 967 / 1,038).  Elsewhere the library's
+    product was level or ahead (by 10 to 25 % from 2,048 rows on)."""
     if PROMPT_PRODUCT == "library" or M <= SKINNY_MAX_ROWS or K % 64:
         return None
     if PROMPT_PRODUCT == "tiles":
@@ -1978,6 +1985,13 @@ def tiles_plan(M: int, N: int, K: int) -> Optional[Tuple[int, int]]:
         while parts > 1 and (K // 64) // parts < 2:
             parts //= 2
         return parts, token_tiles
+    if K >= 16384 and M > 1024:
+        tiles = -(-M // 256) * -(-N // 256)
+        share = tiles / (256.0 * -(-tiles // 256))               # of the compute units that the rounds of tiles keep busy
+        if K > 16384 and tiles <= 128:
+            return 2, 0
+        if tiles > 128 and 0.78 <= share <= 0.92:
+            return 1, 0
     return None
 
 
@@ -2012,6 +2026,28 @@ def gemm_tiles_bf16(a: torch.Tensor, pw: PackedWeight, bias: Optional[torch.Tens
         return None
     _check(code, "gemm_tiles_bf16")
     return out[0] if parts == 1 else out
+
+
+def gemm_tiles_add(x: torch.Tensor, a: torch.Tensor, pw: Optional[PackedWeight]) -> bool:
+    """x [M, N] (float32, in place) += a [M, K] . w^T by the tiled product with the sum in its epilogue, where
+    tiles_plan takes the product in one part; False (and x untouched) otherwise."""
+    if pw is None or pw.gate_rows or RESIDUAL_PRODUCT != "on":
+        return False
+    if not (a.dtype == torch.bfloat16 and a.dim() == 2 and a.is_cuda and x.is_cuda and a.device == x.device == pw.data.device):
+        return False
+    M, K = a.shape
+    if not (x.dtype == torch.float32 and x.shape == (M, pw.N) and x.is_contiguous() and K == pw.K and a.stride(1) == 1
+            and a.stride(0) % 8 == 0 and a.data_ptr() % 16 == 0):
+        return False
+    plan = tiles_plan(M, pw.N, K)
+    if plan is None or plan[0] != 1:
+        return False
+    code = _lib().llogos_gemm_tiles_bf16(_p(x), F32, _p(a), a.stride(0), _p(pw.data), None, M, pw.N, K, pw.N, ctypes.c_longlong(0), 2, 1,
+                                         int(plan[1]), compute_units(a.device), ctypes.c_float(-1.0), _stream())
+    if code == -2:
+        return False
+    _check(code, "gemm_tiles_add")
+    return True
 
 
 def gemm_product(a: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, swiglu_input: bool = False,

@@ -124,8 +124,8 @@ class Linear(Part):
             return None
         x = residual.x
         if a.shape[0] > K.SKINNY_MAX_ROWS:
-            # prompts: the library's product with the sum in its epilogue, where the library serves anyway
-            if self.bias is None and K.gemm_library_add(x, a, self.weight, self.packed):
+            # prompts: the product that serves them, the tiled one or the library's, with the sum in its epilogue
+            if self.bias is None and (K.gemm_tiles_add(x, a, self.packed) or K.gemm_library_add(x, a, self.weight, self.packed)):
                 return K.RowSquares(None, self.weight.shape[0])
             return None
         if self.packed is None or self.packed.gate_rows:

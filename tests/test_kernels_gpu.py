@@ -972,3 +972,43 @@ def test_expert_product_at_the_edges_of_its_tiles(form, N, K_, monkeypatch):
         assert (got.double() - want).abs().max() <= 2.0 ** -23 * K_ ** 0.5 * 4 * max(1.0, want.abs().max().item())
         half = K.moe_product(a, w, order, seg, 1, gather, torch.bfloat16, relu2=True)
         _close(half, _np(want.clamp(min=0) ** 2), "bfloat16")
+
+
+@pytest.mark.parametrize("M,N,K_", [(1, 64, 64), (129, 320, 192), (700, 1100, 128), (2100, 2900, 64), (4700, 260, 128)])
+def test_tiled_product_places_every_tile_and_adds_itself(M, N, K_):
+    """One tile, fewer than XCDs, bands of token tiles that are not full, several rounds of blocks, parts of k: every value is
+    written once, in every cut into tiles; with the sum in its epilogue the stream gets the same values added once."""
+    gen = torch.Generator(device=DEV).manual_seed(M)
+    a = torch.randn((M, K_), device=DEV, generator=gen).to(torch.bfloat16)
+    w = (torch.randn((N, K_), device=DEV, generator=gen) * 0.1).to(torch.bfloat16)
+    pw = K.pack_weights(w)
+    want = a.double() @ w.double().t()
+    bound = 2.0 ** -22 * K_ ** 0.5 * max(1.0, want.abs().max().item())      # products exact in 32 bits; partial sums rounded
+    x = torch.randn((M, N), device=DEV, generator=gen)
+    lib = K._lib()
+    for token_tiles in (0, 2, 4):
+        for parts in (1, 2, 3):
+            if K_ // 64 // parts < 2 and parts > 1:
+                continue
+            got = K.gemm_tiles_bf16(a, pw, None, torch.float32, parts=parts, token_tiles=token_tiles)
+            got = got if parts == 1 else got.sum(0)
+            assert (got.double() - want).abs().max() <= bound * 2, (token_tiles, parts)
+        y = x.clone()
+        K._check(lib.llogos_gemm_tiles_bf16(K._p(y), K.F32, K._p(a), a.stride(0), K._p(pw.data), None, M, N, K_, N, 0, 2, 1, token_tiles,
+                                            K.compute_units(a.device), -1.0, K._stream()), "tiles")
+        assert torch.equal(y, x + K.gemm_tiles_bf16(a, pw, None, torch.float32, token_tiles=token_tiles)), token_tiles
+
+
+def test_long_products_of_prompts_add_themselves_to_the_stream():
+    """Where the plan takes a long product in one part, the stream gets it in the product's epilogue; elsewhere it is untouched."""
+    M, N, K_ = 3400, 4096, 16384
+    assert K.tiles_plan(M, N, K_) == (1, 0) and K.tiles_plan(2000, N, K_ + 64) == (2, 0) and K.tiles_plan(M + 512, N, K_) is None
+    a = torch.randn((M, K_), device=DEV).to(torch.bfloat16)
+    w = (torch.randn((N, K_), device=DEV) * 0.02).to(torch.bfloat16)
+    pw, x = K.pack_weights(w), torch.randn((M, N), device=DEV)
+    y = x.clone()
+    assert K.gemm_tiles_add(y, a, pw)
+    assert (y - (x + a.float() @ w.float().t())).abs().max() <= 2e-3
+    kept = y.clone()
+    assert not K.gemm_tiles_add(y[:M - 1000], a[:M - 1000], pw) and not K.gemm_tiles_add(y, a.float(), pw) and not K.gemm_tiles_add(y, a, None)
+    assert torch.equal(y, kept)
