@@ -23,6 +23,7 @@
 // step 4 KB, its steps follow one another.  Every load then asks for whole cache lines (the
 // row-major form asks for 16 half lines), and the loads are non-temporal: the weights are read
 // once.  llogos_gemm_packed_bf16 at the end of the file.
+#include <type_traits>
 #include "common.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -113,7 +114,7 @@ __device__ __forceinline__ float gated_value(float gate, float up, int bounded, 
     return gate * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * gate)) * up;
 }
 
-template <int RB, int MB, int MODE, typename TO, int CHUNK, int WAVES = kLdsWaves, bool PACKED = false, bool GATED = false>
+template <int RB, int MB, int MODE, typename TO, int CHUNK, int WAVES = kLdsWaves, bool PACKED = false, bool GATED = false, int RING = 0>
 __global__ __launch_bounds__(WAVES * kWave) void gemm_skinny_lds_kernel(
         TO* __restrict__ out, ActSource src, const bf16_t* __restrict__ w, const float* __restrict__ bias,
         int M, int N, int K, int ldo, size_t part_stride, int k_per_block, int parts) {
@@ -224,6 +225,97 @@ __global__ __launch_bounds__(WAVES * kWave) void gemm_skinny_lds_kernel(
             squares_by_part[threadIdx.x] = row_squares;
         }
     };
+    if constexpr (RING > 0) {
+        // Bound by the weights' stream.  A wave keeps the fragments (1 KB each) of the next RING steps on their way at
+        // every moment: a fragment's registers take the load of RING steps on as soon as they are used, and
+        // activations are loaded two chunks ahead, so that the wait for them, which is one for every older load,
+        // ends no load that the stream needs.  All loads of the loop are unconditional (rows past M repeat the last
+        // one, whose products are not stored): a load under a condition makes every later wait one for all.
+        static_assert(PACKED && (MODE == PRODUCE_PLAIN || MODE == PRODUCE_UNSCALED) && RING % (CHUNK / 16) == 0, "an even number of chunks");
+        constexpr int kSteps = CHUNK / 32, kAhead = RING / kSteps;
+        constexpr int kGroup = MB >= 3 ? 2 : 4;                          // steps whose LDS reads go together
+        const int n_steps = (max(k_end - k_begin, 0) + 31) / 32;
+        const u32x4* wq[RB];
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)                                  // a block past the last reads the last, never stored
+            wq[rb] = reinterpret_cast<const u32x4*>(w) + ((size_t)min(n_block * RB + rb, (N + 63) / 64 - 1) * ((K + 31) / 32) +
+                                                          (k_begin >> 5)) * (4 * kWave) + wave * kWave + lane;
+        const bf16_t* arow[kPiecesPerThread];
+#pragma unroll
+        for (int i = 0; i < kPiecesPerThread; ++i) {
+            const int piece = i * (WAVES * kWave) + threadIdx.x;
+            arow[i] = (const bf16_t*)src.ptr + (size_t)min(piece / (CHUNK / 8), M - 1) * src.lda;
+        }
+        auto load_acts = [&](uint4 (&st)[kPiecesPerThread], int k0) {
+#pragma unroll
+            for (int i = 0; i < kPiecesPerThread; ++i) {
+                const int kk = k0 + ((i * (WAVES * kWave) + threadIdx.x) % (CHUNK / 8)) * 8;
+                st[i] = *reinterpret_cast<const uint4*>(arow[i] + min(kk, K - 8));
+            }
+        };
+        auto put_acts = [&](const uint4 (&st)[kPiecesPerThread], int buf, int k0) {
+#pragma unroll
+            for (int i = 0; i < kPiecesPerThread; ++i) {
+                const int piece = i * (WAVES * kWave) + threadIdx.x;
+                const bool in = k0 + (piece % (CHUNK / 8)) * 8 < k_end;
+                const uint4 v = make_uint4(in ? st[i].x : 0, in ? st[i].y : 0, in ? st[i].z : 0, in ? st[i].w : 0);
+                if (kPieces % (WAVES * kWave) == 0 || piece < kPieces)
+                    *reinterpret_cast<uint4*>(&lds[buf][piece / (CHUNK / 8)][(piece % (CHUNK / 8)) * 8]) = v;
+            }
+        };
+        u32x4 ring[RING][RB];
+        uint4 ahead[2][kPiecesPerThread];
+        auto chunks = [&](int c, auto full) {                            // kAhead chunks from chunk c on
+            constexpr bool FULL = decltype(full)::value;                 // every load lies inside the part
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) {
+                const int cc = c + u;
+                if (!FULL && cc >= n_chunks) break;
+                if (FULL || cc + 2 < n_chunks) load_acts(ahead[u & 1], k_begin + (cc + 2) * CHUNK);
+#pragma unroll
+                for (int s0 = 0; s0 < kSteps; s0 += kGroup) {
+#pragma unroll
+                    for (int s = s0; s < s0 + kGroup; ++s) {
+                        const int t = cc * kSteps + s;
+                        if (!FULL && t >= n_steps) break;
+#pragma unroll
+                        for (int mb = 0; mb < MB; ++mb) {
+                            const bf16x8 af = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(&lds[u & 1][mb * 16 + r][s * 32 + g * 8]));
+#pragma unroll
+                            for (int rb = 0; rb < RB; ++rb)
+                                acc[rb][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, ring[u * kSteps + s][rb]), af,
+                                                                                      acc[rb][mb], 0, 0, 0);
+                        }
+                    }
+#pragma unroll
+                    for (int s = s0; s < s0 + kGroup; ++s) {
+                        const int t = cc * kSteps + s + RING;
+                        if (!FULL && t >= n_steps) break;
+#pragma unroll
+                        for (int rb = 0; rb < RB; ++rb) ring[u * kSteps + s][rb] = __builtin_nontemporal_load(wq[rb] + (size_t)t * (4 * kWave));
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                if (FULL || cc + 1 < n_chunks) put_acts(ahead[(u + 1) & 1], (u + 1) & 1, k_begin + (cc + 1) * CHUNK);
+                __syncthreads();
+            }
+        };
+        if (n_chunks > 0) {
+            load_acts(ahead[0], k_begin);
+            load_acts(ahead[1], k_begin + CHUNK);
+#pragma unroll
+            for (int s = 0; s < RING; ++s)
+#pragma unroll
+                for (int rb = 0; rb < RB; ++rb)
+                    ring[s][rb] = __builtin_nontemporal_load(wq[rb] + (size_t)min(s, n_steps - 1) * (4 * kWave));
+            put_acts(ahead[0], 0, k_begin);
+            add_row_squares();
+            __syncthreads();
+        }
+        int c = 0;
+        for (; (c + 2 * kAhead) * kSteps <= n_steps; c += kAhead) chunks(c, std::true_type{});
+        for (; c < n_chunks; c += kAhead) chunks(c, std::false_type{});
+    } else {
     if (n_chunks > 0) {
         fetch_acts(k_begin);
         fetch_w(wf0, k_begin);
@@ -242,6 +334,7 @@ __global__ __launch_bounds__(WAVES * kWave) void gemm_skinny_lds_kernel(
         if (has1) multiply(wf1, 1);
         if (has2) store_acts(0);
         __syncthreads();
+    }
     }
 
     if (MODE == PRODUCE_UNSCALED) {
@@ -264,23 +357,29 @@ __global__ __launch_bounds__(WAVES * kWave) void gemm_skinny_lds_kernel(
         __syncthreads();                                             // the last chunk has been read
         if (wave & 1) {
 #pragma unroll
-            for (int mb = 0; mb < MB; ++mb)
+            for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) xch[(((wave >> 1) * MB + mb) * 4 + i) * kWave + lane] = acc[0][mb][i];
+                for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) xch[((((wave >> 1) * RB + rb) * MB + mb) * 4 + i) * kWave + lane] = acc[rb][mb][i];
         }
         __syncthreads();
         if (wave & 1) return;
-        const int col0 = (n_block * 2 + (wave >> 1)) * 16 + 4 * g;   // column of silu(gate) * up
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb) {
-            const int m = mb * 16 + r;
-            if (m >= M) continue;
+        for (int rb = 0; rb < RB; ++rb) {
+            const int col0 = ((n_block * RB + rb) * 2 + (wave >> 1)) * 16 + 4 * g;   // column of silu(gate) * up
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
+            for (int mb = 0; mb < MB; ++mb) {
+                const int m = mb * 16 + r;
+                if (m >= M) continue;
                 const float row_scale = MODE == PRODUCE_UNSCALED ? inv_rms[m] : 1.0f;
-                const float gate = acc[0][mb][i] * row_scale, up = xch[(((wave >> 1) * MB + mb) * 4 + i) * kWave + lane] * row_scale;
-                const float y = gated_value(gate, up, src.bounded, src.limit);
-                if (col0 + i < N / 2) store_f32(out + (size_t)m * ldo + col0 + i, y);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float gate = acc[rb][mb][i] * row_scale;
+                    const float up = xch[((((wave >> 1) * RB + rb) * MB + mb) * 4 + i) * kWave + lane] * row_scale;
+                    const float y = gated_value(gate, up, src.bounded, src.limit);
+                    if (col0 + i < N / 2) store_f32(out + (size_t)m * ldo + col0 + i, y);
+                }
             }
         }
         return;
@@ -296,7 +395,7 @@ __global__ __launch_bounds__(WAVES * kWave) void gemm_skinny_lds_kernel(
             const float row_scale = MODE == PRODUCE_UNSCALED ? inv_rms[m] : 1.0f;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const int n = n0 + rb * 16 + 4 * g + i;
+                const int n = (PACKED ? ((n_block * RB + rb) * WAVES + wave) * 16 : n0 + rb * 16) + 4 * g + i;
                 if (n < N) store_f32(dst + (size_t)m * ldo + n, acc[rb][mb][i] * row_scale + (bias ? bias[n] : 0.f));
             }
         }
@@ -312,15 +411,15 @@ LLOGOS_EXPORT int llogos_gemm_skinny_lds_parts(int K, int splits) {
     return (K + kpb - 1) / kpb;
 }
 
-template <int RB, int MB, int MODE, int CHUNK = kChunkK, int WAVES = kLdsWaves, bool PACKED = false, bool GATED = false>
+template <int RB, int MB, int MODE, int CHUNK = kChunkK, int WAVES = kLdsWaves, bool PACKED = false, bool GATED = false, int RING = 0>
 static int launch_lds(void* out, int out_dtype, const ActSource& src, const bf16_t* w, const float* bias,
                       int M, int N, int K, int ldo, size_t part_stride, int kpb, int parts, hipStream_t stream) {
     const int n_blocks = (N + 16 * RB * WAVES - 1) / (16 * RB * WAVES);
     if (out_dtype == DT_BF16)
-        gemm_skinny_lds_kernel<RB, MB, MODE, bf16_t, CHUNK, WAVES, PACKED, GATED><<<n_blocks * parts, WAVES * kWave, 0, stream>>>(
+        gemm_skinny_lds_kernel<RB, MB, MODE, bf16_t, CHUNK, WAVES, PACKED, GATED, RING><<<n_blocks * parts, WAVES * kWave, 0, stream>>>(
             (bf16_t*)out, src, w, bias, M, N, K, ldo, part_stride, kpb, parts);
     else
-        gemm_skinny_lds_kernel<RB, MB, MODE, float, CHUNK, WAVES, PACKED, GATED><<<n_blocks * parts, WAVES * kWave, 0, stream>>>(
+        gemm_skinny_lds_kernel<RB, MB, MODE, float, CHUNK, WAVES, PACKED, GATED, RING><<<n_blocks * parts, WAVES * kWave, 0, stream>>>(
             (float*)out, src, w, bias, M, N, K, ldo, part_stride, kpb, parts);
     return LLOGOS_LAUNCH_CHECK();
 }
@@ -422,6 +521,28 @@ LLOGOS_EXPORT int llogos_gemm_packed_parts(int K, int splits, int chunk) {
     return (K + kpb - 1) / kpb;
 }
 
+// Which form a packed product takes.  The ring of RING steps keeps a wave's loads on their way at every moment, where the
+// chunks of the other form leave in a burst and are waited for together; it matters where a compute unit has one block
+// only: gate/up of [16384, 2048] 17.3 -> 12.5 us at 1 row, 20.8 -> 16.3 at 64 (256 blocks).  With more than 16 rows its
+// chunks of 128 k also leave LDS for twice the blocks, which tells from more than two blocks a unit on: [34816, 5120] 70.8 ->
+// 67.4 at 24 rows, [43008, 4096] 61.9 -> 57.6; between those it is even or behind ([28672, 4096] 36.9 against 36.2 at 1 row,
+// 46.7 against 44.3 at 64; [34816, 5120] 62.2 against 55.9 at 1).  From 33 rows on the reads of the activations from LDS
+// are what costs, and two strips a wave halve them: [28672, 4096] 44.3 -> 41.4 at 64 rows, [43008, 4096] 83.1 -> 74.6, the
+// head [128256, 4096] 210 -> 195, where the blocks of 128 rows fill the units evenly ([34816, 5120], 272 of them: 87.6 against
+// 83.8 with one strip) and a block's k is long enough ([4096, 4096] in eight parts of 512: 13.8
+// against 13.0 at 64 rows; parts of 1,792 25.7 against 26.2 at 64 but 23.6 against 22.8 at 40, parts of 2,901 ahead at both).  Rings of
+// 16 steps and chunks of 256 k measured no faster.  All forms add in the same order.
+enum { STREAM_NONE = 0, STREAM_ONE = 1, STREAM_TWO = 2 };
+constexpr int kStreamRing = 8;
+
+static int stream_form(int mb, int N, int k_part, int parts) {
+    constexpr int kUnits = 256;                                          // compute units
+    const long long blocks = (long long)((N + 63) / 64) * parts, pairs = (long long)((N + 127) / 128) * parts;
+    if (mb >= 3 && k_part >= (mb == 3 ? 2560 : 1536) && pairs * 8 >= 7 * ((pairs + kUnits - 1) / kUnits * kUnits)) return STREAM_TWO;
+    if (blocks <= kUnits || (mb >= 2 && blocks > 2 * kUnits)) return STREAM_ONE;
+    return STREAM_NONE;
+}
+
 LLOGOS_EXPORT int llogos_gemm_packed_bf16(void* out, int out_dtype, const void* act, int mode, int lda,
                                           int act_parts, long long act_part_stride, const void* packed_w,
                                           const float* bias, int M, int N, int K, int ldo,
@@ -439,6 +560,14 @@ LLOGOS_EXPORT int llogos_gemm_packed_bf16(void* out, int out_dtype, const void* 
     ActSource src{act, lda, act_parts, (size_t)act_part_stride};
     const bf16_t* W = (const bf16_t*)packed_w;
     const int mb = (M + 15) / 16;
+    if (mode == PRODUCE_PLAIN) {
+        const int form = stream_form(mb, N, min(kpb, K), parts);
+#define STREAM(RB, MB) return launch_lds<RB, MB, PRODUCE_PLAIN, 128, kLdsWaves, true, false, kStreamRing>(out, out_dtype, src, W, bias, M, N, \
+                                                                                                    K, ldo, (size_t)part_stride, kpb, parts, stream)
+        if (form == STREAM_TWO) { if (mb == 3) STREAM(2, 3); STREAM(2, 4); }
+        if (form == STREAM_ONE) { if (mb == 1) STREAM(1, 1); if (mb == 2) STREAM(1, 2); if (mb == 3) STREAM(1, 3); STREAM(1, 4); }
+#undef STREAM
+    }
 #define GO(MB, MODE, CH) return launch_lds<1, MB, MODE, CH, kLdsWaves, true>(out, out_dtype, src, W, bias, M, N, K, ldo, \
                                                                             (size_t)part_stride, kpb, parts, stream)
 #define BY_MODE(MB, CH) do { if (mode == PRODUCE_PLAIN) GO(MB, PRODUCE_PLAIN, CH); \
@@ -467,6 +596,12 @@ LLOGOS_EXPORT int llogos_gemm_packed_gated_bf16(void* out, int out_dtype, const 
     src.limit = limit;
     const bf16_t* W = (const bf16_t*)packed_w;
     const int mb = (M + 15) / 16;
+    const int form = stream_form(mb, N, K, 1);
+#define STREAM(RB, MB) return launch_lds<RB, MB, PRODUCE_PLAIN, 128, kLdsWaves, true, true, kStreamRing>(out, out_dtype, src, W, nullptr, M, N, \
+                                                                                                  K, ldo, 0, kpb, 1, stream)
+    if (form == STREAM_TWO) { if (mb == 3) STREAM(2, 3); STREAM(2, 4); }
+    if (form == STREAM_ONE) { if (mb == 1) STREAM(1, 1); if (mb == 2) STREAM(1, 2); if (mb == 3) STREAM(1, 3); STREAM(1, 4); }
+#undef STREAM
 #define GO(MB, CH) return launch_lds<1, MB, PRODUCE_PLAIN, CH, kLdsWaves, true, true>(out, out_dtype, src, W, nullptr, M, N, K, ldo, \
                                                                                      0, kpb, 1, stream)
 #define BY_ROWS(CH) do { if (mb == 1) GO(1, CH); if (mb == 2) GO(2, CH); if (mb == 3) GO(3, CH); GO(4, CH); } while (0)
@@ -503,6 +638,10 @@ LLOGOS_EXPORT int llogos_gemm_packed_unscaled_bf16(void* out, int out_dtype, con
     src.bounded = bounded;
     src.limit = limit;
     const bf16_t* W = (const bf16_t*)packed_w;
+#define STREAM(GATED) return launch_lds<1, 1, PRODUCE_UNSCALED, 128, kLdsWaves, true, GATED, kStreamRing>(out, out_dtype, src, W, bias, M, N, K, ldo, \
+                                                                                                   (size_t)part_stride, kpb, parts, stream)
+    if (stream_form(1, N, min(kpb, K), parts) == STREAM_ONE) { if (gated) STREAM(true); STREAM(false); }
+#undef STREAM
 #define GO(CH, GATED) return launch_lds<1, 1, PRODUCE_UNSCALED, CH, kLdsWaves, true, GATED>(out, out_dtype, src, W, bias, M, N, K, ldo, \
                                                                                             (size_t)part_stride, kpb, parts, stream)
     if (gated) { if (chunk == 128) GO(128, true); GO(256, true); }

@@ -689,6 +689,27 @@ def test_gemm_on_packed_weights(M, N, K_):
             assert torch.equal(alone[0], K.gemm_packed_bf16(a, pw, None, torch.float32, 1, 256)[0][:1])
 
 
+@pytest.mark.parametrize("M,N,K_,splits", [(1, 200, 40, 1), (16, 200, 2056, 3), (17, 130, 264, 1), (64, 16384, 520, 1),   # one block a unit
+                                           (33, 32840, 264, 1), (17, 32840, 1032, 1),                    # more than two
+                                           (64, 28696, 1544, 1), (33, 28696, 2824, 1), (40, 57400, 2568, 1)])   # two strips a wave
+def test_packed_product_forms_add_alike(M, N, K_, splits):
+    """Every form of the product on packed weights (a ring of loads, one or two strips a wave) gives the bits of the
+    row-major product, which adds in the same order: steps and chunks that the ring's length does not divide, the last
+    block of a pair missing, several parts."""
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    a = torch.randn(M, K_, device=DEV, generator=g).to(torch.bfloat16)
+    w = (torch.randn(N, K_, device=DEV, generator=g) * 0.05).to(torch.bfloat16)
+    want = K.gemm_skinny_lds_bf16(a, w, None, torch.float32, splits)
+    got = K.gemm_packed_bf16(a, K.pack_weights(w), None, torch.float32, splits, 256)
+    assert torch.equal(got, want)
+    if splits == 1:                                   # want in parts adds in another order than the gated product
+        rows = N // 32 * 32
+        y = K.gemm_packed_gated_bf16(a, K.pack_weights(w[:rows].contiguous(), rows // 2), torch.float32, 256)
+        gate, up = want[0][:, :rows // 2].double(), want[0][:, rows // 2:rows].double()
+        # the hardware's exp2 and reciprocal: 1 ulp each on a factor of at most 1, two more roundings
+        assert torch.allclose(y.double(), gate * torch.sigmoid(gate) * up, rtol=2e-6, atol=1e-6)
+
+
 def test_first_rows_of_packed_weights_and_the_fused_swiglu():
     rng = np.random.default_rng(3)
     I, H = 200, 136
