@@ -17,8 +17,8 @@
 // in order.  Many rows (gemm_f32_tiles_kernel): bound by the matrix cores (157 TFLOP/s); tiles of
 // 128 x 64, 64 x 64 or 64 x 32 through two LDS buffers of 32 k.
 // Measured (us; before: plain FMAs in tiles of 64 x 64, up to 32 rows a wave for a few columns).  705 rows of the 1B
-// sizes: gate/up [16384, 2048] 1,507 -> 477 (99 TFLOP/s), o [2048, 2048] about 390 -> 81, down [2048, 8192] about
-// 1,510 -> 300, q/k/v [3072, 2048] 448 -> 123.  2 rows: gate/up 28.3 -> 28.6 (4.7 TB/s), head [128256, 2048] 209 -> 180
+// sizes: gate/up [16384, 2048] 1,507 -> 459 (103 TFLOP/s), o [2048, 2048] about 390 -> 80, down [2048, 8192] about
+// 1,510 -> 305, q/k/v [3072, 2048] 448 -> 115.  2 rows: gate/up 28.3 -> 28.6 (4.7 TB/s), head [128256, 2048] 209 -> 180
 // (5.8 TB/s).  Distance from 64 bits at k = 8192: 1.5e-7 of the result.
 #include "common.h"
 
@@ -157,11 +157,22 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tiles_kernel(
         dst[c] = row * LD + col;
     }
     const int col = (tid & 7) * 4;
-    f32x4 next[COPIES];
+    // a stage is asked for two stages ahead (one: gate/up 477 us against 459, q/k/v 123 against 115); past K the last values are read again (a load under a condition would make
+    // every wait one for all loads) and zeros are stored
+    f32x4 ahead[2][COPIES];
+    auto load = [&](f32x4 (&to)[COPIES], int k) {
 #pragma unroll
-    for (int c = 0; c < COPIES; ++c) next[c] = load4<VEC>(src[c], col, K);
+        for (int c = 0; c < COPIES; ++c)
+            to[c] = VEC ? *reinterpret_cast<const f32x4*>(src[c] + min(k + col, K - 4)) : load4<false>(src[c], k + col, K);
+    };
+    auto store = [&](const f32x4 (&from)[COPIES], float* to, int k) {
+        const bool in = !VEC || k + col < K;
 #pragma unroll
-    for (int c = 0; c < COPIES; ++c) *reinterpret_cast<f32x4*>(&lds[0][dst[c]]) = next[c];
+        for (int c = 0; c < COPIES; ++c) *reinterpret_cast<f32x4*>(to + dst[c]) = in ? from[c] : f32x4{0.f, 0.f, 0.f, 0.f};
+    };
+    load(ahead[0], 0);
+    load(ahead[1], KS);
+    store(ahead[0], lds[0], 0);
     __syncthreads();
 
     f32x4 mid[NT][MT], total[NT][MT];
@@ -169,13 +180,9 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tiles_kernel(
     for (int n = 0; n < NT; ++n)
 #pragma unroll
         for (int m = 0; m < MT; ++m) mid[n][m] = total[n][m] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int k0 = 0, s = 0; k0 < K; k0 += KS, ++s) {
-        const bool another = k0 + KS < K;
-        if (another) {
-#pragma unroll
-            for (int c = 0; c < COPIES; ++c) next[c] = load4<VEC>(src[c], k0 + KS + col, K);
-        }
-        const float* buf = lds[s & 1];
+    auto stage = [&](int k0, int at) {                           // `at`: the stage's buffer, 0 or 1
+        load(ahead[at], k0 + 2 * KS);
+        const float* buf = lds[at];
 #pragma unroll
         for (int p = 0; p < 2; ++p) {
             if (k0 + 16 * p >= K) break;
@@ -204,11 +211,12 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tiles_kernel(
                     for (int m = 0; m < MT; ++m) { total[n][m] += mid[n][m]; mid[n][m] = f32x4{0.f, 0.f, 0.f, 0.f}; }
             }
         }
-        if (another) {                                           // the other buffer was last read before the barrier behind it
-#pragma unroll
-            for (int c = 0; c < COPIES; ++c) *reinterpret_cast<f32x4*>(&lds[(s + 1) & 1][dst[c]]) = next[c];
-        }
+        store(ahead[at ^ 1], lds[at ^ 1], k0 + KS);              // the other buffer was last read before the barrier behind it
         __syncthreads();
+    };
+    for (int k0 = 0; k0 < K; k0 += 2 * KS) {
+        stage(k0, 0);
+        if (k0 + KS < K) stage(k0 + KS, 1);
     }
     const bool open = (((K + 15) / 16) & 15) != 0;              // parts since the last fold
 #pragma unroll
