@@ -508,8 +508,8 @@ LLOGOS_EXPORT int llogos_pack_weights(void* dst, const void* src, int N, int K, 
 // matrix as one contiguous run, with loads that do not stay in the caches.  Measured on the
 // MI355X against the row-major form (16 rows x 64 bytes per load): 8B gate/up at 8 rows 35.8 us
 // against 46.3 (6.6 TB/s against 5.1), o 7.8 against 13.6, the head 156 against 185.
-// Arguments as llogos_gemm_skinny_lds_bf16; `chunk` (128 or 256) is the k an LDS buffer holds and
-// the unit of the parts: parts = llogos_gemm_packed_parts(K, splits, chunk).
+// Arguments as llogos_gemm_skinny_lds_bf16; `chunk` (128 or 256) is the unit of the parts and the k an
+// LDS buffer holds (the ring's forms, stream_form below, always hold 128): parts = llogos_gemm_packed_parts(K, splits, chunk).
 static int packed_k_per_block(int K, int splits, int chunk) {
     return ((K + splits - 1) / splits + chunk - 1) / chunk * chunk;
 }

@@ -1767,8 +1767,8 @@ def packed_plan(M: int, N: int, K: int) -> Tuple[int, int]:
     blocks along k as for the row-major form (the same trade of evenness, enough blocks and the
     cost of partial sums, measured again on packed weights), and the shorter buffer for up to 16
     rows, where it was 2 to 5 % faster.  One plan per class of row count (16, 32, 64); the kernel itself
-    works in tiles of 16 rows, 1 to 4 of them (33 to 48 rows take three: 41.7 us against 46.1 for the 8B
-    gate/up matrix), which changes no sum."""
+    works in tiles of 16 rows, 1 to 4 of them (33 to 48 rows take three: 39.4 us against 41.4 for the 8B
+    gate/up matrix), and picks the form of its loads by the number of blocks; neither changes a sum."""
     return lds_splits(M, N, K), (128 if M <= 16 else 256)
 
 
