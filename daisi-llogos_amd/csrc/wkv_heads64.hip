@@ -73,7 +73,7 @@ __global__ __launch_bounds__(kWkvWaves * kWave) void wkv64_kernel(
     const int count = MODE ? min(seg_len, count0 - seg * seg_len) : count0;
     const size_t at = ((size_t)seq * n_seg + seg) * H + head;
     float* S = MODE ? seg_state + at * D * D : row + (size_t)head * D * D;      // [value channel][key channel]
-    if (MODE && count <= 0) {
+    if (count <= 0) {                                       // (in mode 0 a sequence that brings no token: its state stays)
         if (MODE == 1) {                                    // a segment beyond the sequence's end: nothing added, nothing decayed
             for (int e = lane; e < D * D; e += kWave) S[e] = 0.f;
             seg_decay[at * D + lane] = 1.f;

@@ -462,6 +462,29 @@ def test_recurrence_of_heads_of_64_channels(heads, lens, segments, monkeypatch):
             assert torch.equal(single, y[rows]), t
 
 
+@pytest.mark.parametrize("segments", [1, 3])
+def test_recurrence_with_sequences_that_bring_no_token(segments, monkeypatch):
+    """Sequences without a token in the step, first, in the middle and last: their states stay, and nothing in front of the
+    step's rows or behind them is read (it would be NaN); the others get what they get without them."""
+    monkeypatch.setattr(K, "SCAN_SEGMENTS", segments)
+    lens, heads = [0, 9, 0, 20, 0], 3
+    f, _, _ = _recurrence_case([0, 9, 0, 20, 0], heads, 6)
+    for name in ("r", "k", "v", "d", "gate", "h"):
+        wide = torch.full((f[name].shape[0] + 2, f[name].shape[1]), float("nan"), device=DEV)
+        wide[1:-1] = f[name]
+        f[name] = wide[1:-1]
+    state = f["state"].clone()
+    cu = np.concatenate([[0], np.cumsum(lens)]).tolist()
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    scan = lambda s, slots, offsets: K.wkv_scan(
+        type("Ctx", (), dict(n_tokens=29, batch=len(slots), slots=i32(slots), cu_seqlens=offsets, cu_dev=i32(offsets), is_decode=False))(),
+        f["r"], f["k"], f["v"], f["d"], f["gate"], f["w0"], f["u"], f["g"], 1e-5, s, heads, 64, f["h"], torch.float32)
+    y = scan(state, [1, 2, 3, 4, 5], cu)
+    alone = f["state"].clone()
+    assert torch.equal(y, scan(alone, [2, 4], [0, 9, 29])) and torch.isfinite(y).all()
+    assert torch.equal(state, alone) and torch.equal(state[[0, 1, 3, 5]], f["state"][[0, 1, 3, 5]])
+
+
 @pytest.mark.parametrize("out", ["float32", "bfloat16"])
 @pytest.mark.parametrize("taps", [1, 2, 4, 7, 16])
 def test_long_steps_of_convolution_shift_and_activation(taps, out):
