@@ -1968,14 +1968,8 @@ def tiles_plan(M: int, N: int, K: int) -> Optional[Tuple[int, int]]:
     the library's does.  Measured on the MI355X at the layer sizes of 8B, 14B and 70B models: a matrix that
     is much longer than high (a feed-forward's down projection) with 129 to 1,024 rows of activations is where
     the library is furthest from its best (14B, 256 rows: 119 us against 65; 70B: 291 against 143; 8B, 512 rows:
-    88 against 68), and blocks along k fill the compute units that its few row tiles leave idle.  With k of 16,384
-    and more the library's kernels are far from their best at many sizes beyond that, too, by what they choose for a size:
-    where tiles of 256 x 256 fill at most half of the compute units the product in two parts is ahead at all sizes
-    measured (4,096 x 21,504: 1,100 rows 267 us against 225, 1,700 399 / 280, 2,048 441 / 306; 5,120 x 17,408:
-    1,400 rows 330 / 227), and where they fill between 78 and 92 % of their rounds the product in one part at most
-    (4,096 x 21,504: 3,400 rows 739 / 523, 7,000 1,348 / 1,081; 5,120 x 17,408: 2,400 519 / 422, 5,003 1,033 / 880;
-    8,192 x 28,672: 1,700 937 / 692, 5,003 2,355 / 2,167; behind at 6,400 rows of the first, 967 / 1,038).  Elsewhere the library's
-    product was level or ahead (by 10 to 25 % from 2,048 rows on)."""
+    88 against 68), and blocks along k fill the compute units that its few row tiles leave idle.  For more rows see
+    long_tiles_plan.  Elsewhere the library's product was level or ahead (by 10 to 25 % from 2,048 rows on)."""
     if PROMPT_PRODUCT == "library" or M <= SKINNY_MAX_ROWS or K % 64:
         return None
     if PROMPT_PRODUCT == "tiles":
@@ -1985,14 +1979,38 @@ def tiles_plan(M: int, N: int, K: int) -> Optional[Tuple[int, int]]:
         while parts > 1 and (K // 64) // parts < 2:
             parts //= 2
         return parts, token_tiles
-    if K >= 16384 and M > 1024:
-        tiles = -(-M // 256) * -(-N // 256)
-        share = tiles / (256.0 * -(-tiles // 256))               # of the compute units that the rounds of tiles keep busy
-        if K > 16384 and tiles <= 128:
-            return 2, 0
-        if tiles > 128 and 0.78 <= share <= 0.92:
-            return 1, 0
-    return None
+    return long_tiles_plan(M, N, K) if M > 1024 else None
+
+
+def long_tiles_plan(M: int, N: int, K: int, n_cus: Optional[int] = None) -> Optional[Tuple[int, int]]:
+    """tiles_plan for more than 1,024 rows: with k of 16,384 and more the library's kernels run at 0.55 to 0.95 PFLOP/s at
+    many sizes and at 1.1 to 1.4 at the others, by what they choose for a size, and the tiled product (1.0 to 1.2) serves
+    where they were slow at every size measured.  That is told by how tiles of 256 x 256 fill the compute units; us, library
+    against tiled, with the sum into the stream or the norm that adds the parts:
+
+    two parts of k  tiles for an eighth to a half of the units, k beyond 16,384 (4,096 x 21,504: 1,100 rows 273 / 231, 2,048 457 /
+                    324; 5,120 x 17,408: 1,400 rows 344 / 257).  111 sizes: level at 6,144 x 18,432 with 1,113 rows, ahead by 2 to
+                    52 % at the others; 14 tiles are behind (0.86), and so are at k of 16,384 those of every other size (0.9).
+    one round       78 to 88 % of the units (4,096 x 21,504: 3,456 rows 760 / 547; 8,192 x 28,672: 1,664 rows 956 / 708): ahead
+                    by 17 to 48 % at 111 sizes.  Outside the library is ahead by 10 to 25 %: 198 tiles 0.84, 228 to 232 0.9, 256 0.9.
+    two rounds      79 to 92 % (4,096 x 21,504: 7,168 rows 1,388 / 1,084): ahead by 3 to 42 % at 140 sizes.  At 400 tiles, 78 %, it
+                    depends on k: below 18,000 and from 24,000 on ahead by 16 to 37 % at 69 sizes (5,120 x 17,408: 5,003 rows 1,071 /
+                    843), between them level or behind (4,096 x 21,504: 6,400 rows 1,006 / 1,037; 10,240 x 18,432 0.95).
+    Rows and columns that fill less than 74 % of the units with values of their own are the library's in either case (its tiles
+    are of other heights: 6,400 x 18,944 with 1,832 rows 0.83, with 2,005 1.35), and so are three rounds and more (0.93 to 1.2)."""
+    if K < 16384 or M <= 1024:
+        return None
+    units = n_cus or compute_units()
+    tiles = -(-M // 256) * -(-N // 256)
+    if K > 16384 and units <= 8 * tiles <= 4 * units:
+        return 2, 0
+    rounds = -(-tiles // units)
+    taken, filled = tiles / (units * rounds), M * N / (65536.0 * units * rounds)
+    if rounds > 2 or filled < 0.74:
+        return None
+    if rounds == 1:
+        return (1, 0) if 0.78 <= taken <= 0.88 else None
+    return (1, 0) if 0.79 <= taken <= 0.92 or (0.78 <= taken < 0.79 and not 18000 <= K < 24000) else None
 
 
 def gemm_tiles_bf16(a: torch.Tensor, pw: PackedWeight, bias: Optional[torch.Tensor], out_dtype: torch.dtype,

@@ -96,6 +96,30 @@ def test_where_the_tiled_product_serves_prompts(monkeypatch):
     assert K.tiles_plan(300, 4096, 4096) == (1, 0) and K.tiles_serve_gated(65)
 
 
+def test_long_products_of_prompts_are_tiled_where_that_was_measured_ahead():
+    """k of 16,384 and more with more than 1,024 rows: sizes measured on either side of every line of the plan.  The library's
+    product was 3 to 19 % ahead at the first ones, the tiled one level or ahead at the others."""
+    plan = lambda M, N, K_: K.long_tiles_plan(M, N, K_, n_cus=256)
+    for M, N, K_ in ((6145, 4096, 21504), (6400, 4096, 21504), (2432, 10240, 18432), (2379, 10240, 21504),      # 400 tiles
+                     (10000, 4096, 21504), (10000, 5120, 17408), (6592, 6144, 18432), (5952, 7168, 18432),      # three rounds
+                     (6145, 8192, 28672), (6656, 8192, 28672),                                                  # and four
+                     (7232, 2048, 16384), (4672, 3072, 16384), (5820, 2560, 16384), (1692, 8448, 16384),        # 228 to 231 tiles
+                     (1306, 8448, 16384), (2560, 4096, 21504), (4096, 4096, 21504), (6144, 4096, 21504), (8192, 4096, 21504),
+                     (1832, 6400, 18944), (1133, 10240, 26624), (1899, 12800, 16896), (1916, 12800, 28608),     # tiles not filled
+                     (1723, 512, 32256), (1100, 4096, 16384), (2432, 3072, 16384), (4032, 2048, 16384),
+                     (1024, 4096, 21504), (2048, 4096, 16320)):
+        assert plan(M, N, K_) is None, (M, N, K_)
+    for M, N, K_ in ((1025, 4096, 21504), (2048, 4096, 21504), (1400, 5120, 17408), (1792, 2048, 32256), (1896, 1024, 40960), (2900, 2560, 30720)):
+        assert plan(M, N, K_) == (2, 0), (M, N, K_)
+    for M, N, K_ in ((3400, 4096, 21504), (3400, 4096, 16384), (1700, 8192, 28672), (2500, 5120, 17408), (2005, 6400, 16896),
+                     (6401, 4096, 21504), (7000, 4096, 24576), (7424, 4096, 21504), (5376, 5120, 17408), (3300, 8192, 28672),
+                     (5003, 5120, 17408), (6400, 4096, 16384), (5000, 5120, 25600), (2442, 10240, 26624)):
+        assert plan(M, N, K_) == (1, 0), (M, N, K_)
+    # half of the units: the same shares of them
+    assert K.long_tiles_plan(3400, 2048, 21504, n_cus=128) == (1, 0) and K.long_tiles_plan(3400, 4096, 21504, n_cus=128) == (1, 0)
+    assert K.long_tiles_plan(1100, 2048, 21504, n_cus=128) == (2, 0) and K.long_tiles_plan(2048, 4096, 21504, n_cus=128) is None
+
+
 def test_where_the_product_that_adds_itself_to_the_stream_serves():
     """The one-pass product whose blocks own 16 or 32 rows of w and all of k serves up to 16 rows where its
     blocks fill the compute units evenly (256 of them here): one strip a block up to 256 strips (1B, 3B, 8B), two
