@@ -1956,11 +1956,13 @@ def tiles_serve_gated(M: int, K: int = 0) -> bool:
     119 / 120 at 2,048; 8B 225 / 217 and 405 / 391, level inside the model; 14B 343 / 413 and 614 / 630).
     The library gains with the rows and with k (8B: 1.11 PFLOP/s at 1,024 rows, 1.34 from 4,096 on; 70B 1.41
     to 1.47) where the tiled product stays at 1.2: 8B at 4,096 rows 825 / 727, 70B at 2,048 rows 1,516 / 1,363,
-    a 16,384-token prompt of the 8B sizes 278 ms against 268.  With k beyond 4,096 (14B) it is ahead up to 5,120 rows: 2,500
-    rows 751 / 836, 3,529 1,032 / 1,039, 4,096 1,183 / 1,279, 5,003 1,485 / 1,547, 6,144 1,798 / 1,788)."""
+    a 16,384-token prompt of the 8B sizes 278 ms against 268.  Beyond 2,048 rows neither is ahead for long: with k of 4,608
+    and 5,120 and 8,192 to 65,536 columns the tiled product took between 0.61 and 1.16 of the time of the library with its SwiGLU pass at 204 sizes,
+    by what the library chooses for a size: 14B 4,096 rows 1,153 / 1,258, 3,840 1,082 / 1,059; 24,576 columns, 2,500 rows
+    476 / 444, 3,072 579 / 652)."""
     if PROMPT_PRODUCT == "tiles":
         return True
-    return PROMPT_PRODUCT == "auto" and TILES_MIN_ROWS <= M <= (TILES_MAX_ROWS if K <= 4096 else 5120) and K <= TILES_MAX_K
+    return PROMPT_PRODUCT == "auto" and TILES_MIN_ROWS <= M <= TILES_MAX_ROWS and K <= TILES_MAX_K
 
 
 def tiles_plan(M: int, N: int, K: int) -> Optional[Tuple[int, int]]:

@@ -96,6 +96,14 @@ def test_where_the_tiled_product_serves_prompts(monkeypatch):
     assert K.tiles_plan(300, 4096, 4096) == (1, 0) and K.tiles_serve_gated(65)
 
 
+def test_gated_products_of_long_prompts_are_the_library_s():
+    """Beyond 2,048 rows, whatever k is: sizes at which the library with a SwiGLU pass was measured 2 to 13 % ahead."""
+    for M, N, K_ in ((2500, 24576, 4608), (4096, 24576, 4608), (2304, 8192, 4608), (3072, 8192, 4608), (3329, 27648, 5120),
+                     (3843, 32768, 5120), (4048, 65536, 4352), (2049, 16384, 5120), (5120, 8192, 5120)):
+        assert not K.tiles_serve_gated(M, K_), (M, N, K_)
+    assert K.tiles_serve_gated(2048, 4608) and K.tiles_serve_gated(1024, 5120)
+
+
 def test_long_products_of_prompts_are_tiled_where_that_was_measured_ahead():
     """k of 16,384 and more with more than 1,024 rows: sizes measured on either side of every line of the plan.  The library's
     product was 3 to 19 % ahead at the first ones, the tiled one level or ahead at the others."""
