@@ -1,7 +1,7 @@
 // out[M, N] = a[M, K] . w[N, K]^T (+ bias[N]) with every product and sum in 32-bit
 // floats (plain FMA, no matrix-core input rounding): the fallback of the bfloat16 engine for
-// shapes its fast kernels refuse, and products of mixed types.  Products of float32 alone have
-// a kernel of their own (gemm_f32.hip).  Each output element is summed in the same order whatever M is, so a row's result
+// shapes its fast kernels refuse, and products of mixed types.  Products of float32 alone are
+// handed on to the kernels of their own (gemm_f32.hip).  Each output element is summed in the same order whatever M is, so a row's result
 // does not depend on the other rows of the batch.  The order is blocked: 16 products into a
 // partial sum, 16 of those into a second, those into the total, so that the rounding error
 // of a sum over thousands of k grows with the sum's blocks (about 16 + 16 + K / 256 additions
@@ -72,6 +72,9 @@ __global__ __launch_bounds__(256) void gemm_generic_kernel(
     }
 }
 
+extern "C" int llogos_gemm_f32(float* out, const float* a, const float* w, const float* bias, int M, int N, int K, int lda, int ldo,
+                               int form, hipStream_t stream);
+
 LLOGOS_EXPORT int llogos_gemm_generic(void* out, int out_dtype, const void* a, int a_dtype,
                                       const void* w, int w_dtype, const float* bias,
                                       int M, int N, int K, int lda, int ldo, hipStream_t stream) {
@@ -81,6 +84,7 @@ LLOGOS_EXPORT int llogos_gemm_generic(void* out, int out_dtype, const void* a, i
         (TO*)out, (const TA*)a, (const TW*)w, bias, M, N, K, lda, ldo)
     const int key = a_dtype * 4 + w_dtype * 2 + out_dtype;
     switch (key) {
+        case 0: return llogos_gemm_f32((float*)out, (const float*)a, (const float*)w, bias, M, N, K, lda, ldo, 0, stream);
         case 1: LAUNCH(float, float, bf16_t); break;
         case 2: LAUNCH(float, bf16_t, float); break;
         case 3: LAUNCH(float, bf16_t, bf16_t); break;

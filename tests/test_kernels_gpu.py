@@ -281,6 +281,19 @@ def test_float32_product_of_few_rows_is_the_tiled_product_bit_for_bit(N, K_):
     assert torch.equal(few, many[:5])
 
 
+def test_the_generic_entry_takes_float32_throughout():
+    """The library's entry for any types hands float32 operands on to the float32 product: the same bits, with and without a
+    bias, into rows of a wider result."""
+    rng = np.random.default_rng(2)
+    for M, N, K_ in ((1, 70, 40), (33, 65, 255)):
+        a, w, b = _t(rng.standard_normal((M, K_))), _t(rng.standard_normal((N, K_))), _t(rng.standard_normal(N))
+        for bias in (b, None):
+            out = torch.full((M, N + 3), 7.0, device=DEV)
+            code = K._lib().llogos_gemm_generic(K._p(out), K.F32, K._p(a), K.F32, K._p(w), K.F32, K._p(bias), M, N, K_, K_, N + 3, K._stream())
+            assert code == 0
+            assert torch.equal(out[:, :N], K.gemm_generic(a, w, bias, torch.float32)) and (out[:, N:] == 7.0).all()
+
+
 @pytest.mark.parametrize("M,N,K_", [(1, 16, 16), (17, 33, 40), (33, 70, 272), (64, 129, 4112), (65, 31, 255), (130, 66, 2049), (200, 250, 513)])
 def test_float32_product_gives_the_same_bits_in_every_form(M, N, K_, monkeypatch):
     """The forms of the float32 product (few rows in three heights of blocks, tiles in three sizes) at remainders of
