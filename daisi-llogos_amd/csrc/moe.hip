@@ -465,12 +465,13 @@ LLOGOS_EXPORT int llogos_moe_combine_weighted(float* out, const float* y, const 
 //             [4096, 7168], two a token: 4 tokens (6 and 4 experts) 88 -> 64 us (5.5 TB/s) and 48 -> 43, 64 tokens
 //             (all) 220 -> 178 (5.3 TB/s), against a block that found its tile one segment after the other and
 //             whose loads stood in branches, two in flight a wave;
-//   tiles     64 or 256 sorted rows x 128 rows of the matrix with v_mfma_f32_32x32x16_bf16, stages of 64 k
+//   tiles     64, 128 or 256 sorted rows x 128 rows of the matrix with v_mfma_f32_32x32x16_bf16, stages of 64 k
 //             through LDS (swizzled rows of 128 bytes), the next stage's loads in registers meanwhile.  Bound by
 //             how much of the matrix is in flight and by what the caches give (10 TB/s, matrices and rows
-//             together).  The tall form is taken where experts have 64 rows or more on average: it reads an expert's
-//             matrix once, and waves whose 64 rows a segment does not reach only copy: 1,127 tokens 319 -> 271 us
-//             and 340 -> 246 against tiles of 128 rows, whose second tile a segment of 141 rows barely fills.
+//             together).  A tile costs about the same whatever part of its rows a segment fills (waves whose 64
+//             rows it does not reach only copy): low tiles for short segments, tall ones, which read an expert's
+//             matrix less often, where segments fill several of them (16 experts of [7168, 4096] and 2,048 rows
+//             each: 64 rows 1.27, 256 rows 0.93 of the time of 128).
 // Sums depend on k's order alone, as above.  K must be a multiple of 8 and N of 4.
 typedef __bf16 moe_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float moe_f32x4 __attribute__((ext_vector_type(4)));
@@ -599,11 +600,11 @@ __device__ __forceinline__ int moe_lds_at(int row, int oct) { return row * kMoeB
 // rows of the expert's matrix are the first operand and the sorted rows the second, so a lane ends with the sums
 // of one sorted row (l & 31) for 4 x 4 neighbouring columns: entry 4 q + e is column 8 q + 4 (l >> 5) + e.
 template <int BM, int BN, typename TO>
-__global__ __launch_bounds__(BM == 64 ? 256 : 512) __attribute__((amdgpu_waves_per_eu(BM == 64 ? 3 : 4, BM == 64 ? 3 : 4))) void moe_tiles_kernel(
+__global__ __launch_bounds__(BM == 256 ? 512 : 256) __attribute__((amdgpu_waves_per_eu(BM == 256 ? 4 : 3, BM == 256 ? 4 : 3))) void moe_tiles_kernel(
         TO* __restrict__ out, const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, const int* __restrict__ order,
         const int* __restrict__ seg, int E, int top, int gather, int N, int K, int lda, int act, float scale,
                                                           const float* __restrict__ row_weight, float limit) {
-    constexpr int THREADS = BM == 64 ? 256 : 512;
+    constexpr int THREADS = BM == 256 ? 512 : 256;
     constexpr int CA = BM * 8 / THREADS, CW = BN * 8 / THREADS;   // 16-byte pieces a thread copies a stage
     constexpr int WN = BM == 64 ? BN / 4 : BN / 2, NT = WN / 32, MT = 2;      // a wave's part: 64 rows x WN columns of the tile
     __shared__ __attribute__((aligned(16))) bf16_t As[BM * kMoeBK];
@@ -713,19 +714,20 @@ __global__ __launch_bounds__(BM == 64 ? 256 : 512) __attribute__((amdgpu_waves_p
     }
 }
 
-// form 0: few rows (tiles of 16); 1: tiles of 64 rows; 2: tiles of 256 rows.  -2 for shapes these do not take.
+// form 0: few rows (tiles of 16); 1: tiles of 64 rows; 2: of 128; 3: of 256.  -2 for shapes these do not take.
 LLOGOS_EXPORT int llogos_moe_product_bf16(void* out, int out_dtype, const void* a, const void* w, const int* order, const int* seg,
                                           int E, int top, int gather, int P, int N, int K, int lda, int act, float scale,
                                           const float* row_weight, float limit, int form, hipStream_t stream) {
-    if (P <= 0 || N <= 0 || K <= 0 || E <= 0 || top <= 0 || lda < K || act < 0 || act > 3 || form < 0 || form > 2 || (row_weight && act < 2) || (act == 3 && !(limit >= 0.f))) return LLOGOS_BAD_ARGUMENT;
+    if (P <= 0 || N <= 0 || K <= 0 || E <= 0 || top <= 0 || lda < K || act < 0 || act > 3 || form < 0 || form > 3 || (row_weight && act < 2) || (act == 3 && !(limit >= 0.f))) return LLOGOS_BAD_ARGUMENT;
     if ((K % 8) || (N % 4) || (lda % 8) || ((uintptr_t)a % 16) || ((uintptr_t)w % 16) || ((uintptr_t)out % 16)) return LLOGOS_UNSUPPORTED;
     if (out_dtype != DT_F32 && out_dtype != DT_BF16) return LLOGOS_BAD_ARGUMENT;
-    const int rows = form == 0 ? 16 : (form == 1 ? 64 : 256);
+    const int rows = form == 0 ? 16 : (form == 1 ? 64 : (form == 2 ? 128 : 256));
     const int row_tiles = (P + rows - 1) / rows + E;
-#define MOE_GO(KERNEL, NB, TO) KERNEL<<<dim3((N + NB - 1) / NB, row_tiles), form == 2 ? 512 : 256, 0, stream>>>((TO*)out, (const bf16_t*)a, (const bf16_t*)w, \
+#define MOE_GO(KERNEL, NB, TO) KERNEL<<<dim3((N + NB - 1) / NB, row_tiles), form == 3 ? 512 : 256, 0, stream>>>((TO*)out, (const bf16_t*)a, (const bf16_t*)w, \
         order, seg, E, top, gather, N, K, lda, act, scale, row_weight, limit)
     if (form == 0) { if (out_dtype == DT_F32) MOE_GO(moe_few_kernel<float>, 16, float); else MOE_GO(moe_few_kernel<bf16_t>, 16, bf16_t); }
     else if (form == 1) { if (out_dtype == DT_F32) MOE_GO((moe_tiles_kernel<64, 128, float>), 128, float); else MOE_GO((moe_tiles_kernel<64, 128, bf16_t>), 128, bf16_t); }
+    else if (form == 2) { if (out_dtype == DT_F32) MOE_GO((moe_tiles_kernel<128, 128, float>), 128, float); else MOE_GO((moe_tiles_kernel<128, 128, bf16_t>), 128, bf16_t); }
     else { if (out_dtype == DT_F32) MOE_GO((moe_tiles_kernel<256, 128, float>), 128, float); else MOE_GO((moe_tiles_kernel<256, 128, bf16_t>), 128, bf16_t); }
 #undef MOE_GO
     return LLOGOS_LAUNCH_CHECK();

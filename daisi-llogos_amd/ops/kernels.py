@@ -644,7 +644,7 @@ def activation(x: torch.Tensor, kind: str, out_dtype: torch.dtype, a: float = 0.
 # ----------------------------------------------------------------------------
 MOE_MAX_EXPERTS = 1024
 MOE_FEW_PAIRS = 256          # up to so many (token, choice) pairs a step the experts' product streams the matrices in tiles of 16 rows
-MOE_PRODUCT = "auto"         # "auto": chosen by the step; "plain", "few", "tiles64" (low tiles), "tiles128" (tall ones) force a form (tests)
+MOE_PRODUCT = "auto"         # "auto": chosen by the step; "plain", "few", "tiles64", "tiles128", "tiles256" force a form (tests)
 
 
 def moe_route(ids: Optional[torch.Tensor], table: torch.Tensor, n_experts: int):
@@ -725,6 +725,24 @@ def moe_combine_weighted(y: torch.Tensor, where: torch.Tensor, choice: torch.Ten
     return out if stream is None else new_rows
 
 
+def moe_form(P: int, E: int, N: int, K: int) -> int:
+    """Which form of the experts' product serves P pairs of E experts with matrices of N rows and K values: 0 few rows, 1 to 3
+    tiles of 64, 128 and 256 rows.  Only the average segment is known here; segments around it differ, by chance or because
+    a router prefers some experts.
+    Few rows end at 8 an expert where tiles give every compute unit two blocks (16 experts of 7168 x 4096, 16 rows: 275 us
+    against 232, and 276 against 160 for the way down).  Tiles of 64 rows up to 96 an expert, of 128 above: at 96 rows
+    16 experts of 4096 x 7168 took 283 us in tiles of 64, 190 in tiles of 128; at 64 rows 14 of 7168 x 4096 207 and 231.
+    Tiles of 256 rows only where every expert has several and the product is large (88 million results, k of 4,096 and
+    more): 0.91 to 1.01 of the time of tiles of 128 over seven matrices, even routing and uneven.  Below, what they gain
+    depends on how segments fall on them: at 144 rows an expert 0.65 to 0.95 for even segments, 0.95 to 1.3 for uneven
+    ones; at 64 to 96 rows 1.05 to 1.3 of the time of tiles of 64, at 256 to 350 1.03 to 1.2 of that of 128."""
+    if P <= MOE_FEW_PAIRS and (P <= 8 * E or E * -(-N // 128) < 512):
+        return 0
+    if P < 96 * E:
+        return 1
+    return 3 if P >= 400 * E and K >= 4096 and P * N >= 88_000_000 else 2
+
+
 def moe_product(a: torch.Tensor, w: torch.Tensor, order: torch.Tensor, seg: torch.Tensor, top: int, gather: bool,
                 out_dtype: torch.dtype, relu2: bool = False, scale: float = 1.0, gated: bool = False,
                 pair_weight: Optional[torch.Tensor] = None, limit: Optional[float] = None) -> torch.Tensor:
@@ -754,16 +772,11 @@ def moe_product(a: torch.Tensor, w: torch.Tensor, order: torch.Tensor, seg: torc
     lim = ctypes.c_float(limit or 0.0)
     out = torch.empty((P, N // 2 if gated else N), dtype=out_dtype, device=a.device)
     if a.dtype == torch.bfloat16 and MOE_PRODUCT != "plain" and a.stride(1) == 1:
-        # on the matrix cores: tiles of 16 sorted rows straight from memory for steps of few rows, tiles of 64 or
-        # 256 rows through LDS for more: the tall ones (an expert's matrix is read once) from 64 rows an expert on
-        # average (16 experts of 7168 x 4096: 50 rows 230 us in the low form and 246 in the tall one, 75 rows 260 and 246,
-        # 141 rows 327 and 271)
-        # (and the few-row form ends at 8 rows an expert where tiles give every compute unit two blocks: 16 rows an expert
-        # 275 us against 232, and 276 against 160 for the way down)
-        few = P <= 8 * E or E * -(-N // 128) < 512
-        form = 0 if few and P <= MOE_FEW_PAIRS else (2 if P >= 64 * E else 1)
-        if MOE_PRODUCT in ("few", "tiles64", "tiles128"):
-            form = ("few", "tiles64", "tiles128").index(MOE_PRODUCT)
+        # on the matrix cores: tiles of 16 sorted rows straight from memory for steps of few rows, tiles of 64, 128 or
+        # 256 rows through LDS for more
+        form = moe_form(P, E, N, Kk)
+        if MOE_PRODUCT != "auto":
+            form = ("few", "tiles64", "tiles128", "tiles256").index(MOE_PRODUCT)
         code = _lib().llogos_moe_product_bf16(_p(out), _DT[out_dtype], _p(a), _p(w), _p(order), _p(seg), E, top, 1 if gather else 0,
                                               P, N, Kk, a.stride(0), act, ctypes.c_float(scale), _p(pair_weight), lim, form, _stream())
         if code != -2:

@@ -985,14 +985,14 @@ def test_long_prompts_take_the_tiled_gate_up_product_by_default():
     H.close(got, want, "bfloat16", "long prompt, tiled gate/up product", config=name)
 
 
-@pytest.mark.parametrize("form", ["few", "tiles64", "tiles128"])
+@pytest.mark.parametrize("form", ["few", "tiles64", "tiles128", "tiles256"])
 @pytest.mark.parametrize("N,K_", [(20, 8), (132, 72), (260, 264), (64, 1320)])
 def test_expert_product_at_the_edges_of_its_tiles(form, N, K_, monkeypatch):
-    """Segments of no row, one, and around 16, 64 and 256 rows (in the order of many experts, more than a wave has lanes),
+    """Segments of no row, one, and around 16, 64, 128 and 256 rows (in the order of many experts, more than a wave has lanes),
     matrices that fill no tile, k of no whole stage, and more of k than the few-row form asks for at once."""
     monkeypatch.setattr(K, "MOE_PRODUCT", form)
     rng = np.random.default_rng(N)
-    sizes = [0, 1, 15, 16, 17, 0, 63, 64, 65, 255, 256, 257, 300] + [0, 1] * 40
+    sizes = [0, 1, 15, 16, 17, 0, 63, 64, 65, 127, 128, 129, 255, 256, 257, 300] + [0, 1] * 40
     seg = _t(np.concatenate([[0], np.cumsum(sizes)]), torch.int32)
     P, E = sum(sizes), len(sizes)
     order = _t(rng.permutation(P), torch.int32)

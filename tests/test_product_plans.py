@@ -128,6 +128,20 @@ def test_long_products_of_prompts_are_tiled_where_that_was_measured_ahead():
     assert K.long_tiles_plan(1100, 2048, 21504, n_cus=128) == (2, 0) and K.long_tiles_plan(2048, 4096, 21504, n_cus=128) is None
 
 
+def test_tiles_of_the_experts_product():
+    """Tall tiles only where they were measured level or ahead for even and uneven segments; tiles of 64 rows below 96 rows an
+    expert, of 128 from there on."""
+    for P, E, N, K_ in ((64 * 16, 16, 1024, 2048), (73 * 14, 14, 7168, 4096), (95 * 16, 16, 4096, 7168), (32 * 8, 8, 28672, 4096)):
+        assert K.moe_form(P, E, N, K_) == 1, (P, E, N, K_)
+    for P, E, N, K_ in ((96 * 16, 16, 4096, 7168), (141 * 16, 16, 7168, 4096), (144 * 16, 16, 3584, 2048), (256 * 16, 16, 4096, 7168),
+                        (292 * 14, 14, 7168, 4096), (512 * 8, 8, 4096, 4096), (1024 * 16, 16, 1024, 2048), (1024 * 16, 16, 7168, 2048),
+                        (1024 * 16, 16, 4096, 3584), (336 * 64, 64, 4096, 4096), (1024 * 16, 16, 4096, 5120)):
+        assert K.moe_form(P, E, N, K_) == 2, (P, E, N, K_)
+    for P, E, N, K_ in ((1024 * 16, 16, 7168, 4096), (1500 * 16, 16, 4096, 7168), (1024 * 8, 8, 14336, 4096), (512 * 8, 8, 28672, 4096),
+                        (3000 * 8, 8, 4096, 4096)):
+        assert K.moe_form(P, E, N, K_) == 3, (P, E, N, K_)
+
+
 def test_where_the_product_that_adds_itself_to_the_stream_serves():
     """The one-pass product whose blocks own 16 or 32 rows of w and all of k serves up to 16 rows where its
     blocks fill the compute units evenly (256 of them here): one strip a block up to 256 strips (1B, 3B, 8B), two
