@@ -725,19 +725,27 @@ def moe_combine_weighted(y: torch.Tensor, where: torch.Tensor, choice: torch.Ten
     return out if stream is None else new_rows
 
 
-def moe_form(P: int, E: int, N: int, K: int) -> int:
+def moe_form(P: int, E: int, N: int, K: int, n_cus: Optional[int] = None) -> int:
     """Which form of the experts' product serves P pairs of E experts with matrices of N rows and K values: 0 few rows, 1 to 3
     tiles of 64, 128 and 256 rows.  Only the average segment is known here; segments around it differ, by chance or because
     a router prefers some experts.
-    Few rows end at 8 an expert where tiles give every compute unit two blocks (16 experts of 7168 x 4096, 16 rows: 275 us
-    against 232, and 276 against 160 for the way down).  Tiles of 64 rows up to 96 an expert, of 128 above: at 96 rows
+    Few rows end at about 12 an expert (16 experts of 7168 x 4096, 12 rows 210 us against 224 in tiles of 64, 16 rows 264
+    and 222; 8 of 4096 x 4096, 12 rows 64 and 71, 16 rows 78 and 72), at 4 where the tiles' blocks fill the compute units in
+    one round (4096 x 7168, 4 rows 157 and 155, 8 rows 175 and 156), and not at all where they leave units without a block;
+    MOE_FEW_PAIRS pairs at most, or 4 rows an expert if that is more and k is long enough (128 experts of 1536 x 2048, 384
+    pairs 147 and 176).
+    Tiles of 64 rows up to 96 an expert, of 128 above: at 96 rows
     16 experts of 4096 x 7168 took 283 us in tiles of 64, 190 in tiles of 128; at 64 rows 14 of 7168 x 4096 207 and 231.
     Tiles of 256 rows only where every expert has several and the product is large (88 million results, k of 4,096 and
     more): 0.91 to 1.01 of the time of tiles of 128 over seven matrices, even routing and uneven.  Below, what they gain
     depends on how segments fall on them: at 144 rows an expert 0.65 to 0.95 for even segments, 0.95 to 1.3 for uneven
     ones; at 64 to 96 rows 1.05 to 1.3 of the time of tiles of 64, at 256 to 350 1.03 to 1.2 of that of 128."""
-    if P <= MOE_FEW_PAIRS and (P <= 8 * E or E * -(-N // 128) < 512):
-        return 0
+    if P <= max(MOE_FEW_PAIRS, 4 * E if K >= 1024 else 0):
+        if P <= 4 * E:
+            return 0
+        units, columns = n_cus or compute_units(), E * -(-N // 128)
+        if columns < units or P <= (4 if 1.5 * units <= columns <= 3 * units else (13 if columns < 6 * units else 12)) * E:
+            return 0
     if P < 96 * E:
         return 1
     return 3 if P >= 400 * E and K >= 4096 and P * N >= 88_000_000 else 2

@@ -131,6 +131,13 @@ def test_long_products_of_prompts_are_tiled_where_that_was_measured_ahead():
 def test_tiles_of_the_experts_product():
     """Tall tiles only where they were measured level or ahead for even and uneven segments; tiles of 64 rows below 96 rows an
     expert, of 128 from there on."""
+    few = [(2, 16, 7168, 4096), (64, 16, 4096, 7168), (128, 14, 7168, 4096), (160, 16, 7168, 2048), (100, 8, 4096, 4096), (256, 16, 1024, 2048),
+           (200, 16, 7168, 2048), (384, 128, 1536, 2048), (256, 128, 2048, 768)]
+    for P, E, N, K_ in few:
+        assert K.moe_form(P, E, N, K_, 256) == 0, (P, E, N, K_)
+    for P, E, N, K_ in ((96, 16, 4096, 7168), (128, 16, 4096, 3584), (200, 14, 7168, 4096), (128, 8, 4096, 4096), (257, 16, 1024, 2048),
+                        (384, 128, 2048, 768), (520, 128, 1536, 2048), (196, 16, 14336, 4096)):
+        assert K.moe_form(P, E, N, K_, 256) == 1, (P, E, N, K_)
     for P, E, N, K_ in ((64 * 16, 16, 1024, 2048), (73 * 14, 14, 7168, 4096), (95 * 16, 16, 4096, 7168), (32 * 8, 8, 28672, 4096)):
         assert K.moe_form(P, E, N, K_) == 1, (P, E, N, K_)
     for P, E, N, K_ in ((96 * 16, 16, 4096, 7168), (141 * 16, 16, 7168, 4096), (144 * 16, 16, 3584, 2048), (256 * 16, 16, 4096, 7168),
