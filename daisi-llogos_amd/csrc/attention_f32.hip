@@ -23,12 +23,13 @@
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x8 __attribute__((ext_vector_type(8), aligned(16)));
 
-// cu: token offsets of the sequences [batch + 1]; null: every sequence brings one token
+// cu: token offsets of the sequences [batch + 1]; null: every sequence brings one token.  tok_seq: row of the page table a
+// token's sequence has; null: the sequences' own order.  A sequence's tokens may come in any order of positions.
 template <int HD, int WAVES>
 __global__ __launch_bounds__(WAVES * 64) void attn_f32_kernel(
         float* __restrict__ out, const float* __restrict__ q, int q_stride, const float* __restrict__ k_pool,
         const float* __restrict__ v_pool, PagedKV cache, const int* __restrict__ cu, int batch,
-        const int* __restrict__ tok_pos, int n_heads, int group, float scale, int window, int sinks) {
+        const int* __restrict__ tok_seq, const int* __restrict__ tok_pos, int n_heads, int group, float scale, int window, int sinks) {
     constexpr int DB = HD / 16, OWN = (DB + WAVES - 1) / WAVES;
     __shared__ f32x4 sums[WAVES][DB][64];
     __shared__ float tops[WAVES][16], dens[WAVES][16];
@@ -55,8 +56,12 @@ __global__ __launch_bounds__(WAVES * 64) void attn_f32_kernel(
     const bool real = row < rows;
     const int tok = first + min(row, rows - 1) / group, head = kvh * group + min(row, rows - 1) % group;
     const int pos = real ? tok_pos[tok] : -1;
-    const int last = tok_pos[first + min(tile * 16 + 15, rows - 1) / group];       // the tile's latest position ...
-    const int early = tok_pos[first + tile * 16 / group];                          // ... and its earliest
+    int last = pos, early = real ? pos : 0x7fffffff;             // the tile's latest position and its earliest
+#pragma unroll
+    for (int o = 1; o < 16; o <<= 1) { last = max(last, __shfl_xor(last, o, kWave)); early = min(early, __shfl_xor(early, o, kWave)); }
+    last = __builtin_amdgcn_readfirstlane(last);                // (the same in every lane)
+    early = __builtin_amdgcn_readfirstlane(early);
+    if (tok_seq) seq = tok_seq[first];
 
     f32x8 qv[HD / 32];
 #pragma unroll
@@ -192,8 +197,8 @@ __global__ __launch_bounds__(WAVES * 64) void attn_f32_kernel(
 
 // n_tiles: tiles of 16 (token, head of the group) rows over all sequences; cu null: every sequence brings one token
 LLOGOS_EXPORT int llogos_attention_f32(float* out, const float* q, int q_stride, const float* k_pool, const float* v_pool,
-                                       const int* table, int table_stride, const int* cu, const int* tok_pos, int batch, int n_tiles,
-                                       int n_heads, int n_kv_heads, int head_dim, float scale, int window, int sinks, hipStream_t stream) {
+                                       const int* table, int table_stride, const int* cu, const int* tok_seq, const int* tok_pos,
+                                       int batch, int n_tiles, int n_heads, int n_kv_heads, int head_dim, float scale, int window, int sinks, hipStream_t stream) {
     if (batch <= 0 || n_tiles <= 0 || n_kv_heads <= 0 || n_heads <= 0 || n_heads % n_kv_heads != 0 || window < 0 || sinks < 0) return LLOGOS_BAD_ARGUMENT;
     if ((head_dim != 64 && head_dim != 128) || (q_stride & 3) || (((uintptr_t)q | (uintptr_t)out) & 15)) return LLOGOS_UNSUPPORTED;
     const int group = n_heads / n_kv_heads;
@@ -202,7 +207,7 @@ LLOGOS_EXPORT int llogos_attention_f32(float* out, const float* q, int q_stride,
     // Waves that share a tile's pages: many where there are few tiles (a single-token step: as many as LDS holds results of), few where
     // the tiles alone fill the GPU.
     const bool few = (long long)n_tiles * n_kv_heads < 1024;
-#define ATTN(HD, W) attn_f32_kernel<HD, W><<<grid, W * 64, 0, stream>>>(out, q, q_stride, k_pool, v_pool, cache, cu, batch, tok_pos, \
+#define ATTN(HD, W) attn_f32_kernel<HD, W><<<grid, W * 64, 0, stream>>>(out, q, q_stride, k_pool, v_pool, cache, cu, batch, tok_seq, tok_pos, \
                                                                         n_heads, group, scale, window, sinks)
     if (head_dim == 64) { if (few) ATTN(64, 16); else ATTN(64, 4); }
     else { if (few) ATTN(128, 8); else ATTN(128, 4); }

@@ -2356,27 +2356,36 @@ def attention_decode_fused(ctx, qkv: torch.Tensor, bias: Optional[torch.Tensor],
 def attention_f32(ctx, q: torch.Tensor, q_stride: int, k_pool: torch.Tensor, v_pool: torch.Tensor, table: torch.Tensor,
                   n_heads: int, n_kv_heads: int, head_dim: int, scale: float, window: int = 0, sinks: int = 0) -> Optional[torch.Tensor]:
     """float32 attention on the matrix cores' 32-bit instruction, the same bits for a token whether it comes alone or in a
-    prompt; None for head sizes other than 64 and 128 (and for rows that are not aligned), which the kernel for any shape serves."""
-    if q.dtype != torch.float32 or head_dim not in (64, 128) or q_stride % 4 or q.data_ptr() % 16:
+    prompt; None for what the kernel for any shape serves: head sizes other than 64 and 128, rows that are not aligned, pages
+    whose rows are wider than a head, and steps whose tokens are not laid out by sequences (single tokens, one a sequence, or
+    the token offsets of the sequences on host and device; within a sequence the tokens may come in any order)."""
+    T = ctx.tok_pos.numel()
+    if q.dtype != torch.float32 or head_dim not in (64, 128) or q_stride % 4 or q.data_ptr() % 16 or T == 0 or n_heads % n_kv_heads:
         return None
-    _dev(k_pool, v_pool, table, ctx.tok_pos)
-    _i32(table, "table"); _i32(ctx.tok_pos, "tok_pos")
-    _check_pools(k_pool, v_pool, n_kv_heads, head_dim, "attention")
-    _need(k_pool.dtype == torch.float32 and v_pool.dtype == torch.float32, "attention: q and cache types differ")
-    _need(n_heads % n_kv_heads == 0, "attention: heads must be a multiple of kv heads")
-    T, group = ctx.n_tokens, n_heads // n_kv_heads
-    _need(q.numel() >= (T - 1) * q_stride + n_heads * head_dim and q_stride >= n_heads * head_dim, "attention: q too small")
-    _need(table.dim() == 2 and table.shape[0] == ctx.batch and ctx.tok_pos.numel() == T, "attention: one table row a sequence, one position a token")
-    if ctx.is_decode:
-        _need(T == ctx.batch, "attention: one token a sequence")
-        cu, tiles = None, T * -(-group // 16)
+    shape = (n_kv_heads, PAGE_TOKENS * head_dim)
+    if not (k_pool.dtype == torch.float32 and v_pool is not None and v_pool.dtype == torch.float32 and v_pool.shape == k_pool.shape
+            and tuple(k_pool.shape[1:]) == shape and k_pool.is_contiguous() and v_pool.is_contiguous()
+            and (k_pool.data_ptr() | v_pool.data_ptr()) % 16 == 0):
+        return None
+    batch, cu = getattr(ctx, "batch", 0), None
+    if getattr(ctx, "is_decode", False):
+        if T != batch:
+            return None
     else:
-        cu = ctx.cu_dev
-        _need(cu is not None and cu.numel() == ctx.batch + 1, "attention: the step's token offsets are missing")
-        tiles = sum(-(-(b - a) * group // 16) for a, b in zip(ctx.cu_seqlens, ctx.cu_seqlens[1:]))
+        cu = getattr(ctx, "cu_dev", None)
+        if cu is None or cu.numel() != batch + 1 or len(ctx.cu_seqlens) != batch + 1 or ctx.cu_seqlens[-1] != T:
+            return None
+    tok_seq, group = getattr(ctx, "tok_seq", None), n_heads // n_kv_heads
+    if table.dim() != 2 or (tok_seq is None and table.shape[0] != batch):
+        return None
+    _dev(k_pool, v_pool, table, tok_seq, ctx.tok_pos, cu)
+    _i32(table, "table"); _i32(ctx.tok_pos, "tok_pos"); _i32(tok_seq, "tok_seq"); _i32(cu, "cu_dev")
+    _need(tok_seq is None or tok_seq.numel() == T, "attention: one sequence a token")
+    _need(q.is_cuda and q.numel() >= (T - 1) * q_stride + n_heads * head_dim and q_stride >= n_heads * head_dim, "attention: q too small")
+    tiles = T * -(-group // 16) if cu is None else sum(-(-(b - a) * group // 16) for a, b in zip(ctx.cu_seqlens, ctx.cu_seqlens[1:]))
     out = torch.empty((T, n_heads * head_dim), dtype=torch.float32, device=q.device)
-    _check(_lib().llogos_attention_f32(_p(out), _p(q), q_stride, _p(k_pool), _p(v_pool), _p(table), table.stride(0), _p(cu), _p(ctx.tok_pos),
-                                       ctx.batch, tiles, n_heads, n_kv_heads, head_dim, ctypes.c_float(scale), window, sinks, _stream()),
+    _check(_lib().llogos_attention_f32(_p(out), _p(q), q_stride, _p(k_pool), _p(v_pool), _p(table), table.stride(0), _p(cu), _p(tok_seq), _p(ctx.tok_pos),
+                                       batch, tiles, n_heads, n_kv_heads, head_dim, ctypes.c_float(scale), window, sinks, _stream()),
            "attention_f32")
     return out
 

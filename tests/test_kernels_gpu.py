@@ -476,6 +476,36 @@ def test_float32_attention_of_a_token_alone_and_in_a_prompt(nh, nkv, hd, window,
     _close(after[_t(~sees, torch.bool)], _np(out)[~sees], "float32")
 
 
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("window,sinks", [(0, 0), (70, 5)])
+def test_float32_attention_of_tokens_in_any_order(hd, window, sinks):
+    """Tokens of a sequence in any order of positions, single tokens of sequences in any order, steps of which nothing is known
+    but every token's sequence and position (tokens of the sequences mixed), pages whose rows are wider than a head."""
+    nh, nkv, rng = 6, 2, np.random.default_rng(hd)
+    lens, new = [200, 90, 3], [200, 33, 3]
+    c = _attention_case("float32", nh, nkv, hd, lens, new)
+    want = _plain_attention(c, nh, nkv, hd, window, sinks)
+    cu, T = np.concatenate([[0], np.cumsum(new)]), sum(new)
+    call = lambda rows, **kw: K.attention(
+        type("Ctx", (), dict(tok_seq=_t(c["tok_seq"][rows], torch.int32), tok_pos=_t(c["tok_pos"][rows], torch.int32), batch=3, n_tokens=len(rows), **kw))(),
+        c["q"][_t(rows, torch.int64)], c["stride"], c["kp"], c["vp"], c["table"], nh, nkv, hd, 1 / math.sqrt(hd), window, sinks)
+    shuffled = np.concatenate([rng.permutation(np.arange(a, b)) for a, b in zip(cu, cu[1:])])
+    _close(call(shuffled, is_decode=False, cu_seqlens=cu.tolist(), cu_dev=_t(cu, torch.int32)), want[shuffled], "float32")
+    mixed = rng.permutation(T)
+    _close(call(mixed, is_decode=False, cu_seqlens=None, cu_dev=None), want[mixed], "float32")
+    last = np.array([T - 1, 199, 232])
+    _close(call(last, is_decode=True, cu_seqlens=[0, 1, 2, 3], cu_dev=None), want[last], "float32")
+    if not window:                                                      # key pages of hd + 16 dimensions a row
+        kw_, vw = (torch.zeros((p.shape[0], nkv, 64 * (hd + 16)), device=DEV) for p in (c["kp"], c["vp"]))
+        ki, vi = _page_index(hd + 16)
+        kw_[:, :, ki[:, :hd].reshape(-1)] = c["kp"][:, :, c["ki"].reshape(-1)]
+        vw[:, :, vi[:, :hd].reshape(-1)] = c["vp"][:, :, c["vi"].reshape(-1)]
+        ctx = type("Ctx", (), dict(tok_seq=_t(c["tok_seq"], torch.int32), tok_pos=_t(c["tok_pos"], torch.int32), batch=3, n_tokens=T, is_decode=False,
+                                   cu_seqlens=cu.tolist(), cu_dev=_t(cu, torch.int32)))()
+        got = K.attention(ctx, c["q"], c["stride"], kw_, vw, c["table"], nh, nkv, hd, 1 / math.sqrt(hd))
+        _close(got.view(T, nh, -1)[:, :, :hd].reshape(T, nh * hd), want, "float32")
+
+
 @pytest.mark.parametrize("window,sinks", [(0, 0), (200, 70)])
 @pytest.mark.parametrize("nh,nkv,hd,batch,longest", [(8, 4, 128, 64, 700),      # one block a sequence, three pages a wave
                                                      (8, 4, 64, 70, 1500),       # batches beyond the captured sizes
