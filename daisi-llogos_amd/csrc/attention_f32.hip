@@ -10,7 +10,7 @@
 // depends on the query's position alone, not on how many waves share the pages, on how the tokens
 // were cut into steps or on what else is in the batch: single tokens and prompts run this kernel
 // with the same bits.  (A page of which a row sees no key leaves the row as it was: factors 1 and
-// 0.)
+// 0.)  A key whose weight is 0, unseen or underflowed, counts for nothing whatever its value is.
 //
 // Bound by the latency of a page's loads in single-token steps and by the matrix cores in prompts
 // (a page of 16 rows of 64 dimensions: 128 instructions, 4,096 clocks).  The kernel for any shape
@@ -121,8 +121,6 @@ __global__ __launch_bounds__(WAVES * 64) void attn_f32_kernel(
             l += __shfl_xor(l, 16, kWave);
             l += __shfl_xor(l, 32, kWave);
             // O^T = V^T . P^T; values behind the tile's latest position were never written
-            const bool edge = t0 + kPageTokens - 1 > early || (window > 0 && t0 < max(sinks, last - window + 1));
-            bool odd = false;                                    // a value that is no number, of a token that some row does not see
 #pragma unroll
             for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -132,30 +130,33 @@ __global__ __launch_bounds__(WAVES * 64) void attn_f32_kernel(
 #pragma unroll
                         for (int e = 0; e < 8; ++e) if (t0 + 16 * g + 8 * h + e > last) vv[e] = 0.f;
                     }
-                    if (edge) {
-#pragma unroll
-                        for (int e = 0; e < 8; ++e) odd |= !isfinite(vv[e]);
-                    }
 #pragma unroll
                     for (int e = 0; e < 8; ++e) o[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[e], s[2 * h + (e >> 2)][e & 3], o[d], 0, 0, 0);
                 }
-            if (edge && __any(odd)) {                            // a weight of 0 must not meet it: token by token, seen ones alone
+            // A weight of 0 (a key that the row does not see, or one whose weight underflows) must not meet a value that is no
+            // number, and every such meeting leaves a sum that is no number: then the page is added token by token without
+            // them, in the instruction's order (slot g of step j holds token 16 g + j), so that rows that do not see the value
+            // keep their bits.
+            bool odd = false;
+#pragma unroll
+            for (int d = 0; d < DB; ++d)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) odd |= !isfinite(o[d][c]);
+            if (__any(odd)) {
 #pragma unroll
                 for (int d = 0; d < DB; ++d) o[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int j = 0; j < 16; ++j)
 #pragma unroll 1
-                for (int u = 0; u < 4; ++u)
-#pragma unroll
-                    for (int rb = 0; rb < 4; ++rb)
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            const int t = 16 * u + 4 * rb + r;
-                            const float p = __shfl(s[rb][r], 16 * u + i, kWave);
-                            if (!key_visible(pos, t0 + t, window, sinks)) continue;
+                    for (int u = 0; u < 4; ++u) {
+                        const float p = __shfl(s[j >> 2][j & 3], 16 * u + i, kWave);
+                        if (p != 0.f) {
 #pragma unroll
                             for (int d = 0; d < DB; ++d)
 #pragma unroll
-                                for (int c = 0; c < 4; ++c) o[d][c] = fmaf(p, vp[page_value_offset(t, 16 * d + 4 * g + c)], o[d][c]);
+                                for (int c = 0; c < 4; ++c) o[d][c] = fmaf(p, vp[page_value_offset(16 * u + j, 16 * d + 4 * g + c)], o[d][c]);
                         }
+                    }
             }
         }
 #pragma unroll
@@ -173,7 +174,7 @@ __global__ __launch_bounds__(WAVES * 64) void attn_f32_kernel(
                 if (d < DB) {
                     const f32x4 v = sums[j][d][lane];
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) acc[w][r] = fmaf(v[r], add, acc[w][r] * keep);
+                    for (int r = 0; r < 4; ++r) acc[w][r] = fmaf(add == 0.f ? 0.f : v[r], add, (keep == 0.f ? 0.f : acc[w][r]) * keep);
                 }
             }
             den = fmaf(dens[j][i], add, den * keep);

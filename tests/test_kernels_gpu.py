@@ -473,7 +473,32 @@ def test_float32_attention_of_a_token_alone_and_in_a_prompt(nh, nkv, hd, window,
     sees = np.array([s == 0 and p >= 150 and (not window or p - 150 < window) for s, p in zip(c["tok_seq"], c["tok_pos"])])
     clean = torch.isfinite(after).all(1).cpu().numpy()
     assert np.array_equal(clean, ~sees)
-    _close(after[_t(~sees, torch.bool)], _np(out)[~sees], "float32")
+    assert torch.equal(after[_t(~sees, torch.bool)], out[_t(~sees, torch.bool)])
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("low", [(20,), tuple(range(64, 128)), tuple(range(0, 64)), (0, 70, 130, 190)])
+def test_float32_attention_of_keys_whose_weights_underflow(hd, low):
+    """Keys that a row sees with a weight that underflows to 0, alone in a page, a whole page of them before or behind the
+    others: their values, infinite or not a number, count for nothing, and the result is the bits of values of 0."""
+    nh, nkv, L = 4, 2, 200
+    c = _attention_case("float32", nh, nkv, hd, [L], [L])
+    c["q"][:, :nh * hd] = 1.0 + 0.1 * c["q"][:, :nh * hd].clamp(-1, 1)
+    c["kp"] *= 0.01
+    cu = np.array([0, L])
+    ctx = type("Ctx", (), dict(tok_seq=_t(c["tok_seq"], torch.int32), tok_pos=_t(c["tok_pos"], torch.int32), batch=1, n_tokens=L, is_decode=False,
+                               cu_seqlens=[0, L], cu_dev=_t(cu, torch.int32), max_context=L))()
+    call = lambda: K.attention(ctx, c["q"], c["stride"], c["kp"], c["vp"], c["table"], nh, nkv, hd, 1 / math.sqrt(hd))
+    rows = torch.tensor([t > max(low) if low[0] == 0 else True for t in range(L)], device=DEV)      # rows that see another key
+    outs = []
+    for value in (0.0, float("inf"), float("nan")):
+        for t in low:
+            page = int(c["table"][0, t // 64])
+            c["kp"][page][:, c["ki"][t % 64]] = -40.0                    # a score below -300 beside ones near 0
+            c["vp"][page][:, c["vi"][t % 64]] = value
+        outs.append(call())
+    assert torch.isfinite(outs[0]).all()
+    assert torch.equal(outs[1][rows], outs[0][rows]) and torch.equal(outs[2][rows], outs[0][rows])
 
 
 @pytest.mark.parametrize("hd", [64, 128])
