@@ -39,12 +39,24 @@ __global__ __launch_bounds__(WAVES * 64) void attn_f32_kernel(
     // which sequence this tile of rows belongs to; the tiles of late tokens, which have most pages, go first
     int seq = 0, first = 0, tokens = 1, tile = gridDim.x - 1 - blockIdx.x;
     if (cu) {
-        for (;; ++seq) {
-            first = cu[seq];
-            tokens = cu[seq + 1] - first;
-            const int tiles = (tokens * group + 15) / 16;
-            if (tile < tiles || seq + 1 >= batch) break;
-            tile -= tiles;
+        // (the lanes look at 64 sequences side by side: one after the other each costs a round trip to the cache)
+        for (int s0 = 0;; s0 += kWave) {
+            if (s0 >= batch) return;                             // (the grid has up to a tile a sequence more than there are)
+            const int lo = cu[min(s0 + lane, batch)], hi = cu[min(s0 + lane + 1, batch)];
+            const int tiles = ((hi - lo) * group + 15) / 16;
+            int upto = tiles;                                    // tiles of this sequence and the ones in front of it
+#pragma unroll
+            for (int o = 1; o < kWave; o <<= 1) { const int v = __shfl_up(upto, o, kWave); if (lane >= o) upto += v; }
+            const unsigned long long mine = __ballot(tile < upto);
+            if (mine) {
+                const int at = __ffsll(mine) - 1;
+                seq = s0 + at;
+                first = __builtin_amdgcn_readlane(lo, at);
+                tokens = __builtin_amdgcn_readlane(hi, at) - first;
+                tile -= __builtin_amdgcn_readlane(upto - tiles, at);
+                break;
+            }
+            tile -= __builtin_amdgcn_readlane(upto, kWave - 1);
         }
     } else {
         const int tiles = (group + 15) / 16;
@@ -196,22 +208,28 @@ __global__ __launch_bounds__(WAVES * 64) void attn_f32_kernel(
     }
 }
 
-// n_tiles: tiles of 16 (token, head of the group) rows over all sequences; cu null: every sequence brings one token
+// n_tiles: tiles of 16 (token, head of the group) rows over all sequences, or more; pages: the most a sequence has (0: unknown); cu null:
+// every sequence brings one token
 LLOGOS_EXPORT int llogos_attention_f32(float* out, const float* q, int q_stride, const float* k_pool, const float* v_pool,
                                        const int* table, int table_stride, const int* cu, const int* tok_seq, const int* tok_pos,
-                                       int batch, int n_tiles, int n_heads, int n_kv_heads, int head_dim, float scale, int window, int sinks, hipStream_t stream) {
+                                       int batch, int n_tiles, int pages, int n_heads, int n_kv_heads, int head_dim, float scale, int window, int sinks,
+                                       hipStream_t stream) {
     if (batch <= 0 || n_tiles <= 0 || n_kv_heads <= 0 || n_heads <= 0 || n_heads % n_kv_heads != 0 || window < 0 || sinks < 0) return LLOGOS_BAD_ARGUMENT;
     if ((head_dim != 64 && head_dim != 128) || (q_stride & 3) || (((uintptr_t)q | (uintptr_t)out) & 15)) return LLOGOS_UNSUPPORTED;
     const int group = n_heads / n_kv_heads;
     PagedKV cache{table, table_stride, n_kv_heads, head_dim};
     const dim3 grid(n_tiles, n_kv_heads);
     // Waves that share a tile's pages: many where there are few tiles (a single-token step: as many as LDS holds results of), few where
-    // the tiles alone fill the GPU.
-    const bool few = (long long)n_tiles * n_kv_heads < 1024;
+    // the tiles alone fill the GPU, and no more than there are pages: a wave without one still costs its block's start and its share
+    // of LDS (64 sequences of 40 tokens, 32 heads of 128 by themselves: 62 us with four waves, 26 with one; 42 in the kernel for any shape).
+    int waves = (long long)n_tiles * n_kv_heads >= 1024 ? 4 : (head_dim == 64 ? 16 : 8);
+    while (waves > 1 && pages > 0 && waves / 2 >= pages) waves /= 2;
 #define ATTN(HD, W) attn_f32_kernel<HD, W><<<grid, W * 64, 0, stream>>>(out, q, q_stride, k_pool, v_pool, cache, cu, batch, tok_seq, tok_pos, \
-                                                                        n_heads, group, scale, window, sinks)
-    if (head_dim == 64) { if (few) ATTN(64, 16); else ATTN(64, 4); }
-    else { if (few) ATTN(128, 8); else ATTN(128, 4); }
+                                                                        n_heads, group, scale, window, sinks); break
+#define BY_WAVES(HD) switch (waves) { case 1: ATTN(HD, 1); case 2: ATTN(HD, 2); case 4: ATTN(HD, 4); case 8: ATTN(HD, 8); default: ATTN(64, 16); }
+    if (head_dim == 64) BY_WAVES(64)
+    else BY_WAVES(128)
+#undef BY_WAVES
 #undef ATTN
     return LLOGOS_LAUNCH_CHECK();
 }

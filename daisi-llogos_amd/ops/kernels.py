@@ -2382,11 +2382,11 @@ def attention_f32(ctx, q: torch.Tensor, q_stride: int, k_pool: torch.Tensor, v_p
     _i32(table, "table"); _i32(ctx.tok_pos, "tok_pos"); _i32(tok_seq, "tok_seq"); _i32(cu, "cu_dev")
     _need(tok_seq is None or tok_seq.numel() == T, "attention: one sequence a token")
     _need(q.is_cuda and q.numel() >= (T - 1) * q_stride + n_heads * head_dim and q_stride >= n_heads * head_dim, "attention: q too small")
-    tiles = T * -(-group // 16) if cu is None else sum(-(-(b - a) * group // 16) for a, b in zip(ctx.cu_seqlens, ctx.cu_seqlens[1:]))
+    tiles = T * -(-group // 16) if cu is None else T * group // 16 + batch           # (at most; a sequence's last tile may be part full)
     out = torch.empty((T, n_heads * head_dim), dtype=torch.float32, device=q.device)
     _check(_lib().llogos_attention_f32(_p(out), _p(q), q_stride, _p(k_pool), _p(v_pool), _p(table), table.stride(0), _p(cu), _p(tok_seq), _p(ctx.tok_pos),
-                                       batch, tiles, n_heads, n_kv_heads, head_dim, ctypes.c_float(scale), window, sinks, _stream()),
-           "attention_f32")
+                                       batch, tiles, -(-getattr(ctx, "max_context", 0) // PAGE_TOKENS), n_heads, n_kv_heads, head_dim,
+                                       ctypes.c_float(scale), window, sinks, _stream()), "attention_f32")
     return out
 
 

@@ -477,6 +477,28 @@ def test_float32_attention_of_a_token_alone_and_in_a_prompt(nh, nkv, hd, window,
 
 
 @pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("longest", [3, 64, 65, 200, 500, 1100])
+def test_float32_attention_with_waves_for_the_pages_there_are(hd, longest):
+    """One to sixteen waves a tile by the most pages a sequence has, and more sequences than a wave has lanes, some without a
+    token: the bits of the form that knows nothing of the pages."""
+    nh, nkv, rng = 3, 1, np.random.default_rng(longest)
+    new = [int(n) for n in rng.integers(0, 4, 130)]
+    lens = [n + int(rng.integers(0, 30)) if n else 0 for n in new]
+    lens[70], new[70] = longest, 2
+    c = _attention_case("float32", nh, nkv, hd, [max(l, 1) for l in lens], new)
+    cu = np.concatenate([[0], np.cumsum(new)])
+    pos = np.concatenate([np.arange(l - n, l) for l, n in zip(lens, new)])
+    ctx = lambda **kw: type("Ctx", (), dict(tok_seq=_t(c["tok_seq"], torch.int32), tok_pos=_t(pos, torch.int32), batch=130, n_tokens=sum(new), is_decode=False,
+                                            cu_seqlens=cu.tolist(), cu_dev=_t(cu, torch.int32), **kw))()
+    call = lambda x: K.attention_f32(x, c["q"], c["stride"], c["kp"], c["vp"], c["table"], nh, nkv, hd, 1 / math.sqrt(hd))
+    out = call(ctx(max_context=max(lens)))
+    assert torch.equal(out, call(ctx()))
+    want = K.attention_generic(c["q"], c["stride"], c["kp"], c["vp"], c["table"], _t(c["tok_seq"], torch.int32), _t(pos, torch.int32), nh, nkv, hd,
+                               1 / math.sqrt(hd))
+    _close(out, _np(want), "float32")
+
+
+@pytest.mark.parametrize("hd", [64, 128])
 @pytest.mark.parametrize("low", [(20,), tuple(range(64, 128)), tuple(range(0, 64)), (0, 70, 130, 190)])
 def test_float32_attention_of_keys_whose_weights_underflow(hd, low):
     """Keys that a row sees with a weight that underflows to 0, alone in a page, a whole page of them before or behind the
