@@ -12,10 +12,10 @@
 // So a row's result is the same bits alone and in any batch, and the rounding error of a sum over
 // thousands of k grows with its blocks (16 + 16 + K / 256 additions deep) and not with K.
 //
-// Few rows (gemm_f32_rows_kernel): bound by reading w once.  A block owns 16 or 32 rows of w and
-// all of k; its waves take 256 k in turn straight from memory, a mid each, and LDS adds the mids
-// in order.  Many rows (gemm_f32_tiles_kernel): bound by the matrix cores (157 TFLOP/s); tiles of
-// 128 x 64, 64 x 64 or 64 x 32 through two LDS buffers of 32 k.
+// One to four rows (gemm_f32_lanes_kernel) and few rows (gemm_f32_rows_kernel): bound by reading w once.
+// In the second a block owns 16 or 32 rows of w and all of k; its waves take 256 k in turn straight from
+// memory, a mid each, and LDS adds the mids in order.  Many rows (gemm_f32_tiles_kernel): bound by the
+// matrix cores (157 TFLOP/s); tiles of 128 x 64, 64 x 64 or 64 x 32 through two LDS buffers of 32 k.
 // Measured (us; before: plain FMAs in tiles of 64 x 64, up to 32 rows a wave for a few columns).  705 rows of the 1B
 // sizes: gate/up [16384, 2048] 1,507 -> 459 (103 TFLOP/s), o [2048, 2048] about 390 -> 80, down [2048, 8192] about
 // 1,510 -> 305, q/k/v [3072, 2048] 448 -> 115.  2 rows: gate/up 28.3 -> 28.6 (4.7 TB/s), head [128256, 2048] 209 -> 180
@@ -130,6 +130,56 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_f32_rows_kernel(
         if (tile >= TILES) continue;
         const int m = m0 + 16 * (tile % MT) + i, n = n0 + 16 * (tile / MT) + 4 * g;
         if (m < M) store4(out, bias, total[o], m, n, N, ldo, vec_out != 0);
+    }
+}
+
+// The fewest rows by plain multiply-adds: a wave takes COLS rows of w, a lane 16 consecutive k of them and of every row of a at a
+// time; it chains a part in the order above, sixteen neighbouring lanes hold the parts of a mid, and the mids are added in
+// order.  No wave waits for another, and a matrix of few rows has a wave for each where the kernel above has one block for 16:
+// 1 row, us, that kernel -> this one: [2048, 8192] 27.3 -> 15.6 (4.3 TB/s), [4096, 14336] 49.7 -> 40.4 (5.8), [2048, 2048] 8.5 -> 5.8,
+// [16, 16384] 42.9 -> 14.4, [50000, 768] 40.0 -> 26.8, [1000, 1001] 14.4 -> 5.4.
+template <int MR, int COLS, bool VEC>
+__global__ __launch_bounds__(256) void gemm_f32_lanes_kernel(
+        float* __restrict__ out, const float* __restrict__ a, const float* __restrict__ w,
+        const float* __restrict__ bias, int M, int N, int K, int lda, int ldo) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n0 = (blockIdx.x * 4 + wave) * COLS, m0 = blockIdx.y * MR;
+    if (n0 >= N) return;
+    float total[MR];                                            // lane c: the totals of column n0 + c
+#pragma unroll
+    for (int m = 0; m < MR; ++m) total[m] = 0.f;
+    for (int k0 = 0; k0 < K; k0 += 1024) {
+        f32x4 av[MR][4];
+#pragma unroll
+        for (int m = 0; m < MR; ++m)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) av[m][g] = load4<VEC>(a + (size_t)min(m0 + m, M - 1) * lda, k0 + 16 * lane + 4 * g, K);
+#pragma unroll 1
+        for (int c = 0; c < COLS; ++c) {
+            f32x4 wv[4];
+#pragma unroll
+            for (int g = 0; g < 4; ++g) wv[g] = load4<VEC>(w + (size_t)min(n0 + c, N - 1) * K, k0 + 16 * lane + 4 * g, K);
+#pragma unroll
+            for (int m = 0; m < MR; ++m) {
+                float part = 0.f, mid = 0.f, sum = total[m];
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) part = fmaf(wv[g][e], av[m][g][e], part);
+#pragma unroll
+                for (int j = 0; j < 16; ++j) mid += __shfl(part, (lane & 48) + j, kWave);
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const float m4 = __shfl(mid, 16 * g, kWave);
+                    if (k0 + 256 * g < K) sum += m4;
+                }
+                total[m] = lane == c ? sum : total[m];
+            }
+        }
+    }
+    if (lane < COLS && n0 + lane < N) {
+#pragma unroll
+        for (int m = 0; m < MR; ++m)
+            if (m0 + m < M) out[(size_t)(m0 + m) * ldo + n0 + lane] = bias ? total[m] + bias[n0 + lane] : total[m];
     }
 }
 
@@ -252,6 +302,19 @@ double rows_cost(double M, double N, double K, int mt, int ns) {
     return blocks * (ns + mt) * 64 * K / (ns == 2 ? 5.3e12 : mt == 4 ? 6.7e12 : 9.5e12) / spread + 4e-6;
 }
 
+// Rows of w a wave of the lanes' kernel takes, 0 where the few-row kernel is ahead: matrices whose blocks of 16 rows leave units idle
+// or whose k gives those blocks' waves little to do (1 row, us, few-row kernel and this one: [6144, 4096] 30 and 22, [8192, 8192] 60 and
+// 58, [16384, 2048] 27.3 and 26.7, [12288, 4096] 44 and 46, [128256, 2048] 177 and 196; 2 rows: [8192, 8192] 61 and 70, [24576, 1024] 24
+// and 22).  Rows that are not aligned are read value by value, which the few-row kernel's lanes do at sixteen places of a line
+// each; there it is ahead from 5 rows on ([50000, 769], 1 row 127 and 87, 4 rows 132 and 119; [3000, 4099] 39 and 41).
+int lanes_cols(int M, int N, int K, bool vec) {
+    if (!vec) return M > 4 ? 0 : (N <= 2048 ? 1 : (N > 16384 ? 8 : (K <= 1024 ? 2 : 0)));
+    if (M > 2) return 0;
+    if (N <= 3584 || (M == 1 && K <= 1024)) return 1;
+    if (N <= (M == 1 ? 8192 : 6144)) return 2;
+    return (M == 1 && N <= 16384 && K <= 2048) || (M == 2 && K <= 1024) ? 4 : 0;
+}
+
 }  // namespace
 
 #define ROWS(W, MT, NS) do { \
@@ -259,6 +322,8 @@ double rows_cost(double M, double N, double K, int mt, int ns) {
         if (vec) gemm_f32_rows_kernel<W, MT, NS, true><<<grid, W * 64, 0, stream>>>(out, a, w, bias, M, N, K, lda, ldo, vec_out); \
         else gemm_f32_rows_kernel<W, MT, NS, false><<<grid, W * 64, 0, stream>>>(out, a, w, bias, M, N, K, lda, ldo, vec_out); \
     } while (0)
+#define LANES(MR, COLS, VEC) gemm_f32_lanes_kernel<MR, COLS, VEC><<<dim3((N + 4 * COLS - 1) / (4 * COLS), (M + MR - 1) / MR), 256, 0, stream>>>( \
+        out, a, w, bias, M, N, K, lda, ldo)
 #define TILES(TM, TN) do { \
         const int mt = (M + TM - 1) / TM, nt = (N + TN - 1) / TN; \
         if (vec) gemm_f32_tiles_kernel<TM, TN, true><<<mt * nt, 256, 0, stream>>>(out, a, w, bias, M, N, K, lda, ldo, vec_out, mt, nt); \
@@ -266,12 +331,14 @@ double rows_cost(double M, double N, double K, int mt, int ns) {
     } while (0)
 
 // form: 0 chosen by the costs above; 1 to 4 the few-row kernel with 16, 32, 64 rows of a or 64 rows of a and 32 of w a block; 5 to 7 tiles of
-// 64 x 32, 64 x 64, 128 x 64
+// 64 x 32, 64 x 64, 128 x 64; 8 the lanes' kernel
 LLOGOS_EXPORT int llogos_gemm_f32(float* out, const float* a, const float* w, const float* bias,
                                   int M, int N, int K, int lda, int ldo, int form, hipStream_t stream) {
-    if (M <= 0 || N <= 0 || K <= 0 || lda < K || ldo < N || form < 0 || form > 7) return LLOGOS_BAD_ARGUMENT;
+    if (M <= 0 || N <= 0 || K <= 0 || lda < K || ldo < N || form < 0 || form > 8) return LLOGOS_BAD_ARGUMENT;
     const bool vec = (K & 3) == 0 && (lda & 3) == 0 && (((uintptr_t)a | (uintptr_t)w) & 15) == 0;
     const int vec_out = (ldo & 3) == 0 && ((uintptr_t)out & 15) == 0;
+    const int cols = lanes_cols(M, N, K, vec);
+    if (form == 0 && cols) form = 8;
     if (form == 0) {
         const double cost[8] = {0, 0, rows_cost(M, N, K, 2, 1), rows_cost(M, N, K, 4, 1), rows_cost(M, N, K, 4, 2),
                                 tiles_cost(M, N, K, 64, 32), tiles_cost(M, N, K, 64, 64), tiles_cost(M, N, K, 128, 64)};
@@ -287,7 +354,14 @@ LLOGOS_EXPORT int llogos_gemm_f32(float* out, const float* a, const float* w, co
         case 4: ROWS(8, 4, 2); break;
         case 5: TILES(64, 32); break;
         case 6: TILES(64, 64); break;
-        default: TILES(128, 64); break;
+        case 7: TILES(128, 64); break;
+        default:
+            if (vec && M == 1) { if (cols == 4) LANES(1, 4, true); else if (cols == 2) LANES(1, 2, true); else LANES(1, 1, true); }
+            else if (vec) { if (cols == 4) LANES(2, 4, true); else if (cols == 2) LANES(2, 2, true); else LANES(2, 1, true); }
+            else if (M == 1) { if (cols == 8) LANES(1, 8, false); else if (cols == 2) LANES(1, 2, false); else LANES(1, 1, false); }
+            else if (M == 2) { if (cols == 8) LANES(2, 8, false); else if (cols == 2) LANES(2, 2, false); else LANES(2, 1, false); }
+            else { if (cols == 8) LANES(4, 8, false); else if (cols == 2) LANES(4, 2, false); else LANES(4, 1, false); }
+            break;
     }
     return LLOGOS_LAUNCH_CHECK();
 }

@@ -281,6 +281,21 @@ def test_float32_product_of_few_rows_is_the_tiled_product_bit_for_bit(N, K_):
     assert torch.equal(few, many[:5])
 
 
+@pytest.mark.parametrize("M", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("N,K_", [(1, 1), (5, 1024), (130, 1040), (3585, 2052), (6145, 1028), (8193, 1028), (40, 16), (7, 1025), (2049, 515), (16387, 33)])
+def test_float32_products_of_the_fewest_rows(M, N, K_, monkeypatch):
+    """The lanes' kernel, at the sizes where it takes one, two, four or eight rows of w a wave and where the few-row kernel
+    serves, with k around its lanes' and waves' shares: the few-row kernel's bits."""
+    rng = np.random.default_rng(N)
+    a, w, b = _t(rng.standard_normal((M, K_))), _t(rng.standard_normal((N, K_)) * 0.05), _t(rng.standard_normal(N))
+    got = K.gemm_generic(a, w, b, torch.float32)
+    for form in (8, 1):
+        monkeypatch.setattr(K, "F32_FORM", form)
+        out = torch.full((M, N + 1), 7.0, device=DEV)
+        assert torch.equal(K.gemm_generic(a, w, b, torch.float32, out=out[:, :N]), got), form
+        assert (out[:, N:] == 7.0).all()
+
+
 def test_the_generic_entry_takes_float32_throughout():
     """The library's entry for any types hands float32 operands on to the float32 product: the same bits, with and without a
     bias, into rows of a wider result."""
@@ -296,7 +311,7 @@ def test_the_generic_entry_takes_float32_throughout():
 
 @pytest.mark.parametrize("M,N,K_", [(1, 16, 16), (17, 33, 40), (33, 70, 272), (64, 129, 4112), (65, 31, 255), (130, 66, 2049), (200, 250, 513)])
 def test_float32_product_gives_the_same_bits_in_every_form(M, N, K_, monkeypatch):
-    """The forms of the float32 product (few rows in three heights of blocks, tiles in three sizes) at remainders of
+    """The forms of the float32 product (few rows in three heights of blocks, tiles in three sizes, pairs of rows) at remainders of
     tiles, of blocks of 16 and of 256 k and of 16 bytes: one result, and right (a sum is at most 16 + 16 + K / 256
     additions deep)."""
     rng = np.random.default_rng(M)
@@ -304,7 +319,7 @@ def test_float32_product_gives_the_same_bits_in_every_form(M, N, K_, monkeypatch
     chosen = K.gemm_generic(a, w, b, torch.float32)
     bound = 2.0 ** -24 * (34 + K_ / 256) * (_np(a.abs()) @ _np(w.abs()).T + np.abs(_np(b)))
     assert (np.abs(_np(chosen) - pm.linear(_np(a), _np(w), _np(b))) <= bound).all()
-    for form in range(1, 8):
+    for form in range(1, 9):
         monkeypatch.setattr(K, "F32_FORM", form)
         out = torch.full((M, N + 3), 7.0, device=DEV)
         assert torch.equal(K.gemm_generic(a, w, b, torch.float32, out=out[:, :N]), chosen), form
