@@ -256,18 +256,19 @@ def test_prompt_products_of_random_shapes_on_packed_weights():
 
 
 @pytest.mark.parametrize("N,K_", [(70, 16), (2048, 8192), (17000, 1000), (33000, 2049), (66000, 530), (5, 4099), (300, 7)])
-def test_float32_product_of_few_rows_is_the_tiled_product_bit_for_bit(N, K_):
-    """Up to 32 rows in float32 go to a kernel of their own (a wave a few columns, the rows of a in
-    registers); it adds in the order of the tiled kernel, so a row's result is the same bits
-    whichever of the two a step's row count selects, alone or beside others, and right."""
+def test_float32_product_of_few_rows_is_the_tiled_product_bit_for_bit(N, K_, monkeypatch):
+    """Few rows in float32 go to kernels of their own; they add in the order of the tiled kernel, so a row's
+    result is the same bits whichever of them a step's row count selects, alone or beside others, and right."""
     rng = np.random.default_rng(N)
     a = _t(rng.standard_normal((40, K_)))
     w = _t(rng.standard_normal((N, K_)) * 0.05)
     b = _t(rng.standard_normal(N))
-    tiled = K.gemm_generic(a, w, b, torch.float32)                         # 40 rows: the tiled kernel
+    monkeypatch.setattr(K, "F32_FORM", 6)                                  # the tiled kernel, whatever 40 rows would choose
+    tiled = K.gemm_generic(a, w, b, torch.float32)
+    monkeypatch.setattr(K, "F32_FORM", 0)
     want = pm.linear(_np(a), _np(w), _np(b))
     assert np.abs(_np(tiled) - want).max() <= 2e-6 * max(1.0, np.abs(want).max()) * math.sqrt(K_)
-    for M in (1, 2, 3, 4, 7, 8, 9, 16, 31, 32):
+    for M in (1, 2, 3, 4, 7, 8, 9, 16, 31, 32, 40):
         few = K.gemm_generic(a[:M], w, b, torch.float32)
         assert torch.equal(few, tiled[:M]), (M, N, K_, (few - tiled[:M]).abs().max().item())
     # several tiles of rows: the same bits again
@@ -511,6 +512,44 @@ def test_float32_attention_with_waves_for_the_pages_there_are(hd, longest):
     want = K.attention_generic(c["q"], c["stride"], c["kp"], c["vp"], c["table"], _t(c["tok_seq"], torch.int32), _t(pos, torch.int32), nh, nkv, hd,
                                1 / math.sqrt(hd))
     _close(out, _np(want), "float32")
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+def test_float32_attention_of_a_prompt_of_many_tiles(hd):
+    """600 tokens of 32 heads are 1,200 blocks of four waves: the bits of tokens that come alone, with sixteen waves a tile
+    or eight."""
+    nh, L = 32, 600
+    c = _attention_case("float32", nh, nh, hd, [L], [L])
+    pos = _t(c["tok_pos"], torch.int32)
+    call = lambda x, q: K.attention_f32(x, q, c["stride"], c["kp"], c["vp"], c["table"], nh, nh, hd, 1 / math.sqrt(hd))
+    out = call(type("Ctx", (), dict(tok_pos=pos, is_decode=False, batch=1, n_tokens=L, cu_seqlens=[0, L], cu_dev=_t([0, L], torch.int32), max_context=L))(), c["q"])
+    for t in (0, 63, 64, 127, 255, 256, 511, 598, 599):
+        one = type("Ctx", (), dict(tok_pos=pos[t:t + 1], is_decode=True, batch=1, n_tokens=1, max_context=L))()
+        assert torch.equal(call(one, c["q"][t:t + 1])[0], out[t]), t
+
+
+@pytest.mark.parametrize("types", [("float32", "float32", "float32"), ("float32", "bfloat16", "float32"), ("float32", "bfloat16", "bfloat16"),
+                                   ("bfloat16", "bfloat16", "bfloat16"), ("bfloat16", "bfloat16", "float32")])
+@pytest.mark.parametrize("T,N,K_,odd", [(1, 1, 1, 0), (17, 5, 3, 0), (65, 64, 256, 0), (64, 66, 260, 0), (70, 129, 36, 1), (130, 62, 33, 1), (3, 200, 512, 4)])
+def test_products_of_heads(T, N, K_, odd, types):
+    """One product a head: k below, at and beyond the kernel's blocks of 32, heights and row counts around its tiles of 64, rows
+    and heads that begin anywhere (odd strides: value by value), with and without the gate; what lies between the heads'
+    results stays.  A sum is K products deep; bfloat16 results round once more."""
+    rng, Hn = np.random.default_rng(K_), 3
+    ta, tw, to = (DT[t] for t in types)
+    wide = _t(rng.standard_normal((T, Hn, K_ + odd)), ta)
+    a, w = wide[:, :, :K_], _t(rng.standard_normal((Hn, N, K_)), tw)
+    logits = _t(rng.standard_normal((T, Hn + 2)))
+    plain = np.einsum("thk,hnk->thn", _np(a), _np(w))
+    deep = np.einsum("thk,hnk->thn", np.abs(_np(a)), np.abs(_np(w))) * (K_ + 8) * 2.0 ** -24
+    for gate in (None, logits):
+        buf = torch.full((T, Hn, N + odd), 7.0, dtype=to, device=DEV)
+        K.head_products(a, w, buf[:, :, :N], gate=gate)
+        factor = 1.0 if gate is None else 1 / (1 + np.exp(-_np(gate)[:, :Hn, None]))
+        want = plain * factor
+        bound = deep * factor + np.abs(want) * (2.0 ** -8 if types[2] == "bfloat16" else 2.0 ** -20) + 1e-30
+        assert (np.abs(_np(buf[:, :, :N]) - want) <= bound).all()
+        assert (buf[:, :, N:] == 7.0).all()
 
 
 @pytest.mark.parametrize("hd", [64, 128])
