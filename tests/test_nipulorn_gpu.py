@@ -462,6 +462,32 @@ def test_recurrence_of_heads_of_64_channels(heads, lens, segments, monkeypatch):
             assert torch.equal(single, y[rows]), t
 
 
+@pytest.mark.parametrize("out", ["float32", "bfloat16"])
+@pytest.mark.parametrize("lens,segments", [([1, 1, 1], 1), ([9, 20], 1), ([30, 50], 3)])
+def test_recurrence_of_partial_sums(lens, segments, out, monkeypatch):
+    """Inputs as the partial sums of products split along k, three of r, k, v and the gate and two of the decay: the bits of
+    their sums taken beforehand in the same order, for single tokens, whole prompts and segments; bfloat16 results are the float32
+    ones rounded."""
+    monkeypatch.setattr(K, "SCAN_SEGMENTS", segments)
+    heads, T, rng = 3, sum(lens), np.random.default_rng(8)
+    f, _, _ = _recurrence_case(lens, heads, 9)
+    split = {n: torch.tensor(rng.standard_normal((2 if n == "d" else 3, T, heads * 64)), dtype=torch.float32, device=DEV) for n in ("r", "k", "v", "d", "gate")}
+    cu = np.concatenate([[0], np.cumsum(lens)]).tolist()
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    ctx = type("Ctx", (), dict(n_tokens=T, batch=len(lens), slots=i32(range(1, len(lens) + 1)), cu_seqlens=cu, is_decode=max(lens) == 1,
+                               cu_dev=None if max(lens) == 1 else i32(cu)))()
+    scan = lambda x, state, dtype: K.wkv_scan(ctx, x["r"], x["k"], x["v"], x["d"], x["gate"], f["w0"], f["u"], f["g"], 1e-5, state, heads, 64, f["h"], dtype)
+    summed = {}
+    for n, t in split.items():
+        summed[n] = t[0].clone()
+        for part in t[1:]:
+            summed[n] += part
+    states = [f["state"].clone(), f["state"].clone()]
+    y = scan(split, states[0], torch.float32 if out == "float32" else torch.bfloat16)
+    want = scan(summed, states[1], torch.float32)
+    assert torch.equal(y, want.to(y.dtype)) and torch.equal(states[0], states[1]) and torch.isfinite(want).all()
+
+
 @pytest.mark.parametrize("segments", [1, 3])
 def test_recurrence_with_sequences_that_bring_no_token(segments, monkeypatch):
     """Sequences without a token in the step, first, in the middle and last: their states stay, and nothing in front of the
@@ -505,10 +531,9 @@ def test_long_steps_of_convolution_shift_and_activation(taps, out):
                                tok_pos=i32(np.concatenate([np.arange(s, s + n) for s, n in zip(starts, counts)])), cu_dev=i32(cu), is_decode=False))()
     dtype = torch.float32 if out == "float32" else torch.bfloat16
     tol = 2e-6 if out == "float32" else 8e-3
-    got = _np(K.causal_conv(ctx, h, w, state, dtype)) if taps > 1 else None
+    got = _np(K.causal_conv(ctx, h, w, state, dtype))
     want = np.concatenate([pn.input_convolution(x, _np(w))[s:] for x, s in zip(whole, starts)])
-    if taps > 1:
-        assert np.abs(got - want).max() <= tol * taps * np.abs(want).max()
+    assert np.abs(got - want).max() <= tol * taps * np.abs(want).max()
     if taps == 4:
         mu = torch.tensor(rng.uniform(0, 1, (3, W)), dtype=torch.float32, device=DEV)
         prev = torch.tensor(np.stack([np.zeros(W, np.float32)] + [x[s - 1] if s else np.zeros(W, np.float32) for x, s in zip(whole, starts)]), device=DEV)
