@@ -472,7 +472,7 @@ __global__ void wkv_scan_kernel(TO* __restrict__ y, const float* __restrict__ r,
             if (active && MODE == 1) seg_S[m] = s[m];
             if (keeps_decay) seg_P[m] = pw[m];
         }
-    if (MODE != 1 && head == 0 && blockIdx.z == 0 && h_in) {
+    if (MODE != 1 && head == 0 && blockIdx.z == 0 && h_in && count0 > 0) {      // (a sequence that brings no token keeps its row)
         const float* last = h_in + (size_t)(first0 + count0 - 1) * W;
         for (int c = tid; c < W; c += nthreads) row[prev_offset + c] = last[c];
     }

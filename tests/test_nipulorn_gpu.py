@@ -488,11 +488,13 @@ def test_recurrence_of_partial_sums(lens, segments, out, monkeypatch):
     assert torch.equal(y, want.to(y.dtype)) and torch.equal(states[0], states[1]) and torch.isfinite(want).all()
 
 
-@pytest.mark.parametrize("segments", [1, 3])
-def test_recurrence_with_sequences_that_bring_no_token(segments, monkeypatch):
+@pytest.mark.parametrize("segments,rows", [(1, 0), (3, 0), (1, 4), (3, 4), (1, 16), (3, 16)])
+def test_recurrence_with_sequences_that_bring_no_token(segments, rows, monkeypatch):
     """Sequences without a token in the step, first, in the middle and last: their states stay, and nothing in front of the
-    step's rows or behind them is read (it would be NaN); the others get what they get without them."""
+    step's rows or behind them is read (it would be NaN); the others get what they get without them.  In the kernel with a wave
+    a head, and (rows of the state a thread) in the one with a block a head."""
     monkeypatch.setattr(K, "SCAN_SEGMENTS", segments)
+    monkeypatch.setattr(K, "SCAN_ROWS", rows)
     lens, heads = [0, 9, 0, 20, 0], 3
     f, _, _ = _recurrence_case([0, 9, 0, 20, 0], heads, 6)
     for name in ("r", "k", "v", "d", "gate", "h"):
