@@ -519,7 +519,8 @@ def wkv_scan(ctx, r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, d: torch.Te
     _need(6 * dim * 4 <= 65536, f"wkv_scan: head size {dim} is too large")
     y = torch.empty((ctx.n_tokens, HD), dtype=out_dtype, device=r.device)
     longest = None if ctx.is_decode else max(ctx.cu_seqlens[i + 1] - ctx.cu_seqlens[i] for i in range(ctx.batch))
-    if dim == 64 and state.stride(0) % 4 == 0 and state.data_ptr() % 16 == 0 and not (SCAN_ROWS or SCAN_COLUMN_BLOCKS):
+    if (dim == 64 and state.stride(0) % 4 == 0 and state.data_ptr() % 16 == 0 and not (SCAN_ROWS or SCAN_COLUMN_BLOCKS)
+            and wave_scan_serves(ctx.batch, n_heads, longest)):
         n_seg = wave_scan_segments(ctx.batch, n_heads, longest)
         seg_len, seg_state, seg_decay = 0, None, None
         if n_seg > 1:
@@ -551,22 +552,34 @@ SCAN_SEGMENTS = 0            # 0: chosen by the step; 1, 2, 3, ... force the num
 SCAN_ROWS = 0                # 0: chosen by the step; 4 or 16 force the rows of the state a thread (tests)
 
 
+def wave_scan_serves(batch: int, n_heads: int, longest: Optional[int], n_cus: Optional[int] = None) -> bool:
+    """Whether heads of 64 channels go to the recurrence with a wave a head, rather than the one with a block a head.  That one
+    shares a token's chain of work out over a block's waves, which tells where every head has a compute unit of its own and
+    prompts are too short for segments (us, block a head and wave a head; 64 heads: 3 tokens 7.1 / 8.7, 16 13.1 / 15.5, 40 25.6 /
+    37, 64 24.6 / 30.8, 100 34.6 / 35.2, 128 41.4 / 36.8; eight prompts of 20, 32 heads 17.2 / 21.7, 40 heads 30.5 / 21.8; single
+    tokens 6.3 / 4.5)."""
+    return bool(SCAN_SEGMENTS) or longest is None or longest >= 96 or batch * n_heads > (n_cus or compute_units())
+
+
 def wave_scan_segments(batch: int, n_heads: int, longest: Optional[int], n_cus: Optional[int] = None) -> int:
     """Segments that the prompts of a step are cut into by the recurrence with a wave a head: as many as bring the waves
-    to two a SIMD, of at least 16 tokens.  A segment costs more than half of its tokens' time again for its end state, but a
-    wave alone on its SIMD issues at half the rate and waits for every token's chain: 64 heads, one prompt of 127 tokens
-    whole 98 us, in 8 segments 39; of 2,048 1,505 whole, 178 in 16, 158 in 32; eight of 250 to 600 470 whole, 281 in 4."""
+    to two a SIMD, of 16 tokens (of prompts below 96 of at least 16).  A segment costs more than half of its tokens' time
+    again for its end state, but a wave alone on its SIMD issues at half the rate and waits for every token's chain: 64 heads,
+    one prompt of 100 tokens whole 80 us, in segments of 24 41, of 16 35, of 8 31; of 127 whole 98, in 8 37; of 2,048 1,505 whole,
+    178 in 16, 158 in 32; eight of 250 to 600 470 whole, 281 in 4."""
     if longest is None:
         return 1
     if SCAN_SEGMENTS:
         return SCAN_SEGMENTS
-    return max(1, min(32, longest // 16, -(-(8 * (n_cus or compute_units())) // max(1, batch * n_heads))))
+    of16 = -(-longest // 16) if longest >= 96 else longest // 16
+    return max(1, min(32, of16, -(-(8 * (n_cus or compute_units())) // max(1, batch * n_heads))))
 
 
 def scan_plan(batch: int, n_heads: int, dim: int, longest: Optional[int], n_cus: Optional[int] = None) -> Tuple[int, int, int]:
-    """(rows of the state a thread, blocks a head, segments a prompt) for the recurrence; `longest` is the most
-    tokens a sequence brings (None: a single-token step).  Measured on the MI355X (64 heads of 64, one prompt of
-    2,048 tokens): a block a head with 4 rows a thread 1,014 us, its columns over 4 blocks 550 us (a chain of
+    """(rows of the state a thread, blocks a head, segments a prompt) for the recurrence with a block a head, which serves
+    heads of other sizes than 64 channels, and of 64 where wave_scan_serves says no; `longest` is the most
+    tokens a sequence brings (None: a single-token step).  Measured on the MI355X when it served heads of 64 throughout (64
+    of them, one prompt of 2,048 tokens): a block a head with 4 rows a thread 1,014 us, its columns over 4 blocks 550 us (a chain of
     2,048 dependent steps of 270 ns, whatever else is done); cut into 4 to 16 segments that run side by side
     (each twice: once for its end state from zero, once for its outputs from its true initial state) 455 us, no
     longer bound by the chain but by the instructions a token costs a thread, of which with 4 rows a thread two

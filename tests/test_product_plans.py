@@ -167,3 +167,14 @@ def test_where_the_product_that_adds_itself_to_the_stream_serves():
         assert plan(M, 4096, 4100) == (0, 0)
     assert plan(17, 4096, 4096) == (0, 0) and plan(0, 4096, 4096) == (0, 0)
     assert K.residual_plan(8, 4096, 4096, n_cus=64) == (8, 2)                            # fewer units: two strips a block
+
+
+def test_which_recurrence_serves_short_prompts_of_heads_of_64():
+    """Steps measured on either side of the line: at the first ones the kernel with a block a head was ahead (by 8 to 60 %), at the
+    others the one with a wave a head; and a prompt just above the line is cut into segments of two whole chunks of eight."""
+    for batch, heads, longest in ((1, 64, 2), (1, 64, 16), (1, 8, 40), (1, 128, 64), (1, 64, 80), (8, 32, 20), (8, 32, 5), (6, 40, 2), (4, 32, 64)):
+        assert not K.wave_scan_serves(batch, heads, longest, n_cus=256), (batch, heads, longest)
+    for batch, heads, longest in ((1, 64, None), (64, 64, None), (8, 40, 20), (8, 64, 5), (6, 64, 2), (40, 8, 2), (1, 64, 127), (1, 8, 100), (1, 64, 2048)):
+        assert K.wave_scan_serves(batch, heads, longest, n_cus=256), (batch, heads, longest)
+    assert K.wave_scan_segments(1, 64, 100, n_cus=256) == 7 and K.wave_scan_segments(1, 8, 127, n_cus=256) == 8
+    assert K.wave_scan_segments(8, 64, 20, n_cus=256) == 1 and K.wave_scan_segments(1, 64, 8000, n_cus=256) == 32
