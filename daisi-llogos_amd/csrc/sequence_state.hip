@@ -233,12 +233,19 @@ __global__ __launch_bounds__(128) void token_shift_wide_kernel(TO* __restrict__ 
     }
 }
 
+// Whether a step has enough of tokens x channels for the form of many tokens.  Its threads make the mixes one after the other, which
+// only many blocks hide: us, a channel a thread and this form, bfloat16: 300 x 2,048, five mixes 5.1 and 8.2, 632 x 2,048 7.9 and
+// 9.6, 800 x 2,560 level at 0.93, 2,048 x 2,048 22.9 and 15.4; one or two mixes 1,024 x 1,024 0.90 and 1.06, 500 x 2,560 0.85 and 0.99.
+LLOGOS_EXPORT int llogos_token_shift_wide(int T, int W, int n_mix) {
+    return (long long)T * W >= (n_mix <= 2 ? 1280000 : 2000000);
+}
+
 LLOGOS_EXPORT int llogos_token_shift(void* out, int out_dtype, const float* h, const float* mu, const float* state,
                                      long long state_stride, const int* slots, const int* tok_seq, const int* cu,
                                      int T, int W, int n_mix, hipStream_t stream) {
     if (T <= 0 || W <= 0 || n_mix <= 0) return LLOGOS_BAD_ARGUMENT;
     const int threads = 256;
-    if (cu && T > 64 && (W & 3) == 0 && (state_stride & 3) == 0 && (((uintptr_t)h | (uintptr_t)mu | (uintptr_t)state | (uintptr_t)out) & 15) == 0) {
+    if (cu && llogos_token_shift_wide(T, W, n_mix) && (W & 3) == 0 && (state_stride & 3) == 0 && (((uintptr_t)h | (uintptr_t)mu | (uintptr_t)state | (uintptr_t)out) & 15) == 0) {
         const dim3 wide((T + kShiftTokens - 1) / kShiftTokens, (W / 4 + 127) / 128);
         if (out_dtype == DT_F32)
             token_shift_wide_kernel<float><<<wide, 128, 0, stream>>>((float*)out, h, mu, state, (size_t)state_stride, slots, tok_seq, cu, T, W, n_mix);

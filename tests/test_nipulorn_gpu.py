@@ -513,6 +513,32 @@ def test_recurrence_with_sequences_that_bring_no_token(segments, rows, monkeypat
     assert torch.equal(state, alone) and torch.equal(state[[0, 1, 3, 5]], f["state"][[0, 1, 3, 5]])
 
 
+@pytest.mark.parametrize("mixes", [1, 2, 5])
+def test_token_shift_of_many_tokens_and_of_few(mixes):
+    """The form for many tokens serves where it was measured ahead, and gives the bits of the other form, which shorter steps
+    of the same rows take: sequences that begin anywhere in a thread's four tokens, a width that fills no block."""
+    wide = K._lib().llogos_token_shift_wide
+    for T, W in ((65, 4096), (300, 2048), (632, 1024), (1024, 768)):
+        assert not wide(T, W, mixes), (T, W)
+    assert not wide(632, 2048, 5) and not wide(130, 8192, 2)
+    for T, W in ((2048, 2048), (500, 4096), (800, 2560), (4096, 512)):
+        assert wide(T, W, mixes), (T, W)
+    W, counts, dtype = 2060, [1, 6, 501, 3, 400, 102], torch.bfloat16
+    T, cu = sum(counts), np.concatenate([[0], np.cumsum(counts)])
+    gen = torch.Generator(device=DEV).manual_seed(3)
+    h, mu, prev = (torch.randn(s, device=DEV, generator=gen) for s in ((T, W), (mixes, W), (7, W)))
+    i32 = lambda a: torch.tensor(np.asarray(a), dtype=torch.int32, device=DEV)
+    def shift(lo, hi):                                                   # sequences lo .. hi - 1 in a step
+        n = [int(c) for c in counts[lo:hi]]
+        ctx = type("Ctx", (), dict(n_tokens=sum(n), batch=hi - lo, slots=i32(np.arange(lo + 1, hi + 1)), tok_seq=i32(np.repeat(np.arange(hi - lo), n)),
+                                   cu_dev=i32(np.concatenate([[0], np.cumsum(n)])), is_decode=False))()
+        return K.token_shift(ctx, h[cu[lo]:cu[hi]].contiguous(), mu, prev, dtype)
+    assert wide(T, W, mixes) and not wide(max(counts), W, mixes)
+    whole = shift(0, 6)
+    for i in range(6):
+        assert torch.equal(shift(i, i + 1), whole[:, cu[i]:cu[i + 1]]), i
+
+
 @pytest.mark.parametrize("out", ["float32", "bfloat16"])
 @pytest.mark.parametrize("taps", [1, 2, 4, 7, 16])
 def test_long_steps_of_convolution_shift_and_activation(taps, out):
