@@ -331,19 +331,6 @@ LLOGOS_EXPORT int llogos_batch_class(int batch) {
     return (batch + 63) / 64 * 64;
 }
 
-// compute units of the current device, asked for once per device
-static int compute_units() {
-    static int cached[64];
-    int device = 0;
-    if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 64) return 256;
-    if (cached[device] == 0) {
-        int n = 0;
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || n <= 0) n = 256;
-        cached[device] = n;
-    }
-    return cached[device];
-}
-
 constexpr int kDecodeWaves = 4;
 constexpr int kMaxPagesPerWave = 16;
 
@@ -358,7 +345,7 @@ constexpr int kMaxPagesPerWave = 16;
 // at 32,768 192 from 211; batch 1 at 131,000 102 from 117; batch 32 at 640 25.1 from 23.6.
 static int decode_pages_per_wave(int table_width, int batch, int n_kv_heads) {
     const long long pairs = (long long)llogos_batch_class(batch) * n_kv_heads;
-    const long long units = compute_units();
+    const long long units = device_units();
     int best = 1;
     double best_cost = 0;
     for (int ppw = 1; ppw <= kMaxPagesPerWave; ++ppw) {

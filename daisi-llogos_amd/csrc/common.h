@@ -119,4 +119,17 @@ __device__ __forceinline__ bool key_visible(int q_pos, int k_pos, int window, in
     return k_pos < sinks || k_pos > q_pos - window;
 }
 
+// compute units of the current device, asked for once per device and source file
+static inline int device_units() {
+    static int cached[64];
+    int device = 0;
+    if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 64) return 256;
+    if (cached[device] == 0) {
+        int n = 0;
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || n <= 0) n = 256;
+        cached[device] = n;
+    }
+    return cached[device];
+}
+
 #define LLOGOS_LAUNCH_CHECK() (int)hipGetLastError()

@@ -207,8 +207,8 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tiles_kernel(
         dst[c] = row * LD + col;
     }
     const int col = (tid & 7) * 4;
-    // a stage is asked for two stages ahead (one: gate/up 477 us against 459, q/k/v 123 against 115); past K the last values are read again (a load under a condition would make
-    // every wait one for all loads) and zeros are stored
+    // a stage is asked for two stages ahead (one: gate/up 477 us against 459, q/k/v 123 against 115); past K the last values are
+    // read again (a load under a condition would make every wait one for all loads) and zeros are stored
     f32x4 ahead[2][COPIES];
     auto load = [&](f32x4 (&to)[COPIES], int k) {
 #pragma unroll
@@ -282,24 +282,24 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tiles_kernel(
 
 namespace {
 
-constexpr double kUnits = 256, kUnitFlops = 157.3e12 / 256;
+constexpr double kUnitFlops = 157.3e12 / 256;               // of one compute unit
 
 // Seconds that the two kernels take, fitted to sweeps of 1 to 2,048 rows over eight matrices.  Tiles: a stage of 32 k takes a block that is
 // alone on its compute unit 0.35 us beside its products; blocks that share a unit hide that, and share the matrix cores, which the
 // kernel keeps busy 70 % of the time.
-double tiles_cost(double M, double N, double K, int tm, int tn) {
+double tiles_cost(double M, double N, double K, int tm, int tn, double units) {
     const double blocks = ceil(M / tm) * ceil(N / tn), tile = tm * (double)tn * 2 / kUnitFlops * (tn == 32 ? 1.6 : 1.4);
     const double together = tn == 32 ? 4 : tm == 64 ? 3 : 2;
-    const double busy = ceil(blocks / kUnits) * tile * K, waits = ceil(blocks / (kUnits * together)) * (tile * K + K / 32 * 0.35e-6);
+    const double busy = ceil(blocks / units) * tile * K, waits = ceil(blocks / (units * together)) * (tile * K + K / 32 * 0.35e-6);
     return (busy > waits ? busy : waits) + 3e-6;
 }
 
 // 17 rows and more by the few-row kernel: what its blocks ask of the caches (their strips of w and the rows of a, once a block), at the rates
 // that the three forms were measured at, with compute units idle while a last round of blocks runs.
-double rows_cost(double M, double N, double K, int mt, int ns) {
+double rows_cost(double M, double N, double K, int mt, int ns, double units) {
     const double blocks = ceil(N / (16 * ns)) * ceil(M / (16 * mt));
-    const double spread = blocks < kUnits ? blocks / kUnits : blocks / kUnits / ceil(blocks / kUnits);
-    return blocks * (ns + mt) * 64 * K / (ns == 2 ? 5.3e12 : mt == 4 ? 6.7e12 : 9.5e12) / spread + 4e-6;
+    const double spread = blocks < units ? blocks / units : blocks / units / ceil(blocks / units);
+    return blocks * (ns + mt) * 64 * K / ((ns == 2 ? 5.3e12 : mt == 4 ? 6.7e12 : 9.5e12) * units / 256) / spread + 4e-6;      // (rates of 256 units)
 }
 
 // Rows of w a wave of the lanes' kernel takes, 0 where the few-row kernel is ahead: matrices whose blocks of 16 rows leave units idle
@@ -337,16 +337,16 @@ LLOGOS_EXPORT int llogos_gemm_f32(float* out, const float* a, const float* w, co
     if (M <= 0 || N <= 0 || K <= 0 || lda < K || ldo < N || form < 0 || form > 8) return LLOGOS_BAD_ARGUMENT;
     const bool vec = (K & 3) == 0 && (lda & 3) == 0 && (((uintptr_t)a | (uintptr_t)w) & 15) == 0;
     const int vec_out = (ldo & 3) == 0 && ((uintptr_t)out & 15) == 0;
-    const int cols = lanes_cols(M, N, K, vec);
+    const int cols = lanes_cols(M, N, K, vec), units = device_units();
     if (form == 0 && cols) form = 8;
     if (form == 0) {
-        const double cost[8] = {0, 0, rows_cost(M, N, K, 2, 1), rows_cost(M, N, K, 4, 1), rows_cost(M, N, K, 4, 2),
-                                tiles_cost(M, N, K, 64, 32), tiles_cost(M, N, K, 64, 64), tiles_cost(M, N, K, 128, 64)};
+        const double cost[8] = {0, 0, rows_cost(M, N, K, 2, 1, units), rows_cost(M, N, K, 4, 1, units), rows_cost(M, N, K, 4, 2, units),
+                                tiles_cost(M, N, K, 64, 32, units), tiles_cost(M, N, K, 64, 64, units), tiles_cost(M, N, K, 128, 64, units)};
         form = M <= 16 ? 1 : 2;
         for (int f = 3; form > 1 && f <= 7; ++f) if (cost[f] < cost[form]) form = f;
     }
     // 16 waves a block where a matrix has few blocks and enough of k for all of them
-    const bool wide = K >= 16 * 256 && (N + 15) / 16 * ((M + 15) / 16) <= 512;
+    const bool wide = K >= 16 * 256 && (N + 15) / 16 * ((M + 15) / 16) <= 2 * units;
     switch (form) {
         case 1: if (wide) ROWS(16, 1, 1); else ROWS(8, 1, 1); break;
         case 2: if (wide) ROWS(16, 2, 1); else ROWS(8, 2, 1); break;

@@ -536,10 +536,10 @@ enum { STREAM_NONE = 0, STREAM_ONE = 1, STREAM_TWO = 2 };
 constexpr int kStreamRing = 8;
 
 static int stream_form(int mb, int N, int k_part, int parts) {
-    constexpr int kUnits = 256;                                          // compute units
+    const int units = device_units();
     const long long blocks = (long long)((N + 63) / 64) * parts, pairs = (long long)((N + 127) / 128) * parts;
-    if (mb >= 3 && k_part >= (mb == 3 ? 2560 : 1536) && pairs * 8 >= 7 * ((pairs + kUnits - 1) / kUnits * kUnits)) return STREAM_TWO;
-    if (blocks <= kUnits || (mb >= 2 && blocks > 2 * kUnits)) return STREAM_ONE;
+    if (mb >= 3 && k_part >= (mb == 3 ? 2560 : 1536) && pairs * 8 >= 7 * ((pairs + units - 1) / units * units)) return STREAM_TWO;
+    if (blocks <= units || (mb >= 2 && blocks > 2 * units)) return STREAM_ONE;
     return STREAM_NONE;
 }
 
