@@ -744,7 +744,9 @@ def moe_form(P: int, E: int, N: int, K: int, n_cus: Optional[int] = None) -> int
     a router prefers some experts.
     Few rows end at about 12 an expert (16 experts of 7168 x 4096, 12 rows 210 us against 224 in tiles of 64, 16 rows 264
     and 222; 8 of 4096 x 4096, 12 rows 64 and 71, 16 rows 78 and 72), at 4 where the tiles' blocks fill the compute units in
-    one round (4096 x 7168, 4 rows 157 and 155, 8 rows 175 and 156), and not at all where they leave units without a block;
+    one round (4096 x 7168, 4 rows 157 and 155, 8 rows 175 and 156) unless k is a power of two, whose rows the tiles read from
+    too few memory channels at once (4.3 TB/s against 5.7: 8 of 8192 x 4096, 6 rows 96 and 126, 10 rows 110 and 127, of 8192 x
+    5120 125 and 114, 143 and 115; 32 of 2048 x 2048, 5 rows 53 and 67), and not at all where they leave units without a block;
     MOE_FEW_PAIRS pairs at most, or 4 rows an expert if that is more and k is long enough (128 experts of 1536 x 2048, 384
     pairs 147 and 176).
     Tiles of 64 rows up to 96 an expert, of 128 above: at 96 rows
@@ -757,7 +759,10 @@ def moe_form(P: int, E: int, N: int, K: int, n_cus: Optional[int] = None) -> int
         if P <= 4 * E:
             return 0
         units, columns = n_cus or compute_units(), E * -(-N // 128)
-        if columns < units or P <= (4 if 1.5 * units <= columns <= 3 * units else (13 if columns < 6 * units else 12)) * E:
+        rows = 13 if columns < 6 * units else 12
+        if 1.5 * units <= columns <= 3 * units:
+            rows = 4 if K & (K - 1) else 10
+        if columns < units or P <= rows * E:
             return 0
     if P < 96 * E:
         return 1

@@ -135,7 +135,9 @@ def test_tiles_of_the_experts_product():
            (200, 16, 7168, 2048), (384, 128, 1536, 2048), (256, 128, 2048, 768)]
     for P, E, N, K_ in few:
         assert K.moe_form(P, E, N, K_, 256) == 0, (P, E, N, K_)
-    for P, E, N, K_ in ((96, 16, 4096, 7168), (128, 16, 4096, 3584), (200, 14, 7168, 4096), (128, 8, 4096, 4096), (257, 16, 1024, 2048),
+    for P, E, N, K_ in ((48, 8, 8192, 4096), (80, 16, 4096, 4096), (160, 32, 2048, 2048)):        # k a power of two
+        assert K.moe_form(P, E, N, K_, 256) == 0 and K.moe_form(11 * E, E, N, K_, 256) == 1, (P, E, N, K_)
+    for P, E, N, K_ in ((96, 16, 4096, 7168), (48, 8, 8192, 5120), (128, 16, 4096, 3584), (200, 14, 7168, 4096), (128, 8, 4096, 4096), (257, 16, 1024, 2048),
                         (384, 128, 2048, 768), (520, 128, 1536, 2048), (196, 16, 14336, 4096)):
         assert K.moe_form(P, E, N, K_, 256) == 1, (P, E, N, K_)
     for P, E, N, K_ in ((64 * 16, 16, 1024, 2048), (73 * 14, 14, 7168, 4096), (95 * 16, 16, 4096, 7168), (32 * 8, 8, 28672, 4096)):
