@@ -41,9 +41,9 @@
 //    matrices with few rows, whose tiles do not fill the compute units.
 //  * Epilogues: plain (+ bias) in bfloat16 or float32; added to a float32 result in place; SwiGLU for a matrix packed
 //    with gate_rows.
-//  * Measured, 2,048 tokens of the 8B layer sizes: gate/up with SwiGLU 387 us against the library's 385 with a SwiGLU
-//    pass; down 200 (two parts of k) against 212; qkv 102 against 80; o 72 against 63; 5,003 tokens of the 14B sizes:
-//    gate/up 1,414 against 1,524, down 783 against 1,037.  By the counters the matrix pipe is busy 76 % of a tile's
+//  * Measured, 2,048 tokens of the 8B layer sizes: gate/up with SwiGLU 407 us against the library's 389 with a SwiGLU
+//    pass; down 215 (two parts of k, to be added) against 215; qkv 108 against 92; o 81 against 67; 5,003 tokens of the
+//    14B sizes: gate/up 1,478 against 1,560, down 800 against 1,019 (some machines are 5 % faster, on both sides).  By the counters the matrix pipe is busy 76 % of a tile's
 //    time (86 % with the copies left out, barriers 9 %); the rest of the distance to the library's kernels on the short
 //    matrices is the round of blocks that their tiles do not fill.  (Copies straight into LDS, five stages of 32 k deep,
 //    with a barrier a stage were 8 % slower.)
@@ -297,8 +297,8 @@ __device__ __forceinline__ void tile_body(
 // tiles are counted in bands of eight token tiles, a column of the band before the next, and every XCD takes a run of them, as
 // long as the others' to one tile.  The 32 blocks that run on an XCD so are about 8 x 4 tiles of one part of k: they share
 // their weights and their activations in its L2, and no XCD is left with a round of blocks more than the others.  (With
-// whole columns dealt to the XCDs in turn 11 x 20 tiles took two rounds on four of them: 715 us for 2,600 x 5,120 x 17,408,
-// 404 now; 5,003 x 5,120 x 17,408 889 -> 783, 5,003 x 34,816 x 5,120 with SwiGLU 1,485 -> 1,414, 2,048 x 28,672 x 4,096 402 -> 387.)
+// whole columns dealt to the XCDs in turn 11 x 20 tiles took two rounds on four of them: 708 us for 2,600 x 5,120 x 17,408,
+// 415 now; 5,003 x 5,120 x 17,408 847 -> 800, 5,003 x 34,816 x 5,120 with SwiGLU 1,505 -> 1,478, 2,048 x 28,672 x 4,096 410 -> 407.)
 __device__ __forceinline__ bool tiles_place(int tiles, int rows, int cols, int xcd, int j, int& row, int& col) {
     const int per = tiles >> 3, more = tiles & 7;
     if (j >= per + (xcd < more)) return false;
@@ -342,8 +342,8 @@ static double tiles_cost(int tm, long long tiles, int stages, int compute_units)
 
 // How the tiles are cut: row tiles 0 .. n_full - 1 in tiles of 256 tokens, the rest in tiles of 128 tokens.
 // token_tiles 4: all of 256, 2: all of 128, 0: the cheapest by tiles_cost of all of 256, all of 128 and the last round of
-// blocks in tiles of 128.  (Few rows leave units idle in tiles of 256: 334 x 4,096 x 14,336 in four parts 82 us, in tiles of
-// 128 62; 2,048 x 28,672 x 4,096, three rounds and a half: 413 all of 256, 470 all of 128, 402 mixed.)
+// blocks in tiles of 128.  (Few rows leave units idle in tiles of 256: 334 x 4,096 x 14,336 in four parts 87 us, in tiles of
+// 128 65; 2,048 x 28,672 x 4,096, three rounds and a half: 425 all of 256, 467 all of 128, 407 mixed.)
 static int tiles_n_full(int n_tiles, int m_tiles4, int m_tiles2, int parts, int stages, int token_tiles, int compute_units) {
     if (token_tiles == 4) return n_tiles;
     if (token_tiles == 2) return 0;

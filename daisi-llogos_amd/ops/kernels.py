@@ -1980,8 +1980,9 @@ def gemm_packed_unscaled_bf16(squares: RowSquares, eps: float, pw: PackedWeight,
 
 
 # Which product serves many rows of bfloat16 (prompts): "auto" (the default): the hand-written tiled
-# product (gemm_tiles_bf16 on the packed copy) where it was measured faster than the library's, which is
-# the gate/up product with its SwiGLU epilogue from TILES_MIN_ROWS rows on, and the library's product
+# product (gemm_tiles_bf16 on the packed copy) where it was measured level with the library's or faster, which is
+# the gate/up product with its SwiGLU epilogue from TILES_MIN_ROWS to TILES_MAX_ROWS rows (tiles_serve_gated), down
+# projections of up to 1,024 rows and long ones at some sizes (tiles_plan), and the library's product
 # elsewhere (as the reference uses a library there); "tiles": the hand-written one wherever it applies;
 # "library": the library's everywhere.  LLOGOS_PROMPT_PRODUCT in the environment sets the default.
 PROMPT_PRODUCT = os.environ.get("LLOGOS_PROMPT_PRODUCT", "auto")
@@ -1991,14 +1992,14 @@ TILES_MIN_ROWS, TILES_MAX_ROWS, TILES_MAX_K = 1024, 2048, 5120
 def tiles_serve_gated(M: int, K: int = 0) -> bool:
     """Whether the tiled product makes silu(gate) * up for M rows of K values (rather than the library's product
     and a SwiGLU pass): by default from TILES_MIN_ROWS to TILES_MAX_ROWS rows with k up to TILES_MAX_K, where
-    it was measured level or ahead (tiled against library + SwiGLU, us, sustained: 1B 63 / 67 at 1,024 rows,
-    119 / 120 at 2,048; 8B 225 / 217 and 405 / 391, level inside the model; 14B 343 / 413 and 614 / 630).
+    it was measured level or ahead (tiled against library + SwiGLU, us, sustained: 1B 69 / 77 at 1,024 rows,
+    129 / 131 at 2,048; 8B 218 / 218 and 407 / 389, level inside the model; 14B 343 / 414 and 618 / 627).
     The library gains with the rows and with k (8B: 1.11 PFLOP/s at 1,024 rows, 1.34 from 4,096 on; 70B 1.41
-    to 1.47) where the tiled product stays at 1.2: 8B at 4,096 rows 825 / 727, 70B at 2,048 rows 1,516 / 1,363,
+    to 1.47) where the tiled product stays at 1.2: 8B at 4,096 rows 778 / 721, 70B at 2,048 rows 1,524 / 1,376,
     a 16,384-token prompt of the 8B sizes 278 ms against 268.  Beyond 2,048 rows neither is ahead for long: with k of 4,608
-    and 5,120 and 8,192 to 65,536 columns the tiled product took between 0.61 and 1.16 of the time of the library with its SwiGLU pass at 204 sizes,
-    by what the library chooses for a size: 14B 4,096 rows 1,153 / 1,258, 3,840 1,082 / 1,059; 24,576 columns, 2,500 rows
-    476 / 444, 3,072 579 / 652)."""
+    and 5,120 and 8,192 to 65,536 columns the tiled product took between 0.61 and 1.16 of the time of the library with its
+    SwiGLU pass at 204 sizes, by what the library chooses for a size (14B 4,096 rows 1,153 / 1,258, 3,840 1,082 / 1,059;
+    24,576 columns, 2,500 rows 476 / 444, 3,072 579 / 652)."""
     if PROMPT_PRODUCT == "tiles":
         return True
     return PROMPT_PRODUCT == "auto" and TILES_MIN_ROWS <= M <= TILES_MAX_ROWS and K <= TILES_MAX_K
@@ -2008,8 +2009,8 @@ def tiles_plan(M: int, N: int, K: int) -> Optional[Tuple[int, int]]:
     """(parts of k, token_tiles) with which the tiled product serves a plain product of M rows, or None where
     the library's does.  Measured on the MI355X at the layer sizes of 8B, 14B and 70B models: a matrix that
     is much longer than high (a feed-forward's down projection) with 129 to 1,024 rows of activations is where
-    the library is furthest from its best (14B, 256 rows: 119 us against 65; 70B: 291 against 143; 8B, 512 rows:
-    88 against 68), and blocks along k fill the compute units that its few row tiles leave idle.  For more rows see
+    the library is furthest from its best (14B, 256 rows: 226 us against 78; 70B: 313 against 154; 8B, 512 rows:
+    94 against 77), and blocks along k fill the compute units that its few row tiles leave idle.  For more rows see
     long_tiles_plan.  Elsewhere the library's product was level or ahead (by 10 to 25 % from 2,048 rows on)."""
     if PROMPT_PRODUCT == "library" or M <= SKINNY_MAX_ROWS or K % 64:
         return None
@@ -2117,7 +2118,7 @@ def gemm_product(a: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, swigl
     product is taken of silu(gate) * up.  With `f32_ok` the consumer also takes one float32
     [M, N], which spares the result a rounding to bfloat16.
 
-    float32 operands: plain FMAs in 32-bit throughout.  bfloat16 operands: up to 64 rows the
+    float32 operands: 32-bit throughout (gemm_generic).  bfloat16 operands: up to 64 rows the
     hand-written weight-streaming kernels (on the packed copy of w when there is one: `packed`),
     up to 128 rows too where w is much longer than it has rows (see long_inner); for more rows the
     hand-written tiled product where it was measured ahead (see tiles_plan); otherwise the

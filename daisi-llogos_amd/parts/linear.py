@@ -116,9 +116,9 @@ class Linear(Part):
 
     def add_to(self, a: torch.Tensor, residual: Residual):
         """residual.x += a . W^T + bias in one kernel: for the few rows and the shapes that
-        gemm_residual_bf16 serves, and for prompts that the library's product serves (its epilogue adds).
+        gemm_residual_bf16 serves, and for prompts (the tiled product in one part and the library's add in their epilogues).
         Returns what the product left for the norm that follows (RowSquares: with that norm's rows without
-        their scale if residual.norm has a row weight; empty after the library's product), or None when x
+        their scale if residual.norm has a row weight; empty after a prompt's product), or None when x
         is untouched and the caller takes the product as a tensor."""
         if not isinstance(a, torch.Tensor) or a.dim() != 2:
             return None

@@ -542,7 +542,7 @@ def test_token_shift_of_many_tokens_and_of_few(mixes):
 @pytest.mark.parametrize("out", ["float32", "bfloat16"])
 @pytest.mark.parametrize("taps", [1, 2, 4, 7, 16])
 def test_long_steps_of_convolution_shift_and_activation(taps, out):
-    """The forms for steps of many tokens, four channels a thread: sequences of one token, of fewer than the taps, of a block of
+    """The forms for steps of many tokens, four channels a thread (token shifts of so few take a channel a thread): sequences of one token, of fewer than the taps, of a block of
     eight and more, new ones and ones that go on from their state; widths that fill no block; an activation of a part of rows."""
     rng = np.random.default_rng(taps)
     counts, starts, W = [1, 3, 8, 9, 50, 2], [5, 0, 0, 30, 2, 1], 516
