@@ -18,6 +18,9 @@
 // Measured (us, before -> now): heads of 64, 32 to 8 kv heads, prompts of 515 and 190 tokens 1,019 -> 47, one of 2,048
 // tokens 14,731 -> 288; single tokens behind 515 and 190: 158 -> 17, behind 8,192: 2,625 -> 142.  Heads of 128: 1,496 -> 90,
 // 19,143 -> 536, 180 -> 27, 2,721 -> 259.
+// Behind only where a step's longest context has fewer than some 16 tokens, since a page is worked on whole: one token of heads
+// of 64 by itself 4.9 -> 7.7, of 128 5.9 -> 11.3, a prompt of 16 11.2 -> 11.8 (the other kernel adds in another order, so
+// serving those with it would cost the bits that a token has in common with itself in a longer step).
 #include "common.h"
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
