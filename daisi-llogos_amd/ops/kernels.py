@@ -1903,11 +1903,23 @@ def residual_plan(M: int, N: int, K: int, n_cus: Optional[int] = None) -> Tuple[
     return 8, 2
 
 
+def residual_form(N: int, K: int, waves: int, strips: int, n_cus: Optional[int] = None) -> Tuple[int, int]:
+    """(waves, strips) of residual_plan as the kernel runs it, strips 0 for half a strip of 16 rows of w a block.  Halves where
+    whole strips leave half the compute units or more without a block and k is long enough to be worth a wave's run of it
+    (us at 1 / 8 / 16 rows, whole strips against halves, 256 units): [2048, 8192] 10.5 / 11.2 / 12.8 against 9.0 / 9.8 / 11.1,
+    [2048, 2048] 5.0 / 5.2 / 5.8 against 4.4 / 4.7 / 5.1, [1024, 4096] 5.9 / 6.4 / 7.2 against 5.2 / 5.8 / 6.6; with a strip for
+    every unit ([4096, 4096]) 8.7 / 8.5 / 9.3 against 10.4 / 11.1 / 12.3, since twice as many blocks copy the activations.  16
+    waves up to k = 4096 (8 take 0.2 to 0.3 us more there), 8 above (16 take 0.4 to 1.1 us more)."""
+    if strips == 1 and waves == 8 and 2 * -(-N // 16) <= (n_cus or compute_units()):
+        return (16 if K <= 4096 else 8), 0
+    return waves, strips
+
+
 def gemm_residual_bf16(x: torch.Tensor, a: torch.Tensor, pw: PackedWeight, bias: Optional[torch.Tensor],
                        waves: int, norm_w: Optional[torch.Tensor] = None, strips: int = 1) -> Optional[RowSquares]:
     """x [M, N] (float32, in place) += a [M, K] . w^T (+ bias) for up to 16 rows of bfloat16 activations in
     one kernel, every sum in an order fixed by the shapes; returns the sums of squares of x's new rows, by
-    strips of 16 columns, and with `norm_w` [N] also x * norm_w in bfloat16 (the rows of the rmsnorm with
+    blocks of 16 * strips columns (8 with strips 0), and with `norm_w` [N] also x * norm_w in bfloat16 (the rows of the rmsnorm with
     that weight, without their scale).  None for shapes it does not take."""
     if a.dtype != torch.bfloat16 or a.dim() != 2 or x.dim() != 2 or x.dtype != torch.float32 or pw.gate_rows:
         return None
@@ -1923,7 +1935,8 @@ def gemm_residual_bf16(x: torch.Tensor, a: torch.Tensor, pw: PackedWeight, bias:
     if norm_w is not None:
         _need(norm_w.dtype == torch.float32 and norm_w.shape == (N,) and norm_w.is_contiguous(), "gemm: norm weight must be float32 [N]")
         unscaled = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
-    sums = torch.empty((-(-(-(-N // 16)) // int(strips)), 16), dtype=torch.float32, device=x.device)
+    n16 = -(-N // 16)
+    sums = torch.empty((-(-n16 // int(strips)) if strips else 2 * n16, 16), dtype=torch.float32, device=x.device)
     code = _lib().llogos_gemm_residual_bf16(_p(x), x.stride(0), _p(sums), _p(unscaled), N, _p(norm_w), _p(a), a.stride(0),
                                             _p(pw.data), _p(bias), M, N, K, int(waves), int(strips), _stream())
     if code == -2:

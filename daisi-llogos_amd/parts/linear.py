@@ -135,6 +135,7 @@ class Linear(Part):
         waves, strips = K.residual_plan(a.shape[0], self.packed.N, self.packed.K)
         if not waves:
             return None
+        waves, strips = K.residual_form(self.packed.N, self.packed.K, waves, strips)
         norm_w = residual.norm.row_weight() if residual.norm is not None else None
         return K.gemm_residual_bf16(x, a, self.packed, self.bias, waves, norm_w, strips)
 

@@ -941,6 +941,32 @@ def test_product_that_adds_itself_to_the_residual_stream(M, N, K_, waves, strips
     assert K.gemm_residual_bf16(torch.zeros(17, N, device=DEV), torch.zeros(17, K_, device=DEV, dtype=torch.bfloat16), pw, None, waves) is None
 
 
+@pytest.mark.parametrize("M,N,K_", [(1, 2048, 8192), (8, 2048, 2048), (16, 1024, 4096), (16, 48, 200), (5, 80, 8), (13, 1000, 1000), (3, 16, 72),
+                                    (9, 120, 1032), (2, 7, 16)])
+@pytest.mark.parametrize("waves", [8, 16])
+def test_product_that_adds_itself_to_the_residual_stream_by_half_strips(M, N, K_, waves):
+    """The same with 8 rows of w a block: odd numbers of steps of k and of half strips, parts of them, and rows alone."""
+    rng = np.random.default_rng(M * 100 + N + waves)
+    a, w = _t(rng.standard_normal((M, K_)), torch.bfloat16), _t(rng.standard_normal((N, K_)) * 0.05, torch.bfloat16)
+    bias, norm_w = _t(rng.standard_normal(N)), _t(1 + 0.1 * rng.standard_normal(N))
+    x0 = _t(rng.standard_normal((M, N)) * 3)
+    pw = K.pack_weights(w)
+    want = _np(x0) + _np(a) @ _np(w).T + _np(bias)
+    x = x0.clone()
+    left = K.gemm_residual_bf16(x, a, pw, bias, waves, norm_w, 0)
+    _close(x, want, "float32", scale=np.abs(want).max() * 10)                    # bfloat16 operands, float32 sums
+    blocks = 2 * -(-N // 16)
+    sums, padded = _np(left.sums), np.zeros((M, blocks * 8))
+    padded[:, :N] = _np(x)
+    assert sums.shape == (blocks, 16) and np.all(sums[:, M:] == 0)
+    assert np.allclose(sums[:, :M], (padded ** 2).reshape(M, blocks, 8).sum(2).T, rtol=2e-6, atol=1e-30)
+    assert torch.equal(left.unscaled, (x * norm_w).to(torch.bfloat16))
+    plain, alone = x0.clone(), x0[:1].clone()
+    K.gemm_residual_bf16(plain, a, pw, None, waves, strips=0)
+    K.gemm_residual_bf16(alone, a[:1].contiguous(), pw, None, waves, strips=0)
+    assert torch.equal(alone, plain[:1])
+
+
 def test_library_product_that_adds_itself_to_the_residual_stream():
     """For prompts that the library's product serves, the sum with the residual stream is the product's
     epilogue: the float32 product added to x, bit for bit; refused for few rows, other element types and where

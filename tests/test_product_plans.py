@@ -171,6 +171,14 @@ def test_where_the_product_that_adds_itself_to_the_stream_serves():
     assert K.residual_plan(8, 4096, 4096, n_cus=64) == (8, 2)                            # fewer units: two strips a block
 
 
+def test_where_that_product_takes_half_a_strip_a_block():
+    """Half a strip of 16 rows of w a block where whole strips would leave half of the units without one and k is no short one."""
+    form = lambda N, K_: K.residual_form(N, K_, *K.residual_plan(8, N, K_, n_cus=256), n_cus=256)
+    assert form(2048, 8192) == (8, 0) and form(2048, 2048) == (16, 0) and form(1024, 4096) == (16, 0) and form(2041, 4104) == (8, 0)
+    assert form(2064, 8192) == (8, 1) and form(4096, 14336) == (8, 1) and form(8192, 8192) == (8, 2)
+    assert form(64, 176) == (4, 1) and form(1024, 8192) == (0, 0)
+
+
 def test_which_recurrence_serves_short_prompts_of_heads_of_64():
     """Steps measured on either side of the line: at the first ones the kernel with a block a head was ahead (by 8 to 60 %), at the
     others the one with a wave a head; and a prompt just above the line is cut into segments of two whole chunks of eight."""
