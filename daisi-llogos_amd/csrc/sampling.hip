@@ -112,46 +112,80 @@ struct PenaltyParams {
     int banned[kMaxBanned];
 };
 
-__global__ __launch_bounds__(kSampleThreads) void sample_prepare_kernel(
-        float* __restrict__ work, const float* __restrict__ logits, int V,
-        const int* __restrict__ hist, const int* __restrict__ hist_len, int hist_stride, PenaltyParams pp) {
-    const int r = blockIdx.x;
-    const float* row = logits + (size_t)r * V;
-    float* w = work + (size_t)r * V;
+// The tokens of the window h[0 .. n) that lie in first .. first + count - 1 are made again from the logits, penalty first,
+// then the scale, and put to w[token - first].  A round's threads look at a position of the window each and list those
+// that name such a token; a wave takes a listed position and reads the window 64 tokens at a time: a token's first occurrence
+// does the work.  (One thread a position, reading the window token by token, made this 11 us of a slice's 16.)
+struct WindowLds {
+    int n;
+    int at[kSampleThreads];
+};
+
+__device__ __forceinline__ void apply_penalties(float* w, const float* __restrict__ row, int first, int count, int V,
+                                                const int* __restrict__ h, int n, const PenaltyParams& pp, WindowLds& lds) {
+    const float inv_t = pp.inv_temperature;
+    const bool scaled = inv_t != 1.0f;
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave, waves = blockDim.x / kWave;
+    for (int i0 = 0; i0 < n; i0 += blockDim.x) {
+        __syncthreads();
+        if (threadIdx.x == 0) lds.n = 0;
+        __syncthreads();
+        if (i0 + (int)threadIdx.x < n) {
+            const int tok = h[i0 + threadIdx.x];
+            if (tok >= first && tok - first < count && tok < V && (pp.penalize_newline || (tok != 10 && tok != 13)))
+                lds.at[atomicAdd(&lds.n, 1)] = i0 + threadIdx.x;
+        }
+        __syncthreads();
+        for (int q = wave; q < lds.n; q += waves) {
+            const int i = lds.at[q], tok = h[i];
+            int times = 0;
+            for (int j0 = 0; j0 < n; j0 += kWave) {
+                const uint64_t same = __ballot(j0 + lane < n && h[j0 + lane] == tok);
+                const uint64_t later = j0 >= i ? ~(uint64_t)0 : i - j0 >= kWave ? 0 : ~(uint64_t)0 << (i - j0);
+                if (same & ~later) { times = 0; break; }             // an earlier position names it too
+                times += (int)__popcll(same & later);
+            }
+            if (lane != 0 || times == 0) continue;
+            float l = row[tok];
+            if (pp.repetition != 1.0f)
+                for (int c = 0; c < times; ++c) l = l > 0.f ? l / pp.repetition : l * pp.repetition;
+            if (pp.frequency != 0.f || pp.presence != 0.f) {
+                l -= pp.frequency * (float)times;
+                l -= pp.presence;
+            }
+            w[tok - first] = scaled ? l * inv_t : l;
+        }
+    }
+}
+
+__device__ __forceinline__ bool has_penalties(const PenaltyParams& pp) {
+    return pp.repetition != 1.0f || pp.frequency != 0.f || pp.presence != 0.f;
+}
+
+// a whole row by one block; h: the row's window of n tokens, or null
+__device__ void prepare_row(float* w, const float* __restrict__ row, int V, const int* __restrict__ h, int n, const PenaltyParams& pp,
+                            WindowLds& lds) {
     const float inv_t = pp.inv_temperature;
     const bool scaled = inv_t != 1.0f;
     for_each_value(row, V, [&](int i, float x) { w[i] = scaled ? x * inv_t : x; });
     __syncthreads();
-    // the few tokens that penalties touch are made again from the logits: penalty first, then the scale
-    const bool penalties = pp.repetition != 1.0f || pp.frequency != 0.f || pp.presence != 0.f;
-    if (penalties && hist) {
-        const int* h = hist + (size_t)r * hist_stride;
-        const int n = hist_len[r];
-        // one thread per window position; the first occurrence of a token does the work
-        for (int i = threadIdx.x; i < n; i += blockDim.x) {
-            const int tok = h[i];
-            if (tok < 0 || tok >= V) continue;
-            if (!pp.penalize_newline && (tok == 10 || tok == 13)) continue;
-            bool first = true;
-            for (int j = 0; j < i; ++j) if (h[j] == tok) { first = false; break; }
-            if (!first) continue;
-            int count = 0;
-            for (int j = i; j < n; ++j) count += (h[j] == tok);
-            float l = row[tok];
-            if (pp.repetition != 1.0f)
-                for (int c = 0; c < count; ++c) l = l > 0.f ? l / pp.repetition : l * pp.repetition;
-            if (pp.frequency != 0.f || pp.presence != 0.f) {
-                l -= pp.frequency * (float)count;
-                l -= pp.presence;
-            }
-            w[tok] = scaled ? l * inv_t : l;
-        }
+    if (has_penalties(pp) && h) {
+        apply_penalties(w, row, 0, V, V, h, n, pp, lds);
         __syncthreads();
     }
     if (threadIdx.x < pp.n_banned) {
         const int tok = pp.banned[threadIdx.x];
         if (tok >= 0 && tok < V) w[tok] = -INFINITY;
     }
+}
+
+__global__ __launch_bounds__(kSampleThreads) void sample_prepare_kernel(
+        float* __restrict__ work, const float* __restrict__ logits, int V,
+        const int* __restrict__ hist, const int* __restrict__ hist_len, int hist_stride, PenaltyParams pp) {
+    __shared__ WindowLds lds;
+    const int r = blockIdx.x;
+    prepare_row(work + (size_t)r * V, logits + (size_t)r * V, V, hist ? hist + (size_t)r * hist_stride : nullptr,
+                hist ? hist_len[r] : 0, pp, lds);
 }
 
 LLOGOS_EXPORT int llogos_sample_prepare(float* work, const float* logits, int R, int V,
@@ -438,47 +472,394 @@ __device__ int sorted_head(uint64_t* head, const float* row, int V, int want, fl
 //    with sort_here the block sorts the whole row into `list`, this row's scratch of n_pad
 //    keys, and turns `work` into probabilities in place (slow: one compute unit sorts 10^5
 //    keys in milliseconds); without sort_here it leaves out[row] = -1 for sample_sorted_kernel.
-__global__ __launch_bounds__(kSampleThreads) void sample_pipeline_kernel(
-        int* __restrict__ out, float* __restrict__ work_all, float* __restrict__ prob_all, int V,
-        uint64_t* __restrict__ list_all, int n_pad, const float* __restrict__ uniforms, SampleParams sp,
-        int try_head, int sort_here) {
-    __shared__ float red[16];
-    __shared__ float scan[kSampleThreads];
-    __shared__ int found;
-    __shared__ int counter;
-    __shared__ int bins[kHeadBins];
-    __shared__ uint64_t head[kHeadMax];
-    const int r = blockIdx.x;
-    float* work = work_all + (size_t)r * V;
-    const float u = uniforms[r];
-    const int n = (sp.top_k > 0 && sp.top_k < V) ? sp.top_k : V;
+struct PipelineLds {
+    float red[16];
+    float scan[kSampleThreads];
+    int found;
+    int counter;
+    int bins[kHeadBins];
+    uint64_t head[kHeadMax];
+};
 
+// the token of one row, or -1 where it has to be sorted whole and sort_here is not set
+__device__ int row_token(PipelineLds& s, float* work, float* prob, int V, uint64_t* list, int n_pad, float u,
+                         const SampleParams& sp, int try_head, int sort_here) {
+    const int n = (sp.top_k > 0 && sp.top_k < V) ? sp.top_k : V;
     if (try_head && (n <= kHeadMax / 2 || n == V)) {
         bool complete = false;
-        const int n_head = sorted_head(head, work, V, min(n, kHeadMax / 2), red, scan, bins, &counter, &complete);
+        const int n_head = sorted_head(s.head, work, V, min(n, kHeadMax / 2), s.red, s.scan, s.bins, &s.counter, &complete);
         if (n_head > 0) {
             // a complete head holds every candidate that can be drawn: the rest count for nothing
-            const int token = pipeline_on_sorted(head, n_head, complete ? min(n, n_head) : n, work,
-                                                 prob_all + (size_t)r * V, V, sp, u, red, scan, &found);
-            if (token >= 0) {
-                if (threadIdx.x == 0) out[r] = token;
-                return;
-            }
+            const int token = pipeline_on_sorted(s.head, n_head, complete ? min(n, n_head) : n, work, prob, V, sp, u, s.red, s.scan, &s.found);
+            if (token >= 0) return token;
         }
         __syncthreads();
     }
-    if (!sort_here) {
-        if (threadIdx.x == 0) out[r] = -1;
-        return;
-    }
+    if (!sort_here) return -1;
     // 1. all tokens in descending order of their scaled logit, lower id first among equals;
     //    the first k of them are the candidates (Sampler.cs:249-276)
-    uint64_t* list = list_all + (size_t)r * n_pad;
     for (int i = threadIdx.x; i < n_pad; i += blockDim.x)
         list[i] = i < V ? desc_key(work[i], i) : ~(uint64_t)0;
     __syncthreads();
     bitonic_sort(list, n_pad);
-    const int token = pipeline_on_sorted(list, V, n, work, work, V, sp, u, red, scan, &found);
+    return pipeline_on_sorted(list, V, n, work, work, V, sp, u, s.red, s.scan, &s.found);
+}
+
+__global__ __launch_bounds__(kSampleThreads) void sample_pipeline_kernel(
+        int* __restrict__ out, float* __restrict__ work_all, float* __restrict__ prob_all, int V,
+        uint64_t* __restrict__ list_all, int n_pad, const float* __restrict__ uniforms, SampleParams sp,
+        int try_head, int sort_here) {
+    __shared__ PipelineLds s;
+    const int r = blockIdx.x;
+    const int token = row_token(s, work_all + (size_t)r * V, prob_all + (size_t)r * V, V, list_all + (size_t)r * n_pad, n_pad,
+                                uniforms[r], sp, try_head, sort_here);
+    if (threadIdx.x == 0) out[r] = token;
+}
+
+// ---- few candidates (top-k up to kFewCandidates): a row is read once, by many blocks.
+//
+// One block a row (the kernels above: a pass that prepares the row, then three that look for its head) left three quarters of
+// the compute units idle at 64 rows and moved each row five times.  Here a block takes a slice of a row, prepares it in
+// registers (the tokens that penalties touch are patched through LDS) and keeps what may be among the row's first top-k:
+// every value in the slice's first bins, by the same histogram of the distance to the largest that sorted_head uses, but the
+// slice's own largest.  A second kernel, one block a row, cuts the slices' lists (some tens of keys each) the same way against
+// the row's largest, sorts what is left and draws.  Up to 64 candidates one wave does steps 2 to 6 without a barrier; its sums
+// are the additions of the block's in the same order.  Whatever these lists cannot decide (an infinite value, thousands of
+// values within a bin) is done again by the row's block in the general way.
+// 64 rows of 128,256 logits, top-k 40, penalties: 76 us in the two kernels above, 31 here (one row: 65 and 18;
+// top-k 256: 87 and 39).  Twice or four times as many, shorter slices at 64 rows: 35 and 42 us.
+constexpr int kFewCandidates = 256;      // largest top-k served
+constexpr int kSliceThreads = 512;
+constexpr int kSliceCap = 1024;          // keys a slice can hand on
+
+// the first bin up to which `want` values lie, of counts of kHeadBins bins, by a block of THREADS; the last bin does not
+// count.  *total: values up to it, *outside: all counted (0: none, then -1 comes back).  part: 16 ints of LDS, cut: 2.
+template <int THREADS>
+__device__ int cut_bin(const int* bins, int want, int* part, int* cut, int* total, int* outside) {
+    constexpr int PER = kHeadBins / THREADS;
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    int c[PER], mine = 0;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const int b = threadIdx.x * PER + i;
+        c[i] = b < kHeadBins - 1 ? bins[b] : 0;
+        mine += c[i];
+    }
+    int incl = mine;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+        const int add = __shfl_up(incl, o, kWave);
+        if (lane >= o) incl += add;
+    }
+    if (lane == kWave - 1) part[wave] = incl;
+    if (threadIdx.x == 0) { cut[0] = -1; cut[1] = 0; }
+    __syncthreads();
+    int before = 0, all = 0;
+#pragma unroll
+    for (int w = 0; w < THREADS / kWave; ++w) {
+        if (w < wave) before += part[w];
+        all += part[w];
+    }
+    want = min(want, all);
+    int run = before + incl - mine;
+    if (want > 0 && run < want && run + mine >= want) {
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            if (run < want && run + c[i] >= want) { cut[0] = threadIdx.x * PER + i; cut[1] = run + c[i]; }
+            run += c[i];
+        }
+    }
+    __syncthreads();
+    *total = cut[1];
+    *outside = all;
+    return cut[0];
+}
+
+// grid (slices, rows).  VPT values a thread.  counts, tops: [rows][slices]; keys: [rows][slices][kSliceCap].  count -1: more
+// than kSliceCap keys, or a largest value that is not finite.  hist_at (or null): row r's window is hist[hist_at[r] .. hist_at[r + 1]).
+template <int VPT>
+__global__ __launch_bounds__(kSliceThreads) void sample_slices_kernel(
+        uint64_t* __restrict__ keys, int* __restrict__ counts, float* __restrict__ tops, const float* __restrict__ logits, int V,
+        const int* __restrict__ hist, const int* __restrict__ hist_at, PenaltyParams pp, int top_k) {
+    constexpr int kSlice = VPT * kSliceThreads;
+    constexpr int kLds = kSlice > kHeadBins ? kSlice : kHeadBins;
+    __shared__ __attribute__((aligned(16))) int lds[kLds];        // the slice's values while they are patched, then the bins
+    __shared__ float red[16];
+    __shared__ int part[16], cut[2], counter;
+    __shared__ WindowLds window;
+    const int s = blockIdx.x, r = blockIdx.y, at = r * gridDim.x + s;
+    const float* row = logits + (size_t)r * V;
+    const int first = s * kSlice, count = min(kSlice, V - first);
+    const float inv_t = pp.inv_temperature;
+    const bool scaled = inv_t != 1.0f;
+    const bool wide = (V & 3) == 0 && ((uintptr_t)logits & 15) == 0;   // then four neighbours a load, else threads side by side
+    auto place = [&](int j) { return wide ? ((j >> 2) * kSliceThreads + threadIdx.x) * 4 + (j & 3) : j * kSliceThreads + (int)threadIdx.x; };
+    float v[VPT];
+    if (wide) {
+#pragma unroll
+        for (int j = 0; j < VPT; j += 4) {
+            const int i = place(j);
+            float4 t = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
+            if (i < count) t = *reinterpret_cast<const float4*>(row + first + i);
+            v[j] = t.x; v[j + 1] = t.y; v[j + 2] = t.z; v[j + 3] = t.w;
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < VPT; ++j) v[j] = place(j) < count ? row[first + place(j)] : -INFINITY;
+    }
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) v[j] = scaled ? v[j] * inv_t : v[j];
+    const bool penalties = has_penalties(pp) && hist_at != nullptr;
+    if (penalties || pp.n_banned > 0) {
+        float* vals = reinterpret_cast<float*>(lds);
+        if (wide) {
+#pragma unroll
+            for (int j = 0; j < VPT; j += 4) *reinterpret_cast<float4*>(vals + place(j)) = make_float4(v[j], v[j + 1], v[j + 2], v[j + 3]);
+        } else {
+#pragma unroll
+            for (int j = 0; j < VPT; ++j) vals[place(j)] = v[j];
+        }
+        if (penalties) {
+            apply_penalties(vals, row, first, count, V, hist + hist_at[r], hist_at[r + 1] - hist_at[r], pp, window);
+        }
+        __syncthreads();
+        if (threadIdx.x < pp.n_banned) {
+            const int tok = pp.banned[threadIdx.x] - first;
+            if (tok >= 0 && tok < count) vals[tok] = -INFINITY;
+        }
+        __syncthreads();
+        if (wide) {
+#pragma unroll
+            for (int j = 0; j < VPT; j += 4) {
+                const float4 t = *reinterpret_cast<const float4*>(vals + place(j));
+                v[j] = t.x; v[j + 1] = t.y; v[j + 2] = t.z; v[j + 3] = t.w;
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < VPT; ++j) v[j] = vals[place(j)];
+        }
+    }
+    float m = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) m = fmaxf(m, v[j]);              // (places past the slice hold -inf)
+    const float top = block_max(m, red);
+    if (!(top > -INFINITY && top < INFINITY)) {
+        if (threadIdx.x == 0) { counts[at] = top < INFINITY ? 0 : -1; tops[at] = top; }
+        return;
+    }
+    // The top_k largest of the threads' own largest values bound the slice's top_k from below: counting those alone (a
+    // sixteenth of the values) cuts the slice nearly as short.  Where fewer than top_k threads hold a value that counts, or the
+    // list would overflow, all values are counted.
+    bool fits = false;
+    int total = 0;
+#pragma unroll 1
+    for (int all = 0; all < 2 && !fits; ++all) {
+        __syncthreads();
+        for (int i = threadIdx.x; i < kHeadBins; i += kSliceThreads) lds[i] = 0;
+        if (threadIdx.x == 0) counter = 0;
+        __syncthreads();
+        if (all) {
+#pragma unroll
+            for (int j = 0; j < VPT; ++j) {
+                const int b = head_bin(top, v[j]);
+                if (b < kHeadBins - 1) atomicAdd(&lds[b], 1);
+            }
+        } else {
+            const int b = head_bin(top, m);
+            if (b < kHeadBins - 1) atomicAdd(&lds[b], 1);
+        }
+        __syncthreads();
+        int outside;
+        const int last = cut_bin<kSliceThreads>(lds, top_k, part, cut, &total, &outside);
+        if (all ? total > kSliceCap : outside < top_k) continue;
+#pragma unroll
+        for (int j = 0; j < VPT; ++j)
+            if (head_bin(top, v[j]) <= last) {
+                const int slot = atomicAdd(&counter, 1);
+                if (slot < kSliceCap) keys[(size_t)at * kSliceCap + slot] = desc_key(v[j], first + place(j));
+            }
+        __syncthreads();
+        total = counter;
+        fits = total <= kSliceCap;
+    }
+    if (threadIdx.x == 0) { counts[at] = fits ? total : -1; tops[at] = top; }
+}
+
+__device__ __forceinline__ float key_value(uint64_t k) {            // of a desc_key (-0 comes back as 0)
+    const uint32_t o = ~(uint32_t)(k >> 32);
+    return __uint_as_float(o & 0x80000000u ? o & 0x7fffffffu : ~o);
+}
+
+// Steps 2, 3, 5 and 6 of pipeline_on_sorted for n <= 64 PER candidates, sorted in head, by one wave: value j of lane l is the
+// (64 j + l)-th.  The same sums in the same order: a wave's sums one after the other as block_sum adds them, and the scan over
+// the values step by step.
+template <int PER>
+__device__ int pipeline_on_wave(const uint64_t* head, int n, const SampleParams& sp, float u) {
+    const int lane = threadIdx.x & (kWave - 1);
+    const int keep = max(sp.min_keep, 1);
+    const float top = key_value(head[0]);
+    float x[PER], p[PER];
+#pragma unroll
+    for (int j = 0; j < PER; ++j) x[j] = key_value(head[min(j * kWave + lane, n - 1)]);
+    auto sum_of = [&](const float (&f)[PER]) {
+        float t = 0.f;
+#pragma unroll
+        for (int j = 0; j < PER; ++j) t += wave_sum(j * kWave + lane < n ? f[j] : 0.f);
+        return t;
+    };
+    if (sp.min_p > 0.f && sp.min_p < 1.f && n > keep) {
+        const float thr = top + logf(sp.min_p);
+        int kept = 0;
+#pragma unroll
+        for (int j = 0; j < PER; ++j) kept += (int)__popcll(__ballot(j * kWave + lane < n && x[j] >= thr));
+        n = max(keep, kept);
+    }
+#pragma unroll
+    for (int j = 0; j < PER; ++j) p[j] = expf(x[j] - top);
+    const float inv = 1.0f / sum_of(p);
+#pragma unroll
+    for (int j = 0; j < PER; ++j) p[j] = expf(x[j] - top) * inv;
+    auto crossing = [&](int from, float target) {                    // first i >= from whose running sum exceeds target
+        float incl[PER];
+#pragma unroll
+        for (int j = 0; j < PER; ++j) incl[j] = j * kWave + lane < n ? p[j] : 0.f;
+#pragma unroll
+        for (int o = 1; o < PER * kWave; o <<= 1) {
+            float add[PER];
+#pragma unroll
+            for (int j = 0; j < PER; ++j) {
+                if (o >= kWave) add[j] = j >= o / kWave ? incl[j - o / kWave] : 0.f;
+                else {
+                    const float same = __shfl(incl[j], lane - o, kWave), before = j > 0 ? __shfl(incl[j - 1], lane - o + kWave, kWave) : 0.f;
+                    add[j] = lane >= o ? same : before;
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < PER; ++j) incl[j] += add[j];
+        }
+        int first = -1;
+#pragma unroll
+        for (int j = PER - 1; j >= 0; --j) {
+            const int i = j * kWave + lane;
+            const float own = i < n ? p[j] : 0.f;
+            float run = incl[j] - own;
+            run += own;
+            const uint64_t hits = __ballot(i < n && i >= from && run > target);
+            if (hits) first = j * kWave + __ffsll((unsigned long long)hits) - 1;
+        }
+        return first;
+    };
+    if (sp.top_p > 0.f && sp.top_p < 1.f) {
+        const int cut = crossing(keep - 1, sp.top_p);
+        if (cut >= 0) n = cut + 1;
+        const float sum = sum_of(p);
+        if (sum > 0.f) {
+#pragma unroll
+            for (int j = 0; j < PER; ++j) p[j] *= 1.0f / sum;
+        }
+    }
+    const int pick = crossing(0, u);
+    return key_id(head[pick >= 0 ? pick : 0]);
+}
+
+// One block a row.  work, prob [rows][V] and list [rows][n_pad]: scratch that is written only where a row has to be done in the
+// general way, or for typical-p.
+__global__ __launch_bounds__(kSampleThreads) void sample_few_kernel(
+        int* __restrict__ out, const uint64_t* __restrict__ keys, const int* __restrict__ counts, const float* __restrict__ tops, int slices,
+        const float* __restrict__ logits, int V, const int* __restrict__ hist, const int* __restrict__ hist_at, PenaltyParams pp,
+        float* __restrict__ work_all, float* __restrict__ prob_all, uint64_t* __restrict__ list_all, int n_pad,
+        const float* __restrict__ uniforms, SampleParams sp) {
+    __shared__ PipelineLds s;
+    __shared__ WindowLds window;
+    __shared__ int part[16], cut[2], slice_at[kWave + 1];
+    const int r = blockIdx.x, lane = threadIdx.x & (kWave - 1);
+    float* work = work_all + (size_t)r * V;
+    float* prob = prob_all + (size_t)r * V;
+    const float u = uniforms[r];
+    for (int i = threadIdx.x; i < kHeadBins; i += kSampleThreads) s.bins[i] = 0;
+    if (threadIdx.x == 0) s.counter = 0;
+    // where each slice's keys go among the row's (slices <= kWave): every wave for itself, the first one for all
+    const int mine = lane < slices ? counts[(size_t)r * slices + lane] : 0;
+    const float top = wave_max(lane < slices ? tops[(size_t)r * slices + lane] : -INFINITY);
+    const bool lost = __any(mine < 0) || !(top > -INFINITY && top < INFINITY);
+    int incl = max(mine, 0);
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+        const int add = __shfl_up(incl, o, kWave);
+        if (lane >= o) incl += add;
+    }
+    const int n_keys = __shfl(incl, kWave - 1, kWave);
+    if (threadIdx.x < kWave) slice_at[lane + 1] = incl;
+    if (threadIdx.x == 0) slice_at[0] = 0;
+    __syncthreads();
+    constexpr int PER = kWave * kFewCandidates / kSampleThreads;     // as many keys as slices of kFewCandidates each bring, for one
+    if (!lost && n_keys <= PER * kSampleThreads) {
+        uint64_t key[PER];
+        int bin[PER];
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            const int i = j * kSampleThreads + threadIdx.x;
+            bin[j] = kHeadBins;
+            if (i < n_keys) {
+                int at = 0;                                          // the slice whose run holds i: slice_at[at] <= i < slice_at[at + 1]
+#pragma unroll
+                for (int step = kWave / 2; step > 0; step >>= 1) if (slice_at[at + step] <= i) at += step;
+                key[j] = keys[((size_t)r * slices + at) * kSliceCap + (i - slice_at[at])];
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            if (j * kSampleThreads + (int)threadIdx.x >= n_keys) break;
+            bin[j] = head_bin(top, key_value(key[j]));
+            if (bin[j] < kHeadBins - 1) atomicAdd(&s.bins[bin[j]], 1);
+        }
+        __syncthreads();
+        int total, outside;
+        const int last = cut_bin<kSampleThreads>(s.bins, sp.top_k, part, cut, &total, &outside);
+        if (total <= kHeadMax) {
+        const int n = min(sp.top_k, total);                          // fewer only where fewer have a probability that is not 0
+        // the keys up to that bin, in any order, then each to its rank (all keys differ)
+        uint64_t* some = total <= kHeadMax / 2 ? s.head + kHeadMax / 2 : s.head;
+#pragma unroll
+        for (int j = 0; j < PER; ++j)
+            if (bin[j] <= last) some[atomicAdd(&s.counter, 1)] = key[j];
+        __syncthreads();
+        if (total <= kSampleThreads) {
+            if (threadIdx.x < total) {
+                const uint64_t k = some[threadIdx.x];
+                int rank = 0;
+                for (int i = 0; i < total; ++i) rank += some[i] < k;
+                s.head[rank] = k;
+            }
+            __syncthreads();
+        } else {
+            if (some != s.head) {
+                for (int i = threadIdx.x; i < total; i += kSampleThreads) s.head[i] = some[i];
+                __syncthreads();
+            }
+            int np2 = 1;
+            while (np2 < total) np2 <<= 1;
+            for (int i = total + threadIdx.x; i < np2; i += kSampleThreads) s.head[i] = ~(uint64_t)0;
+            __syncthreads();
+            bitonic_sort(s.head, np2);
+        }
+        int token;
+        if (!(sp.typical_p > 0.f && sp.typical_p < 1.f)) {
+            if (threadIdx.x >= kWave) return;
+            token = n <= kWave ? pipeline_on_wave<1>(s.head, n, sp, u) : n <= 2 * kWave ? pipeline_on_wave<2>(s.head, n, sp, u)
+                                                                                      : pipeline_on_wave<kFewCandidates / kWave>(s.head, n, sp, u);
+        } else {
+            for (int i = threadIdx.x; i < n; i += kSampleThreads) work[key_id(s.head[i])] = key_value(s.head[i]);
+            __syncthreads();
+            token = pipeline_on_sorted(s.head, total, n, work, prob, V, sp, u, s.red, s.scan, &s.found);
+        }
+        if (threadIdx.x == 0) out[r] = token;
+        return;
+        }
+    }
+    prepare_row(work, logits + (size_t)r * V, V, hist_at ? hist + hist_at[r] : nullptr, hist_at ? hist_at[r + 1] - hist_at[r] : 0, pp, window);
+    __syncthreads();
+    const int token = row_token(s, work, prob, V, list_all + (size_t)r * n_pad, n_pad, u, sp, 1, 1);
     if (threadIdx.x == 0) out[r] = token;
 }
 
@@ -580,5 +961,45 @@ LLOGOS_EXPORT int llogos_sample_pipeline(int* out, float* work, float* prob, int
         }
         sample_sorted_kernel<<<R, kSampleThreads, 0, stream>>>(out, work, V, keys, n_pad, uniforms, sp);
     }
+    return LLOGOS_LAUNCH_CHECK();
+}
+
+// values a slice: small ones where there are few rows, at most kWave slices a row and no more keys of a row than sample_few_kernel takes
+static int slice_values(int R, int V, int top_k) {
+    auto slices = [&](int vpt) { return (V + vpt * kSliceThreads - 1) / (vpt * kSliceThreads); };
+    int vpt = 4;
+    while (vpt < 16 && ((long long)R * slices(vpt) > 1024 || slices(vpt) > kWave || slices(vpt) * top_k > kWave * kFewCandidates / 2)) vpt *= 2;
+    return vpt * kSliceThreads;
+}
+
+// slices a row for sample_few, 0: not served (the entry below then refuses too)
+LLOGOS_EXPORT int llogos_sample_few_slices(int R, int V, int top_k) {
+    if (R <= 0 || V <= 0 || top_k <= 0 || top_k > kFewCandidates || top_k >= V) return 0;
+    const int values = slice_values(R, V, top_k), slices = (V + values - 1) / values;
+    return slices <= kWave ? slices : 0;
+}
+
+LLOGOS_EXPORT int llogos_sample_few_cap(void) { return kSliceCap; }
+
+// Preparation and pipeline of rows of which at most top_k <= kFewCandidates tokens can be drawn: the tokens that llogos_sample_prepare
+// and llogos_sample_pipeline give.  keys [R][slices][cap] uint64, counts [R][slices], tops [R][slices]: scratch; work, prob [R][V] and
+// list [R][n_pad]: scratch of the rows that need the general way.  hist_at (or null): offsets [R + 1] of the rows' windows in hist.
+LLOGOS_EXPORT int llogos_sample_few(int* out, const float* logits, int R, int V, const int* hist, const int* hist_at,
+                                    float repetition, float frequency, float presence, float inv_temperature,
+                                    int penalize_newline, const int* banned, int n_banned, void* keys, int* counts, float* tops,
+                                    float* work, float* prob, void* list, int n_pad, const float* uniforms, int top_k, float top_p,
+                                    float min_p, float typical_p, int min_keep, hipStream_t stream) {
+    const int slices = llogos_sample_few_slices(R, V, top_k);
+    if (slices == 0 || n_banned < 0 || n_banned > kMaxBanned || n_pad < V || (n_pad & (n_pad - 1))) return LLOGOS_BAD_ARGUMENT;
+    PenaltyParams pp{repetition, frequency, presence, inv_temperature, penalize_newline, n_banned, {}};
+    for (int i = 0; i < n_banned; ++i) pp.banned[i] = banned[i];
+    const SampleParams sp{top_k, top_p, min_p, typical_p, min_keep};
+    const dim3 grid(slices, R);
+#define GO(VPT) sample_slices_kernel<VPT><<<grid, kSliceThreads, 0, stream>>>((uint64_t*)keys, counts, tops, logits, V, hist, hist_at, pp, top_k)
+    const int vpt = slice_values(R, V, top_k) / kSliceThreads;
+    if (vpt == 4) GO(4); else if (vpt == 8) GO(8); else GO(16);
+#undef GO
+    sample_few_kernel<<<R, kSampleThreads, 0, stream>>>(out, (const uint64_t*)keys, counts, tops, slices, logits, V, hist, hist_at, pp,
+                                                        work, prob, (uint64_t*)list, n_pad, uniforms, sp);
     return LLOGOS_LAUNCH_CHECK();
 }

@@ -36,10 +36,12 @@ class Sampler:
         p = self.params
         if p.is_greedy:
             return K.argmax(logits)
+        if p.has_penalties and histories is None:
+            raise ValueError("penalties need each row's token history")
+        if p.temperature > 0 and logits.dim() == 2 and logits.is_contiguous() and K.sample_few_serves(*logits.shape, p.top_k):
+            return self._sample_few(logits, requests, indices, histories)
         arrays = []
         if p.has_penalties:
-            if histories is None:
-                raise ValueError("penalties need each row's token history")
             win = [list(h[-p.penalty_count:]) if 0 < p.penalty_count < len(h) else list(h) for h in histories]
             width = max(1, max(len(w) for w in win))
             arr = np.zeros((len(win), width), dtype=np.int32)
@@ -56,6 +58,18 @@ class Sampler:
         if p.temperature == 0:
             return K.argmax(work)
         return K.sample_pipeline(work, staged[-1], p.top_k, p.top_p, p.min_p, p.typical_p, p.min_keep)
+
+    def _sample_few(self, logits: torch.Tensor, requests, indices, histories) -> torch.Tensor:
+        """The same for a small top-k, whose rows two kernels take from the logits to the token."""
+        p = self.params
+        arrays = [np.asarray(self.uniforms(requests, indices), dtype=np.float32)]
+        if p.has_penalties:
+            win = [np.asarray(h[-p.penalty_count:] if 0 < p.penalty_count < len(h) else h, dtype=np.int32).reshape(-1) for h in histories]
+            arrays += [np.cumsum([0] + [len(w) for w in win], dtype=np.int32), np.concatenate(win + [np.zeros(1, np.int32)])]
+        staged = self._to_device(arrays, logits.device)
+        at, hist = (staged[1], staged[2]) if p.has_penalties else (None, None)
+        return K.sample_few(logits, hist, at, p.repetition_penalty, p.frequency_penalty, p.presence_penalty, p.temperature, p.penalize_newline,
+                            self.stop_tokens if p.prevent_eos else (), staged[0], p.top_k, p.top_p, p.min_p, p.typical_p, p.min_keep)
 
     def _to_device(self, arrays, device) -> List[torch.Tensor]:
         """The step's small host arrays (int32 or float32) on the device with one copy, without

@@ -358,3 +358,60 @@ def test_zeros_of_either_sign_are_equal_logits():
         head, whole, single = _every_way(rows, us, repetition_penalty=1.0, **opts)
         p = S.GenerationParams(repetition_penalty=1.0, **opts)
         assert head == whole == single == _plain(row, p, us), opts
+
+
+@pytest.mark.parametrize("R,V", [(1, 41), (3, 2048), (5, 2049), (64, 8192), (2, 32000), (7, 50257), (64, 128256), (1, 151936)])
+@pytest.mark.parametrize("opts", [
+    dict(temperature=0.7, top_k=40, top_p=0.9, repetition_penalty=1.1),
+    dict(temperature=1.0, top_k=1, top_p=1.0, repetition_penalty=1.0),
+    dict(temperature=1.3, top_k=64, top_p=0.95, repetition_penalty=0.8, min_p=0.02, min_keep=3, penalize_newline=True),
+    dict(temperature=0.9, top_k=65, top_p=1.0, repetition_penalty=1.0, frequency_penalty=0.3, presence_penalty=0.2, penalty_count=0),
+    dict(temperature=0.8, top_k=256, top_p=0.8, repetition_penalty=1.2, penalty_count=7),
+    dict(temperature=0.8, top_k=40, top_p=0.9, repetition_penalty=1.0, typical_p=0.7),
+    dict(temperature=1.1, top_k=40, top_p=0.99, repetition_penalty=1.1, prevent_eos=True),
+])
+def test_few_candidates_draw_what_the_general_way_draws(R, V, opts):
+    """Slices of rows and one wave's pipeline against a block a row: the same tokens, whatever the row: ordinary, with ties
+    across a slice's end, one value throughout (every list overflows), next to nothing in some slices, infinities and NaN."""
+    K = importlib.import_module("daisi-llogos_amd.ops.kernels")
+    if opts["top_k"] >= V:
+        pytest.skip("every token is a candidate")
+    rng = np.random.default_rng(V + R)
+    p = S.GenerationParams(seed=5, **opts)
+    stop = (3, V - 1) if p.prevent_eos else ()
+    assert K.sample_few_serves(R, V, p.top_k)
+    histories = [rng.integers(0, V, size=int(n)).tolist() for n in rng.integers(0, 100, size=R)]
+    histories[0] = [10, 13, 0, V - 1, 0, 0, 10]
+    kinds = ["ordinary", "ties", "flat", "sparse", "infinite", "nan", "steep"]
+    for at in range(0, len(kinds) if R < len(kinds) else 1, 1):
+        x = rng.standard_normal((R, V)).astype(np.float32) * 3
+        for r in range(R):
+            kind = kinds[(r + at) % len(kinds)]
+            if kind == "ties":
+                x[r] = np.round(x[r])
+            elif kind == "flat" and V <= 8192:
+                x[r] = 1.5
+            elif kind == "sparse":
+                x[r, rng.random(V) < 0.999] = -np.inf
+                x[r, V // 2] = 0.25
+            elif kind == "infinite" and V <= 8192:
+                x[r, V // 3] = np.inf
+            elif kind == "nan":
+                x[r, 1::7] = np.nan
+            elif kind == "steep":
+                x[r] *= 60
+        logits = torch.tensor(x, device=DEV)
+        for step in range(3):
+            us = torch.tensor(S.Sampler(p).uniforms(list(range(R)), [step] * R), dtype=torch.float32, device=DEV)
+            got = S.Sampler(p, stop).sample(logits, list(range(R)), [step] * R, histories)
+            hist = hist_len = None
+            if p.has_penalties:
+                win = [h[-p.penalty_count:] if 0 < p.penalty_count < len(h) else h for h in histories]
+                padded = np.zeros((R, max(1, max(map(len, win)))), np.int32)
+                for i, w in enumerate(win):
+                    padded[i, :len(w)] = w
+                hist, hist_len = torch.tensor(padded, device=DEV), torch.tensor([len(w) for w in win], dtype=torch.int32, device=DEV)
+            work = K.sample_prepare(logits, hist, hist_len, p.repetition_penalty, p.frequency_penalty, p.presence_penalty, p.temperature,
+                                    p.penalize_newline, stop)
+            want = K.sample_pipeline(work, us, p.top_k, p.top_p, p.min_p, p.typical_p, p.min_keep)
+            assert got.cpu().tolist() == want.cpu().tolist(), (at, step)
