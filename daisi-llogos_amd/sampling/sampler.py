@@ -4,6 +4,7 @@ The pipeline is the reference's (Daisi.Llogos/Inference/Sampler.cs:26-85): greed
 penalties, temperature, top-k, min-p, softmax over candidates, typical-p, top-p, draw."""
 from __future__ import annotations
 
+import struct
 from typing import List, Optional, Sequence
 
 import numpy as np
@@ -11,7 +12,7 @@ import torch
 
 from ..ops import kernels as K
 from .params import GenerationParams
-from .rng import uniform
+from .rng import uniforms
 
 
 class Sampler:
@@ -26,7 +27,7 @@ class Sampler:
 
     def uniforms(self, requests: Sequence[int], indices: Sequence[int]) -> List[float]:
         seed = self.params.seed if self.params.seed is not None else self._fresh_seed
-        return [uniform(seed, r, i) for r, i in zip(requests, indices)]
+        return uniforms(seed, requests, indices)
 
     def sample(self, logits: torch.Tensor, requests: Sequence[int], indices: Sequence[int],
                histories: Optional[Sequence[Sequence[int]]] = None) -> torch.Tensor:
@@ -62,14 +63,43 @@ class Sampler:
     def _sample_few(self, logits: torch.Tensor, requests, indices, histories) -> torch.Tensor:
         """The same for a small top-k, whose rows two kernels take from the logits to the token."""
         p = self.params
-        arrays = [np.asarray(self.uniforms(requests, indices), dtype=np.float32)]
+        R = logits.shape[0]
+        us = self.uniforms(requests, indices)
+        flat, at = [], [0]
         if p.has_penalties:
-            win = [np.asarray(h[-p.penalty_count:] if 0 < p.penalty_count < len(h) else h, dtype=np.int32).reshape(-1) for h in histories]
-            arrays += [np.cumsum([0] + [len(w) for w in win], dtype=np.int32), np.concatenate(win + [np.zeros(1, np.int32)])]
-        staged = self._to_device(arrays, logits.device)
-        at, hist = (staged[1], staged[2]) if p.has_penalties else (None, None)
-        return K.sample_few(logits, hist, at, p.repetition_penalty, p.frequency_penalty, p.presence_penalty, p.temperature, p.penalize_newline,
-                            self.stop_tokens if p.prevent_eos else (), staged[0], p.top_k, p.top_p, p.min_p, p.typical_p, p.min_keep)
+            for h in histories:
+                flat += h[-p.penalty_count:] if 0 < p.penalty_count < len(h) else h
+                at.append(len(flat))
+        # one copy: uniform numbers, then each window's place and the windows, packed straight into the staging buffer
+        n = len(us) + len(at) + len(flat)
+        host, copied, numbers = self._staging_buffer(n)
+        try:
+            struct.pack_into(f"={len(us)}f{len(at) + len(flat)}i", numbers, 0, *us, *at, *flat)
+        except (struct.error, TypeError):                # (tokens that are no whole numbers: as numpy rounds them)
+            view = np.frombuffer(numbers, dtype=np.int32)
+            view[:len(us)] = np.asarray(us, dtype=np.float32).view(np.int32)
+            view[len(us):len(us) + len(at)] = at
+            view[len(us) + len(at):n] = flat
+        dev = torch.empty(n, dtype=torch.int32, device=logits.device)
+        dev.copy_(host[:n], non_blocking=True)
+        copied.record()
+        hist, hist_at = (dev[len(us) + len(at):], dev[len(us):len(us) + len(at)]) if p.has_penalties else (None, None)
+        return K.sample_few(logits, hist, hist_at, p.repetition_penalty, p.frequency_penalty, p.presence_penalty, p.temperature,
+                            p.penalize_newline, self.stop_tokens if p.prevent_eos else (), dev[:len(us)].view(torch.float32), p.top_k, p.top_p,
+                            p.min_p, p.typical_p, p.min_keep)
+
+    def _staging_buffer(self, n: int):
+        """A pinned buffer of at least n 32-bit numbers, the event to record behind its copy, and its memory as bytes: one of a
+        few, each free again once its last copy has run."""
+        ring = getattr(self, "_staging", None)
+        if ring is None or ring[0][0].numel() < n:
+            ring = self._staging = [(torch.empty(max(1024, 2 * n), dtype=torch.int32, pin_memory=True),
+                                     torch.cuda.Event()) for _ in range(4)]
+            self._staging_next = 0
+        host, copied = ring[self._staging_next]
+        self._staging_next = (self._staging_next + 1) % len(ring)
+        copied.synchronize()
+        return host, copied, memoryview(host.numpy()).cast("B")
 
     def _to_device(self, arrays, device) -> List[torch.Tensor]:
         """The step's small host arrays (int32 or float32) on the device with one copy, without
@@ -79,14 +109,7 @@ class Sampler:
         if not arrays:
             return []
         n = sum(a.size for a in arrays)
-        ring = getattr(self, "_staging", None)
-        if ring is None or ring[0][0].numel() < n:
-            ring = self._staging = [(torch.empty(max(1024, 2 * n), dtype=torch.int32, pin_memory=True),
-                                     torch.cuda.Event()) for _ in range(4)]
-            self._staging_next = 0
-        host, copied = ring[self._staging_next]
-        self._staging_next = (self._staging_next + 1) % len(ring)
-        copied.synchronize()
+        host, copied, _ = self._staging_buffer(n)
         flat = host.numpy()
         o = 0
         for a in arrays:

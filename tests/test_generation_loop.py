@@ -217,3 +217,16 @@ def test_prevent_eos_refuses_more_stop_tokens_than_the_kernel_bans():
     with pytest.raises(ValueError, match="at most 64"):
         sampler_mod.Sampler(params, stop_tokens=range(65))
     sampler_mod.Sampler(GenerationParams(temperature=0.7), stop_tokens=range(100))      # only stops, nothing to ban
+
+
+def test_uniform_numbers_in_arrays_are_the_same():
+    """Batches of more than eight draw their numbers in arrays of 64-bit numbers: the same, whatever the request and index, also
+    beyond 64 bits and below zero, where the plain form masks."""
+    rng = importlib.import_module("daisi-llogos_amd.sampling.rng")
+    numbers = [0, 1, 7, 63, 2**31, 2**40 + 3, 2**62, 2**63 - 1, -1, -2**63, 12345678901, 5]
+    for seed in (0, 1234, 2**63 + 5, -3, 2**70):
+        want = [rng.uniform(seed, r, i) for r, i in zip(numbers, reversed(numbers))]
+        assert rng.uniforms(seed, numbers, list(reversed(numbers))) == want
+        wide = numbers + [2**64 + 9]
+        assert rng.uniforms(seed, wide, wide) == [rng.uniform(seed, r, r) for r in wide]
+    assert rng.uniforms(3, [4], [5]) == [rng.uniform(3, 4, 5)] and rng.uniforms(3, [], []) == []
