@@ -204,6 +204,24 @@ __device__ __forceinline__ void weigh_values(WaveState<HD>& st, const bf16x8 (&v
 // many of the page's keys have been written (the rest of the page holds whatever was there
 // before: such scores are masked, and such values are zeroed because 0 * NaN is NaN).
 template <int HD>
+__device__ __forceinline__ void attend_loaded(WaveState<HD>& st, const bf16x8 (&qf)[HD / 32], const bf16x8 (&kf)[4][HD / 32],
+                                              const bf16x8 (&vf)[HD / 16][2], int q_pos, int key0, int valid_keys, bool all_visible,
+                                              float scale_log2, int window, int sinks) {
+    f32x4 s[4];
+    page_scores<HD>(s, kf, qf);
+    bf16x8 pf[2];
+    float corr;
+    if (!all_visible) {                                                   // (masked here and not in a second copy of the softmax)
+        const int g = (threadIdx.x & (kWave - 1)) >> 4;
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            if (!(q_pos >= 0 && key_visible(q_pos, key0 + 16 * g + i, window, sinks))) s[i >> 2][i & 3] = -INFINITY;
+    }
+    softmax_page<false, 16, 4, HD>(s, st, scale_log2, q_pos, key0, window, sinks, pf, corr);
+    weigh_values<HD>(st, vf, pf, corr, valid_keys);
+}
+
+template <int HD>
 __device__ __forceinline__ void attend_page(WaveState<HD>& st, const bf16x8 (&qf)[HD / 32],
                                             const bf16_t* __restrict__ kpage, const bf16_t* __restrict__ vpage,
                                             int q_pos, int key0, int valid_keys, bool all_visible,
@@ -212,13 +230,7 @@ __device__ __forceinline__ void attend_page(WaveState<HD>& st, const bf16x8 (&qf
     bf16x8 kf[4][HD / 32], vf[HD / 16][2];
     load_keys<HD>(kf, kpage);
     load_values<HD>(vf, vpage);
-    f32x4 s[4];
-    page_scores<HD>(s, kf, qf);
-    bf16x8 pf[2];
-    float corr;
-    if (all_visible) softmax_page<false, 16, 4, HD>(s, st, scale_log2, q_pos, key0, window, sinks, pf, corr);
-    else             softmax_page<true, 16, 4, HD>(s, st, scale_log2, q_pos, key0, window, sinks, pf, corr);
-    weigh_values<HD>(st, vf, pf, corr, valid_keys);
+    attend_loaded<HD>(st, qf, kf, vf, q_pos, key0, valid_keys, all_visible, scale_log2, window, sinks);
 }
 
 // Whether any key of the page [key0, key0 + 63] can be visible to a query at q_pos.

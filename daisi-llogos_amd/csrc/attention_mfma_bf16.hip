@@ -59,21 +59,86 @@ struct QkvSource {
     bf16_t* v_pool;
 };
 
+// What a step's projection gives one item (a query head, the step's key or its value): lane l's dimensions PER l ..
+// PER l + PER - 1 of up to eight partial products as they come from memory, added (ascending) when they are needed.
+template <int PER>
+struct QkvRow {
+    float y[8][PER];
+    // (a part there is none of is the last one read again: with a branch for each the loads wait for one another)
+    __device__ __forceinline__ void load(const float* p, int parts, size_t part_stride) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+            for (int e = 0; e < PER; ++e) y[i][e] = p[min(i, parts - 1) * part_stride + e];
+    }
+    __device__ __forceinline__ void sum(float (&x)[PER], const float* p, int parts, size_t part_stride) const {
+#pragma unroll
+        for (int e = 0; e < PER; ++e) x[e] = y[0][e];
+#pragma unroll
+        for (int i = 1; i < 8; ++i)
+            if (i < parts) {
+#pragma unroll
+                for (int e = 0; e < PER; ++e) x[e] += y[i][e];
+            }
+        for (int part = 8; part < parts; ++part)
+#pragma unroll
+            for (int e = 0; e < PER; ++e) x[e] += p[part * part_stride + e];
+    }
+};
+
+// The blocks of one (sequence, kv head) hand their partial results on without a kernel of their own: each writes its share
+// with stores that go through to memory (relaxed atomics of agent scope), waits until they have arrived, and takes a ticket;
+// the block with the last ticket reads all shares, past its L2, and adds them in the merge kernel's order.  Nobody waits
+// for another block.  Only the shares go through: a release fence would write back whatever earlier kernels left dirty in
+// the L2 (20 us a layer at batch 8); this takes as long as the merge kernel at two or three blocks and 3 us less at 24 (8
+// contexts of 4,100 to 8,190).  A sequence of one block, of up to 256 positions at the least, has nothing to hand on and takes
+// no ticket: 3 us a layer less.  A ticket counter goes back to zero with the last ticket (atomicInc wraps).
+// Tried too: blocks of 8 waves that take contexts of up to 1,024 whole, with nothing to hand on: level or 0.5 % slower steps.
+constexpr int kTicketBlocks = 64;                     // more blocks along the context than this go to the merge kernel
+
+__device__ __forceinline__ void store_through(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ float load_through(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+// a share's maximum and sum, which lie side by side (8-byte aligned: a share is HD + 2 floats)
+__device__ __forceinline__ float2 load_pair_through(const float* p) {
+    return __builtin_bit_cast(float2, __hip_atomic_load(reinterpret_cast<const unsigned long long*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+}
+
+constexpr int kMergeLanes = 4;                        // partial sums a merge adds by themselves: see attn_decode_merge_kernel
+
 template <int HD, int WAVES, bool FUSED>
 __global__ __launch_bounds__(WAVES * kWave) void attn_decode_kernel(
         bf16_t* __restrict__ out, float* __restrict__ partial, const bf16_t* __restrict__ q, int q_stride,
         QkvSource src, const bf16_t* k_pool, const bf16_t* v_pool,
         const int* __restrict__ table, int table_stride, const int* __restrict__ tok_pos,
-        int n_heads, int n_kv_heads, int group, float scale, int window, int sinks, int ppw) {
+        int n_heads, int n_kv_heads, int group, float scale, int window, int sinks, int ppw, unsigned* tickets) {
     extern __shared__ float lds[];
     float* lds_m = lds;                                   // [WAVES][16]
     float* lds_l = lds + WAVES * 16;                      // [WAVES][16]
     float* lds_o = lds + WAVES * 32;                      // [WAVES][group][HD + 1]
     __shared__ __attribute__((aligned(16))) bf16_t q_lds[FUSED ? 16 : 1][HD];
+    __shared__ __attribute__((aligned(16))) bf16_t kv_lds[2][HD];         // the step's key and value
+    __shared__ unsigned ticket;
     const int b = blockIdx.x, kvh = blockIdx.y, z = blockIdx.z;
-    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int c = lane & 15, g = lane >> 4;
+    constexpr int PER = HD / kWave;
+    static_assert(PER == 1 || PER == 2, "head sizes 64 and 128");
+    const int d = PER * lane;
+    // A block's first reads wait for one another (position, page table, page) unless they are asked for together: the
+    // wave's first two rows of the projection and the rotation need no position, and the first page is asked for before the queries are
+    // made.  (64 sequences of 30 to 400 positions: 2.2 us a launch of 20
+    // less; one of 211: 7.3 -> 6.9, of which a kernel that does nothing lasts some 3.)
     const int pos = tok_pos[b];
+    auto item_head = [&](int item) { return item < group ? kvh * group + item : (item == group ? n_heads : n_heads + n_kv_heads) + kvh; };
+    auto item_row = [&](int item) { return src.qkv + (size_t)b * src.row_stride + (size_t)item_head(item) * HD + d; };
+    QkvRow<PER> first, second;
+    float2 cs[PER];
+    if (FUSED) {
+        if (wave < group + 2) first.load(item_row(wave), src.parts, src.part_stride);
+        if (wave + WAVES < group + 2) second.load(item_row(wave + WAVES), src.parts, src.part_stride);
+#pragma unroll
+        for (int e = 0; e < PER; ++e) cs[e] = src.cs[(size_t)b * (HD / 2) + ((d + e) & (HD / 2 - 1))];
+    }
     const int n_pages = pos / kPageTokens + 1;
     const int first_page = z * WAVES * ppw;
     if (first_page >= n_pages) return;                           // nothing of this sequence here
@@ -88,72 +153,115 @@ __global__ __launch_bounds__(WAVES * kWave) void attn_decode_kernel(
     };
     auto page_base = [&](int j) { return ((size_t)row[page_at(j)] * n_kv_heads + kvh) * kPageTokens * HD; };
     int j = next_from(0);
+    bf16x8 kf[4][HD / 32], vf[HD / 16][2];                       // the wave's page
 
     if (FUSED) {
         // items 0 .. group - 1: the kv head's query heads; then, in the block that holds the
         // step's position, its key and its value.  A wave takes an item; lane l holds
         // dimensions PER l .. PER l + PER - 1 (two for head size 128, one for 64), and the
         // rotation partner, HD / 2 dimensions away, is lane l ^ 32.
-        constexpr int PER = HD / kWave;
-        static_assert(PER == 1 || PER == 2, "head sizes 64 and 128");
         const bool writer = (n_pages - 1) / (WAVES * ppw) == z;
         const int items = group + (writer ? 2 : 0);
-        const int d = PER * lane;
         const size_t wbase = writer ? ((size_t)row[n_pages - 1] * n_kv_heads + kvh) * kPageTokens * HD : 0;
-        for (int item = wave; item < items; item += WAVES) {
-            const bool is_q = item < group, is_k = item == group;
-            const int head = is_q ? kvh * group + item : (is_k ? n_heads + kvh : n_heads + n_kv_heads + kvh);
-            const size_t col = (size_t)head * HD + d;
-            const float* p = src.qkv + (size_t)b * src.row_stride + col;
-            float x[PER];
-#pragma unroll
-            for (int e = 0; e < PER; ++e) x[e] = p[e];
-            for (int part0 = 1; part0 < src.parts; part0 += 8) {     // eight loads in flight, added in ascending order
-                float y[8][PER];
-#pragma unroll
-                for (int jj = 0; jj < 8; ++jj)
-#pragma unroll
-                    for (int e = 0; e < PER; ++e)
-                        y[jj][e] = part0 + jj < src.parts ? p[(part0 + jj) * src.part_stride + e] : 0.f;
-#pragma unroll
-                for (int jj = 0; jj < 8; ++jj)
-                    if (part0 + jj < src.parts) {
-#pragma unroll
-                        for (int e = 0; e < PER; ++e) x[e] += y[jj][e];
-                    }
-            }
+        const size_t base = j >= 0 ? page_base(j) : 0;
+        // (everything that is read before the page is waited for before the page is asked for: one wait serves them all)
+        float x1[PER], x2[PER];
+        auto total = [&](float (&x)[PER], const QkvRow<PER>& from, int item) {
+            from.sum(x, item_row(item), src.parts, src.part_stride);
             if (src.bias) {
 #pragma unroll
-                for (int e = 0; e < PER; ++e) x[e] += src.bias[col + e];
+                for (int e = 0; e < PER; ++e) x[e] += src.bias[(size_t)item_head(item) * HD + d + e];
             }
+        };
+        if (wave < items) total(x1, first, wave);
+        if (wave + WAVES < items) total(x2, second, wave + WAVES);
+        float norm_q[PER], norm_k[PER];
+#pragma unroll
+        for (int e = 0; e < PER; ++e) {
+            norm_q[e] = src.q_norm_w ? src.q_norm_w[d + e] : 1.f;
+            norm_k[e] = src.k_norm_w ? src.k_norm_w[d + e] : 1.f;
+        }
+        if (j >= 0) {
+            load_keys<HD>(kf, k_pool + base);
+            load_values<HD>(vf, v_pool + base);
+        }
+        auto make = [&](float (&x)[PER], int item) {
+            const bool is_q = item < group, is_k = item == group;
             if (!is_q && !is_k) {
                 bf16_t* vdst = src.v_pool + wbase;
 #pragma unroll
-                for (int e = 0; e < PER; ++e) vdst[page_value_offset(pos % kPageTokens, d + e)] = f32_to_bf16(x[e]);
-                continue;
+                for (int e = 0; e < PER; ++e) {
+                    const bf16_t y = f32_to_bf16(x[e]);
+                    kv_lds[1][d + e] = y;
+                    vdst[page_value_offset(pos % kPageTokens, d + e)] = y;
+                }
+                return;
             }
-            const float* norm_w = is_q ? src.q_norm_w : src.k_norm_w;
-            if (norm_w) {
+            if (is_q ? src.q_norm_w != nullptr : src.k_norm_w != nullptr) {
                 float sq = 0.f;
 #pragma unroll
                 for (int e = 0; e < PER; ++e) sq += x[e] * x[e];
                 const float inv = 1.0f / sqrtf(wave_sum(sq) / (float)HD + src.eps);
 #pragma unroll
-                for (int e = 0; e < PER; ++e) x[e] = x[e] * inv * norm_w[d + e];
+                for (int e = 0; e < PER; ++e) x[e] = x[e] * inv * (is_q ? norm_q[e] : norm_k[e]);
             }
             bf16_t y[PER];
 #pragma unroll
             for (int e = 0; e < PER; ++e) {
                 const float partner = __shfl_xor(x[e], 32, kWave);
-                const float2 cs = src.cs[(size_t)b * (HD / 2) + ((d + e) & (HD / 2 - 1))];
-                y[e] = f32_to_bf16(lane < 32 ? x[e] * cs.x - partner * cs.y : partner * cs.y + x[e] * cs.x);
+                const float across = partner * cs[e].y;         // (rounded first, as the rotation kernel's is)
+                y[e] = f32_to_bf16(fmaf(x[e], cs[e].x, lane < 32 ? -across : across));
             }
-            // (a lane's one or two dimensions are neighbours in a key page too)
-            bf16_t* dst = is_q ? &q_lds[item][d] : src.k_pool + wbase + page_key_offset(pos % kPageTokens, d, HD);
+            bf16_t* dst = is_q ? &q_lds[item][d] : &kv_lds[0][d];
 #pragma unroll
             for (int e = 0; e < PER; ++e) dst[e] = y[e];
+            if (is_k) {
+                // (a lane's one or two dimensions are neighbours in a key page too)
+                bf16_t* kdst = src.k_pool + wbase + page_key_offset(pos % kPageTokens, d, HD);
+#pragma unroll
+                for (int e = 0; e < PER; ++e) kdst[e] = y[e];
+            }
+        };
+#pragma unroll 1                                                             // (see below: short code)
+        for (int item = wave; item < items; item += WAVES) {
+            make(x1, item);
+#pragma unroll
+            for (int e = 0; e < PER; ++e) x1[e] = x2[e];
+            if (item + 2 * WAVES < items) {
+                QkvRow<PER> more;
+                more.load(item_row(item + 2 * WAVES), src.parts, src.part_stride);
+                total(x2, more, item + 2 * WAVES);
+            }
         }
-        __syncthreads();          // the queries in LDS, and the key and value in memory, for every wave of the block
+        __syncthreads();          // the queries in LDS, and the key and value there and in memory, for every wave of the block
+        if (j >= 0 && page_at(j) == n_pages - 1) {
+            // the page came before the step's key and value were in it: they are put to where their lanes hold them
+            // (page_key_offset, page_value_offset)
+            const int t = pos % kPageTokens;
+            if (c == (((t >> 4) << 2) | (t & 3))) {
+#pragma unroll
+                for (int rb = 0; rb < 4; ++rb)
+                    if (rb == ((t >> 2) & 3)) {
+#pragma unroll
+                        for (int sk = 0; sk < HD / 32; ++sk) kf[rb][sk] = ld_frag(&kv_lds[0][32 * sk + 8 * g]);
+                    }
+            }
+            if (g == (t >> 4)) {
+                const uint32_t keep = (t & 1) ? 0x0000ffffu : 0xffff0000u;
+#pragma unroll
+                for (int db = 0; db < HD / 16; ++db) {
+                    const uint32_t v = (uint32_t)__builtin_bit_cast(uint16_t, kv_lds[1][16 * db + c]) << (16 * (t & 1));
+#pragma unroll
+                    for (int half = 0; half < 2; ++half) {
+                        u32x4 u = __builtin_bit_cast(u32x4, vf[db][half]);
+#pragma unroll
+                        for (int w = 0; w < 4; ++w)
+                            if (half == ((t >> 3) & 1) && w == ((t & 7) >> 1)) u[w] = (u[w] & keep) | v;
+                        vf[db][half] = __builtin_bit_cast(bf16x8, u);
+                    }
+                }
+            }
+        }
     }
 
     WaveState<HD> st;
@@ -166,12 +274,22 @@ __global__ __launch_bounds__(WAVES * kWave) void attn_decode_kernel(
 #pragma unroll
         for (int sk = 0; sk < HD / 32; ++sk) qf[sk] = col_ok ? ld_frag(qrow + 32 * sk) : zero_frag();
         // unused columns (c >= group) have zero queries and are never stored: they may run unmasked
-        for (; j >= 0; j = next_from(j + 1)) {
-            const int key0 = page_at(j) * kPageTokens;
+        if (!FUSED) {
             const size_t base = page_base(j);
-            attend_page<HD>(st, qf, k_pool + base, v_pool + base, col_ok ? pos : -1, key0,
-                            min(kPageTokens, pos - key0 + 1), page_fully_visible(pos, pos, key0, window, sinks),
-                            scale * kLog2e, window, sinks);
+            load_keys<HD>(kf, k_pool + base);
+            load_values<HD>(vf, v_pool + base);
+        }
+        // (one copy of a page's steps: in a short context a kernel lasts as long as its code takes to arrive)
+#pragma unroll 1
+        for (;;) {
+            const int key0 = page_at(j) * kPageTokens;
+            attend_loaded<HD>(st, qf, kf, vf, col_ok ? pos : -1, key0, min(kPageTokens, pos - key0 + 1),
+                              page_fully_visible(pos, pos, key0, window, sinks), scale * kLog2e, window, sinks);
+            j = next_from(j + 1);
+            if (j < 0) break;
+            const size_t base = page_base(j);
+            load_keys<HD>(kf, k_pool + base);
+            load_values<HD>(vf, v_pool + base);
         }
     }
     // merge the waves
@@ -185,8 +303,11 @@ __global__ __launch_bounds__(WAVES * kWave) void attn_decode_kernel(
     }
     __syncthreads();
     const int n_z = gridDim.z;
+    const int used = (n_pages + WAVES * ppw - 1) / (WAVES * ppw);        // blocks that have pages of this sequence
+    const bool whole = n_z == 1 || (tickets != nullptr && used == 1);
+    const size_t head0 = (size_t)b * n_heads + kvh * group;
     for (int idx = threadIdx.x; idx < group * HD; idx += blockDim.x) {
-        const int col = idx / HD, d = idx % HD;
+        const int col = idx / HD, e = idx % HD;
         float m = -INFINITY;
 #pragma unroll
         for (int w = 0; w < WAVES; ++w) m = fmaxf(m, lds_m[w * 16 + col]);
@@ -196,15 +317,63 @@ __global__ __launch_bounds__(WAVES * kWave) void attn_decode_kernel(
             const float mw = lds_m[w * 16 + col];
             const float f = (mw == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(mw - m);
             l += lds_l[w * 16 + col] * f;
-            o += lds_o[((size_t)w * group + col) * (HD + 1) + d] * f;
+            o += lds_o[((size_t)w * group + col) * (HD + 1) + e] * f;
         }
-        if (n_z == 1) {
-            out[((size_t)b * n_heads + kvh * group + col) * HD + d] = f32_to_bf16(l > 0.f ? o / l : 0.f);
+        if (whole) {
+            out[(head0 + col) * HD + e] = f32_to_bf16(l > 0.f ? o / l : 0.f);
         } else {
-            float* dst = partial + (((size_t)b * n_heads + kvh * group + col) * n_z + z) * (HD + 2);
-            dst[2 + d] = o;
-            if (d == 0) { dst[0] = m; dst[1] = l; }
+            float* dst = partial + ((head0 + col) * n_z + z) * (HD + 2);
+            if (tickets) {
+                store_through(dst + 2 + e, o);
+                if (e == 0) { store_through(dst, m); store_through(dst + 1, l); }
+            } else {
+                dst[2 + e] = o;
+                if (e == 0) { dst[0] = m; dst[1] = l; }
+            }
         }
+    }
+    if (whole || tickets == nullptr) return;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                     // this wave's share has arrived
+    __syncthreads();                                                     // and every wave's
+    if (threadIdx.x == 0) ticket = atomicInc(tickets + (size_t)b * n_kv_heads + kvh, (unsigned)used - 1);
+    __syncthreads();
+    if (ticket < (unsigned)used - 1) return;
+    // the last block of the sequence and kv head; the shares are read eight at a time, all of up to eight at once
+    for (int idx = threadIdx.x; idx < group * HD; idx += blockDim.x) {
+        const int col = idx / HD, e = idx % HD;
+        const float* p = partial + (head0 + col) * n_z * (HD + 2);
+        float2 ml[8];
+        float ov[8];
+        auto read = [&](int i0) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float* share = p + (size_t)min(i0 + i, used - 1) * (HD + 2);
+                ml[i] = load_pair_through(share);
+                ov[i] = load_through(share + 2 + e);
+            }
+        };
+        read(0);
+        float m = ml[0].x;
+#pragma unroll
+        for (int i = 1; i < 8; ++i) m = fmaxf(m, ml[i].x);
+        for (int i = 8; i < used; ++i) m = fmaxf(m, load_through(p + (size_t)i * (HD + 2)));
+        float ls[kMergeLanes] = {}, os[kMergeLanes] = {};
+        for (int i0 = 0;;) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                if (i0 + i < used) {
+                    const float f = (ml[i].x == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(ml[i].x - m);
+                    ls[i % kMergeLanes] += ml[i].y * f;
+                    os[i % kMergeLanes] += ov[i] * f;
+                }
+            i0 += 8;
+            if (i0 >= used) break;
+            read(i0);
+        }
+        float l = ls[0], o = os[0];
+#pragma unroll
+        for (int i = 1; i < kMergeLanes; ++i) { l += ls[i]; o += os[i]; }
+        out[(head0 + col) * HD + e] = f32_to_bf16(l > 0.f ? o / l : 0.f);
     }
 }
 
@@ -212,12 +381,8 @@ __global__ __launch_bounds__(WAVES * kWave) void attn_decode_kernel(
 // the context, each of which covered pages_per_block pages: thread (j, d) takes blocks j,
 // j + kMergeLanes, ... of dimension d, and LDS adds the kMergeLanes sums in ascending j, so the
 // order depends on the sequence's own length alone.  (One thread per dimension walking all
-// blocks took 17 us at 33 blocks: a chain of dependent L2 latencies.  Letting the last block
-// to finish add them, behind a device-wide fence and a ticket counter, was measured too: the
-// fence writes back whatever earlier kernels left dirty in the L2 and cost 20 us a layer at
-// batch 8; this kernel costs 4.6.)
-constexpr int kMergeLanes = 4;
-
+// blocks took 17 us at 33 blocks: a chain of dependent L2 latencies.)  It serves more than kTicketBlocks blocks along the
+// context and callers that bring no ticket counters.
 template <int HD>
 __global__ __launch_bounds__(kMergeLanes * HD) void attn_decode_merge_kernel(
         bf16_t* __restrict__ out, const float* __restrict__ partial, const int* __restrict__ tok_pos,
@@ -381,7 +546,7 @@ static int launch_decode(void* out, const void* q, int q_stride, const QkvSource
                          const void* v_pool, const int* table, int table_stride, int table_width,
                          const int* tok_pos, int batch, int n_heads, int n_kv_heads, int head_dim,
                          float scale, int window, int sinks, float* workspace, long long workspace_floats,
-                         hipStream_t stream) {
+                         unsigned* tickets, hipStream_t stream) {
     if (batch <= 0 || table_width <= 0 || window < 0 || sinks < 0) return LLOGOS_BAD_ARGUMENT;
     if (!mfma_shape_ok(n_heads, n_kv_heads, head_dim)) return LLOGOS_UNSUPPORTED;
     if (workspace_floats < llogos_attn_decode_workspace(batch, n_heads, n_kv_heads, head_dim, table_width))
@@ -390,15 +555,16 @@ static int launch_decode(void* out, const void* q, int q_stride, const QkvSource
     const int waves = kDecodeWaves, ppw = decode_pages_per_wave(table_width, batch, n_kv_heads);
     const int n_z = (table_width + waves * ppw - 1) / (waves * ppw);
     if (n_z > 1 && workspace == nullptr) return LLOGOS_BAD_ARGUMENT;
+    if (n_z > kTicketBlocks || (uintptr_t)workspace % 8) tickets = nullptr;
     dim3 grid(batch, n_kv_heads, n_z), mgrid(batch, n_heads);
     const size_t smem = decode_lds_bytes(waves, group, head_dim);
     const QkvSource none{};
 #define GO(HD, FUSED) do { \
     attn_decode_kernel<HD, kDecodeWaves, FUSED><<<grid, kDecodeWaves * kWave, smem, stream>>>( \
         (bf16_t*)out, workspace, (const bf16_t*)q, q_stride, FUSED ? *src : none, (const bf16_t*)k_pool, \
-        (const bf16_t*)v_pool, table, table_stride, tok_pos, n_heads, n_kv_heads, group, scale, window, sinks, ppw); \
-    if (n_z > 1) attn_decode_merge_kernel<HD><<<mgrid, kMergeLanes * HD, 0, stream>>>((bf16_t*)out, workspace, tok_pos, n_heads, \
-                                                                        n_z, kDecodeWaves * ppw); } while (0)
+        (const bf16_t*)v_pool, table, table_stride, tok_pos, n_heads, n_kv_heads, group, scale, window, sinks, ppw, tickets); \
+    if (n_z > 1 && tickets == nullptr) attn_decode_merge_kernel<HD><<<mgrid, kMergeLanes * HD, 0, stream>>>((bf16_t*)out, workspace, \
+                                                                        tok_pos, n_heads, n_z, kDecodeWaves * ppw); } while (0)
     if (src != nullptr && head_dim == 64) GO(64, true);
     else if (src != nullptr) GO(128, true);
     else if (head_dim == 64) GO(64, false);
@@ -414,7 +580,7 @@ LLOGOS_EXPORT int llogos_attn_decode_bf16(void* out, const void* q, int q_stride
                                           long long workspace_floats, hipStream_t stream) {
     if ((q_stride % 8) || ((uintptr_t)q % 16)) return LLOGOS_UNSUPPORTED;
     return launch_decode(out, q, q_stride, nullptr, k_pool, v_pool, table, table_stride, table_width, tok_pos, batch,
-                         n_heads, n_kv_heads, head_dim, scale, window, sinks, workspace, workspace_floats, stream);
+                         n_heads, n_kv_heads, head_dim, scale, window, sinks, workspace, workspace_floats, nullptr, stream);
 }
 
 // ---------------------------------------------------------------- decode without allocation
@@ -471,18 +637,22 @@ LLOGOS_EXPORT int llogos_attn_decode_static_bf16(void* out, const void* q, int q
     const int code = static_scratch(&ws);
     if (code != 0) return code;
     return launch_decode(out, q, q_stride, nullptr, k_pool, v_pool, table, table_stride, table_width, tok_pos, batch,
-                         n_heads, n_kv_heads, head_dim, scale, window, sinks, ws, kStaticScratchFloats, stream);
+                         n_heads, n_kv_heads, head_dim, scale, window, sinks, ws, kStaticScratchFloats, nullptr,
+                         stream);
 }
 
 // The same from the fused projection (see QkvSource): head sizes 64 and 128; also writes the
-// step's keys and values to their pages.  cs: [batch][head size / 2][2] floats.
+// step's keys and values to their pages.  cs: [batch][head size / 2][2] floats.  tickets: a counter for each sequence and kv
+// head, all zero before the first call and left at zero by every call, which belong to this call alone while it runs (null, or
+// fewer than that: a kernel of its own merges what blocks along the context leave).
 LLOGOS_EXPORT int llogos_attn_decode_fused_bf16(void* out, const float* qkv, int parts, long long part_stride,
                                                 int row_stride, const float* bias, const float* q_norm_w,
                                                 const float* k_norm_w, float eps, const void* cs, void* k_pool,
                                                 void* v_pool, const int* table, int table_stride, int table_width,
                                                 const int* tok_pos, int batch, int n_heads, int n_kv_heads,
                                                 int head_dim, float scale, int window, int sinks, float* workspace,
-                                                long long workspace_floats, hipStream_t stream) {
+                                                long long workspace_floats, unsigned* tickets, long long n_tickets,
+                                                hipStream_t stream) {
     if (head_dim != 128 && head_dim != 64) return LLOGOS_UNSUPPORTED;
     if (parts < 1 || (row_stride % 2) || (part_stride % 2) || ((uintptr_t)qkv % 8) ||
         row_stride < (n_heads + 2 * n_kv_heads) * head_dim)
@@ -490,7 +660,8 @@ LLOGOS_EXPORT int llogos_attn_decode_fused_bf16(void* out, const float* qkv, int
     const QkvSource src{qkv, parts, (size_t)part_stride, row_stride, bias, q_norm_w, k_norm_w, eps,
                         (const float2*)cs, (bf16_t*)k_pool, (bf16_t*)v_pool};
     return launch_decode(out, nullptr, 0, &src, k_pool, v_pool, table, table_stride, table_width, tok_pos, batch,
-                         n_heads, n_kv_heads, head_dim, scale, window, sinks, workspace, workspace_floats, stream);
+                         n_heads, n_kv_heads, head_dim, scale, window, sinks, workspace, workspace_floats,
+                         n_tickets >= (long long)batch * n_kv_heads ? tickets : nullptr, stream);
 }
 
 // tile_rows: 64 for the kernel whose waves read pages from global memory, 128 for the kernel

@@ -2297,6 +2297,23 @@ def _attn_workspace(device: torch.device, floats: int) -> torch.Tensor:
     return held[-1]
 
 
+def _attn_shares(ctx, device: torch.device, floats: int, counters: int) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
+    """Scratch memory and ticket counters of an engine's decode attention, at least so many of each.  Counters are zero before a
+    call and after it, and a call that shared them with another at the same time would leave them wrong for the calls to come:
+    they belong to one engine (its Runtime), whose steps follow one another as its cache demands.  A context without a
+    Runtime gets the device's scratch memory and no counters (a merge kernel then).  Pairs that became too small
+    stay, captured steps keep their addresses."""
+    held = getattr(getattr(ctx, "runtime", None), "attention_shares", None)
+    if held is None:
+        return _attn_workspace(device, floats), None
+    if not held or held[-1][0].numel() < floats or held[-1][1].numel() < counters or held[-1][0].device != device:
+        if torch.cuda.is_current_stream_capturing():
+            raise KernelError("attention workspace must be made before a step is captured")
+        held.append((torch.empty(max(floats, 1 << 18, 2 * held[-1][0].numel() if held else 0), dtype=torch.float32, device=device),
+                     torch.zeros(max(counters, 1 << 12, 2 * held[-1][1].numel() if held else 0), dtype=torch.int32, device=device)))
+    return held[-1]
+
+
 def attention_mfma_bf16(ctx, q: torch.Tensor, q_stride: int, k_pool: torch.Tensor, v_pool: torch.Tensor,
                         table: torch.Tensor, n_heads: int, n_kv_heads: int, head_dim: int, scale: float,
                         window: int = 0, sinks: int = 0) -> Optional[torch.Tensor]:
@@ -2373,12 +2390,13 @@ def attention_decode_fused(ctx, qkv: torch.Tensor, bias: Optional[torch.Tensor],
     out = torch.empty((T, n_heads * head_dim), dtype=torch.bfloat16, device=qkv.device)
     lib = _lib()
     width_pages = table.shape[1]
-    ws = _attn_workspace(qkv.device, lib.llogos_attn_decode_workspace(T, n_heads, n_kv_heads, head_dim, width_pages))
+    ws, tickets = _attn_shares(ctx, qkv.device, lib.llogos_attn_decode_workspace(T, n_heads, n_kv_heads, head_dim, width_pages),
+                               T * n_kv_heads)
     code = lib.llogos_attn_decode_fused_bf16(
         _p(out), _p(qkv), parts, ctypes.c_longlong(part_stride), qkv.stride(-2), _p(bias), _p(q_norm_w), _p(k_norm_w),
         ctypes.c_float(eps), _p(cs), _p(k_pool), _p(v_pool), _p(table), table.stride(0), width_pages, _p(ctx.tok_pos),
         T, n_heads, n_kv_heads, head_dim, ctypes.c_float(scale), window, sinks, _p(ws),
-        ctypes.c_longlong(ws.numel()), _stream())
+        ctypes.c_longlong(ws.numel()), _p(tickets), ctypes.c_longlong(tickets.numel() if tickets is not None else 0), _stream())
     if code == -2:
         return None
     _check(code, "attention_decode_fused")

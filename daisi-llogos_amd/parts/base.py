@@ -31,6 +31,7 @@ class Runtime:
     dtype: torch.dtype                  # torch.float32 or torch.bfloat16: matrices, activations, cache
     pack_weights: bool = True           # bfloat16 matrices get a second copy in the matrix cores' order (few-row products)
     pack_budget: Optional[int] = None   # bytes that the packed copies may take together (None: no limit); bind() counts it down
+    attention_shares: list = field(default_factory=list, repr=False, compare=False)   # scratch of decode attention (ops/kernels.py: _attn_shares)
 
     @property
     def is_f32(self) -> bool:

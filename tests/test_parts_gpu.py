@@ -1115,3 +1115,36 @@ def test_a_toy_mixer_with_cached_keys_and_a_position_scheme_of_its_own(tmp_path)
         for i in live:
             if cut[i] + t + 1 == len(seqs[i]):
                 eng.free_slot(slots[i])
+
+
+@pytest.mark.parametrize("hd,nh,nkv,lens", [(64, 4, 1, [4170]), (128, 8, 2, [3000, 257, 256, 1]), (64, 32, 8, [600, 1025, 64]), (128, 16, 1, [5000, 130])])
+def test_decode_blocks_that_hand_their_shares_on_by_tickets(hd, nh, nkv, lens):
+    """Blocks along the context whose last one adds all shares against the merge kernel, bit for bit: one block, two, a share
+    of nine (beyond the eight that are read at once) and dozens, called again and again on the same counters, which end at
+    zero; and replayed."""
+    rng = np.random.default_rng(hd + nh)
+    B, width = len(lens), max(lens) // 64 + 2
+    table = torch.tensor(rng.permutation(B * width).reshape(B, width), dtype=torch.int32, device=DEV)
+    pool = lambda: torch.from_numpy(rng.standard_normal((B * width, nkv, 64 * hd), dtype=np.float32)).to(DEV).bfloat16()
+    kp, vp = pool(), pool()
+    qkv = torch.from_numpy(rng.standard_normal((3, B, (nh + 2 * nkv) * hd), dtype=np.float32)).to(DEV)
+    cs = torch.from_numpy(rng.standard_normal((B, hd // 2, 2), dtype=np.float32)).to(DEV)
+    pos = torch.tensor([n - 1 for n in lens], dtype=torch.int32, device=DEV)
+    rt = P.Runtime(DEV, torch.bfloat16)
+
+    def call(runtime):
+        ctx = type("Ctx", (), dict(is_decode=True, n_tokens=B, batch=B, tok_pos=pos, runtime=runtime))()
+        return K.attention_decode_fused(ctx, qkv, None, nh, nkv, hd, hd, 0, None, None, 1e-5, cs, kp, vp, table, hd ** -0.5)
+
+    want = call(None)                                   # no Runtime: no counters, the merge kernel
+    for _ in range(3):
+        assert torch.equal(call(rt).view(torch.int16), want.view(torch.int16))
+    tickets = rt.attention_shares[-1][1]
+    assert tickets.numel() >= B * nkv and not tickets.any()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = call(rt)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        assert torch.equal(out.view(torch.int16), want.view(torch.int16)) and not tickets.any()
