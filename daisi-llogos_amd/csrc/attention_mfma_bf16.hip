@@ -90,11 +90,13 @@ struct QkvRow {
 // with stores that go through to memory (relaxed atomics of agent scope), waits until they have arrived, and takes a ticket;
 // the block with the last ticket reads all shares, past its L2, and adds them in the merge kernel's order.  Nobody waits
 // for another block.  Only the shares go through: a release fence would write back whatever earlier kernels left dirty in
-// the L2 (20 us a layer at batch 8); this takes as long as the merge kernel at two or three blocks and 3 us less at 24 (8
-// contexts of 4,100 to 8,190).  A sequence of one block, of up to 256 positions at the least, has nothing to hand on and takes
-// no ticket: 3 us a layer less.  A ticket counter goes back to zero with the last ticket (atomicInc wraps).
+// the L2 (20 us a layer at batch 8); this takes as long as the merge kernel or up to 3 us less (8 contexts of 4,100 to 8,190,
+// four blocks each: 4,301 -> 4,087 us for 4 steps of 16 layers).  A sequence of one block, of up to 256 positions at the least, has nothing to
+// hand on and takes no ticket: 3 us a layer less.  A ticket counter goes back to zero with the last ticket (atomicInc wraps).
+// One block adds all shares of a kv head's query heads, where the merge kernel has a block for each: with more than
+// kTicketBlocks of them it is the slower way (one context of 16,000, 32 shares: 7 us a layer), and the merge kernel stays.
 // Tried too: blocks of 8 waves that take contexts of up to 1,024 whole, with nothing to hand on: level or 0.5 % slower steps.
-constexpr int kTicketBlocks = 64;                     // more blocks along the context than this go to the merge kernel
+constexpr int kTicketBlocks = 8;                      // more blocks along the context than this go to the merge kernel
 
 __device__ __forceinline__ void store_through(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ float load_through(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
@@ -338,38 +340,29 @@ __global__ __launch_bounds__(WAVES * kWave) void attn_decode_kernel(
     if (threadIdx.x == 0) ticket = atomicInc(tickets + (size_t)b * n_kv_heads + kvh, (unsigned)used - 1);
     __syncthreads();
     if (ticket < (unsigned)used - 1) return;
-    // the last block of the sequence and kv head; the shares are read eight at a time, all of up to eight at once
+    // the last block of the sequence and kv head: every share is asked for at once
     for (int idx = threadIdx.x; idx < group * HD; idx += blockDim.x) {
         const int col = idx / HD, e = idx % HD;
         const float* p = partial + (head0 + col) * n_z * (HD + 2);
-        float2 ml[8];
-        float ov[8];
-        auto read = [&](int i0) {
+        float2 ml[kTicketBlocks];
+        float ov[kTicketBlocks];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const float* share = p + (size_t)min(i0 + i, used - 1) * (HD + 2);
-                ml[i] = load_pair_through(share);
-                ov[i] = load_through(share + 2 + e);
-            }
-        };
-        read(0);
+        for (int i = 0; i < kTicketBlocks; ++i) {
+            const float* share = p + (size_t)min(i, used - 1) * (HD + 2);
+            ml[i] = load_pair_through(share);
+            ov[i] = load_through(share + 2 + e);
+        }
         float m = ml[0].x;
 #pragma unroll
-        for (int i = 1; i < 8; ++i) m = fmaxf(m, ml[i].x);
-        for (int i = 8; i < used; ++i) m = fmaxf(m, load_through(p + (size_t)i * (HD + 2)));
+        for (int i = 1; i < kTicketBlocks; ++i) m = fmaxf(m, ml[i].x);
         float ls[kMergeLanes] = {}, os[kMergeLanes] = {};
-        for (int i0 = 0;;) {
 #pragma unroll
-            for (int i = 0; i < 8; ++i)
-                if (i0 + i < used) {
-                    const float f = (ml[i].x == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(ml[i].x - m);
-                    ls[i % kMergeLanes] += ml[i].y * f;
-                    os[i % kMergeLanes] += ov[i] * f;
-                }
-            i0 += 8;
-            if (i0 >= used) break;
-            read(i0);
-        }
+        for (int i = 0; i < kTicketBlocks; ++i)
+            if (i < used) {
+                const float f = (ml[i].x == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(ml[i].x - m);
+                ls[i % kMergeLanes] += ml[i].y * f;
+                os[i % kMergeLanes] += ov[i] * f;
+            }
         float l = ls[0], o = os[0];
 #pragma unroll
         for (int i = 1; i < kMergeLanes; ++i) { l += ls[i]; o += os[i]; }

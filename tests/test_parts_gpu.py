@@ -1117,10 +1117,10 @@ def test_a_toy_mixer_with_cached_keys_and_a_position_scheme_of_its_own(tmp_path)
                 eng.free_slot(slots[i])
 
 
-@pytest.mark.parametrize("hd,nh,nkv,lens", [(64, 4, 1, [4170]), (128, 8, 2, [3000, 257, 256, 1]), (64, 32, 8, [600, 1025, 64]), (128, 16, 1, [5000, 130])])
+@pytest.mark.parametrize("hd,nh,nkv,lens", [(64, 4, 1, [1900]), (128, 8, 2, [1800, 257, 256, 1]), (64, 32, 8, [600, 1025, 64]), (128, 16, 1, [1920, 130]), (64, 4, 1, [2100])])
 def test_decode_blocks_that_hand_their_shares_on_by_tickets(hd, nh, nkv, lens):
-    """Blocks along the context whose last one adds all shares against the merge kernel, bit for bit: one block, two, a share
-    of nine (beyond the eight that are read at once) and dozens, called again and again on the same counters, which end at
+    """Blocks along the context whose last one adds all shares against the merge kernel, bit for bit: one block, two, eight
+    (the most), nine (the merge kernel's again), called again and again on the same counters, which end at
     zero; and replayed."""
     rng = np.random.default_rng(hd + nh)
     B, width = len(lens), max(lens) // 64 + 2
