@@ -47,23 +47,13 @@
 //    time (86 % with the copies left out, barriers 9 %); the rest of the distance to the library's kernels on the short
 //    matrices is the round of blocks that their tiles do not fill.  (Copies straight into LDS, five stages of 32 k deep,
 //    with a barrier a stage were 8 % slower.)
-#include "common.h"
-
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float f32x16_t __attribute__((ext_vector_type(16)));
-typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
-typedef float f32x2_t __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+#include "gemm_tiles.h"
 
 constexpr int kWavesN = 4, kWavesM = 2, kTileWaves = 8;
 constexpr int kStageK = 64;
 constexpr int kStageW = kWavesN * 64 * kStageK * 2;   // 32 KB
 enum { EPI_PLAIN = 0, EPI_SWIGLU = 1, EPI_ADD = 2 };
 
-__device__ __forceinline__ uint32_t tiles_pack_bf16(float lo, float hi) {
-    const f32x2_t v = {lo, hi};
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));
-}
 // silu(gate) * up, or, with limit >= 0, g = min(gate, limit), u = up within -limit .. limit, g * sigmoid(1.702 g) * (u + 1)
 __device__ __forceinline__ float tiles_gated(float gate, float up, float limit) {
     if (limit >= 0.f) {
@@ -72,8 +62,6 @@ __device__ __forceinline__ float tiles_gated(float gate, float up, float limit) 
     }
     return gate / (1.0f + __expf(-gate)) * up;
 }
-#define SB() __builtin_amdgcn_sched_barrier(0)
-
 template <int N> __device__ __forceinline__ void tiles_wait_loads() {
     static_assert(N == 4 || N == 5 || N == 6, "loads of the other sub-steps of a stage");
     if (N == 4) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
@@ -291,21 +279,6 @@ __device__ __forceinline__ void tile_body(
                 }
         }
     }
-}
-
-// Which tile block j of XCD x takes, of `rows` token tiles x `cols` columns (a part of k and a row tile; the parts outermost):
-// tiles are counted in bands of eight token tiles, a column of the band before the next, and every XCD takes a run of them, as
-// long as the others' to one tile.  The 32 blocks that run on an XCD so are about 8 x 4 tiles of one part of k: they share
-// their weights and their activations in its L2, and no XCD is left with a round of blocks more than the others.  (With
-// whole columns dealt to the XCDs in turn 11 x 20 tiles took two rounds on four of them: 708 us for 2,600 x 5,120 x 17,408,
-// 415 now; 5,003 x 5,120 x 17,408 847 -> 800, 5,003 x 34,816 x 5,120 with SwiGLU 1,505 -> 1,478, 2,048 x 28,672 x 4,096 410 -> 407.)
-__device__ __forceinline__ bool tiles_place(int tiles, int rows, int cols, int xcd, int j, int& row, int& col) {
-    const int per = tiles >> 3, more = tiles & 7;
-    if (j >= per + (xcd < more)) return false;
-    const int id = xcd * per + min(xcd, more) + j, band = id / (8 * cols), at = id - band * 8 * cols, high = min(8, rows - 8 * band);
-    col = at / high;
-    row = 8 * band + at % high;
-    return true;
 }
 
 // Blocks 0 .. blocks4 - 1 take tiles of 256 tokens over the first n_full row tiles, the blocks after them tiles of

@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import ctypes
 from dataclasses import dataclass
+import functools
 import os
 from typing import Optional, Sequence, Tuple
 
@@ -2068,6 +2069,64 @@ def long_tiles_plan(M: int, N: int, K: int, n_cus: Optional[int] = None) -> Opti
     return (1, 0) if 0.79 <= taken <= 0.92 or (0.78 <= taken < 0.79 and not 18000 <= K < 24000) else None
 
 
+# Microseconds that a launch of the tiles of 64, 128 or 192 tokens takes: a round of blocks, a stage of 64 k of one, what a stage takes
+# longer when all units work, a MB of results.  Fitted (6 % rms) to 621 launches: 70 to 1,400 rows of fourteen matrices, 1 to 8 parts.
+_SHORT_TILES = {1: (6.95, 0.408, 0.344, 0.10), 2: (11.2, 0.566, 0.292, 0.13), 3: (15.1, 0.697, 0.451, 0.12)}
+
+
+@functools.lru_cache(maxsize=4096)
+def _short_tiles_form(M: int, N: int, K: int, units: int) -> Tuple[int, int]:
+    """(parts of k, token_tiles) of the cheapest short launch: a block a unit or somewhat fewer.  The consumer's reading of the
+    parts counts too, 0.2 us a MB."""
+    stages, columns, best, least = K // 64, -(-N // 256), (1, 1), float("inf")
+    for token_tiles, (start, stage, busy, mb) in _SHORT_TILES.items():
+        tiles = -(-M // (64 * token_tiles)) * columns
+        most = max(1, min(8, units // tiles, stages // 4))
+        for parts in range(most, max(0, most - 3), -1):
+            rounds = -(-tiles * parts // units)
+            cost = rounds * (start + stages / parts * (stage + busy * tiles * parts / (rounds * units))) + parts * M * N * 4e-6 * (mb + 0.2)
+            if cost < least:
+                best, least = (parts, token_tiles), cost
+    return best
+
+
+def short_tiles_plan(M: int, N: int, K: int, n_cus: Optional[int] = None) -> Optional[Tuple[int, int]]:
+    """(parts of k, token_tiles) with which tiles of 64 to 192 tokens (gemm_tiles_short_bf16) serve a plain product of M rows, or
+    None where they do not: they do for matrices of 2,048 to 8,192 rows and k from 2,048 on (fourteen were measured, k up to
+    21,504), with up to 256 rows of activations, and up to 1,024 where k is at least twice the matrix's rows.  us, library (where k is
+    twice the rows, what tiles_plan or the few-row product had taken) against these with the reading of their parts: 128 rows
+    [3,072, 2,048] 20 / 14, [4,096, 4,096] 22 / 18, [7,168, 5,120] 33 / 28, [4,096, 14,336] 44 / 37; 192 rows [6,144, 4,096] 28 / 24;
+    256 rows [5,120, 5,120] 45 / 28, [4,096, 4,096] 20 / 22 (the one behind); 334 rows [4,096, 14,336] 61 / 58, [5,120, 17,408] 82 / 78.  Beyond 256 rows of
+    the square matrices the library is level ([2,048, 2,048] 20 / 20, [4,096, 4,096] 23 / 27), and so it is at 21,504 matrix rows
+    (70 to 256 rows 43 to 64 / 43 to 66)."""
+    if PROMPT_PRODUCT != "auto" or not SKINNY_MAX_ROWS < M <= 1024 or K % 64 or K < 2048 or not 2048 <= N <= 8192:
+        return None
+    if M > 256 and K < 2 * N:
+        return None
+    return _short_tiles_form(M, N, K, n_cus or compute_units())
+
+
+def gemm_tiles_short_bf16(a: torch.Tensor, pw: PackedWeight, out_dtype: torch.dtype, parts: int, token_tiles: int) -> Optional[torch.Tensor]:
+    """a [M, K] . w^T on the packed copy of w in tiles of 64 token_tiles (1 to 3) tokens x 256 rows of w: [M, N], or with parts > 1
+    float32 partial sums [parts, M, N] over ranges of k; the sums are gemm_tiles_bf16's of as many parts.  None for what it does not take (rows of w
+    in another order, K no multiple of 64, parts of fewer than 128 values of k)."""
+    if a.dtype != torch.bfloat16 or a.dim() != 2 or pw.gate_rows:
+        return None
+    M, K = a.shape
+    if not (K == pw.K and M > 0 and K % 64 == 0 and a.stride(1) == 1 and a.stride(0) % 8 == 0 and a.data_ptr() % 16 == 0):
+        return None
+    _dev(pw.data)
+    _need(a.is_cuda and a.device == pw.data.device, "gemm: a and w must be on the same GPU")
+    _need(parts >= 1, "gemm: one part or more")
+    out = torch.empty((parts, M, pw.N), dtype=torch.float32 if parts > 1 else out_dtype, device=a.device)
+    code = _lib().llogos_gemm_tiles_short_bf16(_p(out), _DT[out.dtype], _p(a), a.stride(0), _p(pw.data), M, pw.N, K, pw.N,
+                                               ctypes.c_longlong(M * pw.N), int(parts), int(token_tiles), _stream())
+    if code == -2:
+        return None
+    _check(code, "gemm_tiles_short_bf16")
+    return out[0] if parts == 1 else out
+
+
 def gemm_tiles_bf16(a: torch.Tensor, pw: PackedWeight, bias: Optional[torch.Tensor], out_dtype: torch.dtype,
                     parts: int = 1, token_tiles: int = 0, limit: Optional[float] = None) -> Optional[torch.Tensor]:
     """a [M, K] . w^T on the packed copy of w for any number of rows (tiles of 256 or 128 tokens x 256 rows,
@@ -2113,7 +2172,7 @@ def gemm_tiles_add(x: torch.Tensor, a: torch.Tensor, pw: Optional[PackedWeight])
             and a.stride(0) % 8 == 0 and a.data_ptr() % 16 == 0):
         return False
     plan = tiles_plan(M, pw.N, K)
-    if plan is None or plan[0] != 1:
+    if plan is None or plan[0] != 1 or short_tiles_plan(M, pw.N, K) is not None:
         return False
     code = _lib().llogos_gemm_tiles_bf16(_p(x), F32, _p(a), a.stride(0), _p(pw.data), None, M, pw.N, K, pw.N, ctypes.c_longlong(0), 2, 1,
                                          int(plan[1]), compute_units(a.device), ctypes.c_float(-1.0), _stream())
@@ -2133,8 +2192,8 @@ def gemm_product(a: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, swigl
 
     float32 operands: 32-bit throughout (gemm_generic).  bfloat16 operands: up to 64 rows the
     hand-written weight-streaming kernels (on the packed copy of w when there is one: `packed`),
-    up to 128 rows too where w is much longer than it has rows (see long_inner); for more rows the
-    hand-written tiled product where it was measured ahead (see tiles_plan); otherwise the
+    for more the hand-written tiled products where they were measured ahead (see short_tiles_plan and tiles_plan),
+    up to 128 rows the weight-streaming one too where w is much longer than it has rows (see long_inner); otherwise the
     library product (as the reference uses a library for its prompt products,
     Daisi.Llogos.Cuda/CudaBackend.cs:158-316)."""
     M = a.shape[-2]
@@ -2184,6 +2243,11 @@ def gemm_product(a: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, swigl
                 return out
     if swiglu_input:
         a = swiglu(a, out_dtype)
+    plan = short_tiles_plan(M, packed.N, packed.K) if packed is not None else None
+    if plan is not None and out_dtype == torch.bfloat16:
+        out = gemm_tiles_short_bf16(a, packed, torch.float32 if f32_ok else out_dtype, *plan)
+        if out is not None:
+            return out
     if SKINNY_MAX_ROWS < M <= LDS_MAX_ROWS and long_inner(w) and a.dtype == torch.bfloat16 and out_dtype == torch.bfloat16:
         out = gemm_skinny_lds_bf16(a, w, None, torch.float32 if f32_ok else out_dtype,
                                    lds_splits(M, w.shape[0], w.shape[1]), 1)
@@ -2216,7 +2280,7 @@ def gemm_library_add(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor, packed: 
     M, N = a.shape[0], w.shape[0]
     if M <= LDS_MAX_ROWS or x.shape != (M, N) or a.shape[1] != w.shape[1] or a.shape[1] % 8:
         return False
-    if packed is not None and tiles_plan(M, packed.N, packed.K) is not None:
+    if packed is not None and (tiles_plan(M, packed.N, packed.K) or short_tiles_plan(M, packed.N, packed.K)) is not None:
         return False
     torch.addmm(x, a, w.t(), out_dtype=torch.float32, out=x)
     return True

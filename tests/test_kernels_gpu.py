@@ -1203,3 +1203,40 @@ def test_long_products_of_prompts_add_themselves_to_the_stream():
     kept = y.clone()
     assert not K.gemm_tiles_add(y[:M - 1000], a[:M - 1000], pw) and not K.gemm_tiles_add(y, a.float(), pw) and not K.gemm_tiles_add(y, a, None)
     assert torch.equal(y, kept)
+
+
+@pytest.mark.parametrize("M,N,K_", [(1, 1, 64), (65, 300, 128), (64, 256, 192), (130, 515, 448), (191, 2048, 2048), (193, 4160, 320), (70, 64, 4096), (400, 1030, 576)])
+def test_short_tiled_product_at_the_edges_of_its_tiles(M, N, K_):
+    """Tiles of 64, 128 and 192 tokens: rows and columns at remainders of tiles, one stage of k and several, every split that leaves a
+    part two stages; the sums are the larger tiles' bit for bit, in float32 and bfloat16, and right."""
+    rng = np.random.default_rng(M + N)
+    wide = _t(rng.standard_normal((M, K_ + 8)), torch.bfloat16)
+    a, w = wide[:, :K_], _t(rng.standard_normal((N, K_)) * 0.05, torch.bfloat16)
+    pw = K.pack_weights(w)
+    want = a.double() @ w.double().t()
+    bound = 1e-6 * (a.double().abs() @ w.double().abs().t()).max()      # float32 sums of bfloat16 products: 2^-24 a step of an operand's chain
+    for parts in [p for p in range(1, 9) if p == 1 or K_ // 64 // p >= 2]:
+        big = K.gemm_tiles_bf16(a, pw, None, torch.float32, parts=parts, token_tiles=2)
+        for token_tiles in (1, 2, 3):
+            got = K.gemm_tiles_short_bf16(a, pw, torch.float32, parts, token_tiles)
+            assert torch.equal(got, big), (parts, token_tiles)
+        assert ((got.double().sum(0) if parts > 1 else got.double()) - want).abs().max() <= bound * parts
+    for token_tiles in (1, 2, 3):
+        assert torch.equal(K.gemm_tiles_short_bf16(a, pw, torch.bfloat16, 1, token_tiles), K.gemm_tiles_bf16(a, pw, None, torch.bfloat16, token_tiles=2))
+    assert K.gemm_tiles_short_bf16(a, pw, torch.float32, K_ // 64, 1) is None or K_ == 64                 # parts of one stage
+    assert K.gemm_tiles_short_bf16(a.float(), pw, torch.float32, 1, 1) is None
+
+
+def test_short_tiled_product_serves_prompts_of_some_hundred_rows():
+    """What short_tiles_plan chooses, through the general entry: in parts or not, with the rows of a product that adds itself left to the norm."""
+    for M, N, K_ in ((65, 2048, 2048), (128, 8192, 2048), (256, 3072, 2112), (257, 2048, 4096), (1024, 2048, 8192)):
+        plan = K.short_tiles_plan(M, N, K_)
+        a, w = torch.randn((M, K_), device=DEV).bfloat16(), (torch.randn((N, K_), device=DEV) * 0.05).bfloat16()
+        pw = K.pack_weights(w)
+        got = K.gemm_product(a, w, torch.bfloat16, f32_ok=True, packed=pw)
+        assert got.dtype == torch.float32 and (got.shape == (M, N) if plan[0] == 1 else got.shape == (plan[0], M, N))
+        want = a.double() @ w.double().t()
+        total = got.double() if plan[0] == 1 else got.double().sum(0)
+        assert (total - want).abs().max() <= 2e-5 * want.abs().max()
+        x = torch.zeros((M, N), device=DEV)
+        assert not K.gemm_tiles_add(x, a, pw) and not K.gemm_library_add(x, a, w, pw) and not x.any()

@@ -188,3 +188,20 @@ def test_which_recurrence_serves_short_prompts_of_heads_of_64():
         assert K.wave_scan_serves(batch, heads, longest, n_cus=256), (batch, heads, longest)
     assert K.wave_scan_segments(1, 64, 100, n_cus=256) == 7 and K.wave_scan_segments(1, 8, 127, n_cus=256) == 8
     assert K.wave_scan_segments(8, 64, 20, n_cus=256) == 1 and K.wave_scan_segments(1, 64, 8000, n_cus=256) == 32
+
+
+def test_short_tiles_are_forms_that_the_kernel_takes():
+    """Every plan over its range leaves a part four stages or comes in one part, has no more parts than consumers add, and more than a
+    round of blocks only in one part; outside its range there is none."""
+    for N in (2048, 3072, 4096, 5120, 7168, 8192):
+        for K_ in (2048, 2112, 4096, 14336, 21504):
+            for M in (65, 100, 128, 129, 192, 193, 256, 257, 334, 512, 700, 1024):
+                plan = K.short_tiles_plan(M, N, K_, n_cus=256)
+                if M > 256 and K_ < 2 * N:
+                    assert plan is None
+                    continue
+                parts, token_tiles = plan
+                assert token_tiles in (1, 2, 3) and 1 <= parts <= 8 and (parts == 1 or K_ // 64 // parts >= 4)
+                assert parts == 1 or -(-M // (64 * token_tiles)) * -(-N // 256) * parts <= 256
+    for M, N, K_ in ((64, 4096, 4096), (1025, 4096, 14336), (100, 2047, 4096), (100, 8193, 4096), (100, 4096, 1984), (100, 4096, 4100)):
+        assert K.short_tiles_plan(M, N, K_, n_cus=256) is None
