@@ -1859,6 +1859,47 @@ def gemm_packed_bf16(a: torch.Tensor, pw: PackedWeight, bias: Optional[torch.Ten
     return out
 
 
+def pack_together(packed: Sequence[Optional[PackedWeight]]) -> Optional[torch.Tensor]:
+    """One buffer with the packed copies of several matrices of one shape, one behind the other, for the product of all of
+    them at once; the copies become views of it.  None (and everything as it was) where a copy is missing, shapes differ or
+    rows are no multiple of 64, or where memory for the buffer is short."""
+    first = packed[0]
+    if any(p is None or p.gate_rows or (p.N, p.K) != (first.N, first.K) for p in packed) or first.N % 64:
+        return None
+    each = packed_weight_bytes(first.N, first.K) // 2
+    try:
+        data = torch.empty(len(packed) * each, dtype=torch.bfloat16, device=first.data.device)
+    except torch.cuda.OutOfMemoryError:
+        return None
+    for i, p in enumerate(packed):
+        data[i * each:(i + 1) * each].copy_(p.data)
+        p.data = data[i * each:(i + 1) * each]
+    return data
+
+
+def gemm_packed_group_bf16(a: torch.Tensor, data: torch.Tensor, N: int) -> Optional[torch.Tensor]:
+    """a[g] . w[g]^T for every g in one launch: a bfloat16 [G, M, K], data from pack_together of G matrices [N, K]; float32
+    [G, parts, M, N], parts to be added.  None for more than 64 rows and shapes that the few-row product does not take."""
+    if a.dtype != torch.bfloat16 or a.dim() != 3:
+        return None
+    G, M, K = a.shape
+    if not (0 < M <= SKINNY_MAX_ROWS and K % 8 == 0 and a.stride(2) == 1 and a.stride(1) % 8 == 0 and a.stride(0) % 8 == 0 and a.data_ptr() % 16 == 0):
+        return None
+    _dev(data)
+    _need(a.is_cuda and a.device == data.device, "gemm: a and w must be on the same GPU")
+    _need(N % 64 == 0 and data.numel() == G * (packed_weight_bytes(N, K) // 2), "gemm: the packed matrices do not fit")
+    splits, chunk = packed_plan(M, G * N, K)
+    lib = _lib()
+    parts = lib.llogos_gemm_packed_parts(K, int(splits), int(chunk))
+    out = torch.empty((G, parts, M, N), dtype=torch.float32, device=a.device)
+    code = lib.llogos_gemm_packed_group_bf16(_p(out), _p(a), a.stride(1), ctypes.c_longlong(a.stride(0)), _p(data), G, M, N, K, int(splits), int(chunk),
+                                             _stream())
+    if code == -2:
+        return None
+    _check(code, "gemm_packed_group_bf16")
+    return out
+
+
 RESIDUAL_MAX_ROWS = 16     # rows at most of the product that adds itself to the residual stream
 # "on" (the default): steps of up to 16 rows close a mixer and a feed-forward with gemm_residual_bf16 and
 # open the next with gemm_packed_unscaled_bf16 where the shapes allow; "off": the products in parts and

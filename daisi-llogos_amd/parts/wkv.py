@@ -42,6 +42,7 @@ class WKV(Mixer):
         self.w2 = Linear([prefix + "w2"], self.decay_rank, [inner], suffix=suffix)
         self.o = Linear([prefix + "o"], inner, [hidden], suffix=suffix)
         self.mu = self.w0 = self.u = self.norm_w = None
+        self.rkvg: Optional[torch.Tensor] = None         # the packed copies of r, k, v, g in one buffer
 
     def _linears(self) -> List[Linear]:
         return [self.r, self.k, self.v, self.g, self.w1, self.w2, self.o]
@@ -62,6 +63,7 @@ class WKV(Mixer):
         super().bind(get, rt)
         for lin in self._linears():
             lin.bind(get, rt)
+        self.rkvg = K.pack_together([lin.packed for lin in (self.r, self.k, self.v, self.g)])
         f32 = lambda name: get(self.prefix + name).to(device=rt.device, dtype=torch.float32).contiguous()
         self.mu = torch.stack([f32("mu." + s) for s in MIXES]).contiguous()
         self.w0, self.u, self.norm_w = f32("w0"), f32("u").reshape(-1), f32("norm")
@@ -75,7 +77,10 @@ class WKV(Mixer):
         # (a product may come as float32 partial sums of a split along k: the activation and the recurrence add them
         # themselves; r, k, v, g have one shape and so one split)
         as_f32 = lambda p: (p[0] if p.dim() == 3 and p.shape[0] == 1 else p) if p.dtype == f32 else K.sum_parts(p, None, f32)
-        r, k, v, g = (as_f32(lin.product(m[i], f32_ok=True)) for i, lin in enumerate((self.r, self.k, self.v, self.g)))
+        rows = K.gemm_packed_group_bf16(m[:4], self.rkvg, self.inner) if self.rkvg is not None else None     # few rows: the four at once
+        if rows is None:
+            rows = [lin.product(m[i], f32_ok=True) for i, lin in enumerate((self.r, self.k, self.v, self.g))]
+        r, k, v, g = (as_f32(p) for p in rows)
         low = K.activation(self.w1.product(m[4], f32_ok=True), "tanh", self.rt.dtype)
         d = as_f32(self.w2.product(low, f32_ok=True))
         mark(ctx, "projections")
