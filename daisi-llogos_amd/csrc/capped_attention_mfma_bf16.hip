@@ -212,18 +212,10 @@ __global__ __launch_bounds__(16 * VB) void capped_merge_kernel(bf16_t* __restric
     const int b = blockIdx.x, h = blockIdx.y, d = threadIdx.x;
     const int n_pages = tok_pos[b] / kPageTokens + 1;
     const int used = min(n_z, (n_pages + pages_per_block - 1) / pages_per_block);
-    const float* src = partial + ((size_t)b * n_heads + h) * n_z * (VP + 2);
-    float m = -INFINITY;
-    for (int z = 0; z < used; ++z) m = fmaxf(m, src[(size_t)z * (VP + 2)]);
-    float l = 0.f, o = 0.f;
-    for (int z = 0; z < used; ++z) {
-        const float* p = src + (size_t)z * (VP + 2);
-        const float f = (p[0] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(p[0] - m);
-        l += p[1] * f;
-        o += p[2 + d] * f;
-    }
-    const float f = finish_factor(m, l, head_sink ? head_sink + h : nullptr, gate ? gate + (size_t)b * gate_stride + h : nullptr);
-    out[((size_t)b * n_heads + h) * VP + d] = f32_to_bf16(o * f);
+    float m[1], l[1], o[1];
+    merge_blocks<1, VP>(partial + ((size_t)b * n_heads + h) * n_z * (VP + 2), n_z, used, d, m, l, o);
+    const float f = finish_factor(m[0], l[0], head_sink ? head_sink + h : nullptr, gate ? gate + (size_t)b * gate_stride + h : nullptr);
+    out[((size_t)b * n_heads + h) * VP + d] = f32_to_bf16(o[0] * f);
 }
 
 // ---------------------------------------------------------------- entry points

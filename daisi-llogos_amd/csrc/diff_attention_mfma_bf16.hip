@@ -125,21 +125,9 @@ __global__ __launch_bounds__(16 * VB) void diff_merge_kernel(bf16_t* __restrict_
     const int b = blockIdx.x, h = blockIdx.y, d = threadIdx.x;
     const int n_pages = tok_pos[b] / kPageTokens + 1;
     const int used = min(n_z, (n_pages + pages_per_block - 1) / pages_per_block);
-    float a[2];
-#pragma unroll
-    for (int m = 0; m < 2; ++m) {
-        const float* src = partial + (((size_t)b * n_heads + h) * 2 + m) * n_z * (VP + 2);
-        float mx = -INFINITY;
-        for (int z = 0; z < used; ++z) mx = fmaxf(mx, src[(size_t)z * (VP + 2)]);
-        float l = 0.f, o = 0.f;
-        for (int z = 0; z < used; ++z) {
-            const float* p = src + (size_t)z * (VP + 2);
-            const float f = (p[0] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(p[0] - mx);
-            l += p[1] * f;
-            o += p[2 + d] * f;
-        }
-        a[m] = l > 0.f ? o / l : 0.f;
-    }
+    float m[2], l[2], sums[2];
+    merge_blocks<2, VP>(partial + ((size_t)b * n_heads + h) * 2 * n_z * (VP + 2), n_z, used, d, m, l, sums);
+    const float a[2] = {l[0] > 0.f ? sums[0] / l[0] : 0.f, l[1] > 0.f ? sums[1] / l[1] : 0.f};
     const float o = a[0] - lambda * a[1];
     const float total = block_sum(o * o, red);
     out[((size_t)b * n_heads + h) * VP + d] = f32_to_bf16(o * (out_scale / sqrtf(total / (float)VP + eps)));

@@ -619,3 +619,22 @@ def test_random_configuration(seed, dtype):
     got = eng.step([(slots[0], list(seqs[0][lens[0] + 6:lens[0] + 8])), (slots[1], list(seqs[1][:lens[1]]))], want=[[0, 1], [lens[1] - 1]])
     want = np.stack([plain[0][lens[0] + 6], plain[0][lens[0] + 7], plain[1][lens[1] - 1]])
     H.close(_np(got), want, dtype, f"{name}: a continued prompt beside a new one")
+
+
+@pytest.mark.parametrize("lens", [(1,), (2048, 256), (2049, 4200, 700)])
+def test_blocks_along_a_long_context_are_merged_whole(lens, monkeypatch):
+    """One block of 256 positions, eight (as many as are read at once), nine, and a second reading of eight: single tokens behind such
+    contexts give what the kernel for any shape gives, which walks the context in one block."""
+    rng = np.random.default_rng(len(lens))
+    heads, kv, d, dv, B, width = 8, 2, 64, 128, len(lens), -(-max(lens) // 64)
+    pool = lambda wide: torch.from_numpy(rng.standard_normal((B * width, kv, 64 * wide), dtype=np.float32)).to(DEV).bfloat16()
+    kp, vp = pool(2 * d), pool(dv)
+    q = torch.from_numpy(rng.standard_normal((B, heads * 2 * d), dtype=np.float32)).to(DEV).bfloat16()
+    ctx = type("Ctx", (), dict(n_tokens=B, batch=B, is_decode=True, tok_seq=_i32(range(B)), tok_pos=_i32([n - 1 for n in lens])))()
+    table = _i32(rng.permutation(B * width).reshape(B, width))
+    run = lambda: _np(K.diff_attention(ctx, q, kp, vp, table, heads, kv, d, dv, 0.3, 0.4, 0.6, 1e-5))
+    got = run()
+    monkeypatch.setattr(K, "DIFF_MFMA", False)
+    want = run()
+    # (weights rounded to bfloat16, 2^-9 each, in sums that a norm brings to size one; the result is rounded once more)
+    assert np.abs(got - want).max() <= PART_TOL["bfloat16"] * np.abs(want).max()
