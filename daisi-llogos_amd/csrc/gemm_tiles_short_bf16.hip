@@ -14,10 +14,10 @@
 //    whose 16-byte pieces are swizzled).  One barrier a stage, between the third and the fourth sub-step of 16 k: the stores are
 //    in the first three, the first reads of the next stage in the fourth.
 //  * Sums are those of gemm_tiles_bf16.hip in the same parts, bit for bit.
-//  * Measured (us; the library's product, which also had the sum into the stream or the few-row product in brackets -> this one):
-//    128 rows: [2,048, 2,048] 20.0 -> 11.2, [3,072, 2,048] 20.1 -> 12.3, [4,096, 4,096] 21.5 -> 16.4, [7,168, 5,120] 33.4 -> 25.0,
-//    [4,096, 14,336] (44) -> 33, [5,120, 17,408] (70) -> 47; 256 rows: [6,144, 4,096] 35.8 -> 25.1, [5,120, 5,120] 44.6 -> 24.5;
-//    334 rows of [4,096, 14,336]: 61 (tiles of 128 tokens of gemm_tiles_bf16.hip in 4 parts) -> 53.
+//  * Measured (us, the library's product -> this one, whose parts are still to be added): 128 rows: [2,048, 2,048] 20.0 -> 11.2,
+//    [3,072, 2,048] 20.1 -> 12.3, [4,096, 4,096] 21.5 -> 16.4, [7,168, 5,120] 33.4 -> 25.0, [5,120, 17,408] 150 -> 47; 256 rows:
+//    [6,144, 4,096] 35.8 -> 25.1, [5,120, 5,120] 44.6 -> 24.5.  [4,096, 14,336]: 128 rows 44 (the few-row product) -> 33, 334 rows 61
+//    (tiles of 128 tokens of gemm_tiles_bf16.hip in 4 parts) -> 53.
 #include "gemm_tiles.h"
 
 constexpr int kWavesN = 2, kWavesM = 2, kTileWaves = 4;

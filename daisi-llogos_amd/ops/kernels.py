@@ -2134,12 +2134,12 @@ def _short_tiles_form(M: int, N: int, K: int, units: int) -> Tuple[int, int]:
 def short_tiles_plan(M: int, N: int, K: int, n_cus: Optional[int] = None) -> Optional[Tuple[int, int]]:
     """(parts of k, token_tiles) with which tiles of 64 to 192 tokens (gemm_tiles_short_bf16) serve a plain product of M rows, or
     None where they do not: they do for matrices of 2,048 to 8,192 rows and k from 2,048 on (fourteen were measured, k up to
-    21,504), with up to 256 rows of activations, and up to 1,024 where k is at least twice the matrix's rows.  us, library (where k is
-    twice the rows, what tiles_plan or the few-row product had taken) against these with the reading of their parts: 128 rows
-    [3,072, 2,048] 20 / 14, [4,096, 4,096] 22 / 18, [7,168, 5,120] 33 / 28, [4,096, 14,336] 44 / 37; 192 rows [6,144, 4,096] 28 / 24;
-    256 rows [5,120, 5,120] 45 / 28, [4,096, 4,096] 20 / 22 (the one behind); 334 rows [4,096, 14,336] 61 / 58, [5,120, 17,408] 82 / 78.  Beyond 256 rows of
-    the square matrices the library is level ([2,048, 2,048] 20 / 20, [4,096, 4,096] 23 / 27), and so it is at 21,504 matrix rows
-    (70 to 256 rows 43 to 64 / 43 to 66)."""
+    21,504), with up to 256 rows of activations, and up to 1,024 where k is at least twice the matrix's rows.  us, what served
+    before / these with 0.2 us a MB for the reading of their parts: 128 rows [3,072, 2,048] 20 / 14, [4,096, 4,096] 22 / 18, [7,168, 5,120] 33 / 28,
+    [4,096, 14,336] 44 / 37; 192 rows [6,144, 4,096] 28 / 24; 256 rows [5,120, 5,120] 45 / 28, [4,096, 4,096] 20 / 22 (the one that is
+    behind); 334 rows [4,096, 14,336] 65 / 59.  Whole prompts: 1B 128 tokens 2,775 / 2,274, 1,000 tokens 4,204 / 3,834; 8 layers of 8B 192
+    tokens 2,109 / 1,854, 1,000 tokens 4,353 / 4,278.  Beyond 256 rows of the square matrices the library is level ([2,048, 2,048] 20 / 20, [4,096,
+    4,096] 23 / 27), and so it is at 21,504 matrix rows (70 to 256 rows 43 to 64 / 43 to 66)."""
     if PROMPT_PRODUCT != "auto" or not SKINNY_MAX_ROWS < M <= 1024 or K % 64 or K < 2048 or not 2048 <= N <= 8192:
         return None
     if M > 256 and K < 2 * N:
