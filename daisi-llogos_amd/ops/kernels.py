@@ -2133,14 +2133,15 @@ def _short_tiles_form(M: int, N: int, K: int, units: int) -> Tuple[int, int]:
 
 def short_tiles_plan(M: int, N: int, K: int, n_cus: Optional[int] = None) -> Optional[Tuple[int, int]]:
     """(parts of k, token_tiles) with which tiles of 64 to 192 tokens (gemm_tiles_short_bf16) serve a plain product of M rows, or
-    None where they do not: they do for matrices of 2,048 to 8,192 rows and k from 2,048 on (fourteen were measured, k up to
+    None where they do not: they do for matrices of 2,048 to 8,192 rows, a multiple of four (results are stored four at a time; one by
+    one [7,169, 4,096] took 43 us at 200 rows, the library 31), and k from 2,048 on (fourteen were measured, k up to
     21,504), with up to 256 rows of activations, and up to 1,024 where k is at least twice the matrix's rows.  us, what served
     before / these with 0.2 us a MB for the reading of their parts: 128 rows [3,072, 2,048] 20 / 14, [4,096, 4,096] 22 / 18, [7,168, 5,120] 33 / 28,
     [4,096, 14,336] 44 / 37; 192 rows [6,144, 4,096] 28 / 24; 256 rows [5,120, 5,120] 45 / 28, [4,096, 4,096] 20 / 22 (the one that is
     behind); 334 rows [4,096, 14,336] 65 / 59.  Whole prompts: 1B 128 tokens 2,775 / 2,274, 1,000 tokens 4,204 / 3,834; 8 layers of 8B 192
     tokens 2,109 / 1,854, 1,000 tokens 4,353 / 4,278.  Beyond 256 rows of the square matrices the library is level ([2,048, 2,048] 20 / 20, [4,096,
     4,096] 23 / 27), and so it is at 21,504 matrix rows (70 to 256 rows 43 to 64 / 43 to 66)."""
-    if PROMPT_PRODUCT != "auto" or not SKINNY_MAX_ROWS < M <= 1024 or K % 64 or K < 2048 or not 2048 <= N <= 8192:
+    if PROMPT_PRODUCT != "auto" or not SKINNY_MAX_ROWS < M <= 1024 or K % 64 or K < 2048 or not 2048 <= N <= 8192 or N % 4:
         return None
     if M > 256 and K < 2 * N:
         return None
@@ -2307,12 +2308,15 @@ def gemm_product(a: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, swigl
     return gemm_generic(a, w, None, torch.float32 if f32_ok else out_dtype)
 
 
-def gemm_library_add(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor, packed: Optional[PackedWeight] = None) -> bool:
+def gemm_library_add(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor, packed: Optional[PackedWeight] = None,
+                     norm_adds: bool = True) -> bool:
     """x [M, N] (float32, in place) += a [M, K] . w^T by the library's bfloat16 product with float32
     accumulation and the sum in its epilogue, where the library serves this product anyway (prompts of
     more than 128 rows that the tiled product does not take): the stream is read and written once there
     instead of the product being written, read again and added by the norm's kernel.  False (and x
-    untouched) otherwise.  The result is the float32 product added to x, bit for bit."""
+    untouched) otherwise.  The result is the float32 product added to x, bit for bit.  norm_adds: a norm reads the stream next and adds
+    parts that short tiles leave; without one a sum of the parts and one with the stream would follow ([4,096, 4,096], 200 rows: 20 us
+    and 6 and 5, the library with the sum in it 25), and the library keeps what it can add itself."""
     if RESIDUAL_PRODUCT != "on":
         return False
     if not (a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dtype == torch.float32 and a.dim() == 2
@@ -2321,7 +2325,8 @@ def gemm_library_add(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor, packed: 
     M, N = a.shape[0], w.shape[0]
     if M <= LDS_MAX_ROWS or x.shape != (M, N) or a.shape[1] != w.shape[1] or a.shape[1] % 8:
         return False
-    if packed is not None and (tiles_plan(M, packed.N, packed.K) or short_tiles_plan(M, packed.N, packed.K)) is not None:
+    if packed is not None and (tiles_plan(M, packed.N, packed.K) is not None or
+                               (norm_adds and short_tiles_plan(M, packed.N, packed.K) is not None)):
         return False
     torch.addmm(x, a, w.t(), out_dtype=torch.float32, out=x)
     return True

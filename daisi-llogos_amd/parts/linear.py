@@ -125,7 +125,7 @@ class Linear(Part):
         x = residual.x
         if a.shape[0] > K.SKINNY_MAX_ROWS:
             # prompts: the product that serves them, the tiled one or the library's, with the sum in its epilogue
-            if self.bias is None and (K.gemm_tiles_add(x, a, self.packed) or K.gemm_library_add(x, a, self.weight, self.packed)):
+            if self.bias is None and (K.gemm_tiles_add(x, a, self.packed) or K.gemm_library_add(x, a, self.weight, self.packed, residual.norm is not None)):
                 return K.RowSquares(None, self.weight.shape[0])
             return None
         if self.packed is None or self.packed.gate_rows:
