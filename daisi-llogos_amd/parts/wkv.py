@@ -68,6 +68,10 @@ class WKV(Mixer):
         self.mu = torch.stack([f32("mu." + s) for s in MIXES]).contiguous()
         self.w0, self.u, self.norm_w = f32("w0"), f32("u").reshape(-1), f32("norm")
 
+    def weight_bytes(self) -> int:
+        # (rkvg is where the packed copies lie, which packed_bytes() counts)
+        return super().weight_bytes() - (self.rkvg.numel() * self.rkvg.element_size() if self.rkvg is not None else 0)
+
     def forward(self, ctx: StepContext, h: torch.Tensor, cache: LayerCache, residual: Optional[Residual] = None):
         f32 = torch.float32
         state = cache.state

@@ -191,3 +191,24 @@ def test_random_models_of_the_design_are_written_and_fit_their_description(tmp_p
         ck.close()
         c2, w = pn.load_folder(path)
         assert np.isfinite(pn.forward(c2, w, [1, 2, 3, 4, 5])).all()
+
+
+def test_the_copies_that_one_product_reads_together_are_counted_once(monkeypatch):
+    """r, k, v and g lie packed in one buffer: what a step reads of the mixer is each matrix once, whichever copy, and the packed
+    copies are counted as such, as they are without that buffer."""
+    K = importlib.import_module("daisi-llogos_amd.ops.kernels")
+    packed = lambda w, gate_rows=0: K.PackedWeight(torch.zeros(K.packed_weight_bytes(*w.shape) // 2, dtype=torch.bfloat16), *w.shape, gate_rows)
+    monkeypatch.setattr(K, "pack_weights", packed)
+    make = importlib.import_module("daisi-llogos_amd.parts.base").make
+    mixers = importlib.import_module("daisi-llogos_amd.parts.base").MIXERS
+    counted = []
+    for together in (True, False):
+        if not together:
+            monkeypatch.setattr(K, "pack_together", lambda copies: None)
+        mixer = make(mixers, "mixer", "wkv", prefix="m.", hidden=128, n_heads=2, head_dim=64, decay_rank=64, eps=1e-5)
+        shapes = {s.name: s.shape for s in mixer.tensor_specs()}
+        mixer.bind(lambda name: torch.zeros(shapes[name]), P.Runtime(torch.device("cpu"), torch.bfloat16))
+        assert (mixer.rkvg is not None) == together
+        counted.append((mixer.weight_bytes(), mixer.packed_bytes()))
+    matrices = 5 * 128 * 128 + 2 * 128 * 64
+    assert counted[0] == counted[1] == (2 * matrices + 4 * (5 * 128 + 3 * 128), 2 * matrices)
