@@ -4,7 +4,7 @@ System.Random per sampler (Daisi.Llogos/Inference/Sampler.cs:12-15, 336); with o
 per sampler that is the same property."""
 from __future__ import annotations
 
-from typing import List, Sequence
+from typing import Iterable, List
 
 import numpy as np
 
@@ -34,8 +34,11 @@ def _splitmix64_array(x: np.ndarray) -> np.ndarray:
     return z ^ (z >> np.uint64(31))
 
 
-def uniforms(seed: int, requests: Sequence[int], indices: Sequence[int]) -> List[float]:
+def uniforms(seed: int, requests: Iterable[int], indices: Iterable[int]) -> List[float]:
     """uniform(seed, r, i) of each pair; from a few pairs on in arrays of 64-bit numbers, which wrap as the masks above do."""
+    if not (isinstance(requests, (list, tuple)) and isinstance(indices, (list, tuple))):
+        pairs = list(zip(requests, indices))                # (iterators and views have no length or no slices; one may be endless)
+        requests, indices = [r for r, _ in pairs], [i for _, i in pairs]
     n = min(len(requests), len(indices))
     if n > 8:
         r, i = np.array(requests[:n]), np.array(indices[:n])

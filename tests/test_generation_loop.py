@@ -1,6 +1,7 @@
 """The generation loop's decisions, with a stand-in engine: batching, stop tokens, sequences
 that end earlier, slots given back and used again."""
 import importlib
+import itertools
 
 import numpy as np
 import pytest
@@ -230,3 +231,16 @@ def test_uniform_numbers_in_arrays_are_the_same():
         wide = numbers + [2**64 + 9]
         assert rng.uniforms(seed, wide, wide) == [rng.uniform(seed, r, r) for r in wide]
     assert rng.uniforms(3, [4], [5]) == [rng.uniform(3, 4, 5)] and rng.uniforms(3, [], []) == []
+
+
+@pytest.mark.parametrize("count", [3, 12])
+def test_uniform_numbers_of_requests_and_indices_of_any_kind(count):
+    """Whatever can be gone through names requests and indices: iterators, views of dicts, ranges, arrays; the shorter of the two ends."""
+    rng = importlib.import_module("daisi-llogos_amd.sampling.rng")
+    want = [rng.uniform(7, r, r + 5) for r in range(count)]
+    requests, indices = list(range(count)), list(range(5, count + 5))
+    assert rng.uniforms(7, dict.fromkeys(requests).keys(), indices) == want
+    assert rng.uniforms(7, iter(requests), (i for i in indices)) == want
+    assert rng.uniforms(7, range(count), tuple(indices)) == want and rng.uniforms(7, requests, indices + [99]) == want
+    assert rng.uniforms(7, dict(zip(requests, indices)), iter(indices + [1, 2])) == want
+    assert rng.uniforms(7, requests, itertools.count(5)) == want and rng.uniforms(7, np.arange(count).tolist(), np.arange(5, count + 5).tolist()) == want
