@@ -972,9 +972,9 @@ static int slice_values(int R, int V, int top_k) {
     return vpt * kSliceThreads;
 }
 
-// slices a row for sample_few, 0: not served (the entry below then refuses too)
+// slices a row for sample_few, 0: not served (the entry below then refuses too): among others more rows than a grid is high
 LLOGOS_EXPORT int llogos_sample_few_slices(int R, int V, int top_k) {
-    if (R <= 0 || V <= 0 || top_k <= 0 || top_k > kFewCandidates || top_k >= V) return 0;
+    if (R <= 0 || R > 65535 || V <= 0 || top_k <= 0 || top_k > kFewCandidates || top_k >= V) return 0;
     const int values = slice_values(R, V, top_k), slices = (V + values - 1) / values;
     return slices <= kWave ? slices : 0;
 }

@@ -205,3 +205,9 @@ def test_short_tiles_are_forms_that_the_kernel_takes():
                 assert parts == 1 or -(-M // (64 * token_tiles)) * -(-N // 256) * parts <= 256
     for M, N, K_ in ((64, 4096, 4096), (1025, 4096, 14336), (100, 2047, 4096), (100, 8193, 4096), (100, 4096, 1984), (100, 4096, 4100), (100, 7169, 4096)):
         assert K.short_tiles_plan(M, N, K_, n_cus=256) is None
+
+
+def test_rows_of_logits_beyond_a_grids_height_are_left_to_the_general_sampler():
+    """The sampler for a small top-k has a row of its grid a row of logits, of which a grid has 65,535."""
+    assert K.sample_few_serves(65535, 100, 40) and not K.sample_few_serves(65536, 100, 40)
+    assert K.sample_few_serves(1, 128256, 256) and not K.sample_few_serves(1, 128256, 257) and not K.sample_few_serves(0, 100, 40)
