@@ -605,8 +605,9 @@ LLOGOS_EXPORT int llogos_gemm_packed_bf16(void* out, int out_dtype, const void* 
 
 // `groups` products of one shape in one launch: activations act_group elements apart, packed matrices of N rows (a multiple of 64)
 // one behind the other, results [groups][parts][M][N] float32.  Matrices of 8 to 34 MB by themselves end before the
-// memory is busy (4.0 TB/s of reading at 34 MB, 6.3 at 134): four of [4096, 4096] at 8 rows 32 us
-// one after the other, some 22 in one launch (16 steps of 3 such layers: 20,098 -> 19,590 us; of [2048, 2048] 9,851 -> 9,335).
+// memory is busy (4.0 TB/s of reading at 34 MB, 6.3 at 134).  A step of three such layers and one of latent attention, us, the four
+// one after the other / in one launch, in the same parts: [2,048, 2,048] 386 / 359 at one row, 451 / 418 at 8, 518 / 481 at 16, 521 / 485
+// at 32, 650 / 599 at 64; [4,096, 4,096] 646 / 624, 702 / 675, 779 / 757, 827 / 809, 1,110 / 1,079.
 LLOGOS_EXPORT int llogos_gemm_packed_group_bf16(float* out, const void* act, int lda, long long act_group, const void* packed_w, int groups,
                                                 int M, int N, int K, int splits, int chunk, hipStream_t stream) {
     if (groups < 1 || groups > 64 || N <= 0 || (N % 64) || N > (1 << 24) / groups || (act_group % 8) || act_group < 0) return LLOGOS_BAD_ARGUMENT;

@@ -1879,7 +1879,9 @@ def pack_together(packed: Sequence[Optional[PackedWeight]]) -> Optional[torch.Te
 
 def gemm_packed_group_bf16(a: torch.Tensor, data: torch.Tensor, N: int) -> Optional[torch.Tensor]:
     """a[g] . w[g]^T for every g in one launch: a bfloat16 [G, M, K], data from pack_together of G matrices [N, K]; float32
-    [G, parts, M, N], parts to be added.  None for more than 64 rows and shapes that the few-row product does not take."""
+    [G, parts, M, N], parts to be added: each matrix's result in the parts, and so the bits, that it has by itself (the fewer parts that
+    would do for all matrices as one doubled the error of the sums at 4,096 x 4,096, 2.7e-7 for 1.4e-7, for a step 1 to 5 % shorter).
+    None for more than 64 rows and shapes that the few-row product does not take."""
     if a.dtype != torch.bfloat16 or a.dim() != 3:
         return None
     G, M, K = a.shape
@@ -1888,7 +1890,7 @@ def gemm_packed_group_bf16(a: torch.Tensor, data: torch.Tensor, N: int) -> Optio
     _dev(data)
     _need(a.is_cuda and a.device == data.device, "gemm: a and w must be on the same GPU")
     _need(N % 64 == 0 and data.numel() == G * (packed_weight_bytes(N, K) // 2), "gemm: the packed matrices do not fit")
-    splits, chunk = packed_plan(M, G * N, K)
+    splits, chunk = packed_plan(M, N, K)
     lib = _lib()
     parts = lib.llogos_gemm_packed_parts(K, int(splits), int(chunk))
     out = torch.empty((G, parts, M, N), dtype=torch.float32, device=a.device)

@@ -1242,16 +1242,16 @@ def test_short_tiled_product_serves_prompts_of_some_hundred_rows():
         assert not K.gemm_tiles_add(x, a, pw) and not K.gemm_library_add(x, a, w, pw) and not x.any()
 
 
-@pytest.mark.parametrize("G,M,N,K_", [(4, 1, 64, 8), (4, 8, 256, 1024), (3, 17, 192, 520), (2, 33, 4096, 2048), (4, 64, 128, 4096)])
+@pytest.mark.parametrize("G,M,N,K_", [(4, 1, 64, 8), (4, 8, 256, 1024), (3, 17, 192, 520), (2, 33, 4096, 2048), (4, 64, 128, 4096), (4, 8, 4096, 4096)])
 def test_products_of_one_shape_in_one_launch(G, M, N, K_):
-    """Each of the group is the product by itself in as many parts, bit for bit; the single copies still serve alone."""
+    """Each of the group is the product by itself, in the parts that its own plan gives it, bit for bit; the single copies still serve alone."""
     rng = np.random.default_rng(N + M)
     a = _t(rng.standard_normal((G + 1, M, K_)), torch.bfloat16)[1:]
     ws = [_t(rng.standard_normal((N, K_)) * 0.05, torch.bfloat16) for _ in range(G)]
     packed = [K.pack_weights(w) for w in ws]
     data = K.pack_together(packed)
     got = K.gemm_packed_group_bf16(a, data, N)
-    splits, chunk = K.packed_plan(M, G * N, K_)
+    splits, chunk = K.packed_plan(M, N, K_)
     for g in range(G):
         alone = K.gemm_packed_bf16(a[g], packed[g], None, torch.float32, splits, chunk)
         assert torch.equal(got[g], alone)
