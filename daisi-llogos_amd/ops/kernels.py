@@ -1912,7 +1912,7 @@ RESIDUAL_PRODUCT = os.environ.get("LLOGOS_RESIDUAL_PRODUCT", "on")
 @dataclass
 class RowSquares:
     """What a product that has added itself to the residual stream x leaves beside it: sums [blocks, 16],
-    float32, each of the product's blocks holding for each row of x the sum of the squares of its 16 or 32
+    float32, each of the product's blocks holding for each row of x the sum of the squares of its 8, 16 or 32
     columns.  A norm over the rows of x needs no other pass over them (gemm_packed_unscaled_bf16)."""
     sums: Optional[torch.Tensor]                # None: the product left nothing but the complete stream
     width: int                                  # columns of x that the sums cover
@@ -1951,10 +1951,16 @@ def residual_form(N: int, K: int, waves: int, strips: int, n_cus: Optional[int] 
     """(waves, strips) of residual_plan as the kernel runs it, strips 0 for half a strip of 16 rows of w a block.  Halves where
     whole strips leave half the compute units or more without a block and k is long enough to be worth a wave's run of it
     (us at 1 / 8 / 16 rows, whole strips against halves, 256 units): [2048, 8192] 10.5 / 11.2 / 12.8 against 9.0 / 9.8 / 11.1,
-    [2048, 2048] 5.0 / 5.2 / 5.8 against 4.4 / 4.7 / 5.1, [1024, 4096] 5.9 / 6.4 / 7.2 against 5.2 / 5.8 / 6.6; with a strip for
+    [2048, 5632] 8.7 / 9.8 / 10.6 against 7.6 / 8.6 / 9.5, [2048, 2048] 5.1 / 5.3 / 5.9 against 4.4 / 4.7 / 5.1, [1024, 1536] 4.1 / 4.6 / 4.9
+    against 3.8 / 4.0 / 4.2; level from k = 2,304 to 4,096 with 2,048 rows of w (within 4 % either way); with a strip for
     every unit ([4096, 4096]) 8.7 / 8.5 / 9.3 against 10.4 / 11.1 / 12.3, since twice as many blocks copy the activations.  16
-    waves up to k = 4096 (8 take 0.2 to 0.3 us more there), 8 above (16 take 0.4 to 1.1 us more)."""
-    if strips == 1 and waves == 8 and 2 * -(-N // 16) <= (n_cus or compute_units()):
+    waves up to k = 4096 (8 take 0.2 to 0.3 us more there), 8 above (16 take up to 1.1 us more at 8,192).
+    Not below k = 1,408: 16 waves have hardly more than two steps each there, [2048, 1024] takes 3.9 / 4.1 / 4.3 us for 3.6 / 3.8 / 3.9, and adding so
+    many short sums is up to 6 % further from 64 bits than whole strips (8.7e-8 for 8.2e-8 at 1,024, level at 1,280, nearer from 1,408
+    on: 9.3e-8 for 1.02e-7 at 2,048, 1.39e-7 for 1.93e-7 at 8,192).
+    (residual_plan leaves matrices of more than 4 M elements on fewer than half the units' worth of strips to the product in parts, so
+    that of those only widths next to 16 * units / 2 come here.)"""
+    if strips == 1 and waves == 8 and K >= 1408 and 2 * -(-N // 16) <= (n_cus or compute_units()):
         return (16 if K <= 4096 else 8), 0
     return waves, strips
 

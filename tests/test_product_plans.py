@@ -179,6 +179,13 @@ def test_where_that_product_takes_half_a_strip_a_block():
     assert form(64, 176) == (4, 1) and form(1024, 8192) == (0, 0)
 
 
+def test_short_sums_keep_whole_strips():
+    """A wave with two steps of k or fewer adds no more exactly by halves, and no faster."""
+    form = lambda N, K_: K.residual_form(N, K_, *K.residual_plan(8, N, K_, n_cus=256), n_cus=256)
+    assert {form(N, K_) for N in (64, 1024, 2048) for K_ in (1024, 1032, 1152, 1280, 1400)} == {(8, 1)}
+    assert form(2048, 1408) == (16, 0) and form(64, 1408) == (16, 0)
+
+
 def test_which_recurrence_serves_short_prompts_of_heads_of_64():
     """Steps measured on either side of the line: at the first ones the kernel with a block a head was ahead (by 8 to 60 %), at the
     others the one with a wave a head; and a prompt just above the line is cut into segments of two whole chunks of eight."""
