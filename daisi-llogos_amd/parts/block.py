@@ -171,6 +171,7 @@ class ParallelBlock(Block):
     The two sublayers depend on the norm's rows alone, so in steps of few rows, whose kernels are short and
     wait for one another, the feed-forward is queued on a second stream beside the mixer (also inside a
     captured step, where the two become branches of the graph); both streams meet before the block returns.
+    A feed-forward that would take a second stream itself (RoutedMoE) does not there: a branch does not fork again.
     Every use of the second stream begins by waiting for the first, after the norm that consumed what the
     second stream made last, so memory that either stream's allocator hands out again is no longer read by
     the other.  `LLOGOS_PARALLEL_STREAMS=0` keeps everything on one stream."""
@@ -193,18 +194,15 @@ class ParallelBlock(Block):
         return self.mixer_norm
 
     def forward(self, ctx: StepContext, x: torch.Tensor, pending, caches):
-        from ..ops import kernels as K
+        from ..ops import branches, kernels as K
         cache = self.mixer.caches_of(caches) if isinstance(caches, (list, tuple)) else caches
         h = self.mixer_norm.forward(x, pending)
         mark(ctx, "norm")
         d = side = None
         if self.ffn is not None and h.shape[0] <= self.side_rows and (ctx is None or ctx.probe is None) and h.is_cuda:
-            main = torch.cuda.current_stream(h.device)
-            side = self._side_streams.get(h.device)
-            if side is None:
-                side = self._side_streams[h.device] = torch.cuda.Stream(device=h.device)
-            side.wait_stream(main)                       # the norm's rows are there
-            with torch.cuda.stream(side):
+            side = branches.fork(h.device, self._side_streams)         # behind the norm's rows
+        if side is not None:
+            with branches.branch(side):
                 d = self.ffn.forward(ctx, h)
         if self.mixer.adds_to_residual:
             a = self.mixer.forward(ctx, h, cache, residual=Residual(x, None))
@@ -217,9 +215,8 @@ class ParallelBlock(Block):
             return x, a
         if a is not None:
             K.residual_add(x, K.sum_parts(a, None, torch.float32))
-        if side is not None:
-            torch.cuda.current_stream(h.device).wait_stream(side)
-        else:
+        branches.join(h.device, side)
+        if side is None:
             d = self.ffn.forward(ctx, h)
         mark(ctx, "feed_forward")
         return x, d

@@ -14,7 +14,7 @@ from typing import Callable, List, Optional
 
 import torch
 
-from ..ops import kernels as K
+from ..ops import branches, kernels as K
 from .base import FeedForward, Residual, Runtime, StepContext, TensorSpec, mark, register_feed_forward
 from .linear import Linear
 
@@ -206,12 +206,9 @@ class RoutedMoE(FeedForward):
         shared, side = None, None
         if self.shared is not None and h.shape[0] <= self.side_rows and (ctx is None or ctx.probe is None) and h.is_cuda \
                 and 3 * self.shared_intermediate * self.hidden * h.element_size() >= self.side_bytes:
-            main = torch.cuda.current_stream(h.device)
-            side = self._side_streams.get(h.device)
-            if side is None:
-                side = self._side_streams[h.device] = torch.cuda.Stream(device=h.device)
-            side.wait_stream(main)                       # h is there
-            with torch.cuda.stream(side):
+            side = branches.fork(h.device, self._side_streams)         # behind h
+        if side is not None:
+            with branches.branch(side):
                 shared = _float32(self.shared.forward(ctx, h))
         choice, weight = K.moe_router(h, self.router_w, self.correction, self.groups, self.keep, self.top,
                                       self.scale * self.out_scale, scores=self.scores, renorm=self.renorm, group_score=self.group_score)
@@ -228,9 +225,8 @@ class RoutedMoE(FeedForward):
             where = torch.zeros(T * self.top, dtype=torch.int32, device=h.device)
             y = torch.zeros((T * self.top, W), dtype=torch.float32, device=h.device)
         mark(ctx, "experts")
-        if side is not None:
-            torch.cuda.current_stream(h.device).wait_stream(side)
-        elif self.shared is not None:
+        branches.join(h.device, side)
+        if side is None and self.shared is not None:
             shared = _float32(self.shared.forward(ctx, h))
             mark(ctx, "shared")
         x = residual.x if residual is not None else None

@@ -20,7 +20,7 @@ from typing import Callable, List, Optional, Tuple
 
 import torch
 
-from ..ops import kernels as K
+from ..ops import branches, kernels as K
 from .base import MIXERS, LayerCache, Mixer, NormedAhead, Part, Residual, Runtime, StepContext, TensorSpec, make, mark, register_mixer
 from .norm import RMSNorm
 
@@ -70,18 +70,14 @@ class SideBySide(Mixer):
         n = len(self.left.cache_parts())
         side, rows = None, h if isinstance(h, torch.Tensor) else h.x
         if ctx.n_tokens <= self.side_rows and ctx.probe is None and self._left_bytes >= self.side_bytes:
-            main = torch.cuda.current_stream(rows.device)
-            side = self._side_streams.get(rows.device)
-            if side is None:
-                side = self._side_streams[rows.device] = torch.cuda.Stream(device=rows.device)
-            side.wait_stream(main)                           # the rows are there
-            with torch.cuda.stream(side):
+            side = branches.fork(rows.device, self._side_streams)      # behind the rows
+        if side is not None:
+            with branches.branch(side):
                 a = self.left.forward(ctx, h, self.left.caches_of(caches[:n]))
         else:
             a = self.left.forward(ctx, h, self.left.caches_of(caches[:n]))
         b = self.right.forward(ctx, h, self.right.caches_of(caches[n:]))
-        if side is not None:
-            torch.cuda.current_stream(rows.device).wait_stream(side)
+        branches.join(rows.device, side)
         if residual is None:
             out = K.pair_norm(a, b, *self.norm_w, self.eps)
             mark(ctx, "pair_norm")
