@@ -89,7 +89,8 @@ struct QkvRow {
 // The blocks of one (sequence, kv head) hand their partial results on without a kernel of their own: each writes its share
 // with stores that go through to memory (relaxed atomics of agent scope), waits until they have arrived, and takes a ticket;
 // the block with the last ticket reads all shares, past its L2, and adds them in the merge kernel's order.  Nobody waits
-// for another block.  Only the shares go through: a release fence would write back whatever earlier kernels left dirty in
+// for another block.  (That rests on this chip, where accesses of agent scope pass the L2 both ways, and on the wait; the language's memory
+// model would ask for a release and an acquire.)  Only the shares go through: a release fence would write back whatever earlier kernels left dirty in
 // the L2 (20 us a layer at batch 8); this takes as long as the merge kernel or up to 3 us less (8 contexts of 4,100 to 8,190,
 // four blocks each: 4,301 -> 4,087 us for 4 steps of 16 layers).  A sequence of one block, of up to 256 positions at the least, has nothing to
 // hand on and takes no ticket: 3 us a layer less.  A ticket counter goes back to zero with the last ticket (atomicInc wraps).

@@ -8,6 +8,7 @@ counts; sequences are not padded to a common length.  (A replayed single-token s
 carry whole rows that belong to no sequence, see graph.py; no kernel mixes rows.)"""
 from __future__ import annotations
 
+import dataclasses
 import os
 from typing import List, Optional, Sequence, Tuple, Union
 
@@ -95,6 +96,8 @@ class Engine:
     def __init__(self, model: Model, rt: Runtime, max_tokens: int, n_slots: int = 64, config=None,
                  use_graphs: Optional[bool] = None, max_seq: Optional[int] = None, architecture: str = "",
                  spare_page_per_slot: bool = False):
+        # (what a Runtime holds for one engine's steps is this engine's own, also where several share a model and its Runtime)
+        rt = dataclasses.replace(rt, attention_shares=[], branch_attention_shares=[])
         self.model, self.rt, self.config = model, rt, config
         self.architecture = architecture or type(model).__name__      # the registry name the model was built under
         # The longest a sequence may become: the caller's limit (the reference's --max-context,

@@ -9,7 +9,9 @@ the two become branches of the graph), until both meet again.
     branches.join(device, side)
 
 A branch does not fork again: ending the capture of a step with a fork inside a fork has ended the process (a segmentation fault on
-the host, before any replay)."""
+the host, before any replay).  And since the two branches run at the same time, memory that calls of one stream hand to one
+another in turn (attention's scratch and counters) is there once for each: in_branch() says to which of the two a call belongs,
+in a step that is launched, in the run before a capture and in the capture alike."""
 from __future__ import annotations
 
 import contextlib

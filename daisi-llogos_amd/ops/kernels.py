@@ -14,7 +14,7 @@ from typing import Optional, Sequence, Tuple
 
 import torch
 
-from . import library
+from . import branches, library
 from ..cache.pages import HEAD_DIM_STEP, MAX_HEAD_DIM, PAGE_TOKENS      # the one definition; the library is checked against PAGE_TOKENS when loaded
 
 F32, BF16 = 0, 1
@@ -2403,9 +2403,9 @@ def prefill_halves(lens: Sequence[int], starts: Optional[Sequence[int]], n_heads
 
 
 def _attn_workspace(device: torch.device, floats: int) -> torch.Tensor:
-    """Scratch memory of the decode attention, at least `floats` long.  A workspace that has
-    become too small stays alive beside its successor: captured steps keep its address."""
-    key = (device.type, device.index)
+    """Scratch memory of the decode attention, at least `floats` long, one for each of a step's branches, which run at the same
+    time.  A workspace that has become too small stays alive beside its successor: captured steps keep its address."""
+    key = (device.type, device.index, branches.in_branch())
     held = _attn_workspaces.setdefault(key, [])
     if not held or held[-1].numel() < floats:
         if torch.cuda.is_current_stream_capturing():
@@ -2418,10 +2418,10 @@ def _attn_workspace(device: torch.device, floats: int) -> torch.Tensor:
 def _attn_shares(ctx, device: torch.device, floats: int, counters: int) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
     """Scratch memory and ticket counters of an engine's decode attention, at least so many of each.  Counters are zero before a
     call and after it, and a call that shared them with another at the same time would leave them wrong for the calls to come:
-    they belong to one engine (its Runtime), whose steps follow one another as its cache demands.  A context without a
-    Runtime gets the device's scratch memory and no counters (a merge kernel then).  Pairs that became too small
-    stay, captured steps keep their addresses."""
-    held = getattr(getattr(ctx, "runtime", None), "attention_shares", None)
+    they belong to one engine (its own Runtime), whose steps follow one another as its cache demands, and in it to one of a step's two
+    branches, whose calls follow one another on a stream.  A context without a Runtime gets the device's scratch memory and no
+    counters (a merge kernel then).  Pairs that became too small stay, captured steps keep their addresses."""
+    held = getattr(getattr(ctx, "runtime", None), "branch_attention_shares" if branches.in_branch() else "attention_shares", None)
     if held is None:
         return _attn_workspace(device, floats), None
     if not held or held[-1][0].numel() < floats or held[-1][1].numel() < counters or held[-1][0].device != device:

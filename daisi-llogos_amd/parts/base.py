@@ -31,7 +31,9 @@ class Runtime:
     dtype: torch.dtype                  # torch.float32 or torch.bfloat16: matrices, activations, cache
     pack_weights: bool = True           # bfloat16 matrices get a second copy in the matrix cores' order (few-row products)
     pack_budget: Optional[int] = None   # bytes that the packed copies may take together (None: no limit); bind() counts it down
-    attention_shares: list = field(default_factory=list, repr=False, compare=False)   # scratch of decode attention (ops/kernels.py: _attn_shares)
+    # scratch and counters of decode attention (ops/kernels.py: _attn_shares), those of a step's second branch (ops/branches.py) apart
+    attention_shares: list = field(default_factory=list, repr=False, compare=False)
+    branch_attention_shares: list = field(default_factory=list, repr=False, compare=False)
 
     @property
     def is_f32(self) -> bool:

@@ -102,3 +102,46 @@ def test_a_branch_does_not_fork_again(monkeypatch):
     with pytest.raises(RuntimeError):
         moe.forward(None, Rows())
     assert streams.waits == [("side", "caller")]
+
+
+def test_branches_that_run_at_the_same_time_share_no_scratch_and_no_counters(monkeypatch):
+    """Two attentions side by side: each takes scratch memory and ticket counters of its own, the same ones in every step, launched,
+    run before a capture or captured (where none may be made)."""
+    streams = Streams(monkeypatch)
+    monkeypatch.setattr(P.SideBySide, "side_bytes", 0)
+    monkeypatch.setattr(K, "_attn_workspaces", {})
+    monkeypatch.setattr(K, "pair_norm", lambda *a, **k: None)
+    capturing = []
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: bool(capturing))
+    cpu = torch.device("cpu")
+
+    class Attention(Quiet):
+        def forward(self, ctx, h, cache=None, **more):
+            scratch, counters = K._attn_shares(ctx, cpu, 100, 8)
+            self.ran.append((streams.current.name, scratch.data_ptr(), counters.data_ptr(), K._attn_workspace(cpu, 100).data_ptr()))
+            return h
+
+    beside = P.SideBySide.__new__(P.SideBySide)
+    beside.left, beside.right, beside._left_bytes, beside.norm_w, beside.eps = Attention(streams), Attention(streams), 0, [None, None], 0.0
+    ctx = type("Ctx", (), dict(n_tokens=3, probe=None, runtime=P.Runtime(cpu, torch.bfloat16)))()
+    rows = torch.zeros(3, 64)
+    for step in range(3):
+        if step == 2:
+            capturing.append(True)
+        beside.forward(ctx, rows, [None, None])
+    assert [r[0] for r in beside.left.ran] == ["side"] * 3 and [r[0] for r in beside.right.ran] == ["caller"] * 3
+    assert len(set(beside.left.ran)) == len(set(beside.right.ran)) == 1
+    left, right = beside.left.ran[0][1:], beside.right.ran[0][1:]
+    assert len(set(left + right)) == 6
+
+
+def test_engines_on_one_runtime_share_no_counters():
+    """Two engines over one bound model may step at the same time, each on its own stream: what a Runtime holds for an engine's steps is
+    that engine's."""
+    engine = importlib.import_module("daisi-llogos_amd.engine.step").Engine
+    spec = type("Spec", (), dict(max_position=None, vocab_size=8))
+    model = type("Model", (), dict(spec=spec, graph_safe=False, cache_needs=lambda self: [], cache_reads=lambda self: []))()
+    rt = P.Runtime(torch.device("cpu"), torch.bfloat16)
+    first, second = engine(model, rt, 64), engine(model, rt, 64)
+    held = [id(getattr(e, name)) for e in (rt, first.rt, second.rt) for name in ("attention_shares", "branch_attention_shares")]
+    assert len(set(held)) == 6 and first.rt == rt
