@@ -2,6 +2,7 @@
 // reductions, the paged cache's address arithmetic.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <atomic>
 #include <stdint.h>
 
 #define LLOGOS_EXPORT extern "C" __attribute__((visibility("default")))
@@ -11,6 +12,20 @@ enum { DT_F32 = 0, DT_BF16 = 1 };
 
 // error codes returned by entry points (positive values are hipError_t)
 enum { LLOGOS_BAD_ARGUMENT = -1, LLOGOS_UNSUPPORTED = -2, LLOGOS_TOO_LARGE = -3 };
+
+// Lets launches of `kernel` on the current device ask for up to `bytes` of dynamic LDS; 0 or an error to return.  Once for each device
+// and kernel (`asked`: a bit a device, kept by the caller for this kernel), not per launch, which may be recorded into a graph.
+static inline int allow_dynamic_lds(const void* kernel, int bytes, std::atomic<uint64_t>& asked) {
+    int device = -1;
+    hipError_t e = hipGetDevice(&device);
+    if (e != hipSuccess) return (int)e;
+    const uint64_t bit = device < 64 ? (uint64_t)1 << device : 0;
+    if (asked.load(std::memory_order_acquire) & bit) return 0;
+    e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    if (e != hipSuccess) return (int)e;
+    asked.fetch_or(bit, std::memory_order_release);
+    return 0;
+}
 
 constexpr int kWave = 64;        // CDNA wavefront
 constexpr int kPageTokens = 64;  // tokens per cache page

@@ -158,16 +158,11 @@ LLOGOS_EXPORT int llogos_gemm_strips_bf16(void* out, int out_dtype, const void* 
     const size_t smem = (size_t)stages * (strips * 16 + mbt * 16) * (kStageK * 2);
     if (smem > 160 * 1024) return LLOGOS_UNSUPPORTED;
     const int tiles = (N + strips * 16 - 1) / (strips * 16);
-    // (the attribute is set once per instance, with the most any call can ask for: not per launch,
-    // which may be recorded into a graph)
+    // (the most LDS that any call can ask for)
 #define GOS(MB, ST, TO) do { \
-        static bool ready = false; \
-        if (!ready) { \
-            hipError_t e = hipFuncSetAttribute((const void*)gemm_strips_kernel<MB, ST, TO>, \
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); \
-            if (e != hipSuccess) return (int)e; \
-            ready = true; \
-        } \
+        static std::atomic<uint64_t> asked{0}; \
+        const int code = allow_dynamic_lds((const void*)gemm_strips_kernel<MB, ST, TO>, 160 * 1024, asked); \
+        if (code != 0) return code; \
         gemm_strips_kernel<MB, ST, TO><<<tiles * parts, kStripWaves * kWave, smem, stream>>>( \
             (TO*)out, (const bf16_t*)act, lda, (const bf16_t*)w, bias, M, N, K, ldo, (size_t)part_stride, strips, kpb, parts); \
         return LLOGOS_LAUNCH_CHECK(); } while (0)

@@ -340,14 +340,9 @@ static int launch_tiles(void* out, const void* a, int lda, const void* wp, const
     const int n_full = tiles_n_full(n_tiles, m4, m2, parts, K / kStageK, token_tiles, compute_units);
     const int blocks4 = (m4 * n_full * parts + 7) / 8 * 8, blocks2 = (m2 * (n_tiles - n_full) * parts + 7) / 8 * 8;
     constexpr size_t smem = (size_t)2 * (kStageW + 256 * kStageK * 2);
-    // (the attribute is set once per instance: not per launch, which may be recorded into a graph)
-    static bool ready = false;
-    if (!ready) {
-        hipError_t e = hipFuncSetAttribute((const void*)gemm_tiles_kernel<TO, EPI>,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-        if (e != hipSuccess) return (int)e;
-        ready = true;
-    }
+    static std::atomic<uint64_t> asked{0};
+    const int code = allow_dynamic_lds((const void*)gemm_tiles_kernel<TO, EPI>, (int)smem, asked);
+    if (code != 0) return code;
     gemm_tiles_kernel<TO, EPI><<<blocks4 + blocks2, kTileWaves * kWave, smem, stream>>>(
         (TO*)out, (const bf16_t*)a, lda, (const unsigned char*)wp, bias, M, N, K, ldo, (size_t)part_stride, n_row_blocks,
         m4, m2, n_full, n_tiles, blocks4, parts, limit);

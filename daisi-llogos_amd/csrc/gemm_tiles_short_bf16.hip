@@ -194,13 +194,9 @@ static int launch_short(void* out, const void* a, int lda, const void* wp, int M
     const long long tiles = (long long)m_tiles * n_tiles * parts;
     if (tiles > 1 << 24) return LLOGOS_UNSUPPORTED;
     constexpr size_t smem = (size_t)2 * (kStageW + TM * 64 * kStageK * 2);
-    // (the attribute is set once per instance and device's first use, not per launch, which may be recorded into a graph)
-    static bool ready = false;
-    if (!ready) {
-        hipError_t e = hipFuncSetAttribute((const void*)gemm_tiles_short_kernel<TM, TO>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-        if (e != hipSuccess) return (int)e;
-        ready = true;
-    }
+    static std::atomic<uint64_t> asked{0};
+    const int code = allow_dynamic_lds((const void*)gemm_tiles_short_kernel<TM, TO>, (int)smem, asked);
+    if (code != 0) return code;
     gemm_tiles_short_kernel<TM, TO><<<(unsigned)((tiles + 7) / 8 * 8), kTileWaves * kWave, smem, stream>>>(
         (TO*)out, (const bf16_t*)a, lda, (const unsigned char*)wp, M, N, K, ldo, (size_t)part_stride, n_row_blocks, m_tiles, n_tiles, parts);
     return LLOGOS_LAUNCH_CHECK();
