@@ -2222,7 +2222,7 @@ def gemm_tiles_add(x: torch.Tensor, a: torch.Tensor, pw: Optional[PackedWeight])
             and a.stride(0) % 8 == 0 and a.data_ptr() % 16 == 0):
         return False
     plan = tiles_plan(M, pw.N, K)
-    if plan is None or plan[0] != 1 or short_tiles_plan(M, pw.N, K) is not None:
+    if plan is None or plan[0] != 1:                         # (one part: more than 1,024 rows, which short tiles do not serve)
         return False
     code = _lib().llogos_gemm_tiles_bf16(_p(x), F32, _p(a), a.stride(0), _p(pw.data), None, M, pw.N, K, pw.N, ctypes.c_longlong(0), 2, 1,
                                          int(plan[1]), compute_units(a.device), ctypes.c_float(-1.0), _stream())

@@ -1242,6 +1242,29 @@ def test_short_tiled_product_serves_prompts_of_some_hundred_rows():
         assert not K.gemm_tiles_add(x, a, pw) and not K.gemm_library_add(x, a, w, pw) and not x.any()
 
 
+@pytest.mark.parametrize("M,N,K_", [(129, 2048, 2048), (200, 4096, 4096), (256, 3072, 2112)])
+def test_products_that_no_norm_follows_are_added_by_the_library(M, N, K_):
+    """Where short tiles would leave parts for a norm to add and none follows, the library's product adds itself to the stream: the
+    float32 product added to x, bit for bit; with a norm behind it, and up to 128 rows, it does not and x stays as it was."""
+    base = importlib.import_module("daisi-llogos_amd.parts.base")
+    parts = importlib.import_module("daisi-llogos_amd.parts")
+    a, w = torch.randn((M, K_), device=DEV).bfloat16(), (torch.randn((N, K_), device=DEV) * 0.05).bfloat16()
+    pw, x0 = K.pack_weights(w), torch.randn((M, N), device=DEV)
+    assert K.short_tiles_plan(M, N, K_) is not None
+    want = x0 + torch.mm(a, w.t(), out_dtype=torch.float32)
+    x = x0.clone()
+    assert K.gemm_library_add(x, a, w, pw, norm_adds=False) and torch.equal(x, want)
+    x = x0.clone()
+    assert not K.gemm_library_add(x, a, w, pw) and not K.gemm_library_add(x[:128], a[:128], w, pw, norm_adds=False) and torch.equal(x, x0)
+    lin = parts.Linear(["o"], K_, [N])
+    lin.bind(lambda name: w, base.Runtime(torch.device(DEV), torch.bfloat16))
+    left = lin.add_to(a, base.Residual(x, None))
+    assert isinstance(left, K.RowSquares) and left.sums is None and torch.equal(x, want)
+    x = x0.clone()
+    norm = parts.RMSNorm("n", N, 1e-5)
+    assert lin.add_to(a, base.Residual(x, norm)) is None and torch.equal(x, x0)
+
+
 @pytest.mark.parametrize("G,M,N,K_", [(4, 1, 64, 8), (4, 8, 256, 1024), (3, 17, 192, 520), (2, 33, 4096, 2048), (4, 64, 128, 4096), (4, 8, 4096, 4096)])
 def test_products_of_one_shape_in_one_launch(G, M, N, K_):
     """Each of the group is the product by itself, in the parts that its own plan gives it, bit for bit; the single copies still serve alone."""

@@ -218,3 +218,12 @@ def test_rows_of_logits_beyond_a_grids_height_are_left_to_the_general_sampler():
     """The sampler for a small top-k has a row of its grid a row of logits, of which a grid has 65,535."""
     assert K.sample_few_serves(65535, 100, 40) and not K.sample_few_serves(65536, 100, 40)
     assert K.sample_few_serves(1, 128256, 256) and not K.sample_few_serves(1, 128256, 257) and not K.sample_few_serves(0, 100, 40)
+
+
+def test_no_product_is_both_a_tiled_one_part_and_short_tiles():
+    """What the tiled product adds to the stream by itself (one part) is nothing that short tiles serve."""
+    for N in (2048, 4096, 8192):
+        for K_ in (2048, 4096, 14336, 21504):
+            for M in (65, 128, 129, 256, 257, 512, 513, 1024, 1025, 1664, 2048):
+                plan = K.tiles_plan(M, N, K_)
+                assert plan is None or plan[0] != 1 or K.short_tiles_plan(M, N, K_, n_cus=256) is None
