@@ -2142,13 +2142,19 @@ def _short_tiles_form(M: int, N: int, K: int, units: int) -> Tuple[int, int]:
 def short_tiles_plan(M: int, N: int, K: int, n_cus: Optional[int] = None) -> Optional[Tuple[int, int]]:
     """(parts of k, token_tiles) with which tiles of 64 to 192 tokens (gemm_tiles_short_bf16) serve a plain product of M rows, or
     None where they do not: they do for matrices of 2,048 to 8,192 rows, a multiple of four (results are stored four at a time; one by
-    one [7,169, 4,096] took 43 us at 200 rows, the library 31), and k from 2,048 on (fourteen were measured, k up to
-    21,504), with up to 256 rows of activations, and up to 1,024 where k is at least twice the matrix's rows.  us, what served
-    before / these with 0.2 us a MB for the reading of their parts: 128 rows [3,072, 2,048] 20 / 14, [4,096, 4,096] 22 / 18, [7,168, 5,120] 33 / 28,
-    [4,096, 14,336] 44 / 37; 192 rows [6,144, 4,096] 28 / 24; 256 rows [5,120, 5,120] 45 / 28, [4,096, 4,096] 20 / 22 (the one that is
-    behind); 334 rows [4,096, 14,336] 65 / 59.  Whole prompts: 1B 128 tokens 2,775 / 2,274, 1,000 tokens 4,204 / 3,834; 8 layers of 8B 192
-    tokens 2,109 / 1,854, 1,000 tokens 4,353 / 4,278.  Beyond 256 rows of the square matrices the library is level ([2,048, 2,048] 20 / 20, [4,096,
-    4,096] 23 / 27), and so it is at 21,504 matrix rows (70 to 256 rows 43 to 64 / 43 to 66)."""
+    one [7,169, 4,096] took 43 us at 200 rows, the library 31), and k from 2,048 on, with up to 256 rows of activations, and up to 1,024
+    where k is at least twice the matrix's rows.  us, product and the norm that adds it, what served before / these: 128 rows [3,072,
+    2,048] 18.8 / 17.9, [4,096, 4,096] 29.0 / 21.2, [7,168, 5,120] 39.2 / 31.6; 192 rows [6,144, 4,096] 38.6 / 30.4; 256 rows [5,120, 5,120]
+    55.2 / 33.7, [4,096, 4,096] 27.5 / 26.7, [8,192, 8,192] 89.1 / 56.7; products alone, 128 rows [4,096, 14,336] 44 / 33, 334 rows 61 / 53.
+    The float32 sums are 0.34 to 1.0 of the former route's distance from 64 bits, by the parts.
+    Behind on the GPU's own clock with k near 2,048 (2,048 to 8,192 matrix rows, from 129 to 256 rows of activations 0.77 to 1.20 of the
+    library's time, most at 1.05 to 1.15; at 129 and 160 rows of [8,192, 4,096] 1.04 and 1.08): what the library chooses for a
+    size varies more than that (192 rows of [3,072, 2,048] 25.5 us, 224 rows 17.5), and whole steps of such models, which wait for the
+    host, are shorter with these: 1B, a prompt of 129 to 256 tokens 2,810 to 2,940 us / 2,400 to 2,470, without them for the
+    square matrix alone 2,570 to 2,690.  8B (8 layers) 129 to 256 tokens 1,990 to 2,320 / 1,800 to 2,070, 14B 2,600 to 3,190 / 2,420 to 2,930.
+    Steps of 65 to 128 single tokens too: 0.80 to 0.82 of the former time at the 1B sizes, 0.84 to 0.90 at 8B, 0.90 to 0.95 at 14B.
+    Beyond 256 rows of the square matrices the library is level ([2,048, 2,048] 20 / 20, [4,096, 4,096] 23 / 27), and so it is at 21,504
+    matrix rows (70 to 256 rows 43 to 64 / 43 to 66)."""
     if PROMPT_PRODUCT != "auto" or not SKINNY_MAX_ROWS < M <= 1024 or K % 64 or K < 2048 or not 2048 <= N <= 8192 or N % 4:
         return None
     if M > 256 and K < 2 * N:
