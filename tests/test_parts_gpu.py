@@ -1148,3 +1148,50 @@ def test_decode_blocks_that_hand_their_shares_on_by_tickets(hd, nh, nkv, lens):
         out.zero_()
         graph.replay()
         assert torch.equal(out.view(torch.int16), want.view(torch.int16)) and not tickets.any()
+
+
+def test_attentions_of_two_branches_hand_their_shares_on_apart():
+    """Two attentions of one engine at the same time, the second in a branch on a stream of its own, launched and as the branches of a
+    captured step: each gives what it gives alone, and all counters end at zero."""
+    branches = importlib.import_module("daisi-llogos_amd.ops.branches")
+    rng = np.random.default_rng(3)
+    hd, nh, nkv, width = 128, 8, 2, 32
+    cs = torch.from_numpy(rng.standard_normal((4, hd // 2, 2), dtype=np.float32)).to(DEV)
+    rt = P.Runtime(DEV, torch.bfloat16)
+    device = torch.device("cuda", torch.cuda.current_device())
+
+    def made(lens):
+        table = torch.tensor(rng.permutation(4 * width).reshape(4, width), dtype=torch.int32, device=DEV)
+        kp, vp = (torch.from_numpy(rng.standard_normal((4 * width, nkv, 64 * hd), dtype=np.float32)).to(DEV).bfloat16() for _ in range(2))
+        qkv = torch.from_numpy(rng.standard_normal((2, 4, (nh + 2 * nkv) * hd), dtype=np.float32)).to(DEV)
+        pos = torch.tensor([n - 1 for n in lens], dtype=torch.int32, device=DEV)
+
+        def call(runtime=rt):
+            ctx = type("Ctx", (), dict(is_decode=True, n_tokens=4, batch=4, tok_pos=pos, runtime=runtime))()
+            return K.attention_decode_fused(ctx, qkv, None, nh, nkv, hd, hd, 0, None, None, 1e-5, cs, kp, vp, table, hd ** -0.5)
+        return call
+    one, other = made([1900, 700, 300, 2000]), made([600, 2047, 1300, 5])
+    want = one(None), other(None)
+    streams = {}
+
+    def both():
+        side = branches.fork(device, streams)
+        with branches.branch(side):
+            b = other()
+        a = one()
+        branches.join(device, side)
+        return a, b
+    same = lambda got: all(torch.equal(g.view(torch.int16), w.view(torch.int16)) for g, w in zip(got, want))
+    for _ in range(5):
+        assert same(both())
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = both()
+    for _ in range(5):
+        for g in got:
+            g.zero_()
+        graph.replay()
+        assert same(got)
+    held = [rt.attention_shares[-1], rt.branch_attention_shares[-1]]
+    assert held[0][0].data_ptr() != held[1][0].data_ptr() and not any(counters.any() for _, counters in held)
