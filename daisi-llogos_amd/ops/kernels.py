@@ -2042,39 +2042,30 @@ def gemm_packed_unscaled_bf16(squares: RowSquares, eps: float, pw: PackedWeight,
     return out
 
 
-# Which product serves many rows of bfloat16 (prompts): "auto" (the default): the hand-written tiled
-# product (gemm_tiles_bf16 on the packed copy) where it was measured level with the library's or faster, which is
-# the gate/up product with its SwiGLU epilogue from TILES_MIN_ROWS to TILES_MAX_ROWS rows (tiles_serve_gated), down
-# projections of up to 1,024 rows and long ones at some sizes (tiles_plan), and the library's product
-# elsewhere (as the reference uses a library there); "tiles": the hand-written one wherever it applies;
+# Which product serves many rows of bfloat16 (prompts): "auto" (the default): the hand-written tiled product (gemm_tiles_bf16 on the
+# packed copy) for more than 64 rows, in the parts that prompt_parts says and with the SwiGLU epilogue where wide_tiles_serve_gated or
+# tiles_serve_gated say so, and the library's product elsewhere (matrices without a packed copy or of fewer than 512 rows or columns, gated
+# products of few rows; as the reference uses a library there); "tiles": the hand-written one wherever it applies;
 # "library": the library's everywhere.  LLOGOS_PROMPT_PRODUCT in the environment sets the default.
 PROMPT_PRODUCT = os.environ.get("LLOGOS_PROMPT_PRODUCT", "auto")
 TILES_MIN_ROWS, TILES_MAX_ROWS, TILES_MAX_K = 1024, 2048, 5120
 
 
 def tiles_serve_gated(M: int, K: int = 0) -> bool:
-    """Whether the tiled product makes silu(gate) * up for M rows of K values (rather than the library's product
-    and a SwiGLU pass): by default from TILES_MIN_ROWS to TILES_MAX_ROWS rows with k up to TILES_MAX_K, where
-    it was measured level or ahead (tiled against library + SwiGLU, us, sustained: 1B 69 / 77 at 1,024 rows,
-    129 / 131 at 2,048; 8B 218 / 218 and 407 / 389, level inside the model; 14B 343 / 414 and 618 / 627).
-    The library gains with the rows and with k (8B: 1.11 PFLOP/s at 1,024 rows, 1.34 from 4,096 on; 70B 1.41
-    to 1.47) where the tiled product stays at 1.2: 8B at 4,096 rows 778 / 721, 70B at 2,048 rows 1,524 / 1,376,
-    a 16,384-token prompt of the 8B sizes 278 ms against 268.  Beyond 2,048 rows neither is ahead for long: with k of 4,608
-    and 5,120 and 8,192 to 65,536 columns the tiled product took between 0.61 and 1.16 of the time of the library with its
-    SwiGLU pass at 204 sizes, by what the library chooses for a size (14B 4,096 rows 1,153 / 1,258, 3,840 1,082 / 1,059;
-    24,576 columns, 2,500 rows 476 / 444, 3,072 579 / 652)."""
+    """Whether the tiled product makes silu(gate) * up for M rows of K values (rather than the library's product and a SwiGLU pass)
+    whatever the matrix's height: from TILES_MIN_ROWS to TILES_MAX_ROWS rows with k up to TILES_MAX_K.  Where the height is known
+    wide_tiles_serve_gated takes more.  us, library with SwiGLU pass / tiled: [28,672, 4,096] 1,000 rows 200 / 184, 2,048 383 / 353; [34,816, 5,120]
+    1,000 rows 393 / 300, 2,048 630 / 538; [16,384, 2,048] 2,048 rows 118 / 112."""
     if PROMPT_PRODUCT == "tiles":
         return True
     return PROMPT_PRODUCT == "auto" and TILES_MIN_ROWS <= M <= TILES_MAX_ROWS and K <= TILES_MAX_K
 
 
 def tiles_plan(M: int, N: int, K: int) -> Optional[Tuple[int, int]]:
-    """(parts of k, token_tiles) with which the tiled product serves a plain product of M rows, or None where
-    the library's does.  Measured on the MI355X at the layer sizes of 8B, 14B and 70B models: a matrix that
+    """(parts of k, token_tiles) with which the tiled product serves a plain product of M rows, or None.  A matrix that
     is much longer than high (a feed-forward's down projection) with 129 to 1,024 rows of activations is where
-    the library is furthest from its best (14B, 256 rows: 226 us against 78; 70B: 313 against 154; 8B, 512 rows:
-    94 against 77), and blocks along k fill the compute units that its few row tiles leave idle.  For more rows see
-    long_tiles_plan.  Elsewhere the library's product was level or ahead (by 10 to 25 % from 2,048 rows on)."""
+    the library is furthest from its best, and blocks along k fill the compute units that its few row tiles leave idle ([5,120, 17,408],
+    200 rows: 137 us against 54).  For more rows see long_tiles_plan; where this plan has none, prompt_parts asks wide_tiles_plan."""
     if PROMPT_PRODUCT == "library" or M <= SKINNY_MAX_ROWS or K % 64:
         return None
     if PROMPT_PRODUCT == "tiles":
@@ -2088,21 +2079,10 @@ def tiles_plan(M: int, N: int, K: int) -> Optional[Tuple[int, int]]:
 
 
 def long_tiles_plan(M: int, N: int, K: int, n_cus: Optional[int] = None) -> Optional[Tuple[int, int]]:
-    """tiles_plan for more than 1,024 rows: with k of 16,384 and more the library's kernels run at 0.55 to 0.95 PFLOP/s at
-    many sizes and at 1.1 to 1.4 at the others, by what they choose for a size, and the tiled product (1.0 to 1.2) serves
-    where they were slow at every size measured.  That is told by how tiles of 256 x 256 fill the compute units; us, library
-    against tiled, with the sum into the stream or the norm that adds the parts:
-
-    two parts of k  tiles for an eighth to a half of the units, k beyond 16,384 (4,096 x 21,504: 1,100 rows 273 / 231, 2,048 457 /
-                    324; 5,120 x 17,408: 1,400 rows 344 / 257).  111 sizes: level at 6,144 x 18,432 with 1,113 rows, ahead by 2 to
-                    52 % at the others; 14 tiles are behind (0.86), and so are at k of 16,384 those of every other size (0.9).
-    one round       78 to 88 % of the units (4,096 x 21,504: 3,456 rows 760 / 547; 8,192 x 28,672: 1,664 rows 956 / 708): ahead
-                    by 17 to 48 % at 111 sizes.  Outside the library is ahead by 10 to 25 %: 198 tiles 0.84, 228 to 232 0.9, 256 0.9.
-    two rounds      79 to 92 % (4,096 x 21,504: 7,168 rows 1,388 / 1,084): ahead by 3 to 42 % at 140 sizes.  At 400 tiles, 78 %, it
-                    depends on k: below 18,000 and from 24,000 on ahead by 16 to 37 % at 69 sizes (5,120 x 17,408: 5,003 rows 1,071 /
-                    843), between them level or behind (4,096 x 21,504: 6,400 rows 1,006 / 1,037; 10,240 x 18,432 0.95).
-    Rows and columns that fill less than 74 % of the units with values of their own are the library's in either case (its tiles
-    are of other heights: 6,400 x 18,944 with 1,832 rows 0.83, with 2,005 1.35), and so are three rounds and more (0.93 to 1.2)."""
+    """tiles_plan for more than 1,024 rows: k of 16,384 and more where tiles of 256 x 256 fill one or two rounds of the compute units well, or an
+    eighth to a half of them, which two parts of k then fill: there the product is added to the stream in its epilogue (one part) or by
+    the norm (two) whatever wide_tiles_plan would choose, and the library's kernels run at 0.55 to 0.95 PFLOP/s where this one runs at 1.3 to 1.45
+    (us: 4,096 x 21,504 1,500 rows 377 / 190, 3,400 740 / 413; 5,120 x 17,408 5,003 rows 1,030 / 665)."""
     if K < 16384 or M <= 1024:
         return None
     units = n_cus or compute_units()
@@ -2118,22 +2098,24 @@ def long_tiles_plan(M: int, N: int, K: int, n_cus: Optional[int] = None) -> Opti
     return (1, 0) if 0.79 <= taken <= 0.92 or (0.78 <= taken < 0.79 and not 18000 <= K < 24000) else None
 
 
-# Microseconds that a launch of the tiles of 64, 128 or 192 tokens takes: a round of blocks, a stage of 64 k of one, what a stage takes
-# longer when all units work, a MB of results.  Fitted (6 % rms) to 621 launches: 70 to 1,400 rows of fourteen matrices, 1 to 8 parts.
-_SHORT_TILES = {1: (6.95, 0.408, 0.344, 0.10), 2: (11.2, 0.566, 0.292, 0.13), 3: (15.1, 0.697, 0.451, 0.12)}
+@functools.lru_cache(maxsize=4096)
+def _tiles_cost(M: int, N: int, K: int, parts: int, token_tiles: int, units: int) -> float:
+    """Microseconds that the tiled product is expected to take (gemm_tiles_bf16.hip: tiles_cost), with its consumer's reading of the
+    results, 0.2 us a MB."""
+    cost = _lib().llogos_gemm_tiles_cost
+    cost.restype = ctypes.c_double
+    return cost(M, N, K, parts, token_tiles, units) + parts * M * N * 4e-6 * 0.2
 
 
 @functools.lru_cache(maxsize=4096)
 def _short_tiles_form(M: int, N: int, K: int, units: int) -> Tuple[int, int]:
-    """(parts of k, token_tiles) of the cheapest short launch: a block a unit or somewhat fewer.  The consumer's reading of the
-    parts counts too, 0.2 us a MB."""
+    """(parts of k, token_tiles) of the cheapest launch in tiles of 64, 128 or 192 tokens: a block a unit or somewhat fewer."""
     stages, columns, best, least = K // 64, -(-N // 256), (1, 1), float("inf")
-    for token_tiles, (start, stage, busy, mb) in _SHORT_TILES.items():
+    for token_tiles in (1, 2, 3):
         tiles = -(-M // (64 * token_tiles)) * columns
         most = max(1, min(8, units // tiles, stages // 4))
-        for parts in range(most, max(0, most - 3), -1):
-            rounds = -(-tiles * parts // units)
-            cost = rounds * (start + stages / parts * (stage + busy * tiles * parts / (rounds * units))) + parts * M * N * 4e-6 * (mb + 0.2)
+        for parts in range(most, 0, -1):
+            cost = _tiles_cost(M, N, K, parts, token_tiles, units)
             if cost < least:
                 best, least = (parts, token_tiles), cost
     return best
@@ -2143,18 +2125,9 @@ def short_tiles_plan(M: int, N: int, K: int, n_cus: Optional[int] = None) -> Opt
     """(parts of k, token_tiles) with which tiles of 64 to 192 tokens (gemm_tiles_short_bf16) serve a plain product of M rows, or
     None where they do not: they do for matrices of 2,048 to 8,192 rows, a multiple of four (results are stored four at a time; one by
     one [7,169, 4,096] took 43 us at 200 rows, the library 31), and k from 2,048 on, with up to 256 rows of activations, and up to 1,024
-    where k is at least twice the matrix's rows.  us, product and the norm that adds it, what served before / these: 128 rows [3,072,
-    2,048] 18.8 / 17.9, [4,096, 4,096] 29.0 / 21.2, [7,168, 5,120] 39.2 / 31.6; 192 rows [6,144, 4,096] 38.6 / 30.4; 256 rows [5,120, 5,120]
-    55.2 / 33.7, [4,096, 4,096] 27.5 / 26.7, [8,192, 8,192] 89.1 / 56.7; products alone, 128 rows [4,096, 14,336] 44 / 33, 334 rows 61 / 53.
-    The float32 sums are 0.34 to 1.0 of the former route's distance from 64 bits, by the parts.
-    Behind on the GPU's own clock with k near 2,048 (2,048 to 8,192 matrix rows, from 129 to 256 rows of activations 0.77 to 1.20 of the
-    library's time, most at 1.05 to 1.15; at 129 and 160 rows of [8,192, 4,096] 1.04 and 1.08): what the library chooses for a
-    size varies more than that (192 rows of [3,072, 2,048] 25.5 us, 224 rows 17.5), and whole steps of such models, which wait for the
-    host, are shorter with these: 1B, a prompt of 129 to 256 tokens 2,810 to 2,940 us / 2,400 to 2,470, without them for the
-    square matrix alone 2,570 to 2,690.  8B (8 layers) 129 to 256 tokens 1,990 to 2,320 / 1,800 to 2,070, 14B 2,600 to 3,190 / 2,420 to 2,930.
-    Steps of 65 to 128 single tokens too: 0.80 to 0.82 of the former time at the 1B sizes, 0.84 to 0.90 at 8B, 0.90 to 0.95 at 14B.
-    Beyond 256 rows of the square matrices the library is level ([2,048, 2,048] 20 / 20, [4,096, 4,096] 23 / 27), and so it is at 21,504
-    matrix rows (70 to 256 rows 43 to 64 / 43 to 66)."""
+    where k is at least twice the matrix's rows.  us, the library's product / these, whose parts are still to be added: 130 rows [3,072,
+    2,048] 19.3 / 9.3, [4,096, 4,096] 20.9 / 13.6, [7,168, 5,120] 29.9 / 23.0; 200 rows [6,144, 4,096] 25.5 / 22.2, [5,120, 5,120] 28.6 / 24.0; 130 rows
+    [4,096, 14,336] 62 / 34, 334 rows 74 / 44.  Where no norm follows that adds the parts, the library adds its product to the stream itself."""
     if PROMPT_PRODUCT != "auto" or not SKINNY_MAX_ROWS < M <= 1024 or K % 64 or K < 2048 or not 2048 <= N <= 8192 or N % 4:
         return None
     if M > 256 and K < 2 * N:
@@ -2162,10 +2135,54 @@ def short_tiles_plan(M: int, N: int, K: int, n_cus: Optional[int] = None) -> Opt
     return _short_tiles_form(M, N, K, n_cus or compute_units())
 
 
+@functools.lru_cache(maxsize=4096)
+def _wide_parts(M: int, N: int, K: int, units: int) -> int:
+    return min(range(1, max(1, min(8, K // 256)) + 1), key=lambda parts: _tiles_cost(M, N, K, parts, 0, units))
+
+
+def wide_tiles_plan(M: int, N: int, K: int, n_cus: Optional[int] = None) -> int:
+    """Parts of k in which the tiled product serves a plain product of M rows beyond short_tiles_plan, or 0 where it does not: it does for
+    more than 64 rows wherever the matrix has 512 rows and columns.  us, the library's product with float32 results / this one, whose parts
+    are still to be added: 2,048 rows [4,096, 14,336] 200 / 166, [28,672, 4,096] 383 with a SwiGLU pass / 353 with it, [4,096, 4,096] 61 / 61;
+    5,003 rows [5,120, 17,408] 1,030 / 665, [7,168, 5,120] 287 / 269, [5,120, 5,120] 219 / 200, [34,816, 5,120] 1,571 / 1,297; 334 rows
+    [6,144, 4,096] 35 / 27, [4,096, 14,336] 74 / 44; 2,500 rows [21,504, 4,096] 442 / 345.  Of 227 sizes (65 to 5,003 rows of 25 matrices, [512, 4,096] to
+    [10,240, 8,192]) it was behind, by 3 to 14 %, at 6: 2,048 rows [6,144, 4,096] and [6,144, 1,536], 1,000 rows [10,240, 8,192] and three level ones."""
+    if PROMPT_PRODUCT != "auto" or M <= SKINNY_MAX_ROWS or K % 64 or K < 512 or N < 512 or N % 4:
+        return 0
+    return _wide_parts(M, N, K, n_cus or compute_units())
+
+
+def wide_tiles_serve_gated(M: int, N: int, K: int) -> bool:
+    """Whether the tiled product makes silu(gate) * up of M rows with a packed matrix of N rows, beyond tiles_serve_gated: where the rows
+    of w are enough for the compute units, which the gated product cannot share by parts of k.  us, library with SwiGLU pass / this:
+    [28,672, 4,096] 100 rows 56 / 63, 130 60 / 64, 200 72 / 67, 334 90 / 79; [16,384, 2,048] 200 rows 31.2 / 32.3, 334 36.6 / 33.8, 1,000 65 / 57;
+    [34,816, 5,120] 130 rows 104 / 91, 1,000 393 / 300, 5,003 1,571 / 1,297."""
+    return PROMPT_PRODUCT == "auto" and M > SKINNY_MAX_ROWS and K % 64 == 0 and K >= 512 and M * N >= 1 << 22
+
+
+def prompt_parts(M: int, N: int, K: int) -> int:
+    """Parts of k of a plain product of M rows that the tiled product serves, or 0: as short_tiles_plan has them, else as tiles_plan for
+    matrices of less than 4 M values (whose products both serve), else as wide_tiles_plan."""
+    plan = short_tiles_plan(M, N, K)
+    if plan is None and N * K < 1 << 22:
+        plan = tiles_plan(M, N, K)
+    return plan[0] if plan is not None else wide_tiles_plan(M, N, K)
+
+
+def gemm_wide_bf16(a: torch.Tensor, pw: PackedWeight, out_dtype: torch.dtype, parts: int) -> Optional[torch.Tensor]:
+    """a [M, K] . w^T on the packed copy of w, in tiles chosen by the launch: [M, N], or with parts > 1 float32 partial sums [parts, M, N] over
+    ranges of k.  None for what it does not take (see gemm_tiles_short_bf16)."""
+    return _gemm_tiles_plain(a, pw, out_dtype, parts, 0)
+
+
 def gemm_tiles_short_bf16(a: torch.Tensor, pw: PackedWeight, out_dtype: torch.dtype, parts: int, token_tiles: int) -> Optional[torch.Tensor]:
     """a [M, K] . w^T on the packed copy of w in tiles of 64 token_tiles (1 to 3) tokens x 256 rows of w: [M, N], or with parts > 1
     float32 partial sums [parts, M, N] over ranges of k; the sums are gemm_tiles_bf16's of as many parts.  None for what it does not take (rows of w
     in another order, K no multiple of 64, parts of fewer than 128 values of k)."""
+    return _gemm_tiles_plain(a, pw, out_dtype, parts, token_tiles) if token_tiles in (1, 2, 3) else None
+
+
+def _gemm_tiles_plain(a: torch.Tensor, pw: PackedWeight, out_dtype: torch.dtype, parts: int, token_tiles: int) -> Optional[torch.Tensor]:
     if a.dtype != torch.bfloat16 or a.dim() != 2 or pw.gate_rows:
         return None
     M, K = a.shape
@@ -2175,20 +2192,20 @@ def gemm_tiles_short_bf16(a: torch.Tensor, pw: PackedWeight, out_dtype: torch.dt
     _need(a.is_cuda and a.device == pw.data.device, "gemm: a and w must be on the same GPU")
     _need(parts >= 1, "gemm: one part or more")
     out = torch.empty((parts, M, pw.N), dtype=torch.float32 if parts > 1 else out_dtype, device=a.device)
-    code = _lib().llogos_gemm_tiles_short_bf16(_p(out), _DT[out.dtype], _p(a), a.stride(0), _p(pw.data), M, pw.N, K, pw.N,
-                                               ctypes.c_longlong(M * pw.N), int(parts), int(token_tiles), _stream())
+    code = _lib().llogos_gemm_tiles_bf16(_p(out), _DT[out.dtype], _p(a), a.stride(0), _p(pw.data), None, M, pw.N, K, pw.N, ctypes.c_longlong(M * pw.N),
+                                         0, int(parts), int(token_tiles), compute_units(a.device), ctypes.c_float(-1.0), _stream())
     if code == -2:
         return None
-    _check(code, "gemm_tiles_short_bf16")
+    _check(code, "gemm_tiles")
     return out[0] if parts == 1 else out
 
 
 def gemm_tiles_bf16(a: torch.Tensor, pw: PackedWeight, bias: Optional[torch.Tensor], out_dtype: torch.dtype,
                     parts: int = 1, token_tiles: int = 0, limit: Optional[float] = None) -> Optional[torch.Tensor]:
-    """a [M, K] . w^T on the packed copy of w for any number of rows (tiles of 256 or 128 tokens x 256 rows,
-    v_mfma_f32_32x32x16_bf16): [M, N] with the bias added, or, for a matrix packed with gate_rows,
+    """a [M, K] . w^T on the packed copy of w for any number of rows (tiles of 64 to 256 tokens x 256 rows of w): [M, N]
+    with the bias added, or, for a matrix packed with gate_rows,
     [M, gate_rows] = silu(gate) * up (with `limit` the form of clamped_glu); with parts > 1 float32 partial sums [parts, M, N] over ranges of k.
-    token_tiles: 4 or 2 force tiles of 256 or 128 tokens, 0 lets the launch choose.
+    token_tiles: 4 or 2 force tiles of 256 or 128 tokens, 0 lets the launch choose among all heights.
     None for shapes it does not take (K no multiple of 64, parts of fewer than 128 values of k)."""
     if a.dtype != torch.bfloat16 or a.dim() != 2:
         return None
@@ -2238,6 +2255,29 @@ def gemm_tiles_add(x: torch.Tensor, a: torch.Tensor, pw: Optional[PackedWeight])
     return True
 
 
+def gemm_wide_add(x: torch.Tensor, a: torch.Tensor, pw: Optional[PackedWeight], norm_adds: bool = True) -> bool:
+    """gemm_tiles_add where wide_tiles_plan takes the product in one part, or in any number where no norm follows that would add them."""
+    if pw is None or pw.gate_rows or RESIDUAL_PRODUCT != "on":
+        return False
+    if not (a.dtype == torch.bfloat16 and a.dim() == 2 and a.is_cuda and x.is_cuda and a.device == x.device == pw.data.device):
+        return False
+    M, K = a.shape
+    if not (x.dtype == torch.float32 and x.shape == (M, pw.N) and x.is_contiguous() and K == pw.K and a.stride(1) == 1
+            and a.stride(0) % 8 == 0 and a.data_ptr() % 16 == 0):
+        return False
+    if short_tiles_plan(M, pw.N, K) is not None:
+        return False
+    parts = wide_tiles_plan(M, pw.N, K)
+    if parts == 0 or (parts > 1 and norm_adds):
+        return False
+    code = _lib().llogos_gemm_tiles_bf16(_p(x), F32, _p(a), a.stride(0), _p(pw.data), None, M, pw.N, K, pw.N, ctypes.c_longlong(0), 2, 1,
+                                         0, compute_units(a.device), ctypes.c_float(-1.0), _stream())
+    if code == -2:
+        return False
+    _check(code, "gemm_wide_add")
+    return True
+
+
 def gemm_product(a: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, swiglu_input: bool = False,
                  f32_ok: bool = False, packed: Optional[PackedWeight] = None) -> torch.Tensor:
     """a [M, K] . w [N, K]^T without bias, as [M, N] of `out_dtype` or as float32 partial sums
@@ -2248,7 +2288,7 @@ def gemm_product(a: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, swigl
 
     float32 operands: 32-bit throughout (gemm_generic).  bfloat16 operands: up to 64 rows the
     hand-written weight-streaming kernels (on the packed copy of w when there is one: `packed`),
-    for more the hand-written tiled products where they were measured ahead (see short_tiles_plan and tiles_plan),
+    for more the hand-written tiled product (see prompt_parts),
     up to 128 rows the weight-streaming one too where w is much longer than it has rows (see long_inner); otherwise the
     library product (as the reference uses a library for its prompt products,
     Daisi.Llogos.Cuda/CudaBackend.cs:158-316)."""
@@ -2299,9 +2339,9 @@ def gemm_product(a: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, swigl
                 return out
     if swiglu_input:
         a = swiglu(a, out_dtype)
-    plan = short_tiles_plan(M, packed.N, packed.K) if packed is not None else None
-    if plan is not None and out_dtype == torch.bfloat16:
-        out = gemm_tiles_short_bf16(a, packed, torch.float32 if f32_ok else out_dtype, *plan)
+    parts = prompt_parts(M, packed.N, packed.K) if packed is not None else 0
+    if parts and out_dtype == torch.bfloat16:
+        out = gemm_wide_bf16(a, packed, torch.float32 if f32_ok else out_dtype, parts)
         if out is not None:
             return out
     if SKINNY_MAX_ROWS < M <= LDS_MAX_ROWS and long_inner(w) and a.dtype == torch.bfloat16 and out_dtype == torch.bfloat16:
@@ -2339,8 +2379,7 @@ def gemm_library_add(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor, packed: 
     M, N = a.shape[0], w.shape[0]
     if M <= LDS_MAX_ROWS or x.shape != (M, N) or a.shape[1] != w.shape[1] or a.shape[1] % 8:
         return False
-    if packed is not None and (tiles_plan(M, packed.N, packed.K) is not None or
-                               (norm_adds and short_tiles_plan(M, packed.N, packed.K) is not None)):
+    if packed is not None and (tiles_plan(M, packed.N, packed.K) is not None or (norm_adds and prompt_parts(M, packed.N, packed.K) > 1)):
         return False
     torch.addmm(x, a, w.t(), out_dtype=torch.float32, out=x)
     return True

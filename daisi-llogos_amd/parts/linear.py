@@ -125,7 +125,9 @@ class Linear(Part):
         x = residual.x
         if a.shape[0] > K.SKINNY_MAX_ROWS:
             # prompts: the product that serves them, the tiled one or the library's, with the sum in its epilogue
-            if self.bias is None and (K.gemm_tiles_add(x, a, self.packed) or K.gemm_library_add(x, a, self.weight, self.packed, residual.norm is not None)):
+            norm_adds = residual.norm is not None
+            if self.bias is None and (K.gemm_tiles_add(x, a, self.packed) or K.gemm_wide_add(x, a, self.packed, norm_adds)
+                                      or K.gemm_library_add(x, a, self.weight, self.packed, norm_adds)):
                 return K.RowSquares(None, self.weight.shape[0])
             return None
         if self.packed is None or self.packed.gate_rows:
@@ -152,7 +154,8 @@ class Linear(Part):
         if a.dim() != 2:
             return None
         if a.shape[0] > K.SKINNY_MAX_ROWS:
-            return K.gemm_tiles_bf16(a, self.packed, None, self.rt.dtype, limit=limit) if K.tiles_serve_gated(a.shape[0], a.shape[1]) else None
+            serves = K.tiles_serve_gated(a.shape[0], a.shape[1]) or K.wide_tiles_serve_gated(a.shape[0], self.packed.N, a.shape[1])
+            return K.gemm_tiles_bf16(a, self.packed, None, self.rt.dtype, limit=limit) if serves else None
         return K.gemm_packed_gated_bf16(a, self.packed, self.rt.dtype, K.packed_plan(a.shape[0], self.packed.N, self.packed.K)[1], limit=limit)
 
     def bias_rows(self, rows_out: Optional[int] = None) -> Optional[torch.Tensor]:

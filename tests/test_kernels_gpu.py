@@ -1,6 +1,7 @@
 """Each kernel alone against a plain float64 / torch reference of the same op, at sizes
 other than the engine's tests use (head sizes in steps of 16, widths and vocabularies that
 are no power of two, many heads and groups)."""
+import ctypes
 import importlib
 import math
 
@@ -1225,6 +1226,70 @@ def test_short_tiled_product_at_the_edges_of_its_tiles(M, N, K_):
         assert torch.equal(K.gemm_tiles_short_bf16(a, pw, torch.bfloat16, 1, token_tiles), K.gemm_tiles_bf16(a, pw, None, torch.bfloat16, token_tiles=2))
     assert K.gemm_tiles_short_bf16(a, pw, torch.float32, K_ // 64, 1) is None or K_ == 64                 # parts of one stage
     assert K.gemm_tiles_short_bf16(a.float(), pw, torch.float32, 1, 1) is None
+
+
+@pytest.mark.parametrize("M,N,K_", [(1, 32, 64), (97, 512, 128), (255, 544, 320), (256, 260, 256), (257, 1024, 576), (161, 96, 1088), (450, 1088, 192)])
+def test_tiles_of_every_height_and_epilogue(M, N, K_):
+    """Tiles of 64, 96, .. 256 tokens: rows and columns at remainders, one stage of k to several rounds of the ring of four and what is left of one,
+    rows of a wider than k, results narrower than whole lines, every epilogue.  Every height gives the same bits; they are right."""
+    rng = np.random.default_rng(M * N)
+    lib = K._lib()
+    wide = _t(rng.standard_normal((M, K_ + 8)), torch.bfloat16)
+    a, w = wide[:, :K_], _t(rng.standard_normal((N, K_)) * 0.05, torch.bfloat16)
+    pw, pg = K.pack_weights(w), (K.pack_weights(w, gate_rows=N // 2) if N % 32 == 0 else None)
+    exact = a.double() @ w.double().t()
+    bound = 1e-6 * (a.double().abs() @ w.double().abs().t()).max()      # float32 sums of bfloat16 products: 2^-24 a step of an operand's chain
+    x = _t(rng.standard_normal((M, N)))
+    gate, up = exact[:, :N // 2], exact[:, N // 2:]
+    seen = None
+    for token_tiles in (1, 6, 2, 10, 3, 14, 4, 0):
+        def call(out, packed, epilogue, parts=1, limit=-1.0):
+            K._check(lib.llogos_gemm_tiles_bf16(K._p(out), K._DT[out.dtype], K._p(a), a.stride(0), K._p(packed.data), None, M, N, K_, out.shape[-1],
+                                                ctypes.c_longlong(M * out.shape[-1]), epilogue, parts, token_tiles, 256, ctypes.c_float(limit), K._stream()), "tiles")
+            return out
+        empty = lambda *shape, dtype=torch.float32: torch.full(shape, float("nan"), device=DEV, dtype=dtype)
+        got = [call(empty(M, N), pw, 0), call(empty(M, N, dtype=torch.bfloat16), pw, 0), call(x.clone(), pw, 2)]
+        assert (got[0].double() - exact).abs().max() <= bound and torch.equal(got[1], got[0].bfloat16()) and torch.equal(got[2], x + got[0])
+        for parts in (2, 3):
+            if K_ // 64 // parts >= 2:
+                split = call(empty(parts, M, N), pw, 0, parts)
+                assert (split.double().sum(0) - exact).abs().max() <= bound * parts
+                got.append(split)
+        if pg is not None:
+            got += [call(empty(M, N // 2), pg, 1), call(empty(M, N // 2, dtype=torch.bfloat16), pg, 1), call(empty(M, N // 2), pg, 1, limit=0.7)]
+            # (the product's own error through silu, whose slope is below 1.1, and a few roundings of the rest)
+            room = 1.2 * bound * (1 + up.abs().max() + gate.abs().max()) + 2e-6 * (gate.abs() * up.abs()).max()
+            assert (got[-3].double() - torch.nn.functional.silu(gate) * up).abs().max() <= room and torch.equal(got[-2], got[-3].bfloat16())
+            g, u = gate.clamp(max=0.7), up.clamp(-0.7, 0.7)
+            assert (got[-1].double() - g * torch.sigmoid(1.702 * g) * (u + 1)).abs().max() <= room + 4 * bound
+        seen = seen or got
+        assert all(torch.equal(p, q) for p, q in zip(seen, got)), token_tiles
+
+
+def test_wide_tiles_serve_prompts():
+    """What wide_tiles_plan chooses, through the general entry and added to the stream: one part in place, more parts left to the norm that
+    adds them, all in one where none follows; matrices and operands that it does not take go the way they went."""
+    for M, N, K_ in ((1200, 2048, 2048), (2048, 4096, 14336), (300, 512, 4096), (700, 8320, 4096)):
+        parts = K.prompt_parts(M, N, K_)
+        a, w = torch.randn((M, K_), device=DEV).bfloat16(), (torch.randn((N, K_), device=DEV) * 0.05).bfloat16()
+        pw, x0 = K.pack_weights(w), torch.randn((M, N), device=DEV)
+        want = a.double() @ w.double().t()
+        got = K.gemm_product(a, w, torch.bfloat16, f32_ok=True, packed=pw)
+        assert parts and got.dtype == torch.float32 and got.shape == ((M, N) if parts == 1 else (parts, M, N))
+        total = got.double() if parts == 1 else got.double().sum(0)
+        assert (total - want).abs().max() <= 2e-5 * want.abs().max()
+        x = x0.clone()
+        adds = K.wide_tiles_plan(M, N, K_) == 1
+        assert K.gemm_wide_add(x, a, pw) == adds and (adds or (torch.equal(x, x0) and not K.gemm_library_add(x, a, w, pw)))
+        if K.short_tiles_plan(M, N, K_) is None:
+            x = x0.clone()
+            assert K.gemm_wide_add(x, a, pw, norm_adds=False) and (x.double() - x0.double() - want).abs().max() <= 2e-5 * want.abs().max()
+        x = x0.clone()
+        assert not K.gemm_wide_add(x[:, :N - 4], a, pw) and not K.gemm_wide_add(x, a.float(), pw) and not K.gemm_wide_add(x.t(), a, pw) and torch.equal(x, x0)
+        odd = torch.randn((M, K_ + 4), device=DEV).bfloat16()[:, 4:]          # rows that are not 16 bytes apart
+        assert K.gemm_wide_bf16(odd, pw, torch.float32, 1) is None
+        got = K.gemm_product(odd, w, torch.bfloat16, f32_ok=True, packed=pw)
+        assert (got.double() - odd.double() @ w.double().t()).abs().max() <= 2e-5 * want.abs().max() * (1 if got.dtype == torch.float32 else 500)
 
 
 def test_short_tiled_product_serves_prompts_of_some_hundred_rows():

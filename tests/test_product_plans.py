@@ -227,3 +227,23 @@ def test_no_product_is_both_a_tiled_one_part_and_short_tiles():
             for M in (65, 128, 129, 256, 257, 512, 513, 1024, 1025, 1664, 2048):
                 plan = K.tiles_plan(M, N, K_)
                 assert plan is None or plan[0] != 1 or K.short_tiles_plan(M, N, K_, n_cus=256) is None
+
+
+def test_wide_tiles_have_parts_that_the_kernel_takes(monkeypatch):
+    """More than 64 rows of matrices of 512 rows and columns on, each part of four stages or more; where another plan of tiles serves, its parts."""
+    for N in (512, 1536, 2048, 6144, 10240, 28672):
+        for K_ in (512, 576, 4096, 14336, 21504):
+            for M in (65, 129, 334, 1024, 1025, 2048, 5003, 16384):
+                parts = K.wide_tiles_plan(M, N, K_, n_cus=256)
+                assert 1 <= parts <= 8 and (parts == 1 or K_ // 64 // parts >= 4)
+                chosen, short = K.prompt_parts(M, N, K_), K.short_tiles_plan(M, N, K_)
+                assert chosen == (short[0] if short else (K.tiles_plan(M, N, K_) or (parts,))[0] if N * K_ < 1 << 22 else K.wide_tiles_plan(M, N, K_))
+    assert K.wide_tiles_plan(128, 4096, 14336, n_cus=256) > 2 and K.wide_tiles_plan(5003, 28672, 4096, n_cus=256) == 1
+    for M, N, K_ in ((64, 4096, 4096), (2048, 4096, 4100), (2048, 511, 4096), (2048, 514, 4096), (2048, 4096, 448)):
+        assert K.wide_tiles_plan(M, N, K_, n_cus=256) == 0
+    assert K.wide_tiles_serve_gated(334, 28672, 4096) and K.wide_tiles_serve_gated(5003, 34816, 5120) and K.wide_tiles_serve_gated(256, 16384, 2048)
+    assert not K.wide_tiles_serve_gated(100, 28672, 4096) and not K.wide_tiles_serve_gated(255, 16384, 2048) and not K.wide_tiles_serve_gated(64, 1 << 20, 4096)
+    assert not K.wide_tiles_serve_gated(2048, 28672, 4100)
+    for how in ("library", "tiles"):
+        monkeypatch.setattr(K, "PROMPT_PRODUCT", how)
+        assert K.wide_tiles_plan(2048, 4096, 4096, n_cus=256) == 0 and not K.wide_tiles_serve_gated(2048, 28672, 4096)
