@@ -34,7 +34,7 @@ constexpr int kTileWaves = 4;
 constexpr int kTileBlocks = 4;                         // packed blocks of 64 rows of w a tile: 256 rows, a block a wave
 constexpr int kStageK = 64;
 constexpr int kRing = 4;                               // stages of 64 k in LDS and in registers
-enum { EPI_PLAIN = 0, EPI_SWIGLU = 1, EPI_ADD = 2 };
+enum { EPI_PLAIN = 0, EPI_SWIGLU = 1, EPI_ADD = 2, EPI_ROWS = 3, EPI_ROWS_GATED = 4 };   // (the last two: sorted rows of experts, moe_packed.hip)
 
 constexpr int tiles_lds_bytes(int tm) { return kRing * tm * 16 * kStageK * 2; }
 
@@ -46,20 +46,28 @@ __device__ __forceinline__ float tiles_gated(float gate, float up, float limit) 
     return g / (1.0f + __expf((bounded ? -1.702f : -1.0f) * g)) * u;
 }
 
+// the same for experts, whose other kernels take the exact exponential
+__device__ __forceinline__ float tiles_rows_gated(float gate, float up, float limit) {
+    const bool bounded = limit >= 0.f;
+    const float g = bounded ? fminf(gate, limit) : gate, u = bounded ? fminf(fmaxf(up, -limit), limit) + 1.0f : up;
+    return g / (1.0f + expf((bounded ? -1.702f : -1.0f) * g)) * u;
+}
+
 template <int N> __device__ __forceinline__ void tiles_wait_loads() {
     static_assert(N < 64, "the counter has six bits");
     asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory");
 }
 
-// One tile: 16 TM tokens by 256 rows of w, stages [stage_begin, stage_end) of k.  out: EPI_SWIGLU [M][N / 2], else [M][N], rows ldo apart.
-template <int TM, int EPI, typename TO>
-__device__ __forceinline__ void tile_body(
-        unsigned char* lds, TO* __restrict__ out, const bf16_t* __restrict__ a, int lda, const unsigned char* __restrict__ wp,
-        const float* __restrict__ bias, int M, int N, int K, int ldo, int n_row_blocks, int m_tile, int n_tile, int stage_begin,
-        int stage_end, float limit) {
+// The products of one tile: acc[token tile][strip] += 16 TM rows of activations . a wave's 64 rows of w over `stages` stages of 64 k.  w_base:
+// the wave's packed block at the first stage; a_base + a_off[i]: where lane l finds octet (l & 7) ^ ((row >> 1) & 7) of row
+// 8 (wave TM / 2 + i) + (l >> 3) of the tile at the first stage (tiles_a_row), offsets below 2^31.
+template <int TM> __device__ __forceinline__ int tiles_a_row(int i) { return 8 * ((int)(threadIdx.x / kWave) * (TM / 2) + i) + ((threadIdx.x & (kWave - 1)) >> 3); }
+
+template <int TM>
+__device__ __forceinline__ void tile_products(unsigned char* lds, f32x4_t (&acc)[TM][4], const unsigned char* w_base, const unsigned char* a_base,
+                                              const unsigned (&a_off)[TM / 2], int stages) {
 #ifdef __HIP_DEVICE_COMPILE__
-    constexpr int BM = TM * 16;
-    constexpr int kBuf = BM * kStageK * 2;
+    constexpr int kBuf = TM * 16 * kStageK * 2;
     constexpr int kCopies = TM / 2;                          // copies of 8 rows of activations, a wave and stage
     constexpr int kLoads = 8 + kCopies;                      // and 8 operands of w
     constexpr int kUnits = 2 * TM;                           // of a stage: 32 k of 16 tokens against the wave's 64 rows, four products
@@ -72,30 +80,17 @@ __device__ __forceinline__ void tile_body(
 
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int stages = stage_end - stage_begin;
-    const int m0 = m_tile * BM;
     const int i16 = lane & 15, g = lane >> 4;
-    const int nb = n_tile * kTileBlocks + wave;
-
     // The weights' pointer is hidden from the compiler: it could otherwise tell that nothing writes what it points to, and move
     // loads past the barriers.
-    const unsigned char* w_base = wp + ((size_t)min(nb, n_row_blocks - 1) * (K / 32) + 2 * stage_begin) * 4096;
     asm volatile("" : "+s"(w_base));
-    const unsigned char* a_base = reinterpret_cast<const unsigned char*>(a + (size_t)m0 * lda + (size_t)stage_begin * kStageK);
     const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)w_base, 0, 0x7fffffff, 0x00020000);
     const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)a_base, 0, 0x7fffffff, 0x00020000);
     const unsigned w_off = lane * 16;
-    unsigned a_off[kCopies];
-#pragma unroll
-    for (int i = 0; i < kCopies; ++i) {
-        const int row = 8 * (wave * kCopies + i) + (lane >> 3), oct = (lane & 7) ^ ((row >> 1) & 7);
-        a_off[i] = (unsigned)min(row, M - 1 - m0) * (unsigned)(lda * 2) + 16 * oct;
-    }
     int a_read[2];
 #pragma unroll
     for (int j = 0; j < 2; ++j) a_read[j] = i16 * 128 + (((4 * j + g) ^ ((i16 >> 1) & 7)) * 16);
 
-    f32x4_t acc[TM][4];
 #pragma unroll
     for (int tt = 0; tt < TM; ++tt)
 #pragma unroll
@@ -178,24 +173,48 @@ __device__ __forceinline__ void tile_body(
     tiles_wait_loads<0>();                                   // copies still on their way into LDS
     __syncthreads();
 
-    if (nb >= n_row_blocks) return;
+#endif
+}
+
+// What an epilogue needs of its tile.  out: rows ldo apart, width values each; token rows m0 .. m_end - 1; the wave's packed block of rows nb of n_row_blocks.
+struct TileEnd {
+    int m0, m_end, N, ldo, nb, n_row_blocks;
+    const float* bias;
+    float limit;
+    // of experts: the epilogue (0 as they are, 1 squares of what is above 0, 2 and 3 gated, 3 bounded), a factor, a weight for each row
+    int act;
+    float scale;
+    const float* row_weight;
+    const int* order;
+};
+
+template <int TM, int EPI, typename TO>
+__device__ __forceinline__ void tile_store(unsigned char* lds, f32x4_t (&acc)[TM][4], TO* __restrict__ out, const TileEnd& at) {
+#ifdef __HIP_DEVICE_COMPILE__
+    constexpr int BM = TM * 16, kBuf = BM * kStageK * 2;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int i16 = lane & 15, g = lane >> 4, nb = at.nb, N = at.N, ldo = at.ldo, m0 = at.m0;
+    float limit = at.limit;
+    if (nb >= at.n_row_blocks) return;
     // Results go through the wave's own quarter of LDS, so that rows of 64 to 256 bytes are stored 16 bytes a lane: tokens a pass,
     // 16-byte pieces of a row, tokens a store.
-    constexpr int kVals = EPI == EPI_SWIGLU ? 32 : 64, kEach = 16 / (int)sizeof(TO), kPieces = kVals / kEach;
+    constexpr bool kGated = EPI == EPI_SWIGLU || EPI == EPI_ROWS_GATED;
+    constexpr int kVals = kGated ? 32 : 64, kEach = 16 / (int)sizeof(TO), kPieces = kVals / kEach;
     constexpr int kRegion = kRing * kBuf / kTileWaves, kRowBytes = kPieces * 16;
     constexpr int kPass = kRegion / kRowBytes < BM ? kRegion / kRowBytes : BM, kTokens = kWave / kPieces;
     static_assert(kPass % 16 == 0 && BM % kPass == 0, "whole token tiles a pass");
     unsigned char* mine = lds + wave * kRegion;
-    const int width = EPI == EPI_SWIGLU ? N / 2 : N, col0 = kVals * nb;
+    const int width = kGated ? N / 2 : N, col0 = kVals * nb;
     const bool wide = (ldo % kEach) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
-    if (EPI == EPI_SWIGLU) asm("" : "+v"(limit));           // (not known to be the same in all lanes: selects instead of branches)
+    if (kGated) asm("" : "+v"(limit));           // (not known to be the same in all lanes: selects instead of branches)
     f32x4_t more[4];
 #pragma unroll
     for (int rt = 0; rt < 4; ++rt)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const int n = 64 * nb + 16 * rt + 4 * g + e;
-            more[rt][e] = EPI == EPI_PLAIN && bias && n < N ? bias[n] : 0.f;
+            more[rt][e] = EPI == EPI_PLAIN && at.bias && n < N ? at.bias[n] : 0.f;
         }
     auto put = [&](int t, int value, f32x4_t y) {            // values value .. value + 3 of token t of the pass
         const int piece = value / kEach;
@@ -222,11 +241,32 @@ __device__ __forceinline__ void tile_body(
                     SB();
                     put(t, 16 * i + 4 * g, y);
                 }
+            } else if (EPI == EPI_ROWS_GATED) {              // gate and up in turn: a lane's four sums are two of the result's columns
+                const float rw = at.row_weight ? at.row_weight[at.order[min(m0 + 16 * tt + i16, at.m_end - 1)]] : 1.0f;
+#pragma unroll
+                for (int rt = 0; rt < 4; ++rt) {
+                    f32x4_t y = acc[tt][rt] * one;
+                    asm volatile("" : "+v"(y));
+                    const float lo = tiles_rows_gated(y[0] * rw, y[1] * rw, limit) * at.scale, hi = tiles_rows_gated(y[2] * rw, y[3] * rw, limit) * at.scale;
+                    const int value = 8 * rt + 2 * g, piece = value / kEach;
+                    unsigned char* to = mine + t * kRowBytes + ((piece ^ (t & (kPieces - 1))) * 16) + value % kEach * (int)sizeof(TO);
+                    if (sizeof(TO) == 4) *reinterpret_cast<float2*>(to) = make_float2(lo, hi);
+                    else *reinterpret_cast<uint32_t*>(to) = tiles_pack_bf16(lo, hi);
+                    SB();
+                }
             } else {
 #pragma unroll
                 for (int rt = 0; rt < 4; ++rt) {
                     f32x4_t y = acc[tt][rt] * one;
-                    if (EPI == EPI_PLAIN && bias) y += more[rt];
+                    if (EPI == EPI_ROWS) {
+                        asm volatile("" : "+v"(y));
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const float v = fmaxf(y[e], 0.f);
+                            y[e] = (at.act == 1 ? v * v : y[e]) * at.scale;
+                        }
+                    }
+                    if (EPI == EPI_PLAIN && at.bias) y += more[rt];
                     put(t, 16 * rt + 4 * g, y);
                 }
             }
@@ -238,7 +278,7 @@ __device__ __forceinline__ void tile_body(
         for (int it = 0; it < kPass / kTokens; ++it) {
             const int t = kTokens * it + lane / kPieces, token = m0 + p0 + t;
             const u32x4_t v = *reinterpret_cast<const u32x4_t*>(mine + t * kRowBytes + ((piece ^ (t & (kPieces - 1))) * 16));
-            if (token >= M) continue;
+            if (token >= at.m_end) continue;
             TO* o = out + (size_t)token * ldo + col;
             if (wide && col + kEach <= width) {
                 if (EPI == EPI_ADD) {
@@ -263,6 +303,28 @@ __device__ __forceinline__ void tile_body(
         asm volatile("" ::: "memory");
     }
 #endif
+}
+
+// One tile: 16 TM tokens by 256 rows of w, stages [stage_begin, stage_end) of k.  out: EPI_SWIGLU [M][N / 2], else [M][N], rows ldo apart.
+template <int TM, int EPI, typename TO>
+__device__ __forceinline__ void tile_body(
+        unsigned char* lds, TO* __restrict__ out, const bf16_t* __restrict__ a, int lda, const unsigned char* __restrict__ wp,
+        const float* __restrict__ bias, int M, int N, int K, int ldo, int n_row_blocks, int m_tile, int n_tile, int stage_begin,
+        int stage_end, float limit) {
+    const int m0 = m_tile * TM * 16, nb = n_tile * kTileBlocks + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const unsigned char* w_base = wp + ((size_t)min(nb, n_row_blocks - 1) * (K / 32) + 2 * stage_begin) * 4096;
+    const unsigned char* a_base = reinterpret_cast<const unsigned char*>(a + (size_t)m0 * lda + (size_t)stage_begin * kStageK);
+    unsigned a_off[TM / 2];
+#pragma unroll
+    for (int i = 0; i < TM / 2; ++i) {
+        const int row = tiles_a_row<TM>(i);
+        a_off[i] = (unsigned)min(row, M - 1 - m0) * (unsigned)(lda * 2) + 16 * ((threadIdx.x & 7) ^ ((row >> 1) & 7));
+    }
+    f32x4_t acc[TM][4];
+    tile_products<TM>(lds, acc, w_base, a_base, a_off, stage_end - stage_begin);
+    TileEnd at{};
+    at.m0 = m0, at.m_end = M, at.N = N, at.ldo = ldo, at.nb = nb, at.n_row_blocks = n_row_blocks, at.bias = bias, at.limit = limit;
+    tile_store<TM, EPI, TO>(lds, acc, out, at);
 }
 
 // A launch, as the entry points hand it to the file that holds its kernels.  rows, rows_last: units of 16 tokens a tile; row tiles

@@ -9,6 +9,7 @@ carry whole rows that belong to no sequence, see graph.py; no kernel mixes rows.
 from __future__ import annotations
 
 import dataclasses
+import math
 import os
 from typing import List, Optional, Sequence, Tuple, Union
 
@@ -78,6 +79,14 @@ def _packing(rt: Runtime, model: Model, max_tokens: int, pack_weights: Optional[
     """pack_weights None: packed copies as far as the GPU's memory allows; True: all; False: none."""
     rt.pack_weights = pack_weights is not False and rt.dtype == torch.bfloat16
     rt.pack_budget = packed_weight_budget(model, rt.dtype, max_tokens, rt.device) if pack_weights is None else None
+    if rt.pack_budget is None:
+        rt.expert_budget = None
+        return
+    # experts get what the matrices that every token is multiplied with leave (embedding tables' copies, of tied heads, among them)
+    element = torch.empty((), dtype=rt.dtype).element_size()
+    others = sum(math.prod(spec.shape) for spec in model.tensor_specs() if spec.kind in ("matrix", "table")) - model.expert_elements()
+    rt.expert_budget = max(0, rt.pack_budget - element * others)
+    rt.pack_budget -= rt.expert_budget
 
 
 def require_gpu(device: Union[str, torch.device] = "cuda:0") -> torch.device:

@@ -204,6 +204,10 @@ class Model:
         runs += sum(self.stream_parts[e.enter[0]].weight_bytes() for e in self.schedule if e.enter is not None)
         return runs + self.final_norm.weight_bytes() + self.head.weight_bytes()
 
+    def expert_elements(self) -> int:
+        """Elements of all experts' matrices (each layer once)."""
+        return sum(p.expert_elements() for p in self.layers + self.stream_parts)
+
     def packed_weight_bytes(self) -> int:
         """Bytes of device memory that the packed second copies of the matrices take (each layer once)."""
         return sum(p.packed_bytes() for p in self.layers + self.stream_parts) + self.head.packed_bytes()

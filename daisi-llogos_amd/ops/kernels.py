@@ -770,9 +770,30 @@ def moe_form(P: int, E: int, N: int, K: int, n_cus: Optional[int] = None) -> int
     return 3 if P >= 400 * E and K >= 4096 and P * N >= 88_000_000 else 2
 
 
+def moe_packed_form(P: int, E: int) -> Tuple[int, int]:
+    """Lowest and highest tiles, in units of 64 sorted rows, among which the experts' product on packed matrices chooses for P pairs of E experts;
+    (0, 0): the form for few rows, up to 10 an expert (us, few rows / tiles of 64: 16 experts of 7168 x 4096, 8 rows 143 / 159, 12 rows 167 / 161; 64 of 1536 x
+    2048 64 / 75 and 75 / 76; 32 of 2048 x 768 19.5 / 21.7 and 23.8 / 22.2; 8 of 8192 x 4096 83 / 94 and 96 / 95).  The lower the
+    lowest, the more blocks of the grid find no tile; tiles of 64 rows gain nothing from 96 an expert on (16 of 7168 x 4096: 211 / 171 in tiles
+    of 128) and those of 128 from 600 on."""
+    if P <= 10 * E:
+        return 0, 0
+    return (1 if P < 96 * E else 2 if P < 600 * E else 3), 4
+
+
+def pack_experts(w: torch.Tensor) -> Optional["PackedWeight"]:
+    """A packed copy of experts' matrices w [E, N, K] bfloat16 as one matrix of E N rows, for moe_product; None where rows of a matrix are no multiple of 64 or
+    values no multiple of 32 (an expert would not begin with a block of its own)."""
+    E, N, K = w.shape
+    if w.dtype != torch.bfloat16 or N % 64 or K % 32 or not w.is_contiguous():
+        return None
+    return pack_weights(w.view(E * N, K))
+
+
 def moe_product(a: torch.Tensor, w: torch.Tensor, order: torch.Tensor, seg: torch.Tensor, top: int, gather: bool,
                 out_dtype: torch.dtype, relu2: bool = False, scale: float = 1.0, gated: bool = False,
-                pair_weight: Optional[torch.Tensor] = None, limit: Optional[float] = None) -> torch.Tensor:
+                pair_weight: Optional[torch.Tensor] = None, limit: Optional[float] = None,
+                packed: Optional["PackedWeight"] = None) -> torch.Tensor:
     """[P, N]: sorted row r, which belongs to the expert e whose segment holds it, is a_row(r) . w[e]^T, with
     a_row(r) = a[order[r] // top] (gather: a holds the step's token rows) or a[r] (a is sorted already);
     w [E, N, K]; relu2 squares max(., 0) in the epilogue, scale multiplies the result.  gated: the rows of
@@ -780,7 +801,7 @@ def moe_product(a: torch.Tensor, w: torch.Tensor, order: torch.Tensor, seg: torc
     silu(gate_i sum) * (up_i sum), with `limit` g * sigmoid(1.702 g) * (u + 1) of the sums bounded to g = min(gate_i, limit) and
     u = up_i within -limit .. limit; pair_weight float32 [P] (with gated): pair p's row counts as pair_weight[p] times
     itself, which multiplies both sums.  `seg` may hold more segments than w has experts: rows in those belong
-    to choices without a matrix and are left unwritten."""
+    to choices without a matrix and are left unwritten.  packed: pack_experts of w, which is then read instead of it where the form takes it."""
     _dev(a, w, order, seg)
     _i32(order, "order"); _i32(seg, "seg")
     _need(a.dim() == 2 and w.dim() == 3 and a.shape[1] == w.shape[2] and seg.numel() >= w.shape[0] + 1, "moe_product: a [M, K], w [E, N, K]")
@@ -804,6 +825,15 @@ def moe_product(a: torch.Tensor, w: torch.Tensor, order: torch.Tensor, seg: torc
         form = moe_form(P, E, N, Kk)
         if MOE_PRODUCT != "auto":
             form = ("few", "tiles64", "tiles128", "tiles256").index(MOE_PRODUCT)
+        if packed is not None:
+            _need(packed.N == E * N and packed.K == Kk and not packed.gate_rows and packed.data.device == w.device, "moe_product: packed must be the experts' matrices")
+            least, most = moe_packed_form(P, E) if MOE_PRODUCT == "auto" else ((0, 0), (1, 1), (2, 2), (4, 4))[form]
+            code = _lib().llogos_moe_product_packed_bf16(_p(out), _DT[out_dtype], _p(a), a.shape[0], _p(packed.data), _p(order), _p(seg), E, top,
+                                                         1 if gather else 0, P, N, Kk, a.stride(0), act, ctypes.c_float(scale), _p(pair_weight), lim,
+                                                         least, most, compute_units(w.device), _stream())
+            if code != -2:
+                _check(code, "moe_product_packed")
+                return out
         code = _lib().llogos_moe_product_bf16(_p(out), _DT[out_dtype], _p(a), _p(w), _p(order), _p(seg), E, top, 1 if gather else 0,
                                               P, N, Kk, a.stride(0), act, ctypes.c_float(scale), _p(pair_weight), lim, form, _stream())
         if code != -2:

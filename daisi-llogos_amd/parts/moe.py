@@ -26,6 +26,27 @@ def _float32(product: torch.Tensor) -> torch.Tensor:
     return product if product.dtype == torch.float32 else K.sum_parts(product, None, torch.float32)
 
 
+def _packed(w: torch.Tensor, rt: Runtime) -> Optional[K.PackedWeight]:
+    """The experts' packed copy, if the runtime wants packed weights, what is left for experts still holds this one and the shape has one."""
+    if not (rt.pack_weights and w.dtype == torch.bfloat16):
+        return None
+    need = w.numel() * w.element_size()
+    if rt.expert_budget is not None and need > rt.expert_budget:
+        return None
+    try:
+        packed = K.pack_experts(w)
+    except torch.cuda.OutOfMemoryError:
+        rt.expert_budget = 0                                 # (no room after all: the row-major matrices serve)
+        return None
+    if rt.expert_budget is not None and packed is not None:
+        rt.expert_budget -= need
+    return packed
+
+
+def _packed_bytes(*packed: Optional[K.PackedWeight]) -> int:
+    return sum(p.data.numel() * p.data.element_size() for p in packed if p is not None)
+
+
 @register_feed_forward("table_moe")
 class TableMoE(FeedForward):
     graph_safe = True
@@ -40,6 +61,8 @@ class TableMoE(FeedForward):
         self.n_experts, self.top, self.intermediate = int(n_experts), int(top), int(intermediate)
         self.shared_intermediate, self.activation = int(shared_intermediate), activation
         self.table = self.up = self.down = None
+        self.packed_up: Optional[K.PackedWeight] = None      # the copies that steps and prompts read
+        self.packed_down: Optional[K.PackedWeight] = None
         self.shared_up = self.shared_down = None
         if self.shared_intermediate:
             # the gate's row rides behind the shared expert's up matrix: one product for both
@@ -65,6 +88,7 @@ class TableMoE(FeedForward):
         for e in range(E):
             self.up[e].copy_(get(f"{p}e{e}.up"))
             self.down[e].copy_(get(f"{p}e{e}.down"))
+        self.packed_up, self.packed_down = _packed(self.up, rt), _packed(self.down, rt)
         table = get(p + "table")
         if table.dtype.is_floating_point:
             raise ValueError(f"{p}table must hold integers")
@@ -76,14 +100,20 @@ class TableMoE(FeedForward):
             self.shared_up.bind(get, rt)
             self.shared_down.bind(get, rt)
 
+    def packed_bytes(self) -> int:
+        return super().packed_bytes() + _packed_bytes(self.packed_up, self.packed_down)
+
+    def expert_elements(self) -> int:
+        return 2 * self.n_experts * self.intermediate * self.hidden
+
     def matrix_elements(self) -> int:
         """What a token is multiplied with: its `top` experts and the shared one."""
         return super().matrix_elements() + 2 * self.top * self.intermediate * self.hidden
 
     def forward(self, ctx: StepContext, h: torch.Tensor):
         order, seg, where = K.moe_route(ctx.ids, self.table, self.n_experts)
-        act = K.moe_product(h, self.up, order, seg, self.top, True, self.rt.dtype, relu2=True)
-        y = K.moe_product(act, self.down, order, seg, self.top, False, torch.float32)
+        act = K.moe_product(h, self.up, order, seg, self.top, True, self.rt.dtype, relu2=True, packed=self.packed_up)
+        y = K.moe_product(act, self.down, order, seg, self.top, False, torch.float32, packed=self.packed_down)
         mark(ctx, "experts")
         shared = gate = None
         if self.shared_up is not None:
@@ -158,6 +188,8 @@ class RoutedMoE(FeedForward):
         self.groups, self.keep, self.scale = int(groups), int(keep), float(scale)
         self.shared_intermediate, self.has_correction = int(shared_intermediate), bool(correction)
         self.router_w = self.correction = self.gate_up = self.down = None
+        self.packed_up: Optional[K.PackedWeight] = None      # the copies that steps and prompts read
+        self.packed_down: Optional[K.PackedWeight] = None
         self.shared = None
         self.probed = None          # {"choice": int32 [T, top]} of the last step that was run part by part (measurements)
         if self.shared_intermediate:
@@ -193,10 +225,17 @@ class RoutedMoE(FeedForward):
                 self.gate_up[e, 0::2].copy_(get(f"{p}e{e}.gate"))
                 self.gate_up[e, 1::2].copy_(get(f"{p}e{e}.up"))
                 self.down[e].copy_(get(f"{p}e{e}.down"))
+            self.packed_up, self.packed_down = _packed(self.gate_up, rt), _packed(self.down, rt)
         self.router_w = get(p + "router").to(device=rt.device, dtype=torch.float32).contiguous()
         self.correction = get(p + "correction").to(device=rt.device, dtype=torch.float32).contiguous() if self.has_correction else None
         if self.shared is not None:
             self.shared.bind(get, rt)
+
+    def packed_bytes(self) -> int:
+        return super().packed_bytes() + _packed_bytes(self.packed_up, self.packed_down)
+
+    def expert_elements(self) -> int:
+        return 3 * self.n_experts * self.intermediate * self.hidden
 
     def matrix_elements(self) -> int:
         """What a token is multiplied with: the router, its `top` experts (as if all had matrices) and the shared one."""
@@ -219,8 +258,8 @@ class RoutedMoE(FeedForward):
         if self.n_experts:
             order, seg, where = K.moe_route(None, choice, self.outputs)
             act = K.moe_product(h, self.gate_up, order, seg, self.top, True, self.rt.dtype, gated=True,
-                                pair_weight=weight.view(-1) if self.weigh == "input" else None, limit=self.limit)
-            y = K.moe_product(act, self.down, order, seg, self.top, False, torch.float32)
+                                pair_weight=weight.view(-1) if self.weigh == "input" else None, limit=self.limit, packed=self.packed_up)
+            y = K.moe_product(act, self.down, order, seg, self.top, False, torch.float32, packed=self.packed_down)
         else:
             where = torch.zeros(T * self.top, dtype=torch.int32, device=h.device)
             y = torch.zeros((T * self.top, W), dtype=torch.float32, device=h.device)

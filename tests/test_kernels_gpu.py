@@ -1166,6 +1166,43 @@ def test_expert_product_at_the_edges_of_its_tiles(form, N, K_, monkeypatch):
         _close(half, _np(want.clamp(min=0) ** 2), "bfloat16")
 
 
+@pytest.mark.parametrize("form", ["few", "tiles64", "tiles128", "tiles256", "auto"])
+@pytest.mark.parametrize("N,K_", [(64, 64), (192, 96), (320, 1088), (576, 256)])
+def test_expert_product_on_packed_matrices(form, N, K_, monkeypatch):
+    """The edges of test_expert_product_at_the_edges_of_its_tiles with the matrices packed, every epilogue and type: columns that fill no tile of
+    256, k of no whole round of the ring (and of no whole stage, which the tiles leave to the row-major form); the few-row form gives the
+    row-major one's bits."""
+    monkeypatch.setattr(K, "MOE_PRODUCT", form)
+    rng = np.random.default_rng(N)
+    sizes = [0, 1, 15, 16, 17, 0, 63, 64, 65, 127, 128, 129, 191, 192, 193, 255, 256, 257, 300] + [0, 1] * 40
+    seg = _t(np.concatenate([[0], np.cumsum(sizes)]), torch.int32)
+    P, E = sum(sizes), len(sizes)
+    order = _t(rng.permutation(P), torch.int32)
+    a = _t(rng.standard_normal((P, K_)), torch.bfloat16)
+    w = _t(rng.standard_normal((E, N, K_)) * 0.1, torch.bfloat16)
+    packed = K.pack_experts(w)
+    pair = _t(rng.uniform(0.1, 1.0, P))
+    for gather in (True, False):
+        rows = a[order.long()] if gather else a
+        want = torch.cat([rows[int(seg[e]):int(seg[e + 1])].double() @ w[e].double().t() for e in range(E)])
+        # (products of bfloat16 are exact in 32 bits; a sum in any order is off by a few roundings of its partial sums)
+        bound = 2.0 ** -23 * K_ ** 0.5 * 4 * max(1.0, want.abs().max().item())
+        got = K.moe_product(a, w, order, seg, 1, gather, torch.float32, packed=packed)
+        assert (got.double() - want).abs().max() <= bound
+        if form == "few":
+            assert torch.equal(got, K.moe_product(a, w, order, seg, 1, gather, torch.float32))
+        _close(K.moe_product(a, w, order, seg, 1, gather, torch.bfloat16, relu2=True, packed=packed), _np(want.clamp(min=0) ** 2), "bfloat16")
+        weight = pair[order.long()].double()[:, None]
+        gate, up = want[:, 0::2] * weight, want[:, 1::2] * weight
+        room = 1.2 * bound * (1 + up.abs().max() + gate.abs().max()) + 2e-6 * (gate.abs() * up.abs()).max()
+        got = K.moe_product(a, w, order, seg, 1, gather, torch.float32, gated=True, scale=0.5, pair_weight=pair, packed=packed)
+        assert (got.double() - 0.5 * torch.nn.functional.silu(gate) * up).abs().max() <= room
+        g, u = want[:, 0::2].clamp(max=0.7), want[:, 1::2].clamp(-0.7, 0.7)
+        got = K.moe_product(a, w, order, seg, 1, gather, torch.float32, gated=True, limit=0.7, packed=packed)
+        assert (got.double() - g * torch.sigmoid(1.702 * g) * (u + 1)).abs().max() <= room
+    assert K.pack_experts(w[:, :N - 32].contiguous()) is None and K.pack_experts(w[:, :, :K_ - 8].contiguous()) is None and K.pack_experts(w.float()) is None
+
+
 @pytest.mark.parametrize("M,N,K_", [(1, 64, 64), (129, 320, 192), (700, 1100, 128), (2100, 2900, 64), (4700, 260, 128)])
 def test_tiled_product_places_every_tile_and_adds_itself(M, N, K_):
     """One tile, fewer than XCDs, bands of token tiles that are not full, several rounds of blocks, parts of k: every value is

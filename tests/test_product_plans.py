@@ -247,3 +247,12 @@ def test_wide_tiles_have_parts_that_the_kernel_takes(monkeypatch):
     for how in ("library", "tiles"):
         monkeypatch.setattr(K, "PROMPT_PRODUCT", how)
         assert K.wide_tiles_plan(2048, 4096, 4096, n_cus=256) == 0 and not K.wide_tiles_serve_gated(2048, 28672, 4096)
+
+
+def test_packed_experts_tiles():
+    """Few rows up to ten an expert; then heights that the kernel has, the lowest not above what an average segment fills."""
+    assert K.moe_packed_form(160, 16) == (0, 0) and K.moe_packed_form(1, 1) == (0, 0)
+    for E in (1, 16, 1024):
+        for n in (11, 95, 96, 599, 600, 5000):
+            least, most = K.moe_packed_form(E * n, E)
+            assert 1 <= least <= most == 4 and (least == 1 or 64 * least <= n + 63)
