@@ -2132,9 +2132,7 @@ def long_tiles_plan(M: int, N: int, K: int, n_cus: Optional[int] = None) -> Opti
 def _tiles_cost(M: int, N: int, K: int, parts: int, token_tiles: int, units: int) -> float:
     """Microseconds that the tiled product is expected to take (gemm_tiles_bf16.hip: tiles_cost), with its consumer's reading of the
     results, 0.2 us a MB."""
-    cost = _lib().llogos_gemm_tiles_cost
-    cost.restype = ctypes.c_double
-    return cost(M, N, K, parts, token_tiles, units) + parts * M * N * 4e-6 * 0.2
+    return _lib().llogos_gemm_tiles_cost(M, N, K, parts, token_tiles, units) + parts * M * N * 4e-6 * 0.2
 
 
 @functools.lru_cache(maxsize=4096)

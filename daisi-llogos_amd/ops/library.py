@@ -12,6 +12,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 import tempfile
 import threading
 import time
@@ -20,6 +21,7 @@ from concurrent.futures import ThreadPoolExecutor
 _CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "csrc")
 _PKG = os.path.dirname(_CSRC)
 LIB_NAME = "libllogos_hip.so"
+HOST_NAME = f"libllogos_host.{sysconfig.get_config_var('SOABI') or 'python'}.so"      # what reads Python's own objects, for this interpreter alone
 ARCH = "gfx950"
 
 HIPCC_FLAGS = [
@@ -31,6 +33,7 @@ HIPCC_FLAGS = [
 
 _lock = threading.Lock()
 _lib = None
+_host = None
 
 
 class KernelLibraryError(RuntimeError):
@@ -48,7 +51,7 @@ def sources() -> list:
 def _source_hash() -> str:
     h = hashlib.sha256()
     for name in sorted(os.listdir(_CSRC)):
-        if name.endswith((".hip", ".h")):
+        if name.endswith((".hip", ".h", ".cpp")):
             h.update(name.encode())
             with open(os.path.join(_CSRC, name), "rb") as fh:
                 h.update(fh.read())
@@ -187,9 +190,54 @@ def build(verbose: bool = True) -> str:
                 pass
     if verbose:
         _log(f"built {lib_path} in {time.time() - t0:.0f} s")
-    global _lib
-    _lib = None
+    _build_host(out_dir, env)
+    global _lib, _host
+    _lib = _host = None
     return lib_path
+
+
+def _build_host(out_dir: str, env: dict) -> None:
+    """The helpers that pack Python's lists (host_pack.cpp), beside the kernel library.  Without Python's headers or a compiler for the host there
+    are none, and the callers do the same in Python."""
+    path, tmp = os.path.join(out_dir, HOST_NAME), os.path.join(out_dir, f".{HOST_NAME}.{os.getpid()}")
+    compiler = shutil.which("g++") or shutil.which("clang++") or shutil.which("c++")
+    include = sysconfig.get_paths().get("include", "")
+    try:
+        if compiler is None or not os.path.isfile(os.path.join(include, "Python.h")):
+            raise KernelLibraryError("no compiler or no Python.h")
+        _run_with_progress([compiler, "-O3", "-std=c++17", "-shared", "-fPIC", "-I", include, os.path.join(_CSRC, "host_pack.cpp"), "-o", tmp], "host_pack.cpp", env)
+        os.replace(tmp, path)
+    except (KernelLibraryError, OSError) as e:
+        _log(f"without the host's helpers: {e}")
+        for leftover in (tmp, path):
+            try:
+                os.remove(leftover)
+            except OSError:
+                pass
+
+
+def host():
+    """The helpers of host_pack.cpp, which hold the interpreter's lock, or None where they are not built."""
+    global _host
+    if _host is None:
+        load()
+        path = find_library()
+        path = os.path.join(os.path.dirname(path), HOST_NAME) if path else ""
+        found = False
+        if os.path.isfile(path):
+            try:
+                found = ctypes.PyDLL(path)
+                for name, result, args in (("llogos_host_windows_size", ctypes.c_longlong, [ctypes.py_object, ctypes.c_longlong]),
+                                           ("llogos_host_windows", ctypes.c_longlong, [ctypes.py_object, ctypes.c_longlong, ctypes.c_longlong,
+                                                                                       ctypes.c_void_p, ctypes.c_void_p, ctypes.c_longlong]),
+                                           ("llogos_host_uniforms", ctypes.c_int, [ctypes.py_object] * 3 + [ctypes.c_longlong, ctypes.c_void_p])):
+                    f = getattr(found, name)
+                    f.restype, f.argtypes = result, args
+            except (OSError, AttributeError) as e:
+                _log(f"without the host's helpers: {e}")
+                found = False
+        _host = found
+    return _host or None
 
 
 _C_TYPES = {"int": ctypes.c_int, "float": ctypes.c_float, "double": ctypes.c_double, "long long": ctypes.c_longlong,

@@ -10,7 +10,7 @@ from typing import List, Optional, Sequence
 import numpy as np
 import torch
 
-from ..ops import kernels as K
+from ..ops import kernels as K, library
 from .params import GenerationParams
 from .rng import uniforms
 
@@ -64,15 +64,48 @@ class Sampler:
         """The same for a small top-k, whose rows two kernels take from the logits to the token."""
         p = self.params
         R = logits.shape[0]
+        # one copy: uniform numbers, then each window's place and the windows, packed straight into the staging buffer
+        starts, n, host, copied = self._pack(R, requests, indices, histories) or self._pack_in_python(requests, indices, histories)
+        dev = torch.empty(n, dtype=torch.int32, device=logits.device)
+        dev.copy_(host[:n], non_blocking=True)
+        copied.record(torch.cuda.current_stream(logits.device.index))    # (named by its number, which is quicker than finding the current device)
+        us = dev[:starts[0]].view(torch.float32)
+        hist, hist_at = (dev[starts[1]:], dev[starts[0]:starts[1]]) if p.has_penalties else (None, None)
+        return K.sample_few(logits, hist, hist_at, p.repetition_penalty, p.frequency_penalty, p.presence_penalty, p.temperature,
+                            p.penalize_newline, self.stop_tokens if p.prevent_eos else (), us, p.top_k, p.top_p, p.min_p, p.typical_p, p.min_keep)
+
+    def _pack(self, R: int, requests, indices, histories):
+        """((where the windows' places begin, where the windows do), 32-bit numbers in all, staging buffer, its event) with R rows' uniform numbers and
+        windows in the buffer; None for what the host's helpers leave to Python (anything but lists and tuples of plain integers)."""
+        p, helpers = self.params, library.host()
+        if helpers is None or getattr(self.uniforms, "__func__", None) is not Sampler.uniforms:      # (or the numbers come from elsewhere)
+            return None
+        count = p.penalty_count
+        if not (p.has_penalties and -1 << 62 < count < 1 << 62):
+            size = -1 if p.has_penalties else 0
+        else:
+            size = helpers.llogos_host_windows_size(histories, count)
+        if size < 0:
+            return None
+        rows = R + 1 if p.has_penalties else 1
+        host, copied, _, address = self._staging_buffer(R + rows + size)
+        seed = p.seed if p.seed is not None else self._fresh_seed
+        if helpers.llogos_host_uniforms(seed, requests, indices, R, address) != 0:
+            return None
+        if p.has_penalties and helpers.llogos_host_windows(histories, count, R, address + 4 * R, address + 4 * (R + rows), size) != size:
+            return None
+        return (R, R + rows), R + rows + size, host, copied
+
+    def _pack_in_python(self, requests, indices, histories):
+        p = self.params
         us = self.uniforms(requests, indices)
         flat, at = [], [0]
         if p.has_penalties:
             for h in histories:
                 flat += h[-p.penalty_count:] if 0 < p.penalty_count < len(h) else h
                 at.append(len(flat))
-        # one copy: uniform numbers, then each window's place and the windows, packed straight into the staging buffer
         n = len(us) + len(at) + len(flat)
-        host, copied, numbers = self._staging_buffer(n)
+        host, copied, numbers, _ = self._staging_buffer(n)
         try:
             struct.pack_into(f"={len(us)}f{len(at) + len(flat)}i", numbers, 0, *us, *at, *flat)
         except (struct.error, TypeError):                # (tokens that are no whole numbers: as numpy rounds them)
@@ -80,26 +113,20 @@ class Sampler:
             view[:len(us)] = np.asarray(us, dtype=np.float32).view(np.int32)
             view[len(us):len(us) + len(at)] = at
             view[len(us) + len(at):n] = flat
-        dev = torch.empty(n, dtype=torch.int32, device=logits.device)
-        dev.copy_(host[:n], non_blocking=True)
-        copied.record()
-        hist, hist_at = (dev[len(us) + len(at):], dev[len(us):len(us) + len(at)]) if p.has_penalties else (None, None)
-        return K.sample_few(logits, hist, hist_at, p.repetition_penalty, p.frequency_penalty, p.presence_penalty, p.temperature,
-                            p.penalize_newline, self.stop_tokens if p.prevent_eos else (), dev[:len(us)].view(torch.float32), p.top_k, p.top_p,
-                            p.min_p, p.typical_p, p.min_keep)
+        return (len(us), len(us) + len(at)), n, host, copied
 
     def _staging_buffer(self, n: int):
-        """A pinned buffer of at least n 32-bit numbers, the event to record behind its copy, and its memory as bytes: one of a
+        """A pinned buffer of at least n 32-bit numbers, the event to record behind its copy, its memory as bytes and its address: one of a
         few, each free again once its last copy has run."""
         ring = getattr(self, "_staging", None)
         if ring is None or ring[0][0].numel() < n:
-            ring = self._staging = [(torch.empty(max(1024, 2 * n), dtype=torch.int32, pin_memory=True),
-                                     torch.cuda.Event()) for _ in range(4)]
+            hosts = [torch.empty(max(1024, 2 * n), dtype=torch.int32, pin_memory=True) for _ in range(4)]
+            ring = self._staging = [(h, torch.cuda.Event(), memoryview(h.numpy()).cast("B"), h.data_ptr()) for h in hosts]
             self._staging_next = 0
-        host, copied = ring[self._staging_next]
+        place = ring[self._staging_next]
         self._staging_next = (self._staging_next + 1) % len(ring)
-        copied.synchronize()
-        return host, copied, memoryview(host.numpy()).cast("B")
+        place[1].synchronize()
+        return place
 
     def _to_device(self, arrays, device) -> List[torch.Tensor]:
         """The step's small host arrays (int32 or float32) on the device with one copy, without
@@ -109,7 +136,7 @@ class Sampler:
         if not arrays:
             return []
         n = sum(a.size for a in arrays)
-        host, copied, _ = self._staging_buffer(n)
+        host, copied, _, _ = self._staging_buffer(n)
         flat = host.numpy()
         o = 0
         for a in arrays:
