@@ -14,11 +14,12 @@
 //
 // One to four rows (gemm_f32_lanes_kernel) and few rows (gemm_f32_rows_kernel): bound by reading w once.
 // In the second a block owns 16 or 32 rows of w and all of k; its waves take 256 k in turn straight from
-// memory, a mid each, and LDS adds the mids in order.  Many rows (gemm_f32_tiles_kernel): bound by the
-// matrix cores (157 TFLOP/s); tiles of 128 x 64, 64 x 64 or 64 x 32 through two LDS buffers of 32 k.
+// memory, a mid each, and LDS adds the mids in order.  Many rows: bound by the matrix cores (157 TFLOP/s at 2.4 GHz, of which no form
+// reached more than 117); gemm_f32_ring_kernel where K is a multiple of 32, else gemm_f32_tiles_kernel: tiles of 128 x 64, 64 x 64 or 64 x 32
+// through two LDS buffers of 32 k.
 // Measured (us; before: plain FMAs in tiles of 64 x 64, up to 32 rows a wave for a few columns).  705 rows of the 1B
-// sizes: gate/up [16384, 2048] 1,507 -> 459 (103 TFLOP/s), o [2048, 2048] about 390 -> 80, down [2048, 8192] about
-// 1,510 -> 305, q/k/v [3072, 2048] 448 -> 115.  2 rows: gate/up 28.3 -> 28.6 (4.7 TB/s), head [128256, 2048] 209 -> 180
+// sizes, these / tiles / ring: gate/up [16384, 2048] 1,507 / 478 / 436 (109 TFLOP/s), o [2048, 2048] about 390 / 70 / 62, down [2048, 8192] about
+// 1,510 / 270 / 238, q/k/v [3072, 2048] 448 / 108 / 97.  2 rows: gate/up 28.3 -> 28.6 (4.7 TB/s), head [128256, 2048] 209 -> 180
 // (5.8 TB/s).  Distance from 64 bits at k = 8192: 1.5e-7 of the result.
 #include "common.h"
 
@@ -280,6 +281,140 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tiles_kernel(
         }
 }
 
+// Many rows, K a multiple of 32: the same sums with the matrix cores kept at work by each wave alone.  4 waves, WM along the rows of a by WN along the
+// rows of w, each 16 MT x 16 NT of the result.  A ring of four stages of 32 k in LDS, filled by buffer loads (rows of 128 bytes, their eight 16-byte
+// pieces swizzled); one raw barrier a stage, in front of it a wait for the copies of the next stage alone.  A step of 16 k is MT NT chains of four
+// products; between them, pinned, one to a product: the additions of the step before to its mids (a chain's last product is long done by then), the
+// reads of the next step's operands, the copies of the stage after next but one.  Eight stages are written out, so that the additions to the total
+// stand in one place; stages past K bring zeros, and zeros change no sum.
+template <int MT, int NT, int WM, int WN>
+__global__ __launch_bounds__(256, 2) void gemm_f32_ring_kernel(
+        float* __restrict__ out, const float* __restrict__ a, const float* __restrict__ w, const float* __restrict__ bias, int M, int N, int K,
+        int lda, int ldo, int vec_out, int m_tiles, int n_tiles) {
+#ifdef __HIP_DEVICE_COMPILE__
+    constexpr int BM = 16 * MT * WM, BN = 16 * NT * WN, ROWS = BM + BN, BUF = ROWS * 128, RING = 4;
+    constexpr int COPIES = (ROWS / 8 + 3) / 4, LEAST = ROWS / 8 / 4;         // of 8 rows a wave and stage; what every wave has of them
+    constexpr int TILES = MT * NT, READS = MT + NT, PRODUCTS = 4 * TILES;
+    static_assert(WM * WN == 4 && ROWS % 8 == 0, "four waves");
+    extern __shared__ __attribute__((aligned(1024))) unsigned char f32_lds[];
+    const int tiles = m_tiles * n_tiles, per = tiles >> 3, more = tiles & 7, xcd = blockIdx.x & 7;
+    const int tile = xcd * per + min(xcd, more) + (blockIdx.x >> 3);
+    const int m0 = (tile % m_tiles) * BM, n0 = (tile / m_tiles) * BN;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), i = lane & 15, g = lane >> 4;
+    const int wm = (wave % WM) * 16 * MT, wn = (wave / WM) * 16 * NT;
+    const int stages = K / 32;
+
+    const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(a + (size_t)m0 * lda), 0, 0x7fffffff, 0x00020000);
+    const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(w + (size_t)n0 * K), 0, 0x7fffffff, 0x00020000);
+    unsigned off[COPIES];
+#pragma unroll
+    for (int c = 0; c < COPIES; ++c) {
+        const int row = 8 * (4 * c + wave) + (lane >> 3), piece = (lane & 7) ^ ((row >> 1) & 7);
+        off[c] = (row < BM ? (unsigned)min(row, M - 1 - m0) * (unsigned)(4 * lda) : (unsigned)min(row - BM, N - 1 - n0) * (unsigned)(4 * K)) + 16 * piece;
+    }
+    auto copy = [&](int slot, int c, int stage, unsigned past) {
+        const int q = 4 * c + wave;                                          // (the same for a whole wave)
+        if (ROWS / 8 % 4 != 0 && c == COPIES - 1 && q >= ROWS / 8) return;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(q < BM / 8 ? a_rsrc : w_rsrc, (__attribute__((address_space(3))) void*)(f32_lds + slot * BUF + q * 1024), 16,
+                                                 off[c] | past, stage * 128, 0, 0);
+    };
+    auto past_end = [&](int stage) { return stage < stages ? 0u : 0x80000000u; };
+    int at[2];
+#pragma unroll
+    for (int p = 0; p < 2; ++p) at[p] = i * 128 + (((4 * p + g) ^ ((i >> 1) & 7)) * 16);
+    struct Frags { f32x4 a[MT], w[NT]; };
+    auto read_one = [&](Frags& f, int slot, int p, int r) {
+        const unsigned char* base = f32_lds + slot * BUF + at[p];
+        if (r < MT) f.a[r] = *reinterpret_cast<const f32x4*>(base + (wm + 16 * r) * 128);
+        else f.w[r - MT] = *reinterpret_cast<const f32x4*>(base + (BM + wn + 16 * (r - MT)) * 128);
+    };
+    float mid[NT][MT][4], total[NT][MT][4];
+    f32x4 part[2][NT][MT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            part[0][n][m] = part[1][n][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int v = 0; v < 4; ++v) mid[n][m][v] = total[n][m][v] = 0.f;
+        }
+    auto meet = [&]() {
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // step p of the stage in `slot`, of the products cur; next: the step behind it
+    auto step = [&](const Frags& cur, Frags& next, int slot, int p, int stage) {
+        const unsigned past = past_end(stage + 3);
+        f32x4 (&now)[NT][MT] = part[p];
+        const f32x4 (&before)[NT][MT] = part[p ^ 1];
+#pragma unroll
+        for (int x = 0; x < PRODUCTS; ++x) {
+            const int e = x / TILES, n = x % TILES / MT, m = x % MT;
+            now[n][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.w[n][e], cur.a[m][e], e ? now[n][m] : f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            {                                                                // one addition a product: tile x / 4, value x % 4
+                const int tn = x / 4 / MT, tm = x / 4 % MT;
+                asm volatile("v_add_f32 %0, %1, %0" : "+v"(mid[tn][tm][x % 4]) : "v"(before[tn][tm][x % 4]));
+            }
+            if (p == 0) {
+#pragma unroll
+                for (int c = COPIES * x / PRODUCTS; c < COPIES * (x + 1) / PRODUCTS; ++c) copy((slot + 3) & 3, c, stage + 3, past);
+#pragma unroll
+                for (int r = READS * x / PRODUCTS; r < READS * (x + 1) / PRODUCTS; ++r) read_one(next, slot, 1, r);
+            } else if (x == TILES - 1) {
+                // every operand of this buffer is here (the products above took them), and so are this wave's copies of the next stage
+                asm volatile("s_waitcnt vmcnt(%0)" :: "n"(2 * LEAST) : "memory");
+                meet();
+            } else if (x >= TILES) {
+#pragma unroll
+                for (int r = READS * (x - TILES) / (PRODUCTS - TILES); r < READS * (x - TILES + 1) / (PRODUCTS - TILES); ++r) read_one(next, (slot + 1) & 3, 0, r);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+#pragma unroll
+    for (int s = 0; s < 3; ++s)
+#pragma unroll
+        for (int c = 0; c < COPIES; ++c) copy(s, c, s, past_end(s));
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt vmcnt(%0)" :: "n"(2 * LEAST) : "memory");
+    meet();
+    Frags f0, f1;
+#pragma unroll
+    for (int r = 0; r < READS; ++r) read_one(f0, 0, 0, r);
+    int s = 0;
+    do {                                                         // 256 k
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            step(f0, f1, j & 3, 0, s + j);
+            if (j == 0) {                                        // the last step of the 256 k before is in: their mids are whole
+#pragma unroll
+                for (int n = 0; n < NT; ++n)
+#pragma unroll
+                    for (int m = 0; m < MT; ++m)
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) { total[n][m][v] += mid[n][m][v]; mid[n][m][v] = 0.f; }
+            }
+            step(f1, f0, j & 3, 1, s + j);
+        }
+        s += 8;
+    } while (s < stages);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");             // copies still on their way into LDS
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            f32x4 v;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = total[n][m][e] + (mid[n][m][e] + part[1][n][m][e]);
+            const int row = m0 + wm + 16 * m + i;
+            if (row < M) store4(out, bias, v, row, n0 + wn + 16 * n + 4 * g, N, ldo, vec_out != 0);
+        }
+#endif
+}
+
 namespace {
 
 constexpr double kUnitFlops = 157.3e12 / 256;               // of one compute unit
@@ -292,6 +427,17 @@ double tiles_cost(double M, double N, double K, int tm, int tn, double units) {
     const double together = tn == 32 ? 4 : tm == 64 ? 3 : 2;
     const double busy = ceil(blocks / units) * tile * K, waits = ceil(blocks / (units * together)) * (tile * K + K / 32 * 0.35e-6);
     return (busy > waits ? busy : waits) + 3e-6;
+}
+
+// Microseconds of the ring: forms 9 to 12.  A stage of 32 k of a block alone on its compute unit takes `alone`, of each of `together` blocks that
+// share one `shared` (the matrix cores at 72 to 75 % of their rate, whatever runs beside them).  Fitted to 64 to 1,024 rows of six matrices, within 6 %.
+struct RingForm { int tm, tn, together; double alone, shared; };
+constexpr RingForm kRing[4] = {{64, 64, 2, 0.66, 0.573}, {64, 32, 3, 0.46, 0.288}, {48, 64, 2, 0.556, 0.48}, {80, 64, 2, 0.89, 0.746}};
+
+double ring_cost(double M, double N, double K, const RingForm& f, double units) {
+    const int blocks = (int)ceil(ceil(M / f.tm) * ceil(N / f.tn) / units), rest = blocks % f.together;
+    const double stage = (blocks - rest) * f.shared + (rest ? (rest * f.shared > f.alone ? rest * f.shared : f.alone) : 0.0);
+    return (5.0 + ceil(K / 256) * 8 * stage) * 1e-6;
 }
 
 // 17 rows and more by the few-row kernel: what its blocks ask of the caches (their strips of w and the rows of a, once a block), at the rates
@@ -330,20 +476,37 @@ int lanes_cols(int M, int N, int K, bool vec) {
         else gemm_f32_tiles_kernel<TM, TN, false><<<mt * nt, 256, 0, stream>>>(out, a, w, bias, M, N, K, lda, ldo, vec_out, mt, nt); \
     } while (0)
 
+#define RING(MT, NT, WM, WN) do { \
+        const int mt = (M + 16 * MT * WM - 1) / (16 * MT * WM), nt = (N + 16 * NT * WN - 1) / (16 * NT * WN); \
+        constexpr int smem = 4 * 128 * 16 * (MT * WM + NT * WN); \
+        static std::atomic<uint64_t> asked{0}; \
+        const int code = allow_dynamic_lds((const void*)gemm_f32_ring_kernel<MT, NT, WM, WN>, smem, asked); \
+        if (code != 0) return code; \
+        gemm_f32_ring_kernel<MT, NT, WM, WN><<<mt * nt, 256, smem, stream>>>(out, a, w, bias, M, N, K, lda, ldo, vec_out, mt, nt); \
+    } while (0)
+
 // form: 0 chosen by the costs above; 1 to 4 the few-row kernel with 16, 32, 64 rows of a or 64 rows of a and 32 of w a block; 5 to 7 tiles of
-// 64 x 32, 64 x 64, 128 x 64; 8 the lanes' kernel
+// 64 x 32, 64 x 64, 128 x 64; 8 the lanes' kernel; 9 to 12 the ring's tiles of 64 x 64, 64 x 32, 48 x 64, 80 x 64
 LLOGOS_EXPORT int llogos_gemm_f32(float* out, const float* a, const float* w, const float* bias,
                                   int M, int N, int K, int lda, int ldo, int form, hipStream_t stream) {
-    if (M <= 0 || N <= 0 || K <= 0 || lda < K || ldo < N || form < 0 || form > 8) return LLOGOS_BAD_ARGUMENT;
+    if (M <= 0 || N <= 0 || K <= 0 || lda < K || ldo < N || form < 0 || form > 12) return LLOGOS_BAD_ARGUMENT;
     const bool vec = (K & 3) == 0 && (lda & 3) == 0 && (((uintptr_t)a | (uintptr_t)w) & 15) == 0;
     const int vec_out = (ldo & 3) == 0 && ((uintptr_t)out & 15) == 0;
     const int cols = lanes_cols(M, N, K, vec), units = device_units();
     if (form == 0 && cols) form = 8;
+    // (the ring counts a tile's bytes from its first row in 31 bits, and asks for whole stages of aligned rows)
+    const bool ring = vec && K % 32 == 0 && lda <= 1 << 22 && K <= 1 << 22;
+    if (form > 8 && !ring) return LLOGOS_UNSUPPORTED;
     if (form == 0) {
-        const double cost[8] = {0, 0, rows_cost(M, N, K, 2, 1, units), rows_cost(M, N, K, 4, 1, units), rows_cost(M, N, K, 4, 2, units),
-                                tiles_cost(M, N, K, 64, 32, units), tiles_cost(M, N, K, 64, 64, units), tiles_cost(M, N, K, 128, 64, units)};
+        const double cost[5] = {0, 0, rows_cost(M, N, K, 2, 1, units), rows_cost(M, N, K, 4, 1, units), rows_cost(M, N, K, 4, 2, units)};
         form = M <= 16 ? 1 : 2;
-        for (int f = 3; form > 1 && f <= 7; ++f) if (cost[f] < cost[form]) form = f;
+        double least = cost[2];
+        for (int f = 3; form > 1 && f <= (ring ? 12 : 7); ++f) {
+            if (f == 5 && ring) f = 9;
+            const double c = f < 5 ? cost[f] : f == 5 ? tiles_cost(M, N, K, 64, 32, units) : f == 6 ? tiles_cost(M, N, K, 64, 64, units)
+                           : f == 7 ? tiles_cost(M, N, K, 128, 64, units) : ring_cost(M, N, K, kRing[f - 9], units);
+            if (c < least) { least = c; form = f; }
+        }
     }
     // 16 waves a block where a matrix has few blocks and enough of k for all of them
     const bool wide = K >= 16 * 256 && (N + 15) / 16 * ((M + 15) / 16) <= 2 * units;
@@ -355,6 +518,10 @@ LLOGOS_EXPORT int llogos_gemm_f32(float* out, const float* a, const float* w, co
         case 5: TILES(64, 32); break;
         case 6: TILES(64, 64); break;
         case 7: TILES(128, 64); break;
+        case 9: RING(2, 2, 2, 2); break;
+        case 10: RING(2, 1, 2, 2); break;
+        case 11: RING(3, 1, 1, 4); break;
+        case 12: RING(5, 1, 1, 4); break;
         default:
             if (vec && M == 1) { if (cols == 4) LANES(1, 4, true); else if (cols == 2) LANES(1, 2, true); else LANES(1, 1, true); }
             else if (vec) { if (cols == 4) LANES(2, 4, true); else if (cols == 2) LANES(2, 2, true); else LANES(2, 1, true); }

@@ -212,7 +212,7 @@ def concat_rows(a: torch.Tensor, b: torch.Tensor, out_dtype: torch.dtype, delta:
     return out
 
 
-F32_FORM = 0                 # 0: chosen by the sizes; 1 to 8 force a form of the float32 product (tests)
+F32_FORM = 0                 # 0: chosen by the sizes; 1 to 12 force a form of the float32 product (tests; 9 to 12 take K of whole stages of 32 alone)
 
 
 def gemm_generic(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out_dtype: torch.dtype,

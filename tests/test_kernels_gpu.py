@@ -311,6 +311,28 @@ def test_the_generic_entry_takes_float32_throughout():
             assert torch.equal(out[:, :N], K.gemm_generic(a, w, bias, torch.float32)) and (out[:, N:] == 7.0).all()
 
 
+@pytest.mark.parametrize("M,N,K_", [(17, 1, 32), (48, 64, 256), (49, 65, 288), (79, 130, 64), (81, 63, 544), (161, 200, 2048), (321, 33, 224)])
+def test_float32_ring_gives_the_bits_of_the_tiles(M, N, K_, monkeypatch):
+    """The ring's tiles at remainders of their rows and columns, one stage of k, groups of 256 k that are whole and that are not, rows of a
+    and of the result that are wider than their values, a bias, values that are no number in one row and one matrix row."""
+    rng = np.random.default_rng(M + K_)
+    wide, w, b = _t(rng.standard_normal((M, K_ + 8))), _t(rng.standard_normal((N, K_)) * 0.1), _t(rng.standard_normal(N))
+    for special in (False, True):
+        if special:
+            wide[M // 2, 5], wide[M - 1, K_ - 1], w[N // 2, K_ // 2] = float("inf"), float("nan"), float("-inf")
+        for a, out in ((wide[:, :K_], torch.zeros((M, N + 3), device=DEV)[:, :N]), (wide[:, :K_].contiguous(), torch.zeros((M, N), device=DEV))):
+            for bias in (None, b):
+                monkeypatch.setattr(K, "F32_FORM", 6)
+                want = K.gemm_generic(a, w, bias, torch.float32, out=torch.zeros_like(out))
+                for form in range(9, 13):
+                    monkeypatch.setattr(K, "F32_FORM", form)
+                    got = K.gemm_generic(a, w, bias, torch.float32, out=out)
+                    assert torch.equal(got.view(torch.int32) if got.is_contiguous() else got.contiguous().view(torch.int32),
+                                       want.contiguous().view(torch.int32)) or (special and torch.allclose(got, want, rtol=0, atol=0, equal_nan=True)), form
+                monkeypatch.setattr(K, "F32_FORM", 0)
+                assert special or torch.equal(K.gemm_generic(a, w, bias, torch.float32, out=out), want)
+
+
 @pytest.mark.parametrize("M,N,K_", [(1, 16, 16), (17, 33, 40), (33, 70, 272), (64, 129, 4112), (65, 31, 255), (130, 66, 2049), (200, 250, 513)])
 def test_float32_product_gives_the_same_bits_in_every_form(M, N, K_, monkeypatch):
     """The forms of the float32 product (few rows in three heights of blocks, tiles in three sizes, pairs of rows) at remainders of
