@@ -1,5 +1,6 @@
 // The tiled product for many rows on packed weights (gemm_tiles_bf16.hip): which block takes which tile, and one tile.
 #pragma once
+#include "activation.h"
 #include "common.h"
 #include <type_traits>
 
@@ -34,7 +35,8 @@ constexpr int kTileWaves = 4;
 constexpr int kTileBlocks = 4;                         // packed blocks of 64 rows of w a tile: 256 rows, a block a wave
 constexpr int kStageK = 64;
 constexpr int kRing = 4;                               // stages of 64 k in LDS and in registers
-enum { EPI_PLAIN = 0, EPI_SWIGLU = 1, EPI_ADD = 2, EPI_ROWS = 3, EPI_ROWS_GATED = 4 };   // (the last two: sorted rows of experts, moe_packed.hip)
+enum { EPI_PLAIN = 0, EPI_SWIGLU = 1, EPI_ADD = 2, EPI_ROWS = 3, EPI_ROWS_GATED = 4,   // (sorted rows of experts, moe_packed.hip)
+       EPI_RELU2 = 5, EPI_XIELU = 6 };                              // activations with what activation.h takes (TileEnd: act_a, act_b)
 
 constexpr int tiles_lds_bytes(int tm) { return kRing * tm * 16 * kStageK * 2; }
 
@@ -186,6 +188,7 @@ struct TileEnd {
     float scale;
     const float* row_weight;
     const int* order;
+    float act_a, act_b;
 };
 
 template <int TM, int EPI, typename TO>
@@ -266,6 +269,11 @@ __device__ __forceinline__ void tile_store(unsigned char* lds, f32x4_t (&acc)[TM
                             y[e] = (at.act == 1 ? v * v : y[e]) * at.scale;
                         }
                     }
+                    if (EPI == EPI_RELU2 || EPI == EPI_XIELU) {
+                        asm volatile("" : "+v"(y));
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) y[e] = activate(y[e], EPI == EPI_RELU2 ? ACT_RELU2 : ACT_XIELU, at.act_a, at.act_b);
+                    }
                     if (EPI == EPI_PLAIN && at.bias) y += more[rt];
                     put(t, 16 * rt + 4 * g, y);
                 }
@@ -305,12 +313,13 @@ __device__ __forceinline__ void tile_store(unsigned char* lds, f32x4_t (&acc)[TM
 #endif
 }
 
-// One tile: 16 TM tokens by 256 rows of w, stages [stage_begin, stage_end) of k.  out: EPI_SWIGLU [M][N / 2], else [M][N], rows ldo apart.
+// One tile: 16 TM tokens by 256 rows of w, stages [stage_begin, stage_end) of k.  out: EPI_SWIGLU [M][N / 2], else [M][N], rows ldo apart.  limit: of the
+// gated form, or an activation's first number.
 template <int TM, int EPI, typename TO>
 __device__ __forceinline__ void tile_body(
         unsigned char* lds, TO* __restrict__ out, const bf16_t* __restrict__ a, int lda, const unsigned char* __restrict__ wp,
         const float* __restrict__ bias, int M, int N, int K, int ldo, int n_row_blocks, int m_tile, int n_tile, int stage_begin,
-        int stage_end, float limit) {
+        int stage_end, float limit, float act_b) {
     const int m0 = m_tile * TM * 16, nb = n_tile * kTileBlocks + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const unsigned char* w_base = wp + ((size_t)min(nb, n_row_blocks - 1) * (K / 32) + 2 * stage_begin) * 4096;
     const unsigned char* a_base = reinterpret_cast<const unsigned char*>(a + (size_t)m0 * lda + (size_t)stage_begin * kStageK);
@@ -323,7 +332,7 @@ __device__ __forceinline__ void tile_body(
     f32x4_t acc[TM][4];
     tile_products<TM>(lds, acc, w_base, a_base, a_off, stage_end - stage_begin);
     TileEnd at{};
-    at.m0 = m0, at.m_end = M, at.N = N, at.ldo = ldo, at.nb = nb, at.n_row_blocks = n_row_blocks, at.bias = bias, at.limit = limit;
+    at.m0 = m0, at.m_end = M, at.N = N, at.ldo = ldo, at.nb = nb, at.n_row_blocks = n_row_blocks, at.bias = bias, at.limit = limit, at.act_a = limit, at.act_b = act_b;
     tile_store<TM, EPI, TO>(lds, acc, out, at);
 }
 
@@ -336,7 +345,7 @@ struct TilesCall {
     const float* bias;
     int lda, M, N, K, ldo, parts, rows, rows_last, n_full;
     long long part_stride;
-    float limit;
+    float limit, act_b;
     hipStream_t stream;
 };
 // (one file each, so that they are compiled side by side)
@@ -345,6 +354,8 @@ int tiles_plain_bf16(const TilesCall& c);
 int tiles_add_f32(const TilesCall& c);
 int tiles_gated_f32(const TilesCall& c);
 int tiles_gated_bf16(const TilesCall& c);
+int tiles_relu2_bf16(const TilesCall& c);
+int tiles_xielu_bf16(const TilesCall& c);
 
 // Blocks 0 .. blocks_full - 1 take tiles of 16 TM tokens over the first n_full row tiles, the blocks after them tiles of 16 TS tokens
 // over the remaining row tiles (TS = 0: there are none).
@@ -352,7 +363,7 @@ template <int TM, int TS, int EPI, typename TO>
 __global__ __launch_bounds__(kTileWaves * kWave, 1) void gemm_tiles_kernel(
         TO* __restrict__ out, const bf16_t* __restrict__ a, int lda, const unsigned char* __restrict__ wp,
         const float* __restrict__ bias, int M, int N, int K, int ldo, size_t part_stride, int n_row_blocks,
-        int m_full, int m_last, int n_full, int n_tiles, int blocks_full, int parts, float limit) {
+        int m_full, int m_last, int n_full, int n_tiles, int blocks_full, int parts, float limit, float act_b) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char tiles_lds[];
     const int stages = K / kStageK;
     const bool full = TS == 0 || (int)blockIdx.x < blocks_full;
@@ -365,8 +376,8 @@ __global__ __launch_bounds__(kTileWaves * kWave, 1) void gemm_tiles_kernel(
     // when there are at least as many stages as parts
     const int s0 = (int)((long long)stages * part / parts), s1 = (int)((long long)stages * (part + 1) / parts);
     TO* dst = out + (size_t)part * part_stride;
-    if (full) tile_body<TM, EPI, TO>(tiles_lds, dst, a, lda, wp, bias, M, N, K, ldo, n_row_blocks, m_tile, n_tile, s0, s1, limit);
-    else if (TS > 0) tile_body<(TS > 0 ? TS : 4), EPI, TO>(tiles_lds, dst, a, lda, wp, bias, M, N, K, ldo, n_row_blocks, m_tile, n_tile, s0, s1, limit);
+    if (full) tile_body<TM, EPI, TO>(tiles_lds, dst, a, lda, wp, bias, M, N, K, ldo, n_row_blocks, m_tile, n_tile, s0, s1, limit, act_b);
+    else if (TS > 0) tile_body<(TS > 0 ? TS : 4), EPI, TO>(tiles_lds, dst, a, lda, wp, bias, M, N, K, ldo, n_row_blocks, m_tile, n_tile, s0, s1, limit, act_b);
 }
 
 template <int TM, int TS, int EPI, typename TO>
@@ -381,7 +392,7 @@ int launch_tile_kernel(const TilesCall& c) {
     if (code != 0) return code;
     gemm_tiles_kernel<TM, TS, EPI, TO><<<(unsigned)(full + last), kTileWaves * kWave, smem, c.stream>>>(
         (TO*)c.out, (const bf16_t*)c.a, c.lda, (const unsigned char*)c.wp, c.bias, c.M, c.N, c.K, c.ldo, (size_t)c.part_stride, n_row_blocks,
-        m_full, m_last, n_full, n_tiles, (int)full, c.parts, c.limit);
+        m_full, m_last, n_full, n_tiles, (int)full, c.parts, c.limit, c.act_b);
     return LLOGOS_LAUNCH_CHECK();
 }
 

@@ -25,7 +25,9 @@
 //    through registers -> these, the library between): 2,048 tokens, 28,672 x 4,096 with SwiGLU 407 (383) 353, 4,096 x 14,336 in two parts
 //    215 (200) 166, 4,096 x 4,096 70 (61) 61, 6,144 x 4,096 96 (80) 88; 5,003 tokens, 34,816 x 5,120 with SwiGLU 1,492 (1,571) 1,297,
 //    5,120 x 17,408 800 (1,030) 665; 334 tokens, 28,672 x 4,096 with SwiGLU 107 (90) 79.  8,192^3: 1.54 PFLOP/s random, 1.92 zeros.
-//  * Epilogues: plain (+ bias) in bfloat16 or float32; added to a float32 result in place; SwiGLU for a matrix packed with gate_rows.
+//  * Epilogues: plain (+ bias) in bfloat16 or float32; added to a float32 result in place; SwiGLU for a matrix packed with gate_rows; the activations of
+//    two-matrix feed-forwards in bfloat16 (a float32 result and a kernel of its own took 50 us more a layer at 2,500 rows of 21,504 values:
+//    215 MB written and read; a pass of that prompt and 16 steps 25,113 -> 24,461 us).
 #include "gemm_tiles.h"
 
 // What tiles of 64, 96, .. 256 tokens take, in microseconds: a launch, a round of blocks, a stage of 64 k, what a stage takes longer when
@@ -81,6 +83,8 @@ static int tiles_launch(TilesCall c, int out_dtype, int epilogue, int token_tile
     }
     if (epilogue == EPI_SWIGLU) return out_dtype == DT_BF16 ? tiles_gated_bf16(c) : tiles_gated_f32(c);
     if (epilogue == EPI_ADD) return tiles_add_f32(c);
+    if (epilogue == EPI_RELU2) return tiles_relu2_bf16(c);
+    if (epilogue == EPI_XIELU) return tiles_xielu_bf16(c);
     return out_dtype == DT_BF16 ? tiles_plain_bf16(c) : tiles_plain_f32(c);
 }
 
@@ -109,6 +113,18 @@ LLOGOS_EXPORT int llogos_gemm_tiles_bf16(void* out, int out_dtype, const void* a
     c.out = out, c.a = a, c.wp = packed_w, c.bias = bias, c.lda = lda, c.M = M, c.N = N, c.K = K, c.ldo = ldo, c.parts = parts;
     c.part_stride = part_stride, c.limit = limit, c.stream = stream;
     return tiles_launch(c, out_dtype, epilogue, token_tiles, compute_units);
+}
+
+// out [M][ldo] bfloat16 = act(a . w^T) in one part, kinds of activation.h: the square of relu, or xIELU with its two numbers.
+LLOGOS_EXPORT int llogos_gemm_tiles_activated_bf16(void* out, const void* a, int lda, const void* packed_w, int M, int N, int K, int ldo, int kind, float act_a,
+                                                   float act_b, int compute_units, hipStream_t stream) {
+    if (M <= 0 || N <= 0 || K <= 0 || out == nullptr || a == nullptr || packed_w == nullptr || lda < K || ldo < N || compute_units < 1) return LLOGOS_BAD_ARGUMENT;
+    if (kind != ACT_RELU2 && kind != ACT_XIELU) return LLOGOS_UNSUPPORTED;
+    if ((K % kStageK) || (lda % 8) || lda > 1 << 21 || ((uintptr_t)a % 16) || ((uintptr_t)packed_w % 16)) return LLOGOS_UNSUPPORTED;
+    TilesCall c{};
+    c.out = out, c.a = a, c.wp = packed_w, c.lda = lda, c.M = M, c.N = N, c.K = K, c.ldo = ldo, c.parts = 1;
+    c.limit = act_a, c.act_b = act_b, c.stream = stream;
+    return tiles_launch(c, DT_BF16, kind == ACT_RELU2 ? EPI_RELU2 : EPI_XIELU, 0, compute_units);
 }
 
 // The same in tiles of 64 tokens times 1, 2 or 3 (token_tiles): out [parts][M][ldo] float32 (or, in one part, bfloat16).

@@ -4,6 +4,7 @@
 // is zero when its slot is handed out.  All arithmetic is 32-bit; inputs and outputs may be
 // stored as float or bfloat16.
 #include "common.h"
+#include "activation.h"
 
 // ---------------------------------------------------------------- short causal convolution
 // out[t, c] = [h[t, c] +] sum_j w[c, j] * h_(t - taps + 1 + j)[c]   (w[c, taps - 1] multiplies token t;
@@ -687,24 +688,7 @@ LLOGOS_EXPORT int llogos_sandwich_norm(float* x, const void* a, int a_dtype, int
 }
 
 // ---------------------------------------------------------------- activations of a product
-// out = act(sum of the parts of `in`) element by element.  kinds:
-//   0 tanh;  1 silu;  2 gelu (tanh form);
-//   3 the piecewise xIELU with a = softplus(p), b = 1/2 + softplus(q):
-//       z > 0: a z^2 + z / 2;   z <= 0: b (exp(z) - 1 - z) + z / 2
-//   4 the square of relu: max(z, 0)^2;  5 the sum as it is
-enum { ACT_TANH = 0, ACT_SILU = 1, ACT_GELU_TANH = 2, ACT_XIELU = 3, ACT_RELU2 = 4, ACT_NONE = 5 };
-
-__device__ __forceinline__ float activate(float z, int kind, float a, float b) {
-    switch (kind) {
-        case ACT_TANH: return tanhf(z);
-        case ACT_SILU: return z / (1.0f + expf(-z));
-        case ACT_GELU_TANH: return 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
-        case ACT_RELU2: { const float r = fmaxf(z, 0.f); return r * r; }
-        case ACT_NONE: return z;
-        default: return z > 0.f ? fmaf(a * z, z, 0.5f * z) : fmaf(b, expm1f(z) - z, 0.5f * z);
-    }
-}
-
+// out = act(sum of the parts of `in`) element by element (kinds: activation.h)
 // VEC values a thread (8 with 16-byte loads where rows and sizes allow; else 1).  Bound by memory: 3,529 rows of 21,504 values from
 // float32 to bfloat16 75 us (455 MB; a value a thread 187).
 template <int VEC, int KIND, typename TO, typename TI>

@@ -2261,6 +2261,25 @@ def gemm_tiles_bf16(a: torch.Tensor, pw: PackedWeight, bias: Optional[torch.Tens
     return out[0] if parts == 1 else out
 
 
+def gemm_tiles_activated(a: torch.Tensor, pw: PackedWeight, kind: str, act_a: float = 0.0, act_b: float = 0.0) -> Optional[torch.Tensor]:
+    """activation(a [M, K] . w^T, kind, act_a, act_b) as bfloat16 [M, N] in one kernel on the packed copy of w: the float32 product's values,
+    activated, rounded once.  None for kinds other than relu2 and xielu and what the tiled product does not take."""
+    if kind not in ("relu2", "xielu") or a.dtype != torch.bfloat16 or a.dim() != 2 or pw.gate_rows:
+        return None
+    M, K = a.shape
+    if not (K == pw.K and M > 0 and K % 64 == 0 and a.stride(1) == 1 and a.stride(0) % 8 == 0 and a.data_ptr() % 16 == 0):
+        return None
+    _dev(pw.data)
+    _need(a.is_cuda and a.device == pw.data.device, "gemm: a and w must be on the same GPU")
+    out = torch.empty((M, pw.N), dtype=torch.bfloat16, device=a.device)
+    code = _lib().llogos_gemm_tiles_activated_bf16(_p(out), _p(a), a.stride(0), _p(pw.data), M, pw.N, K, pw.N, ACTIVATIONS[kind], ctypes.c_float(act_a),
+                                                   ctypes.c_float(act_b), compute_units(a.device), _stream())
+    if code == -2:
+        return None
+    _check(code, "gemm_tiles_activated")
+    return out
+
+
 def gemm_tiles_add(x: torch.Tensor, a: torch.Tensor, pw: Optional[PackedWeight]) -> bool:
     """x [M, N] (float32, in place) += a [M, K] . w^T by the tiled product with the sum in its epilogue, where
     tiles_plan takes the product in one part; False (and x untouched) otherwise."""

@@ -158,6 +158,15 @@ class Linear(Part):
             return K.gemm_tiles_bf16(a, self.packed, None, self.rt.dtype, limit=limit) if serves else None
         return K.gemm_packed_gated_bf16(a, self.packed, self.rt.dtype, K.packed_plan(a.shape[0], self.packed.N, self.packed.K)[1], limit=limit)
 
+    def activated_product(self, a, kind: str, act_a: float = 0.0, act_b: float = 0.0) -> Optional[torch.Tensor]:
+        """ops.kernels.activation of a . W^T in the runtime's type, made in one kernel from the packed copy; None where that does not apply (few
+        rows, no packed copy, a bias, float32, an activation that the product has not)."""
+        if self.packed is None or self.bias is not None or self.rt.dtype != torch.bfloat16 or not isinstance(a, torch.Tensor) or a.dim() != 2:
+            return None
+        if not K.wide_tiles_serve_gated(a.shape[0], self.packed.N, a.shape[1]):
+            return None
+        return K.gemm_tiles_activated(a, self.packed, kind, act_a, act_b)
+
     def bias_rows(self, rows_out: Optional[int] = None) -> Optional[torch.Tensor]:
         return self.bias if (self.bias is None or rows_out is None) else self.bias[:rows_out]
 

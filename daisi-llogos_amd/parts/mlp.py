@@ -129,9 +129,10 @@ class ActivatedMLP(FeedForward):
             self.a, self.b = _softplus(p), 0.5 + _softplus(q)
 
     def forward(self, ctx: StepContext, h):
-        z = self.up.product(h, f32_ok=True)
+        act = self.up.activated_product(h, self.activation, self.a, self.b)         # (prompts: in the product's epilogue)
+        if act is None:
+            act = K.activation(self.up.product(h, f32_ok=True), self.activation, self.rt.dtype, self.a, self.b)
         mark(ctx, "up")
-        act = K.activation(z, self.activation, self.rt.dtype, self.a, self.b)
         out = self.down.product(act, f32_ok=True)
         mark(ctx, "down")
         return out

@@ -1325,6 +1325,22 @@ def test_tiles_of_every_height_and_epilogue(M, N, K_):
         assert all(torch.equal(p, q) for p, q in zip(seen, got)), token_tiles
 
 
+@pytest.mark.parametrize("M,N,K_", [(1, 8, 64), (130, 300, 320), (257, 517, 192), (700, 1088, 576)])
+def test_tiles_that_activate_their_product(M, N, K_):
+    """The activation in the product's epilogue gives the bits of the activation's kernel on the float32 product, in heights of tiles that the launch
+    chooses for the sizes, results at remainders of their lines, and for sums that are no number; other kinds are left alone."""
+    rng = np.random.default_rng(M + N)
+    a, w = _t(rng.standard_normal((M, K_)) * 2, torch.bfloat16), _t(rng.standard_normal((N, K_)) * 0.1, torch.bfloat16)
+    a[M // 2, 3], a[M - 1, K_ - 1] = float("inf"), float("nan")
+    pw = K.pack_weights(w)
+    z = K.gemm_tiles_bf16(a, pw, None, torch.float32)
+    for kind, numbers in (("relu2", ()), ("xielu", (0.8, 1.1))):
+        got, want = K.gemm_tiles_activated(a, pw, kind, *numbers), K.activation(z, kind, torch.bfloat16, *numbers)
+        number = ~torch.isnan(want)
+        assert got.dtype == torch.bfloat16 and torch.equal(torch.isnan(got), ~number) and torch.equal(got[number], want[number])
+    assert K.gemm_tiles_activated(a, pw, "silu") is None and K.gemm_tiles_activated(a.float(), pw, "relu2") is None
+
+
 def test_wide_tiles_serve_prompts():
     """What wide_tiles_plan chooses, through the general entry and added to the stream: one part in place, more parts left to the norm that
     adds them, all in one where none follows; matrices and operands that it does not take go the way they went."""
