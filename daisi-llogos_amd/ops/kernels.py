@@ -2613,6 +2613,24 @@ def attention_decode_fused(ctx, qkv: torch.Tensor, bias: Optional[torch.Tensor],
     return out
 
 
+F32_PAGES_TILES = {"tickets": 128, "merge": 96}        # tiles of query rows times kv heads up to which pages go to several blocks
+F32_SHARED_PAGES = 16              # pages of a table whose shares one kernel adds (attention_f32.hip: kSharedPages)
+F32_PAGES_FLOATS = 1 << 25         # scratch of the second kernel's form
+
+
+def f32_pages_form(tiles: int, pages: int, longest: int) -> Optional[str]:
+    """How a single-token step's pages are shared out among blocks, or None for one block a tile: "tickets" in one kernel, for tables of 5 to 16
+    pages, "merge" with a second kernel for more.  A second kernel costs some 2 us, which the four and more pages that a matrix unit
+    works on with one block a tile repay from some 400 tokens on; a captured step knows its table alone, whose widths come in sixteens.  us, one
+    block a tile / shared: 8 tiles of heads of 64 7.7 / 6.6 at 40 tokens, 12.1 / 10.1 at 500, 19.4 / 10.9 at 1,000, 134 / 38 at 8,000; of 128 11.2 / 10.6,
+    17.4 / 15.2, 30.9 / 16.0, 269 / 47; 128 tiles 13.9 / 12.9 and 22.7 / 21.8 at 500, but 184 / 196 at 8,000 (64 dimensions); 256 tiles
+    18.0 / 19.2 and 27.6 / 31.3 at 500."""
+    form = "tickets" if pages <= F32_SHARED_PAGES else "merge"
+    if tiles > F32_PAGES_TILES[form] or (pages <= 4 if form == "tickets" else longest <= F32_SHARED_PAGES * PAGE_TOKENS):
+        return None
+    return form
+
+
 def attention_f32(ctx, q: torch.Tensor, q_stride: int, k_pool: torch.Tensor, v_pool: torch.Tensor, table: torch.Tensor,
                   n_heads: int, n_kv_heads: int, head_dim: int, scale: float, window: int = 0, sinks: int = 0) -> Optional[torch.Tensor]:
     """float32 attention on the matrix cores' 32-bit instruction, the same bits for a token whether it comes alone or in a
@@ -2644,6 +2662,21 @@ def attention_f32(ctx, q: torch.Tensor, q_stride: int, k_pool: torch.Tensor, v_p
     _need(q.is_cuda and q.numel() >= (T - 1) * q_stride + n_heads * head_dim and q_stride >= n_heads * head_dim, "attention: q too small")
     tiles = T * -(-group // 16) if cu is None else T * group // 16 + batch           # (at most; a sequence's last tile may be part full)
     out = torch.empty((T, n_heads * head_dim), dtype=torch.float32, device=q.device)
+    form = f32_pages_form(tiles * n_kv_heads, table.shape[1], getattr(ctx, "max_context", 0)) if cu is None else None
+    if form:
+        floats, tickets = _lib().llogos_attention_f32_pages_floats(T, table.shape[1], n_heads, n_kv_heads, head_dim), None
+        if form == "tickets":
+            try:
+                shares, tickets = _attn_shares(ctx, q.device, floats, tiles * n_kv_heads)
+            except KernelError:                                  # (captured before such a step was run: the kernel without scratch)
+                pass
+        elif floats <= F32_PAGES_FLOATS:
+            shares = torch.empty(floats, dtype=torch.float32, device=q.device)
+        if tickets is not None or form == "merge" and floats <= F32_PAGES_FLOATS:
+            _check(_lib().llogos_attention_f32_pages(_p(out), _p(shares), _p(tickets), _p(q), q_stride, _p(k_pool), _p(v_pool), _p(table), table.stride(0),
+                                                     table.shape[1], _p(tok_seq), _p(ctx.tok_pos), T, n_heads, n_kv_heads, head_dim, ctypes.c_float(scale),
+                                                     window, sinks, _stream()), "attention_f32_pages")
+            return out
     _check(_lib().llogos_attention_f32(_p(out), _p(q), q_stride, _p(k_pool), _p(v_pool), _p(table), table.stride(0), _p(cu), _p(tok_seq), _p(ctx.tok_pos),
                                        batch, tiles, -(-getattr(ctx, "max_context", 0) // PAGE_TOKENS), n_heads, n_kv_heads, head_dim,
                                        ctypes.c_float(scale), window, sinks, _stream()), "attention_f32")

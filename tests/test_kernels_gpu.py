@@ -551,6 +551,40 @@ def test_float32_attention_of_a_prompt_of_many_tiles(hd):
         assert torch.equal(call(one, c["q"][t:t + 1])[0], out[t]), t
 
 
+@pytest.mark.parametrize("window,sinks", [(0, 0), (100, 70)])
+@pytest.mark.parametrize("nh,nkv,hd", [(8, 2, 64), (3, 1, 128), (1, 1, 64), (20, 1, 128)])
+@pytest.mark.parametrize("width", [5, 16, 17, 70])
+def test_float32_attention_with_pages_in_several_blocks(nh, nkv, hd, width, window, sinks):
+    """Single tokens whose pages go to several blocks, added by the block with the last ticket or by a second kernel: the bits of one block a tile, at
+    the edges of pages and of a block's four, for groups that fill no tile and more than one, with pages given back; the counters end at zero."""
+    longest = min(64 * width, 1100 if width > 16 else 1024)
+    lens = sorted({1, 64, 65, 256, 257, 320, longest - 1, longest})
+    lens = [n for n in lens if n <= longest]
+    assert K.f32_pages_form(len(lens) * -(-nh // nkv // 16) * nkv, width, longest) == ("tickets" if width <= 16 else "merge")
+    c = _attention_case("float32", nh, nkv, hd, lens, [1] * len(lens))
+    table = torch.full((len(lens), width), 10 ** 6, dtype=torch.int32, device=DEV)
+    for b, n in enumerate(lens):
+        table[b, :-(-n // 64)] = c["table"][b, :-(-n // 64)]
+        if window:
+            table[b, max(0, -(-sinks // 64)):max(0, (n - window) // 64)] = 10 ** 6
+    shares = type("Runtime", (), dict(attention_shares=[], branch_attention_shares=[]))()
+    ctx = lambda **kw: type("Ctx", (), dict(tok_pos=_t(np.array(lens) - 1, torch.int32), is_decode=True, batch=len(lens), n_tokens=len(lens), **kw))()
+    call = lambda x: K.attention_f32(x, c["q"], c["stride"], c["kp"], c["vp"], table, nh, nkv, hd, 1 / math.sqrt(hd), window, sinks)
+    want = call(ctx())                                                   # (neither a longest context nor counters: one block a tile)
+    x = ctx(runtime=shares, max_context=longest)
+    for _ in range(3):
+        assert torch.equal(call(x), want)
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        got = call(x)
+    for _ in range(3):
+        got.zero_()
+        graph.replay()
+        assert torch.equal(got, want)
+    assert (len(shares.attention_shares) == 1) == (width <= 16) and all(int(t.abs().sum()) == 0 for _, t in shares.attention_shares)
+
+
 @pytest.mark.parametrize("types", [("float32", "float32", "float32"), ("float32", "bfloat16", "float32"), ("float32", "bfloat16", "bfloat16"),
                                    ("bfloat16", "bfloat16", "bfloat16"), ("bfloat16", "bfloat16", "float32")])
 @pytest.mark.parametrize("T,N,K_,odd", [(1, 1, 1, 0), (17, 5, 3, 0), (65, 64, 256, 0), (64, 66, 260, 0), (70, 129, 36, 1), (130, 62, 33, 1), (3, 200, 512, 4)])
