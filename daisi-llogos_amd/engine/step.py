@@ -51,7 +51,8 @@ def resolve_dtype(dtype: Union[str, torch.dtype]) -> torch.dtype:
 
 def packed_weight_budget(model: Model, dtype: torch.dtype, max_tokens: int, device: torch.device) -> int:
     """Bytes that the packed copies of the bfloat16 matrices may take (the few-row products stream
-    a packed copy a quarter faster; prompts need the row-major one): what is free on the GPU now,
+    a packed copy a quarter faster and the tiled product of prompts reads nothing else; the
+    row-major one serves what has no copy): what is free on the GPU now,
     when the model is about to be bound, less the matrices themselves and the cache, which are
     still to be allocated, and less a margin of 15 % of the GPU's memory for activations and
     workspaces.  At the Llama-3.1-70B sizes, 141 GB of matrices, about two thirds of the layers get
