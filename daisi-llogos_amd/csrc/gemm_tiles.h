@@ -77,7 +77,8 @@ __device__ __forceinline__ void tile_products(unsigned char* lds, f32x4_t (&acc)
     constexpr int kAhead = TM == 4 ? 3 : TM == 6 ? 4 : TM == 8 ? 4 : 6;
     constexpr int kLag = kAhead > 4 ? 2 : 1, kMeet = kUnits - kAhead + kLag;
     constexpr int kBefore = kLoads * kMeet / kUnits;         // loads of a stage that are asked for before the barrier ...
-    constexpr int kWait = kCopies + kCopies * kBefore / kLoads;   // ... and the copies among them, with the whole stage before
+    constexpr int kWait = kLoads + kBefore;                  // ... and the whole stage before: what may still be on its way then
+    static_assert(kWait > kLoads && kWait < 64, "a whole stage stays on its way, in a counter of six bits");
     static_assert(TM % 2 == 0 && kUnits % kFrags == 0 && kAhead < kFrags && 2 * kLag <= kAhead, "a tile's schedule");
 
     const int lane = threadIdx.x & (kWave - 1);
@@ -128,7 +129,10 @@ __device__ __forceinline__ void tile_products(unsigned char* lds, f32x4_t (&acc)
         for (int u = 0; u < kUnits; ++u) {
             if (u == kMeet) {
                 // this stage's fragments are all here (its buffer is the next to be written), and this wave's copies of the next
-                // stage too: of the copies asked for since, no more are on their way than there are (whatever loads of w are)
+                // stage too: loads come back in the order in which they were asked for (the compiler's own waits for w, which count
+                // copies and loads alike, rest on that too), so all but the kWait youngest are here.  (A wait that counted
+                // copies alone left no stage on its way: [2,048, 8,192], 65 rows in eight parts 19.2 us, 16.5 now; [4,096, 14,336] 32.3
+                // and 27.6; in one part a fifth; from 3,000 rows on level.)
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
                 tiles_wait_loads<kWait>();
                 meet();
@@ -159,7 +163,7 @@ __device__ __forceinline__ void tile_products(unsigned char* lds, f32x4_t (&acc)
 #pragma unroll
         for (int l = 0; l < kLoads; ++l) load(p, l, p, past_end(p));
     SB();
-    tiles_wait_loads<2 * kCopies>();
+    tiles_wait_loads<2 * kLoads>();
     meet();
 #pragma unroll
     for (int u = 0; u < kAhead; ++u) read_a(0, u);
