@@ -31,18 +31,19 @@
 #include "gemm_tiles.h"
 
 // What tiles of 64, 96, .. 256 tokens take, in microseconds: a launch, a round of blocks, a stage of 64 k, what a stage takes longer when
-// every unit works, a MB of results (gated: a MB per 1,024 x 1,024 rows and tokens), a MB of weights.  Fitted to 3,541 launches of 65 to 5,003 rows
-// of 25 matrices ([512, 4,096] to [10,240, 8,192]) in 1 to 8 parts, and to 217 gated ones of three; rms 4 to 5 % from 160 tokens a tile on, 9 to
-// 13 % below (few-row launches wait for the host).  The form it chooses takes 0.3 % longer than the best of them on average (gated 0.7 %).
+// every unit works, a MB of results (gated: a MB per 1,024 x 1,024 rows and tokens), a MB of weights.  Fitted to 25,000 launches of 65 to 16,384 rows
+// of 33 matrices ([512, 4,096] to [32,768, 2,048]) in 1 to 8 parts, and to 2,800 gated ones of 15 ([2,816, 896] to [57,344, 8,192]); rms 3.5 to 6 % from
+// 128 tokens a tile on, 7 to 10 % below.  The height it chooses takes 0.6 % longer than the best of them on average, gated 0.5 % (a fit to
+// three gated matrices took 3 %, and for up to 256 rows of [4,096, 768] and [9,728, 1,024] 1.2 to 2 times as long).
 struct TilesTimes { double start, round, stage, busy, result, weight; };
 static const TilesTimes kTilesPlain[7] = {
-    {4.20, 0.0, 0.543, 0.0, 0.026, 0.133}, {4.70, 0.0, 0.572, 0.035, 0.040, 0.121}, {0.29, 5.09, 0.577, 0.154, 0.062, 0.096},
-    {0.38, 6.98, 0.668, 0.165, 0.038, 0.067}, {0.0, 8.98, 0.745, 0.229, 0.028, 0.031}, {0.0, 10.55, 0.860, 0.250, 0.023, 0.027},
-    {0.0, 10.64, 0.996, 0.292, 0.063, 0.007}};
+    {3.43, 0.82, 0.399, 0.114, 0.018, 0.121}, {3.12, 2.65, 0.423, 0.169, 0.0, 0.104}, {0.22, 6.49, 0.525, 0.210, 0.032, 0.074},
+    {0.54, 7.35, 0.654, 0.168, 0.048, 0.059}, {0.12, 9.44, 0.739, 0.265, 0.029, 0.034}, {0.03, 10.61, 0.860, 0.312, 0.030, 0.024},
+    {0.0, 11.39, 0.983, 0.358, 0.045, 0.022}};
 static const TilesTimes kTilesGated[7] = {
-    {10.92, 0.0, 0.423, 0.123, 0.0, 0.073}, {10.57, 0.0, 0.527, 0.097, 0.003, 0.058}, {5.90, 0.0, 0.783, 0.021, 0.483, 0.028},
-    {5.43, 0.0, 0.821, 0.055, 0.596, 0.027}, {5.19, 0.27, 0.816, 0.246, 0.416, 0.007}, {3.20, 2.92, 0.951, 0.206, 0.432, 0.022},
-    {2.75, 3.83, 1.015, 0.315, 0.398, 0.016}};
+    {3.43, 0.0, 0.437, 0.099, 0.0, 0.106}, {3.65, 0.0, 0.578, 0.031, 0.168, 0.075}, {0.48, 4.24, 0.683, 0.087, 0.181, 0.050},
+    {0.44, 6.96, 0.710, 0.144, 0.104, 0.045}, {0.94, 9.22, 0.712, 0.322, 0.0, 0.028}, {1.40, 10.05, 0.818, 0.396, 0.0, 0.018},
+    {1.56, 11.23, 0.934, 0.455, 0.0, 0.014}};
 
 static double tiles_cost(int rows, int M, int N, int K, int parts, int units, bool gated) {
     const TilesTimes& t = (gated ? kTilesGated : kTilesPlain)[rows / 2 - 2];
@@ -140,4 +141,10 @@ LLOGOS_EXPORT double llogos_gemm_tiles_cost(int M, int N, int K, int parts, int 
     if (M <= 0 || N <= 0 || K < kStageK || parts < 1 || compute_units < 1 || token_tiles < 0 || token_tiles > 4) return 1e30;
     if (token_tiles > 0) return tiles_cost(4 * token_tiles, M, N, K, parts, compute_units, false);
     return tiles_choose(M, N, K, parts, compute_units, false).cost;
+}
+
+// Tokens a tile that token_tiles = 0 chooses, less the half tiles of a last round.
+LLOGOS_EXPORT int llogos_gemm_tiles_height(int M, int N, int K, int parts, int compute_units, int gated) {
+    if (M <= 0 || N <= 0 || K < kStageK || parts < 1 || compute_units < 1) return LLOGOS_BAD_ARGUMENT;
+    return 16 * tiles_choose(M, N, K, parts, compute_units, gated != 0).rows;
 }

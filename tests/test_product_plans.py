@@ -256,3 +256,16 @@ def test_packed_experts_tiles():
         for n in (11, 95, 96, 599, 600, 5000):
             least, most = K.moe_packed_form(E * n, E)
             assert 1 <= least <= most == 4 and (least == 1 or 64 * least <= n + 63)
+
+
+def test_heights_of_tiles_at_sizes_measured():
+    """Sizes at which the other heights were measured 5 % behind the ones named here, or more: gated matrices that the fit of the costs once
+    left out (tiles of 128 and 192 tokens took 1.2 to 2 times as long there), and plain ones in parts."""
+    height = lambda M, N, K_, parts=1, gated=0: K._lib().llogos_gemm_tiles_height(M, N, K_, parts, 256, gated)
+    for M in (65, 100, 160, 256, 512, 1000):
+        assert height(M, 4096, 768, gated=1) == 64, M
+    for M in (129, 200, 300):
+        assert height(M, 9728, 1024, gated=1) in (64, 96), M
+    for M, N, K_, parts, best in ((300, 3072, 3072, 8, (64,)), (300, 5120, 17408, 4, (128,)), (1000, 7168, 5120, 4, (256,)), (400, 8192, 1024, 4, (64, 224)),
+                                  (200, 8192, 28672, 4, (128,)), (2048, 3072, 2048, 4, (64,))):
+        assert height(M, N, K_, parts) in best, (M, N, K_, parts)
