@@ -31,26 +31,28 @@
 #include "gemm_tiles.h"
 
 // What tiles of 64, 96, .. 256 tokens take, in microseconds: a launch, a round of blocks, a stage of 64 k, what a stage takes longer when
-// every unit works, a MB of results (gated: a MB per 1,024 x 1,024 rows and tokens), a MB of weights.  Fitted to 25,000 launches of 65 to 16,384 rows
-// of 33 matrices ([512, 4,096] to [32,768, 2,048]) in 1 to 8 parts, and to 2,800 gated ones of 15 ([2,816, 896] to [57,344, 8,192]); rms 3.5 to 6 % from
-// 128 tokens a tile on, 7 to 10 % below.  The height it chooses takes 0.6 % longer than the best of them on average, gated 0.5 % (a fit to
-// three gated matrices took 3 %, and for up to 256 rows of [4,096, 768] and [9,728, 1,024] 1.2 to 2 times as long).
-struct TilesTimes { double start, round, stage, busy, result, weight; };
+// every unit works, a MB of results (gated: a MB per 1,024 x 1,024 rows and tokens), a MB of weights; rounds and weights side by side but for a
+// share of the shorter.  Fitted to 25,000 launches of 65 to 16,384 rows of 33 matrices ([512, 4,096] to [32,768, 2,048]) in 1 to 8 parts, and to
+// 2,800 gated ones of 15 ([2,816, 896] to [57,344, 8,192]); rms 4 to 6 % from 128 tokens a tile on, 7 to 10 % below.  The height it chooses takes
+// 0.2 to 0.7 % longer than the best of them on average, gated 0.5 % (a fit to three gated matrices took 3 %, and for up to 256 rows of
+// [4,096, 768] and [9,728, 1,024] 1.2 to 2 times as long).
+struct TilesTimes { double start, round, stage, busy, result, weight, both; };
 static const TilesTimes kTilesPlain[7] = {
-    {3.43, 0.82, 0.399, 0.114, 0.018, 0.121}, {3.12, 2.65, 0.423, 0.169, 0.0, 0.104}, {0.22, 6.49, 0.525, 0.210, 0.032, 0.074},
-    {0.54, 7.35, 0.654, 0.168, 0.048, 0.059}, {0.12, 9.44, 0.739, 0.265, 0.029, 0.034}, {0.03, 10.61, 0.860, 0.312, 0.030, 0.024},
-    {0.0, 11.39, 0.983, 0.358, 0.045, 0.022}};
+    {3.56, 0.73, 0.431, 0.062, 0.034, 0.118, 0.91}, {3.57, 1.98, 0.462, 0.127, 0.017, 0.109, 0.88}, {0.11, 6.19, 0.554, 0.182, 0.049, 0.144, 0.48},
+    {0.59, 7.03, 0.667, 0.168, 0.059, 0.168, 0.31}, {0.15, 9.28, 0.732, 0.289, 0.034, 0.156, 0.21}, {0.22, 10.28, 0.852, 0.337, 0.035, 0.126, 0.22},
+    {0.0, 11.24, 0.972, 0.395, 0.049, 0.119, 0.20}};
 static const TilesTimes kTilesGated[7] = {
-    {3.43, 0.0, 0.437, 0.099, 0.0, 0.106}, {3.65, 0.0, 0.578, 0.031, 0.168, 0.075}, {0.48, 4.24, 0.683, 0.087, 0.181, 0.050},
-    {0.44, 6.96, 0.710, 0.144, 0.104, 0.045}, {0.94, 9.22, 0.712, 0.322, 0.0, 0.028}, {1.40, 10.05, 0.818, 0.396, 0.0, 0.018},
-    {1.56, 11.23, 0.934, 0.455, 0.0, 0.014}};
+    {3.43, 0.0, 0.437, 0.099, 0.0, 0.106, 1.0}, {3.65, 0.0, 0.578, 0.031, 0.168, 0.075, 1.0}, {0.48, 4.24, 0.683, 0.087, 0.181, 0.050, 1.0},
+    {0.44, 6.96, 0.710, 0.144, 0.104, 0.045, 1.0}, {0.94, 9.22, 0.712, 0.322, 0.0, 0.028, 1.0}, {1.40, 10.05, 0.818, 0.396, 0.0, 0.018, 1.0},
+    {1.56, 11.23, 0.934, 0.455, 0.0, 0.014, 1.0}};
 
 static double tiles_cost(int rows, int M, int N, int K, int parts, int units, bool gated) {
     const TilesTimes& t = (gated ? kTilesGated : kTilesPlain)[rows / 2 - 2];
     const double tiles = (double)((M + 16 * rows - 1) / (16 * rows)) * ((N + 255) / 256) * parts;
     const double rounds = ceil(ceil(tiles / 8.0) / (units / 8.0)), busy = tiles / (rounds * units);
     const int per = (K / kStageK + parts - 1) / parts, whole = (per + kRing - 1) / kRing * kRing;
-    return t.start + rounds * (t.round + whole * (t.stage + t.busy * busy)) + (double)M * N * (gated ? 1e-6 : 4e-6 * parts) * t.result + (double)N * K * 2e-6 * t.weight;
+    const double work = rounds * (t.round + whole * (t.stage + t.busy * busy)), weights = (double)N * K * 2e-6 * t.weight;
+    return t.start + fmax(work, weights) + t.both * fmin(work, weights) + (double)M * N * (gated ? 1e-6 : 4e-6 * parts) * t.result;
 }
 
 struct TilesChoice { int rows, rows_last, n_full; double cost; };
@@ -128,18 +130,9 @@ LLOGOS_EXPORT int llogos_gemm_tiles_activated_bf16(void* out, const void* a, int
     return tiles_launch(c, DT_BF16, kind == ACT_RELU2 ? EPI_RELU2 : EPI_XIELU, 0, compute_units);
 }
 
-// The same in tiles of 64 tokens times 1, 2 or 3 (token_tiles): out [parts][M][ldo] float32 (or, in one part, bfloat16).
-LLOGOS_EXPORT int llogos_gemm_tiles_short_bf16(void* out, int out_dtype, const void* a, int lda, const void* packed_w, int M, int N, int K,
-                                               int ldo, long long part_stride, int parts, int token_tiles, hipStream_t stream) {
-    if (token_tiles < 1 || token_tiles > 3) return LLOGOS_BAD_ARGUMENT;
-    return llogos_gemm_tiles_bf16(out, out_dtype, a, lda, packed_w, nullptr, M, N, K, ldo, part_stride, EPI_PLAIN, parts, token_tiles, 1, -1.f, stream);
-}
-
-// Microseconds that a product in `parts` parts is expected to take in the tiles that token_tiles = 0 chooses, or in tiles of 64 token_tiles (1 .. 4)
-// tokens.
-LLOGOS_EXPORT double llogos_gemm_tiles_cost(int M, int N, int K, int parts, int token_tiles, int compute_units) {
-    if (M <= 0 || N <= 0 || K < kStageK || parts < 1 || compute_units < 1 || token_tiles < 0 || token_tiles > 4) return 1e30;
-    if (token_tiles > 0) return tiles_cost(4 * token_tiles, M, N, K, parts, compute_units, false);
+// Microseconds that a product in `parts` parts is expected to take in the tiles that token_tiles = 0 chooses.
+LLOGOS_EXPORT double llogos_gemm_tiles_cost(int M, int N, int K, int parts, int compute_units) {
+    if (M <= 0 || N <= 0 || K < kStageK || parts < 1 || compute_units < 1) return 1e30;
     return tiles_choose(M, N, K, parts, compute_units, false).cost;
 }
 

@@ -2129,52 +2129,21 @@ def long_tiles_plan(M: int, N: int, K: int, n_cus: Optional[int] = None) -> Opti
 
 
 @functools.lru_cache(maxsize=4096)
-def _tiles_cost(M: int, N: int, K: int, parts: int, token_tiles: int, units: int) -> float:
+def _tiles_cost(M: int, N: int, K: int, parts: int, units: int) -> float:
     """Microseconds that the tiled product is expected to take (gemm_tiles_bf16.hip: tiles_cost), with its consumer's reading of the
-    results, 0.2 us a MB."""
-    return _lib().llogos_gemm_tiles_cost(M, N, K, parts, token_tiles, units) + parts * M * N * 4e-6 * 0.2
-
-
-@functools.lru_cache(maxsize=4096)
-def _short_tiles_form(M: int, N: int, K: int, units: int) -> Tuple[int, int]:
-    """(parts of k, token_tiles) of the cheapest launch in tiles of 64, 128 or 192 tokens: a block a unit or somewhat fewer."""
-    stages, columns, best, least = K // 64, -(-N // 256), (1, 1), float("inf")
-    for token_tiles in (1, 2, 3):
-        tiles = -(-M // (64 * token_tiles)) * columns
-        most = max(1, min(8, units // tiles, stages // 4))
-        for parts in range(most, 0, -1):
-            cost = _tiles_cost(M, N, K, parts, token_tiles, units)
-            if cost < least:
-                best, least = (parts, token_tiles), cost
-    return best
-
-
-def short_tiles_plan(M: int, N: int, K: int, n_cus: Optional[int] = None) -> Optional[Tuple[int, int]]:
-    """(parts of k, token_tiles) with which tiles of 64 to 192 tokens (gemm_tiles_short_bf16) serve a plain product of M rows, or
-    None where they do not: they do for matrices of 2,048 to 8,192 rows, a multiple of four (results are stored four at a time; one by
-    one [7,169, 4,096] took 43 us at 200 rows, the library 31), and k from 2,048 on, with up to 256 rows of activations, and up to 1,024
-    where k is at least twice the matrix's rows.  us, the library's product / these, whose parts are still to be added: 130 rows [3,072,
-    2,048] 19.3 / 9.3, [4,096, 4,096] 20.9 / 13.6, [7,168, 5,120] 29.9 / 23.0; 200 rows [6,144, 4,096] 25.5 / 22.2, [5,120, 5,120] 28.6 / 24.0; 130 rows
-    [4,096, 14,336] 62 / 34, 334 rows 74 / 44.  Where no norm follows that adds the parts, the library adds its product to the stream itself."""
-    if PROMPT_PRODUCT != "auto" or not SKINNY_MAX_ROWS < M <= 1024 or K % 64 or K < 2048 or not 2048 <= N <= 8192 or N % 4:
-        return None
-    if M > 256 and K < 2 * N:
-        return None
-    return _short_tiles_form(M, N, K, n_cus or compute_units())
+    results, 0.3 us a MB (0.23 to 0.29 measured; what a part more costs the norm beside that is not in it)."""
+    return _lib().llogos_gemm_tiles_cost(M, N, K, parts, units) + parts * M * N * 4e-6 * 0.3
 
 
 @functools.lru_cache(maxsize=4096)
 def _wide_parts(M: int, N: int, K: int, units: int) -> int:
-    return min(range(1, max(1, min(8, K // 256)) + 1), key=lambda parts: _tiles_cost(M, N, K, parts, 0, units))
+    return min(range(1, max(1, min(8, K // 256)) + 1), key=lambda parts: _tiles_cost(M, N, K, parts, units))
 
 
 def wide_tiles_plan(M: int, N: int, K: int, n_cus: Optional[int] = None) -> int:
-    """Parts of k in which the tiled product serves a plain product of M rows beyond short_tiles_plan, or 0 where it does not: it does for
-    more than 64 rows wherever the matrix has 512 rows and columns.  us, the library's product with float32 results / this one, whose parts
-    are still to be added: 2,048 rows [4,096, 14,336] 200 / 166, [28,672, 4,096] 383 with a SwiGLU pass / 353 with it, [4,096, 4,096] 61 / 61;
-    5,003 rows [5,120, 17,408] 1,030 / 665, [7,168, 5,120] 287 / 269, [5,120, 5,120] 219 / 200, [34,816, 5,120] 1,571 / 1,297; 334 rows
-    [6,144, 4,096] 35 / 27, [4,096, 14,336] 74 / 44; 2,500 rows [21,504, 4,096] 442 / 345.  Of 227 sizes (65 to 5,003 rows of 25 matrices, [512, 4,096] to
-    [10,240, 8,192]) it was behind, by 3 to 14 %, at 6: 2,048 rows [6,144, 4,096] and [6,144, 1,536], 1,000 rows [10,240, 8,192] and three level ones."""
+    """Parts of k in which the tiled product takes a plain product of M rows, in the tiles that the launch chooses for them, or 0 where it is not
+    asked: it is for more than 64 rows of matrices of 512 rows, a multiple of four, and columns, a multiple of 64.  What the parts cost with
+    their consumer is within 1.3 % of the cheapest on average over 860 sizes that a norm reads, 1.5 % over those that another kernel reads."""
     if PROMPT_PRODUCT != "auto" or M <= SKINNY_MAX_ROWS or K % 64 or K < 512 or N < 512 or N % 4:
         return 0
     return _wide_parts(M, N, K, n_cus or compute_units())
@@ -2189,28 +2158,13 @@ def wide_tiles_serve_gated(M: int, N: int, K: int) -> bool:
 
 
 def prompt_parts(M: int, N: int, K: int) -> int:
-    """Parts of k of a plain product of M rows that the tiled product serves, or 0: as short_tiles_plan has them, else as tiles_plan for
-    matrices of less than 4 M values (whose products both serve), else as wide_tiles_plan."""
-    plan = short_tiles_plan(M, N, K)
-    if plan is None and N * K < 1 << 22:
-        plan = tiles_plan(M, N, K)
-    return plan[0] if plan is not None else wide_tiles_plan(M, N, K)
+    """Parts of k of a plain product of M rows that the tiled product serves, or 0 (see wide_tiles_plan)."""
+    return wide_tiles_plan(M, N, K)
 
 
 def gemm_wide_bf16(a: torch.Tensor, pw: PackedWeight, out_dtype: torch.dtype, parts: int) -> Optional[torch.Tensor]:
     """a [M, K] . w^T on the packed copy of w, in tiles chosen by the launch: [M, N], or with parts > 1 float32 partial sums [parts, M, N] over
-    ranges of k.  None for what it does not take (see gemm_tiles_short_bf16)."""
-    return _gemm_tiles_plain(a, pw, out_dtype, parts, 0)
-
-
-def gemm_tiles_short_bf16(a: torch.Tensor, pw: PackedWeight, out_dtype: torch.dtype, parts: int, token_tiles: int) -> Optional[torch.Tensor]:
-    """a [M, K] . w^T on the packed copy of w in tiles of 64 token_tiles (1 to 3) tokens x 256 rows of w: [M, N], or with parts > 1
-    float32 partial sums [parts, M, N] over ranges of k; the sums are gemm_tiles_bf16's of as many parts.  None for what it does not take (rows of w
-    in another order, K no multiple of 64, parts of fewer than 128 values of k)."""
-    return _gemm_tiles_plain(a, pw, out_dtype, parts, token_tiles) if token_tiles in (1, 2, 3) else None
-
-
-def _gemm_tiles_plain(a: torch.Tensor, pw: PackedWeight, out_dtype: torch.dtype, parts: int, token_tiles: int) -> Optional[torch.Tensor]:
+    ranges of k.  None for what it does not take (rows of w in another order, K no multiple of 64, parts of fewer than 128 values of k)."""
     if a.dtype != torch.bfloat16 or a.dim() != 2 or pw.gate_rows:
         return None
     M, K = a.shape
@@ -2221,7 +2175,7 @@ def _gemm_tiles_plain(a: torch.Tensor, pw: PackedWeight, out_dtype: torch.dtype,
     _need(parts >= 1, "gemm: one part or more")
     out = torch.empty((parts, M, pw.N), dtype=torch.float32 if parts > 1 else out_dtype, device=a.device)
     code = _lib().llogos_gemm_tiles_bf16(_p(out), _DT[out.dtype], _p(a), a.stride(0), _p(pw.data), None, M, pw.N, K, pw.N, ctypes.c_longlong(M * pw.N),
-                                         0, int(parts), int(token_tiles), compute_units(a.device), ctypes.c_float(-1.0), _stream())
+                                         0, int(parts), 0, compute_units(a.device), ctypes.c_float(-1.0), _stream())
     if code == -2:
         return None
     _check(code, "gemm_tiles")
@@ -2292,7 +2246,7 @@ def gemm_tiles_add(x: torch.Tensor, a: torch.Tensor, pw: Optional[PackedWeight])
             and a.stride(0) % 8 == 0 and a.data_ptr() % 16 == 0):
         return False
     plan = tiles_plan(M, pw.N, K)
-    if plan is None or plan[0] != 1:                         # (one part: more than 1,024 rows, which short tiles do not serve)
+    if plan is None or plan[0] != 1:
         return False
     code = _lib().llogos_gemm_tiles_bf16(_p(x), F32, _p(a), a.stride(0), _p(pw.data), None, M, pw.N, K, pw.N, ctypes.c_longlong(0), 2, 1,
                                          int(plan[1]), compute_units(a.device), ctypes.c_float(-1.0), _stream())
@@ -2303,7 +2257,7 @@ def gemm_tiles_add(x: torch.Tensor, a: torch.Tensor, pw: Optional[PackedWeight])
 
 
 def gemm_wide_add(x: torch.Tensor, a: torch.Tensor, pw: Optional[PackedWeight], norm_adds: bool = True) -> bool:
-    """gemm_tiles_add where wide_tiles_plan takes the product in one part, or in any number where no norm follows that would add them."""
+    """gemm_tiles_add where prompt_parts has the product in one part.  norm_adds: whether a norm reads the stream next."""
     if pw is None or pw.gate_rows or RESIDUAL_PRODUCT != "on":
         return False
     if not (a.dtype == torch.bfloat16 and a.dim() == 2 and a.is_cuda and x.is_cuda and a.device == x.device == pw.data.device):
@@ -2312,10 +2266,7 @@ def gemm_wide_add(x: torch.Tensor, a: torch.Tensor, pw: Optional[PackedWeight], 
     if not (x.dtype == torch.float32 and x.shape == (M, pw.N) and x.is_contiguous() and K == pw.K and a.stride(1) == 1
             and a.stride(0) % 8 == 0 and a.data_ptr() % 16 == 0):
         return False
-    if short_tiles_plan(M, pw.N, K) is not None:
-        return False
-    parts = wide_tiles_plan(M, pw.N, K)
-    if parts == 0 or (parts > 1 and norm_adds):
+    if prompt_parts(M, pw.N, K) != 1:
         return False
     code = _lib().llogos_gemm_tiles_bf16(_p(x), F32, _p(a), a.stride(0), _p(pw.data), None, M, pw.N, K, pw.N, ctypes.c_longlong(0), 2, 1,
                                          0, compute_units(a.device), ctypes.c_float(-1.0), _stream())

@@ -1106,8 +1106,8 @@ def test_gate_up_product_on_norm_rows_without_their_scale(M, I, H):
                                     (1500, 2300, 640), (190, 136, 576), (318, 40, 576)])
 @pytest.mark.parametrize("token_tiles", [0, 4, 2])
 def test_tiled_product_for_many_rows_on_packed_weights(M, N, K_, token_tiles):
-    """The hand-written prompt-size product (tiles of 256 or 128 tokens x 256 rows, 32x32x16 MFMAs on the
-    packed copy): token counts and heights that fill no tile, float32 and bfloat16 results, bias, parts of k."""
+    """The hand-written prompt-size product (tiles of 64 to 256 tokens x 256 rows, 16x16x32 MFMAs on the
+    packed copy; the heights that the launch chooses, 256 and 128): token counts and heights that fill no tile, float32 and bfloat16 results, bias, parts of k."""
     rng = np.random.default_rng(M + N)
     a, w = _t(rng.standard_normal((M, K_)), torch.bfloat16), _t(rng.standard_normal((N, K_)) * 0.05, torch.bfloat16)
     bias = _t(rng.standard_normal(N))
@@ -1312,13 +1312,13 @@ def test_short_tiled_product_at_the_edges_of_its_tiles(M, N, K_):
     for parts in [p for p in range(1, 9) if p == 1 or K_ // 64 // p >= 2]:
         big = K.gemm_tiles_bf16(a, pw, None, torch.float32, parts=parts, token_tiles=2)
         for token_tiles in (1, 2, 3):
-            got = K.gemm_tiles_short_bf16(a, pw, torch.float32, parts, token_tiles)
+            got = K.gemm_tiles_bf16(a, pw, None, torch.float32, parts=parts, token_tiles=token_tiles)
             assert torch.equal(got, big), (parts, token_tiles)
         assert ((got.double().sum(0) if parts > 1 else got.double()) - want).abs().max() <= bound * parts
     for token_tiles in (1, 2, 3):
-        assert torch.equal(K.gemm_tiles_short_bf16(a, pw, torch.bfloat16, 1, token_tiles), K.gemm_tiles_bf16(a, pw, None, torch.bfloat16, token_tiles=2))
-    assert K.gemm_tiles_short_bf16(a, pw, torch.float32, K_ // 64, 1) is None or K_ == 64                 # parts of one stage
-    assert K.gemm_tiles_short_bf16(a.float(), pw, torch.float32, 1, 1) is None
+        assert torch.equal(K.gemm_tiles_bf16(a, pw, None, torch.bfloat16, token_tiles=token_tiles), K.gemm_tiles_bf16(a, pw, None, torch.bfloat16, token_tiles=2))
+    assert K.gemm_wide_bf16(a, pw, torch.float32, K_ // 64) is None or K_ == 64                 # parts of one stage
+    assert K.gemm_wide_bf16(a.float(), pw, torch.float32, 1) is None
 
 
 @pytest.mark.parametrize("M,N,K_", [(1, 32, 64), (97, 512, 128), (255, 544, 320), (256, 260, 256), (257, 1024, 576), (161, 96, 1088), (450, 1088, 192)])
@@ -1377,7 +1377,7 @@ def test_tiles_that_activate_their_product(M, N, K_):
 
 def test_wide_tiles_serve_prompts():
     """What wide_tiles_plan chooses, through the general entry and added to the stream: one part in place, more parts left to the norm that
-    adds them, all in one where none follows; matrices and operands that it does not take go the way they went."""
+    adds them or to the library where none follows; matrices and operands that it does not take go the way they went."""
     for M, N, K_ in ((1200, 2048, 2048), (2048, 4096, 14336), (300, 512, 4096), (700, 8320, 4096)):
         parts = K.prompt_parts(M, N, K_)
         a, w = torch.randn((M, K_), device=DEV).bfloat16(), (torch.randn((N, K_), device=DEV) * 0.05).bfloat16()
@@ -1390,9 +1390,8 @@ def test_wide_tiles_serve_prompts():
         x = x0.clone()
         adds = K.wide_tiles_plan(M, N, K_) == 1
         assert K.gemm_wide_add(x, a, pw) == adds and (adds or (torch.equal(x, x0) and not K.gemm_library_add(x, a, w, pw)))
-        if K.short_tiles_plan(M, N, K_) is None:
-            x = x0.clone()
-            assert K.gemm_wide_add(x, a, pw, norm_adds=False) and (x.double() - x0.double() - want).abs().max() <= 2e-5 * want.abs().max()
+        x = x0.clone()
+        assert K.gemm_wide_add(x, a, pw, norm_adds=False) == adds and (not adds or (x.double() - x0.double() - want).abs().max() <= 2e-5 * want.abs().max())
         x = x0.clone()
         assert not K.gemm_wide_add(x[:, :N - 4], a, pw) and not K.gemm_wide_add(x, a.float(), pw) and not K.gemm_wide_add(x.t(), a, pw) and torch.equal(x, x0)
         odd = torch.randn((M, K_ + 4), device=DEV).bfloat16()[:, 4:]          # rows that are not 16 bytes apart
@@ -1402,16 +1401,16 @@ def test_wide_tiles_serve_prompts():
 
 
 def test_short_tiled_product_serves_prompts_of_some_hundred_rows():
-    """What short_tiles_plan chooses, through the general entry: in parts or not, with the rows of a product that adds itself left to the norm."""
+    """What prompt_parts chooses for some hundred rows, through the general entry: in parts or not, with the rows of a product that adds itself left
+    to the norm."""
     for M, N, K_ in ((65, 2048, 2048), (128, 8192, 2048), (256, 3072, 2112), (257, 2048, 4096), (1024, 2048, 8192)):
-        plan = K.short_tiles_plan(M, N, K_)
+        parts = K.prompt_parts(M, N, K_)
         a, w = torch.randn((M, K_), device=DEV).bfloat16(), (torch.randn((N, K_), device=DEV) * 0.05).bfloat16()
         pw = K.pack_weights(w)
         got = K.gemm_product(a, w, torch.bfloat16, f32_ok=True, packed=pw)
-        assert got.dtype == torch.float32 and (got.shape == (M, N) if plan[0] == 1 else got.shape == (plan[0], M, N))
+        assert got.dtype == torch.float32 and parts > 1 and got.shape == (parts, M, N)
         want = a.double() @ w.double().t()
-        total = got.double() if plan[0] == 1 else got.double().sum(0)
-        assert (total - want).abs().max() <= 2e-5 * want.abs().max()
+        assert (got.double().sum(0) - want).abs().max() <= 2e-5 * want.abs().max()
         x = torch.zeros((M, N), device=DEV)
         assert not K.gemm_tiles_add(x, a, pw) and not K.gemm_library_add(x, a, w, pw) and not x.any()
 
@@ -1424,7 +1423,7 @@ def test_products_that_no_norm_follows_are_added_by_the_library(M, N, K_):
     parts = importlib.import_module("daisi-llogos_amd.parts")
     a, w = torch.randn((M, K_), device=DEV).bfloat16(), (torch.randn((N, K_), device=DEV) * 0.05).bfloat16()
     pw, x0 = K.pack_weights(w), torch.randn((M, N), device=DEV)
-    assert K.short_tiles_plan(M, N, K_) is not None
+    assert K.prompt_parts(M, N, K_) > 1
     want = x0 + torch.mm(a, w.t(), out_dtype=torch.float32)
     x = x0.clone()
     assert K.gemm_library_add(x, a, w, pw, norm_adds=False) and torch.equal(x, want)

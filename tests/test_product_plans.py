@@ -197,47 +197,32 @@ def test_which_recurrence_serves_short_prompts_of_heads_of_64():
     assert K.wave_scan_segments(8, 64, 20, n_cus=256) == 1 and K.wave_scan_segments(1, 64, 8000, n_cus=256) == 32
 
 
-def test_short_tiles_are_forms_that_the_kernel_takes():
-    """Every plan over its range leaves a part four stages or comes in one part, has no more parts than consumers add, and more than a
-    round of blocks only in one part; outside its range there is none."""
-    for N in (2048, 3072, 4096, 5120, 7168, 8192):
-        for K_ in (2048, 2112, 4096, 14336, 21504):
-            for M in (65, 100, 128, 129, 192, 193, 256, 257, 334, 512, 700, 1024):
-                plan = K.short_tiles_plan(M, N, K_, n_cus=256)
-                if M > 256 and K_ < 2 * N:
-                    assert plan is None
-                    continue
-                parts, token_tiles = plan
-                assert token_tiles in (1, 2, 3) and 1 <= parts <= 8 and (parts == 1 or K_ // 64 // parts >= 4)
-                assert parts == 1 or -(-M // (64 * token_tiles)) * -(-N // 256) * parts <= 256
-    for M, N, K_ in ((64, 4096, 4096), (1025, 4096, 14336), (100, 2047, 4096), (100, 8193, 4096), (100, 4096, 1984), (100, 4096, 4100), (100, 7169, 4096)):
-        assert K.short_tiles_plan(M, N, K_, n_cus=256) is None
-
-
 def test_rows_of_logits_beyond_a_grids_height_are_left_to_the_general_sampler():
     """The sampler for a small top-k has a row of its grid a row of logits, of which a grid has 65,535."""
     assert K.sample_few_serves(65535, 100, 40) and not K.sample_few_serves(65536, 100, 40)
     assert K.sample_few_serves(1, 128256, 256) and not K.sample_few_serves(1, 128256, 257) and not K.sample_few_serves(0, 100, 40)
 
 
-def test_no_product_is_both_a_tiled_one_part_and_short_tiles():
-    """What the tiled product adds to the stream by itself (one part) is nothing that short tiles serve."""
-    for N in (2048, 4096, 8192):
-        for K_ in (2048, 4096, 14336, 21504):
-            for M in (65, 128, 129, 256, 257, 512, 513, 1024, 1025, 1664, 2048):
-                plan = K.tiles_plan(M, N, K_)
-                assert plan is None or plan[0] != 1 or K.short_tiles_plan(M, N, K_, n_cus=256) is None
+def test_parts_are_chosen_for_the_height_that_the_launch_takes():
+    """Parts were once chosen for tiles of 64, 128 or 192 tokens and launched in tiles of another height.  By the costs of the launch no number of parts is
+    cheaper than the one chosen, and each part holds four stages or more."""
+    for N in (2048, 3072, 4096, 5120, 7168, 8192):
+        for K_ in (2048, 2112, 4096, 14336, 21504):
+            for M in (65, 100, 128, 129, 192, 193, 209, 256, 257, 334, 512, 700, 1024):
+                parts = K.wide_tiles_plan(M, N, K_, n_cus=256)
+                assert 1 <= parts <= 8 and (parts == 1 or K_ // 64 // parts >= 4)
+                cost = lambda p: K._lib().llogos_gemm_tiles_cost(M, N, K_, p, 256) + p * M * N * 1.2e-6
+                assert all(cost(parts) <= cost(p) for p in range(1, 9)), (M, N, K_)
+    assert K.prompt_parts(200, 4096, 14336) == K.wide_tiles_plan(200, 4096, 14336) > 1
 
 
 def test_wide_tiles_have_parts_that_the_kernel_takes(monkeypatch):
-    """More than 64 rows of matrices of 512 rows and columns on, each part of four stages or more; where another plan of tiles serves, its parts."""
+    """More than 64 rows of matrices of 512 rows and columns on, each part of four stages or more."""
     for N in (512, 1536, 2048, 6144, 10240, 28672):
         for K_ in (512, 576, 4096, 14336, 21504):
             for M in (65, 129, 334, 1024, 1025, 2048, 5003, 16384):
                 parts = K.wide_tiles_plan(M, N, K_, n_cus=256)
                 assert 1 <= parts <= 8 and (parts == 1 or K_ // 64 // parts >= 4)
-                chosen, short = K.prompt_parts(M, N, K_), K.short_tiles_plan(M, N, K_)
-                assert chosen == (short[0] if short else (K.tiles_plan(M, N, K_) or (parts,))[0] if N * K_ < 1 << 22 else K.wide_tiles_plan(M, N, K_))
     assert K.wide_tiles_plan(128, 4096, 14336, n_cus=256) > 2 and K.wide_tiles_plan(5003, 28672, 4096, n_cus=256) == 1
     for M, N, K_ in ((64, 4096, 4096), (2048, 4096, 4100), (2048, 511, 4096), (2048, 514, 4096), (2048, 4096, 448)):
         assert K.wide_tiles_plan(M, N, K_, n_cus=256) == 0
@@ -266,6 +251,6 @@ def test_heights_of_tiles_at_sizes_measured():
         assert height(M, 4096, 768, gated=1) == 64, M
     for M in (129, 200, 300):
         assert height(M, 9728, 1024, gated=1) in (64, 96), M
-    for M, N, K_, parts, best in ((300, 3072, 3072, 8, (64,)), (300, 5120, 17408, 4, (128,)), (1000, 7168, 5120, 4, (256,)), (400, 8192, 1024, 4, (64, 224)),
+    for M, N, K_, parts, best in ((300, 3072, 3072, 8, (64,)), (300, 5120, 17408, 4, (128,)), (65, 4096, 14336, 8, (64,)), (400, 8192, 1024, 4, (64, 224)),
                                   (200, 8192, 28672, 4, (128,)), (2048, 3072, 2048, 4, (64,))):
         assert height(M, N, K_, parts) in best, (M, N, K_, parts)
