@@ -2074,8 +2074,8 @@ def gemm_packed_unscaled_bf16(squares: RowSquares, eps: float, pw: PackedWeight,
 
 # Which product serves many rows of bfloat16 (prompts): "auto" (the default): the hand-written tiled product (gemm_tiles_bf16 on the
 # packed copy) for more than 64 rows, in the parts that prompt_parts says and with the SwiGLU epilogue where wide_tiles_serve_gated or
-# tiles_serve_gated say so, and the library's product elsewhere (matrices without a packed copy or of fewer than 512 rows or columns, gated
-# products of few rows; as the reference uses a library there); "tiles": the hand-written one wherever it applies;
+# tiles_serve_gated say so, and the library's product elsewhere (matrices without a packed copy or of fewer than 512 rows or columns, where
+# library_serves, gated products of few rows; as the reference uses a library there); "tiles": the hand-written one wherever it applies;
 # "library": the library's everywhere.  LLOGOS_PROMPT_PRODUCT in the environment sets the default.
 PROMPT_PRODUCT = os.environ.get("LLOGOS_PROMPT_PRODUCT", "auto")
 TILES_MIN_ROWS, TILES_MAX_ROWS, TILES_MAX_K = 1024, 2048, 5120
@@ -2131,8 +2131,8 @@ def long_tiles_plan(M: int, N: int, K: int, n_cus: Optional[int] = None) -> Opti
 @functools.lru_cache(maxsize=4096)
 def _tiles_cost(M: int, N: int, K: int, parts: int, units: int) -> float:
     """Microseconds that the tiled product is expected to take (gemm_tiles_bf16.hip: tiles_cost), with its consumer's reading of the
-    results, 0.3 us a MB (0.23 to 0.29 measured; what a part more costs the norm beside that is not in it)."""
-    return _lib().llogos_gemm_tiles_cost(M, N, K, parts, units) + parts * M * N * 4e-6 * 0.3
+    results: 0.2 us a MB and 0.4 a part (a norm takes 0.20 to 0.28 a MB, other kernels 0.21 to 0.29)."""
+    return _lib().llogos_gemm_tiles_cost(M, N, K, parts, units) + parts * (M * N * 4e-6 * 0.2 + 0.4)
 
 
 @functools.lru_cache(maxsize=4096)
@@ -2143,7 +2143,7 @@ def _wide_parts(M: int, N: int, K: int, units: int) -> int:
 def wide_tiles_plan(M: int, N: int, K: int, n_cus: Optional[int] = None) -> int:
     """Parts of k in which the tiled product takes a plain product of M rows, in the tiles that the launch chooses for them, or 0 where it is not
     asked: it is for more than 64 rows of matrices of 512 rows, a multiple of four, and columns, a multiple of 64.  What the parts cost with
-    their consumer is within 1.3 % of the cheapest on average over 860 sizes that a norm reads, 1.5 % over those that another kernel reads."""
+    their consumer is within 0.7 % of the cheapest on average over 805 sizes that a norm reads, 1.4 % over 915 that another kernel reads."""
     if PROMPT_PRODUCT != "auto" or M <= SKINNY_MAX_ROWS or K % 64 or K < 512 or N < 512 or N % 4:
         return 0
     return _wide_parts(M, N, K, n_cus or compute_units())
@@ -2157,9 +2157,30 @@ def wide_tiles_serve_gated(M: int, N: int, K: int) -> bool:
     return PROMPT_PRODUCT == "auto" and M > SKINNY_MAX_ROWS and K % 64 == 0 and K >= 512 and M * N >= 1 << 22
 
 
-def prompt_parts(M: int, N: int, K: int) -> int:
-    """Parts of k of a plain product of M rows that the tiled product serves, or 0 (see wide_tiles_plan)."""
-    return wide_tiles_plan(M, N, K)
+def library_serves(M: int, N: int, K: int, adds: bool = False) -> bool:
+    """Whether the library makes a plain product of M rows that wide_tiles_plan would take (adds: in the stream, before a norm).  Its kernels are
+    ahead by 5 to 20 % where a matrix is small, level or ahead by some percent where the rows are many, behind by 5 to 60 % where k is long or
+    the rows some hundred, and change by as much from one size to the next; the lines lie where 33 matrices of 65 to 16,384 rows changed sides on
+    average.  Product and what reads it, us, library / tiled.  In the stream: 2,048 rows [2,048, 2,048] 31.1 / 32.2, [4,096, 4,096] 75 / 82, 16,384
+    rows [4,096, 4,096] 507 / 576; 600 rows [5,120, 5,120] 58 / 54, 1,200 rows [4,096, 11,008] 129 / 110, 2,500 rows [4,096, 14,336] 250 / 239.  Read by
+    another kernel: 512 rows [2,048, 2,048] 15.9 / 18.4, [3,072, 2,048] 18.6 / 20.8; [7,168, 5,120] 300 rows 54 / 42, 2,048 148 / 155, 5,003 370 / 362;
+    [6,144, 4,096] 2,048 rows 107 / 117.  Never where a hand-written product has served all along: some hundred rows of matrices of 2,048 to 8,192
+    rows and k from 2,048 on, few rows of long matrices, what tiles_plan names."""
+    if 2048 <= N <= 8192 and K >= 2048 and (M <= 256 or (M <= 1024 and K >= 2 * N)):
+        return False
+    if (M <= LDS_MAX_ROWS and K >= 2 * N) or tiles_plan(M, N, K) is not None:
+        return False
+    if adds and N > 8192:                                    # (parts of such rows take the norm longer than the product takes)
+        return True
+    if (K >= 2.5 * N and M <= 1800) or (K >= 3 * N and M <= 3600) or (K >= 4608 and 4096 <= N <= 8192 and M <= 700):
+        return False
+    return adds or K < 2560 or M > 700 or N * K < 1 << 23 or (M <= LDS_MAX_ROWS and N > 16384)
+
+
+def prompt_parts(M: int, N: int, K: int, adds: bool = False) -> int:
+    """Parts of k of a plain product of M rows that the tiled product serves (see wide_tiles_plan), or 0 where it does not (see library_serves)."""
+    parts = wide_tiles_plan(M, N, K)
+    return 0 if parts and library_serves(M, N, K, adds) else parts
 
 
 def gemm_wide_bf16(a: torch.Tensor, pw: PackedWeight, out_dtype: torch.dtype, parts: int) -> Optional[torch.Tensor]:
@@ -2256,8 +2277,8 @@ def gemm_tiles_add(x: torch.Tensor, a: torch.Tensor, pw: Optional[PackedWeight])
     return True
 
 
-def gemm_wide_add(x: torch.Tensor, a: torch.Tensor, pw: Optional[PackedWeight], norm_adds: bool = True) -> bool:
-    """gemm_tiles_add where prompt_parts has the product in one part.  norm_adds: whether a norm reads the stream next."""
+def gemm_wide_add(x: torch.Tensor, a: torch.Tensor, pw: Optional[PackedWeight]) -> bool:
+    """gemm_tiles_add where prompt_parts has the product in one part."""
     if pw is None or pw.gate_rows or RESIDUAL_PRODUCT != "on":
         return False
     if not (a.dtype == torch.bfloat16 and a.dim() == 2 and a.is_cuda and x.is_cuda and a.device == x.device == pw.data.device):
@@ -2266,7 +2287,7 @@ def gemm_wide_add(x: torch.Tensor, a: torch.Tensor, pw: Optional[PackedWeight], 
     if not (x.dtype == torch.float32 and x.shape == (M, pw.N) and x.is_contiguous() and K == pw.K and a.stride(1) == 1
             and a.stride(0) % 8 == 0 and a.data_ptr() % 16 == 0):
         return False
-    if prompt_parts(M, pw.N, K) != 1:
+    if prompt_parts(M, pw.N, K, adds=True) != 1:
         return False
     code = _lib().llogos_gemm_tiles_bf16(_p(x), F32, _p(a), a.stride(0), _p(pw.data), None, M, pw.N, K, pw.N, ctypes.c_longlong(0), 2, 1,
                                          0, compute_units(a.device), ctypes.c_float(-1.0), _stream())
@@ -2367,7 +2388,7 @@ def gemm_library_add(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor, packed: 
     more than 128 rows that the tiled product does not take): the stream is read and written once there
     instead of the product being written, read again and added by the norm's kernel.  False (and x
     untouched) otherwise.  The result is the float32 product added to x, bit for bit.  norm_adds: a norm reads the stream next and adds
-    parts that short tiles leave; without one a sum of the parts and one with the stream would follow ([4,096, 4,096], 200 rows: 20 us
+    parts that the tiled product leaves; without one a sum of the parts and one with the stream would follow ([4,096, 4,096], 200 rows: 20 us
     and 6 and 5, the library with the sum in it 25), and the library keeps what it can add itself."""
     if RESIDUAL_PRODUCT != "on":
         return False
@@ -2377,7 +2398,7 @@ def gemm_library_add(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor, packed: 
     M, N = a.shape[0], w.shape[0]
     if M <= LDS_MAX_ROWS or x.shape != (M, N) or a.shape[1] != w.shape[1] or a.shape[1] % 8:
         return False
-    if packed is not None and (tiles_plan(M, packed.N, packed.K) is not None or (norm_adds and prompt_parts(M, packed.N, packed.K) > 1)):
+    if packed is not None and (tiles_plan(M, packed.N, packed.K) is not None or (norm_adds and prompt_parts(M, packed.N, packed.K, adds=True) > 0)):
         return False
     torch.addmm(x, a, w.t(), out_dtype=torch.float32, out=x)
     return True

@@ -126,7 +126,7 @@ class Linear(Part):
         if a.shape[0] > K.SKINNY_MAX_ROWS:
             # prompts: the product that serves them, the tiled one or the library's, with the sum in its epilogue
             norm_adds = residual.norm is not None
-            if self.bias is None and (K.gemm_tiles_add(x, a, self.packed) or K.gemm_wide_add(x, a, self.packed, norm_adds)
+            if self.bias is None and (K.gemm_tiles_add(x, a, self.packed) or (norm_adds and K.gemm_wide_add(x, a, self.packed))
                                       or K.gemm_library_add(x, a, self.weight, self.packed, norm_adds)):
                 return K.RowSquares(None, self.weight.shape[0])
             return None

@@ -1376,9 +1376,9 @@ def test_tiles_that_activate_their_product(M, N, K_):
 
 
 def test_wide_tiles_serve_prompts():
-    """What wide_tiles_plan chooses, through the general entry and added to the stream: one part in place, more parts left to the norm that
-    adds them or to the library where none follows; matrices and operands that it does not take go the way they went."""
-    for M, N, K_ in ((1200, 2048, 2048), (2048, 4096, 14336), (300, 512, 4096), (700, 8320, 4096)):
+    """What prompt_parts chooses, through the general entry and added to the stream: one part in place, more parts left to the norm that
+    adds them, none to the library; matrices and operands that it does not take go the way they went."""
+    for M, N, K_ in ((600, 3072, 3072), (2048, 4096, 14336), (300, 512, 4096), (700, 8320, 4096), (1100, 5120, 16384)):
         parts = K.prompt_parts(M, N, K_)
         a, w = torch.randn((M, K_), device=DEV).bfloat16(), (torch.randn((N, K_), device=DEV) * 0.05).bfloat16()
         pw, x0 = K.pack_weights(w), torch.randn((M, N), device=DEV)
@@ -1388,10 +1388,13 @@ def test_wide_tiles_serve_prompts():
         total = got.double() if parts == 1 else got.double().sum(0)
         assert (total - want).abs().max() <= 2e-5 * want.abs().max()
         x = x0.clone()
-        adds = K.wide_tiles_plan(M, N, K_) == 1
-        assert K.gemm_wide_add(x, a, pw) == adds and (adds or (torch.equal(x, x0) and not K.gemm_library_add(x, a, w, pw)))
-        x = x0.clone()
-        assert K.gemm_wide_add(x, a, pw, norm_adds=False) == adds and (not adds or (x.double() - x0.double() - want).abs().max() <= 2e-5 * want.abs().max())
+        adds = K.prompt_parts(M, N, K_, adds=True)
+        assert K.gemm_wide_add(x, a, pw) == (adds == 1)
+        if adds > 1:
+            assert not K.gemm_library_add(x, a, w, pw) and torch.equal(x, x0)
+        elif adds == 0:
+            assert K.gemm_library_add(x, a, w, pw)
+        assert adds > 1 or (x.double() - x0.double() - want).abs().max() <= 2e-5 * want.abs().max()
         x = x0.clone()
         assert not K.gemm_wide_add(x[:, :N - 4], a, pw) and not K.gemm_wide_add(x, a.float(), pw) and not K.gemm_wide_add(x.t(), a, pw) and torch.equal(x, x0)
         odd = torch.randn((M, K_ + 4), device=DEV).bfloat16()[:, 4:]          # rows that are not 16 bytes apart

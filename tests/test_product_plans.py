@@ -211,7 +211,7 @@ def test_parts_are_chosen_for_the_height_that_the_launch_takes():
             for M in (65, 100, 128, 129, 192, 193, 209, 256, 257, 334, 512, 700, 1024):
                 parts = K.wide_tiles_plan(M, N, K_, n_cus=256)
                 assert 1 <= parts <= 8 and (parts == 1 or K_ // 64 // parts >= 4)
-                cost = lambda p: K._lib().llogos_gemm_tiles_cost(M, N, K_, p, 256) + p * M * N * 1.2e-6
+                cost = lambda p: K._lib().llogos_gemm_tiles_cost(M, N, K_, p, 256) + p * (M * N * 0.8e-6 + 0.4)
                 assert all(cost(parts) <= cost(p) for p in range(1, 9)), (M, N, K_)
     assert K.prompt_parts(200, 4096, 14336) == K.wide_tiles_plan(200, 4096, 14336) > 1
 
@@ -254,3 +254,21 @@ def test_heights_of_tiles_at_sizes_measured():
     for M, N, K_, parts, best in ((300, 3072, 3072, 8, (64,)), (300, 5120, 17408, 4, (128,)), (65, 4096, 14336, 8, (64,)), (400, 8192, 1024, 4, (64, 224)),
                                   (200, 8192, 28672, 4, (128,)), (2048, 3072, 2048, 4, (64,))):
         assert height(M, N, K_, parts) in best, (M, N, K_, parts)
+
+
+def test_the_library_serves_what_it_served_before_and_is_ahead_at():
+    """Prompts' products that the library made before the tiled one took all of them, measured with what reads them: at the first ones the library
+    is ahead, in the stream and for another kernel; at the second ones in the stream alone; at the others the tiled product is, or a hand-written one
+    served all along."""
+    for M, N, K_ in ((334, 2048, 2048), (512, 2048, 2048), (2048, 2048, 2048), (16384, 2048, 2048), (700, 1536, 1536), (4096, 1536, 1536), (512, 3072, 2048),
+                     (334, 2304, 768), (8192, 3072, 3072), (16384, 4096, 4096), (8192, 4096, 4096), (16384, 1536, 8960), (65, 1536, 1536), (100, 1024, 1024),
+                    (2048, 4096, 4096), (2048, 6144, 4096), (2048, 7168, 5120), (65, 21504, 4096)):
+        assert K.library_serves(M, N, K_, adds=True) and K.library_serves(M, N, K_), (M, N, K_)
+        assert K.prompt_parts(M, N, K_) == 0 and K.wide_tiles_plan(M, N, K_) > 0
+    for M, N, K_ in ((300, 3072, 3072), (600, 4096, 4096), (300, 6144, 4096), (700, 21504, 4096), (256, 12288, 4096)):
+        assert K.library_serves(M, N, K_, adds=True) and not K.library_serves(M, N, K_), (M, N, K_)
+        assert K.prompt_parts(M, N, K_, adds=True) == 0 < K.prompt_parts(M, N, K_)
+    for M, N, K_ in ((200, 4096, 4096), (256, 2048, 2048), (65, 8192, 8192), (1000, 4096, 14336), (2048, 4096, 14336), (1200, 4096, 11008), (1500, 1024, 4096),
+                     (3529, 2048, 8192), (600, 5120, 5120), (300, 512, 4096), (100, 768, 3072), (5003, 5120, 17408), (2048, 4096, 21504)):
+        assert not K.library_serves(M, N, K_, adds=True) and not K.library_serves(M, N, K_), (M, N, K_)
+    assert K.library_serves(1200, 10240, 28672, adds=True) and not K.library_serves(1200, 10240, 28672)
