@@ -60,34 +60,33 @@ def packed_weight_budget(model: Model, dtype: torch.dtype, max_tokens: int, devi
     same process, another process) is not counted on: only free memory is."""
     if dtype != torch.bfloat16:
         return 0
-    element = torch.empty((), dtype=dtype).element_size()
-    elements = 0
-    for spec in model.tensor_specs():
-        if spec.kind in ("matrix", "table"):
-            n = 1
-            for d in spec.shape:
-                n *= int(d)
-            elements += n
-    cache = max_tokens * sum(kv.n_kv_heads * (kv.head_dim + (kv.value_dim if kv.values else 0)) * element
-                             for kv, _ in model.cache_needs() if kv is not None)
     with torch.cuda.device(device):
         free, total = torch.cuda.mem_get_info()
         free += torch.cuda.memory_reserved() - torch.cuda.memory_allocated()      # what torch holds but does not use
-    return max(0, int(free - 0.15 * total) - element * elements - cache)
+    return max(0, int(free - 0.15 * total) - _own_bytes(model, dtype, max_tokens))
+
+
+def _own_bytes(model: Model, dtype: torch.dtype, max_tokens: int) -> int:
+    """Bytes of the matrices and the key/value cache."""
+    element = torch.empty((), dtype=dtype).element_size()
+    elements = sum(math.prod(spec.shape) for spec in model.tensor_specs() if spec.kind in ("matrix", "table"))
+    return element * (elements + max_tokens * sum(kv.n_kv_heads * (kv.head_dim + (kv.value_dim if kv.values else 0))
+                                                  for kv, _ in model.cache_needs() if kv is not None))
 
 
 def _packing(rt: Runtime, model: Model, max_tokens: int, pack_weights: Optional[bool]) -> None:
-    """pack_weights None: packed copies as far as the GPU's memory allows; True: all; False: none."""
+    """pack_weights None: packed copies as far as the GPU's memory allows; True: of all matrices that every token is multiplied with; False: none.
+    Experts, of which a token is multiplied with a few, get what the other matrices' copies leave, less room for a second
+    engine like this one without copies of its experts."""
     rt.pack_weights = pack_weights is not False and rt.dtype == torch.bfloat16
     rt.pack_budget = packed_weight_budget(model, rt.dtype, max_tokens, rt.device) if pack_weights is None else None
-    if rt.pack_budget is None:
-        rt.expert_budget = None
-        return
-    # experts get what the matrices that every token is multiplied with leave (embedding tables' copies, of tied heads, among them)
-    element = torch.empty((), dtype=rt.dtype).element_size()
-    others = sum(math.prod(spec.shape) for spec in model.tensor_specs() if spec.kind in ("matrix", "table")) - model.expert_elements()
-    rt.expert_budget = max(0, rt.pack_budget - element * others)
-    rt.pack_budget -= rt.expert_budget
+    rt.expert_budget = 0
+    if rt.pack_weights and model.expert_elements():
+        free = packed_weight_budget(model, rt.dtype, max_tokens, rt.device) if rt.pack_budget is None else rt.pack_budget
+        others = model.packable_bytes()
+        rt.expert_budget = max(0, free - 2 * others - _own_bytes(model, rt.dtype, max_tokens))
+        if rt.pack_budget is not None:
+            rt.pack_budget -= rt.expert_budget
 
 
 def require_gpu(device: Union[str, torch.device] = "cuda:0") -> torch.device:

@@ -208,6 +208,10 @@ class Model:
         """Elements of all experts' matrices (each layer once)."""
         return sum(p.expert_elements() for p in self.layers + self.stream_parts)
 
+    def packable_bytes(self) -> int:
+        """What the packed copies of all matrices but the experts' take (each layer once)."""
+        return sum(p.packable_bytes() for p in self.layers + self.stream_parts) + self.head.packable_bytes()
+
     def packed_weight_bytes(self) -> int:
         """Bytes of device memory that the packed second copies of the matrices take (each layer once)."""
         return sum(p.packed_bytes() for p in self.layers + self.stream_parts) + self.head.packed_bytes()

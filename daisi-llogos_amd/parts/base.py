@@ -31,7 +31,7 @@ class Runtime:
     dtype: torch.dtype                  # torch.float32 or torch.bfloat16: matrices, activations, cache
     pack_weights: bool = True           # bfloat16 matrices get a second copy in the matrix cores' order (few-row products)
     pack_budget: Optional[int] = None   # bytes that the packed copies may take together (None: no limit); bind() counts it down
-    expert_budget: Optional[int] = None # the same for the copies of experts, beside it
+    expert_budget: Optional[int] = None # the same for the copies of experts, apart from it
     # scratch and counters of decode attention (ops/kernels.py: _attn_shares), those of a step's second branch (ops/branches.py) apart
     attention_shares: list = field(default_factory=list, repr=False, compare=False)
     branch_attention_shares: list = field(default_factory=list, repr=False, compare=False)
@@ -150,6 +150,16 @@ class Part:
                 total += v.packed_bytes()
             elif isinstance(v, (list, tuple)):
                 total += sum(x.packed_bytes() for x in v if isinstance(x, Part))
+        return total
+
+    def packable_bytes(self) -> int:
+        """What the packed copies of all matrices of this part and its sub-parts take but those of experts, bound or not."""
+        total = 0
+        for v in vars(self).values():
+            if isinstance(v, Part):
+                total += v.packable_bytes()
+            elif isinstance(v, (list, tuple)):
+                total += sum(x.packable_bytes() for x in v if isinstance(x, Part))
         return total
 
     def expert_elements(self) -> int:

@@ -84,6 +84,9 @@ class Linear(Part):
         """Bytes of the packed copy that this product holds beside the matrix (0 without one)."""
         return 0 if self.packed is None else self.packed.data.numel() * self.packed.data.element_size()
 
+    def packable_bytes(self) -> int:
+        return K.packed_weight_bytes(self.total_out, self.in_features)
+
     def _packed_rows(self, rows_out: Optional[int]) -> Optional[K.PackedWeight]:
         if self.packed is None or rows_out is None:
             return self.packed
