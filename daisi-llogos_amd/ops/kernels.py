@@ -772,19 +772,33 @@ def moe_form(P: int, E: int, N: int, K: int, n_cus: Optional[int] = None) -> int
 
 def moe_packed_form(P: int, E: int) -> Tuple[int, int]:
     """Lowest and highest tiles, in units of 64 sorted rows, among which the experts' product on packed matrices chooses for P pairs of E experts;
-    (0, 0): the form for few rows, up to 10 an expert (us, few rows / tiles of 64: 16 experts of 7168 x 4096, 8 rows 143 / 159, 12 rows 167 / 161; 64 of 1536 x
-    2048 64 / 75 and 75 / 76; 32 of 2048 x 768 19.5 / 21.7 and 23.8 / 22.2; 8 of 8192 x 4096 83 / 94 and 96 / 95).  The lower the
-    lowest, the more blocks of the grid find no tile; tiles of 64 rows gain nothing from 96 an expert on (16 of 7168 x 4096: 211 / 171 in tiles
+    (0, 0): the form for few rows, up to 10 an expert (us, few rows / tiles of 64: 16 experts of 7168 x 4096, 10 rows 149 / 165, 16 rows 215 / 164; 64 of 1536 x
+    2048 69 / 82 and 92 / 82; 32 of 2048 x 768 21.5 / 25.0 and 28.9 / 24.8; 8 of 8192 x 4096 85 / 97 and 122 / 98).  The lower the
+    lowest, the more blocks of the grid find no tile; tiles of 64 rows gain little from 96 an expert on (16 of 7168 x 4096, 200 rows: 364 / 286 in tiles
     of 128) and those of 128 from 600 on."""
     if P <= 10 * E:
         return 0, 0
     return (1 if P < 96 * E else 2 if P < 600 * E else 3), 4
 
 
+MOE_PACKED_EXPERTS = 256          # experts up to which their matrices get a packed copy
+
+
+def moe_packed_serves(P: int, E: int, K: int) -> bool:
+    """Whether the experts' product for P pairs reads the packed matrices: few rows, up to 10 an expert, always; more of them with k of 1,536 and
+    more, or from 300 an expert on.  A stage of the tiles' ring costs a block with a short k more than it saves.  us, row-major / packed: 11 rows an
+    expert, 128 of [2,048, 768] 80 / 91, 256 of [1,024, 1,024] 104 / 116; 32 rows (uneven) 89 / 103; 600 rows level; k of 2,048, 11 rows, 32 of
+    [2,048, 2,048] 64 / 56, 256 of [512, 2,048] 141 / 108.  Not for 1,024 experts, whose blocks look for their segment longer than they multiply: [512, 512] 59 /
+    122 at half a row an expert, 128 / 226 at 10, 151 / 213 at 32."""
+    return E <= MOE_PACKED_EXPERTS and (P <= 10 * E or K >= 1536 or P >= 300 * E)
+
+
 def pack_experts(w: torch.Tensor) -> Optional["PackedWeight"]:
     """A packed copy of experts' matrices w [E, N, K] bfloat16 as one matrix of E N rows, for moe_product; None where rows of a matrix are no multiple of 64 or
-    values no multiple of 32 (an expert would not begin with a block of its own)."""
+    values no multiple of 32 (an expert would not begin with a block of its own), and for more experts than moe_packed_serves takes."""
     E, N, K = w.shape
+    if E > MOE_PACKED_EXPERTS:
+        return None
     if w.dtype != torch.bfloat16 or N % 64 or K % 32 or not w.is_contiguous():
         return None
     return pack_weights(w.view(E * N, K))
@@ -827,6 +841,7 @@ def moe_product(a: torch.Tensor, w: torch.Tensor, order: torch.Tensor, seg: torc
             form = ("few", "tiles64", "tiles128", "tiles256").index(MOE_PRODUCT)
         if packed is not None:
             _need(packed.N == E * N and packed.K == Kk and not packed.gate_rows and packed.data.device == w.device, "moe_product: packed must be the experts' matrices")
+        if packed is not None and (MOE_PRODUCT != "auto" or moe_packed_serves(P, E, Kk)):
             least, most = moe_packed_form(P, E) if MOE_PRODUCT == "auto" else ((0, 0), (1, 1), (2, 2), (4, 4))[form]
             code = _lib().llogos_moe_product_packed_bf16(_p(out), _DT[out_dtype], _p(a), a.shape[0], _p(packed.data), _p(order), _p(seg), E, top,
                                                          1 if gather else 0, P, N, Kk, a.stride(0), act, ctypes.c_float(scale), _p(pair_weight), lim,
