@@ -1259,6 +1259,27 @@ def test_expert_product_on_packed_matrices(form, N, K_, monkeypatch):
     assert K.pack_experts(w[:, :N - 32].contiguous()) is None and K.pack_experts(w[:, :, :K_ - 8].contiguous()) is None and K.pack_experts(w.float()) is None
 
 
+@pytest.mark.parametrize("sizes", [[700, 0, 131, 257, 1, 64], [193, 192, 191], [1025]])
+@pytest.mark.parametrize("least,most", [(3, 3), (1, 4), (2, 4), (3, 4)])
+def test_expert_tiles_of_chosen_heights(sizes, least, most):
+    """Tiles whose height the launch's blocks choose among several, on GPUs of several sizes, so that one round of low tiles, several of high ones and what
+    lies between are cheapest in turn: grids sized by the lowest height and shared out by the chosen one; tiles of 192 rows forced."""
+    N, K_, E, P = 320, 320, len(sizes), sum(sizes)
+    rng = np.random.default_rng(P + least)
+    seg = _t(np.concatenate([[0], np.cumsum(sizes)]), torch.int32)
+    order = _t(rng.permutation(P), torch.int32)
+    a = _t(rng.standard_normal((P, K_)), torch.bfloat16)
+    w = _t(rng.standard_normal((E, N, K_)) * 0.1, torch.bfloat16)
+    packed, rows = K.pack_experts(w), a[order.long()].double()
+    want = torch.cat([rows[int(seg[e]):int(seg[e + 1])] @ w[e].double().t() for e in range(E)])
+    bound = 2.0 ** -23 * K_ ** 0.5 * 4 * max(1.0, want.abs().max().item())      # as in test_expert_product_on_packed_matrices
+    for units in (1, 4, 8, 16, 24, 40, 64, 256):
+        out = torch.full((P, N), float("nan"), device=DEV)
+        K._check(K._lib().llogos_moe_product_packed_bf16(K._p(out), K.F32, K._p(a), P, K._p(packed.data), K._p(order), K._p(seg), E, 1, 1, P, N, K_, K_, 0,
+                                                         ctypes.c_float(1.0), None, ctypes.c_float(0.0), least, most, units, K._stream()), "moe")
+        assert (out.double() - want).abs().max() <= bound, units
+
+
 @pytest.mark.parametrize("M,N,K_", [(1, 64, 64), (129, 320, 192), (700, 1100, 128), (2100, 2900, 64), (4700, 260, 128)])
 def test_tiled_product_places_every_tile_and_adds_itself(M, N, K_):
     """One tile, fewer than XCDs, bands of token tiles that are not full, several rounds of blocks, parts of k: every value is
