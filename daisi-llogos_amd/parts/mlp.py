@@ -131,8 +131,11 @@ class ActivatedMLP(FeedForward):
     def forward(self, ctx: StepContext, h):
         act = self.up.activated_product(h, self.activation, self.a, self.b)         # (prompts: in the product's epilogue)
         if act is None:
-            act = K.activation(self.up.product(h, f32_ok=True), self.activation, self.rt.dtype, self.a, self.b)
-        mark(ctx, "up")
+            z = self.up.product(h, f32_ok=True)
+            mark(ctx, "up")
+            act = K.activation(z, self.activation, self.rt.dtype, self.a, self.b)
+        else:
+            mark(ctx, "up")
         out = self.down.product(act, f32_ok=True)
         mark(ctx, "down")
         return out

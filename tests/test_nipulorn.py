@@ -212,3 +212,19 @@ def test_the_copies_that_one_product_reads_together_are_counted_once(monkeypatch
         counted.append((mixer.weight_bytes(), mixer.packed_bytes()))
     matrices = 5 * 128 * 128 + 2 * 128 * 64
     assert counted[0] == counted[1] == (2 * matrices + 4 * (5 * 128 + 3 * 128), 2 * matrices)
+
+
+@pytest.mark.parametrize("in_one", [False, True])
+def test_the_up_product_is_marked_before_its_activation(monkeypatch, in_one):
+    """A step timed part by part: "up" is the product's time where the activation is a kernel of its own, and both where they are one."""
+    K = importlib.import_module("daisi-llogos_amd.ops.kernels")
+    linear, seen, h = importlib.import_module("daisi-llogos_amd.parts.linear"), [], torch.zeros(2, 8)
+    ctx = P.StepContext(runtime=None, n_tokens=2, batch=1, ids=None, tok_seq=None, tok_pos=None, slots=None, cu_seqlens=[0, 2], starts=[0], slot_ids=[0],
+                        is_decode=False, max_context=2, probe=lambda name: seen.append(name))
+    ff = P.ActivatedMLP("f.", 8, 16, "relu2")
+    ff.rt = P.Runtime(torch.device("cpu"), torch.bfloat16)
+    monkeypatch.setattr(linear.Linear, "activated_product", lambda self, a, *rest: seen.append("both") or a if in_one else None)
+    monkeypatch.setattr(linear.Linear, "product", lambda self, a, **kw: seen.append("product") or a)
+    monkeypatch.setattr(K, "activation", lambda z, *rest: seen.append("activation") or z)
+    ff.forward(ctx, h)
+    assert seen == (["both", "up"] if in_one else ["product", "up", "activation"]) + ["product", "down"]
