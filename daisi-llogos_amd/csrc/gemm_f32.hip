@@ -296,6 +296,9 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_ring_kernel(
     constexpr int COPIES = (ROWS / 8 + 3) / 4, LEAST = ROWS / 8 / 4;         // of 8 rows a wave and stage; what every wave has of them
     constexpr int TILES = MT * NT, READS = MT + NT, PRODUCTS = 4 * TILES;
     static_assert(WM * WN == 4 && ROWS % 8 == 0, "four waves");
+    // (the additions behind the products are assembly, for which the compiler adds no waits: a chain's last product has another tile's product and
+    // the next step's first one behind it when it is read, 64 clocks; with one tile a wave nothing would stand between them)
+    static_assert(TILES >= 2, "additions one step behind their products");
     extern __shared__ __attribute__((aligned(1024))) unsigned char f32_lds[];
     const int tiles = m_tiles * n_tiles, per = tiles >> 3, more = tiles & 7, xcd = blockIdx.x & 7;
     const int tile = xcd * per + min(xcd, more) + (blockIdx.x >> 3);
