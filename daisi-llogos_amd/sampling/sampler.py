@@ -81,7 +81,7 @@ class Sampler:
         if helpers is None or getattr(self.uniforms, "__func__", None) is not Sampler.uniforms:      # (or the numbers come from elsewhere)
             return None
         count = p.penalty_count
-        if not (p.has_penalties and isinstance(count, int) and -1 << 62 < count < 1 << 62):
+        if not (p.has_penalties and -1 << 62 < count < 1 << 62):
             size = -1 if p.has_penalties else 0
         else:
             size = helpers.llogos_host_windows_size(histories, count)

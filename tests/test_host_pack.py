@@ -76,19 +76,3 @@ def test_sampler_packs_the_same_either_way(helpers):
         buffer[:] = 0
         assert s._pack_in_python(requests, indices, histories)[:2] == (starts, n) and (buffer == native).all()
         assert s._pack(9, requests, indices[:-1], histories) is None and s._pack(9, map(int, requests), indices, histories) is None
-
-
-def test_a_count_that_is_no_plain_integer_is_left_to_python(helpers):
-    """A penalty's window given as numpy's integer, or as anything that Python's slices take, is packed as it was."""
-    llogos = importlib.import_module("daisi-llogos_amd")
-    histories = [[1, 2, 3, 4, 5], [6], []]
-
-    class Count(int):
-        pass
-    for count in (np.int64(3), np.int32(3), Count(3), 3, True):
-        s = llogos.Sampler(llogos.GenerationParams(temperature=0.7, top_k=40, repetition_penalty=1.2, seed=3, penalty_count=count))
-        buffer = np.zeros(100, np.int32)
-        s._staging_buffer = lambda n: (buffer, None, memoryview(buffer).cast("B"), buffer.ctypes.data)
-        starts, n, _, _ = s._pack(3, [0, 1, 2], [0, 0, 0], histories) or s._pack_in_python([0, 1, 2], [0, 0, 0], histories)
-        want = sum((h[-count:] if 0 < count < len(h) else h for h in histories), [])
-        assert buffer[starts[1]:n].tolist() == want, count
