@@ -2173,23 +2173,25 @@ def wide_tiles_serve_gated(M: int, N: int, K: int) -> bool:
 
 
 def library_serves(M: int, N: int, K: int, adds: bool = False) -> bool:
-    """Whether the library makes a plain product of M rows that wide_tiles_plan would take (adds: in the stream, before a norm).  Its kernels are
-    ahead by 5 to 20 % where a matrix is small, level or ahead by some percent where the rows are many, behind by 5 to 60 % where k is long or
-    the rows some hundred, and change by as much from one size to the next; the lines lie where 33 matrices of 65 to 16,384 rows changed sides on
-    average.  Product and what reads it, us, library / tiled.  In the stream: 2,048 rows [2,048, 2,048] 31.1 / 32.2, [4,096, 4,096] 75 / 82, 16,384
-    rows [4,096, 4,096] 507 / 576; 600 rows [5,120, 5,120] 58 / 54, 1,200 rows [4,096, 11,008] 129 / 110, 2,500 rows [4,096, 14,336] 250 / 239.  Read by
-    another kernel: 512 rows [2,048, 2,048] 15.9 / 18.4, [3,072, 2,048] 18.6 / 20.8; [7,168, 5,120] 300 rows 54 / 42, 2,048 148 / 155, 5,003 370 / 362;
-    [6,144, 4,096] 2,048 rows 107 / 117.  Never where a hand-written product has served all along: some hundred rows of matrices of 2,048 to 8,192
-    rows and k from 2,048 on, few rows of long matrices, what tiles_plan names."""
+    """Whether the library makes a plain product of M rows that wide_tiles_plan would take (adds: in the stream, before a norm). Its kernels
+    change by up to 60 % from one size to the next; the lines lie where 33 matrices of 65 to 16,384 rows changed sides on average. In the stream
+    the sum is in the library's epilogue at little cost, and it is ahead but for long k and, level there on the GPU but called in less time, for
+    some hundred rows of larger matrices (334 rows of eight layers with [4,096, 4,096]: 2,124 / 2,079); product and norm, us, library / tiled:
+    2,048 rows [2,048, 2,048] 31.1 / 32.2, [4,096, 4,096] 75 / 82, 16,384 rows [4,096, 4,096] 507 / 576; 600 rows [5,120, 5,120] 58 / 54, 1,200
+    rows [4,096, 11,008] 129 / 110, 2,500 rows [4,096, 14,336] 250 / 239. Elsewhere it is ahead for few rows of small matrices, whose product the
+    parts to add make longer (512 rows [1,536, 1,536] 9.5 / 9.1 in four); of 496 other sizes the tiled product took 0.90 of the library's time on
+    average and more than 1.05 at 20: 300 rows [7,168, 5,120] 49 / 32, 3,529 rows [4,096, 4,096] 98 / 93 (inside a model 115 / 103), 2,500 rows
+    [21,504, 4,096] 439 / 361, but 2,048 rows [6,144, 4,096] 81 / 89. Never where a hand-written product has served all along: some hundred rows
+    of matrices of 2,048 to 8,192 rows and k from 2,048 on, few rows of long matrices, what tiles_plan names."""
     if 2048 <= N <= 8192 and K >= 2048 and (M <= 256 or (M <= 1024 and K >= 2 * N)):
         return False
     if (M <= LDS_MAX_ROWS and K >= 2 * N) or tiles_plan(M, N, K) is not None:
         return False
     if adds and N > 8192:                                    # (parts of such rows take the norm longer than the product takes)
         return True
-    if (K >= 2.5 * N and M <= 1800) or (K >= 3 * N and M <= 3600) or (K >= 4608 and 4096 <= N <= 8192 and M <= 700):
+    if (K >= 2.5 * N and M <= 1800) or (K >= 3 * N and M <= 3600) or (N * K >= 1 << 23 and N <= 8192 and M <= 700):
         return False
-    return adds or K < 2560 or M > 700 or N * K < 1 << 23 or (M <= LDS_MAX_ROWS and N > 16384)
+    return adds or N * K < (1 << 23 if M < 300 else 1 << 22 if M < 1000 else 0) or (M <= LDS_MAX_ROWS and N > 16384)
 
 
 def prompt_parts(M: int, N: int, K: int, adds: bool = False) -> int:

@@ -1399,7 +1399,7 @@ def test_tiles_that_activate_their_product(M, N, K_):
 def test_wide_tiles_serve_prompts():
     """What prompt_parts chooses, through the general entry and added to the stream: one part in place, more parts left to the norm that
     adds them, none to the library; matrices and operands that it does not take go the way they went."""
-    for M, N, K_ in ((600, 3072, 3072), (2048, 4096, 14336), (300, 512, 4096), (700, 8320, 4096), (1100, 5120, 16384)):
+    for M, N, K_ in ((800, 3072, 3072), (2048, 4096, 14336), (300, 512, 4096), (700, 8320, 4096), (1100, 5120, 16384)):
         parts = K.prompt_parts(M, N, K_)
         a, w = torch.randn((M, K_), device=DEV).bfloat16(), (torch.randn((N, K_), device=DEV) * 0.05).bfloat16()
         pw, x0 = K.pack_weights(w), torch.randn((M, N), device=DEV)
