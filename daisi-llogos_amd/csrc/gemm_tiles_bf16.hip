@@ -21,10 +21,11 @@
 //  * Blocks are numbered so that the 32 that run on an XCD are about 8 x 4 neighbouring tiles (tiles_place).
 //  * Tiles of 64 to 256 tokens, blocks along k (float32 partial sums [parts][M][N] that the consumer adds), and the last round of blocks in tiles
 //    of half the height, by a cost fitted to measurements (tiles_choose).
-//  * Measured (us, weights from memory, the chip at its power limit; the tiles on eight waves of 32x32x16 products with both operands copied
-//    through registers -> these, the library between): 2,048 tokens, 28,672 x 4,096 with SwiGLU 407 (383) 353, 4,096 x 14,336 in two parts
-//    215 (200) 166, 4,096 x 4,096 70 (61) 61, 6,144 x 4,096 96 (80) 88; 5,003 tokens, 34,816 x 5,120 with SwiGLU 1,492 (1,571) 1,297,
-//    5,120 x 17,408 800 (1,030) 665; 334 tokens, 28,672 x 4,096 with SwiGLU 107 (90) 79.  8,192^3: 1.54 PFLOP/s random, 1.92 zeros.
+//  * Measured (us, weights from memory, in turn with other products; the tiles on eight waves of 32x32x16 products with both operands copied
+//    through registers -> these, the library between): 2,048 tokens, 28,672 x 4,096 with SwiGLU 407 (380) 362, 4,096 x 14,336 in two parts
+//    215 (217) 184, 4,096 x 4,096 70 (62) 63, 6,144 x 4,096 96 (81) 89; 5,003 tokens, 34,816 x 5,120 with SwiGLU 1,492 (1,541) 1,355,
+//    5,120 x 17,408 800 (1,044) 680; 300 tokens, 28,672 x 4,096 with SwiGLU (86) 73; 65 tokens, 4,096 x 14,336 in eight parts (49) 28.  8,192^3:
+//    1.54 PFLOP/s random, 1.92 zeros.
 //  * Epilogues: plain (+ bias) in bfloat16 or float32; added to a float32 result in place; SwiGLU for a matrix packed with gate_rows; the activations of
 //    two-matrix feed-forwards in bfloat16 (a float32 result and a kernel of its own took 50 us more a layer at 2,500 rows of 21,504 values:
 //    215 MB written and read; a pass of that prompt and 16 steps 25,113 -> 24,461 us).

@@ -2099,8 +2099,8 @@ TILES_MIN_ROWS, TILES_MAX_ROWS, TILES_MAX_K = 1024, 2048, 5120
 def tiles_serve_gated(M: int, K: int = 0) -> bool:
     """Whether the tiled product makes silu(gate) * up for M rows of K values (rather than the library's product and a SwiGLU pass)
     whatever the matrix's height: from TILES_MIN_ROWS to TILES_MAX_ROWS rows with k up to TILES_MAX_K.  Where the height is known
-    wide_tiles_serve_gated takes more.  us, library with SwiGLU pass / tiled: [28,672, 4,096] 1,000 rows 200 / 184, 2,048 383 / 353; [34,816, 5,120]
-    1,000 rows 393 / 300, 2,048 630 / 538; [16,384, 2,048] 2,048 rows 118 / 112."""
+    wide_tiles_serve_gated takes more.  us, library with SwiGLU pass / tiled: [28,672, 4,096] 1,000 rows 208 / 200, 2,048 380 / 362; [34,816, 5,120]
+    1,000 rows 404 / 314, 2,048 639 / 563; [16,384, 2,048] 2,048 rows 122 / 119."""
     if PROMPT_PRODUCT == "tiles":
         return True
     return PROMPT_PRODUCT == "auto" and TILES_MIN_ROWS <= M <= TILES_MAX_ROWS and K <= TILES_MAX_K
@@ -2110,7 +2110,8 @@ def tiles_plan(M: int, N: int, K: int) -> Optional[Tuple[int, int]]:
     """(parts of k, token_tiles) with which the tiled product serves a plain product of M rows, or None.  A matrix that
     is much longer than high (a feed-forward's down projection) with 129 to 1,024 rows of activations is where
     the library is furthest from its best, and blocks along k fill the compute units that its few row tiles leave idle ([5,120, 17,408],
-    200 rows: 137 us against 54).  For more rows see long_tiles_plan; where this plan has none, prompt_parts asks wide_tiles_plan."""
+    200 rows: 137 us against 54).  For more rows see long_tiles_plan.  What wide_tiles_plan takes comes in its parts; this plan serves the rest, says where
+    the library need not be asked (library_serves), and what adds itself to the stream in one part (gemm_tiles_add)."""
     if PROMPT_PRODUCT == "library" or M <= SKINNY_MAX_ROWS or K % 64:
         return None
     if PROMPT_PRODUCT == "tiles":
@@ -2167,8 +2168,9 @@ def wide_tiles_plan(M: int, N: int, K: int, n_cus: Optional[int] = None) -> int:
 def wide_tiles_serve_gated(M: int, N: int, K: int) -> bool:
     """Whether the tiled product makes silu(gate) * up of M rows with a packed matrix of N rows, beyond tiles_serve_gated: where the rows
     of w are enough for the compute units, which the gated product cannot share by parts of k.  us, library with SwiGLU pass / this:
-    [28,672, 4,096] 100 rows 56 / 63, 130 60 / 64, 200 72 / 67, 334 90 / 79; [16,384, 2,048] 200 rows 31.2 / 32.3, 334 36.6 / 33.8, 1,000 65 / 57;
-    [34,816, 5,120] 130 rows 104 / 91, 1,000 393 / 300, 5,003 1,571 / 1,297."""
+    [28,672, 4,096] 100 rows 56 / 55, 200 71 / 64, 300 86 / 73, 8,192 1,415 / 1,399; [16,384, 2,048] 300 rows 34.6 / 31.6, 1,000 68 / 61; [34,816, 5,120] 129 rows
+    104 / 92, 1,000 404 / 314, 5,003 1,541 / 1,355; [8,192, 4,608] 400 rows 49 / 50, 600 59 / 54; [4,096, 768] 1,200 rows 20 / 15.  Of 15 matrices' sizes it is
+    behind by more than 5 % at two ([8,192, 4,608], 512 rows, [57,344, 8,192], 16,384)."""
     return PROMPT_PRODUCT == "auto" and M > SKINNY_MAX_ROWS and K % 64 == 0 and K >= 512 and M * N >= 1 << 22
 
 
