@@ -1441,7 +1441,7 @@ def test_short_tiled_product_serves_prompts_of_some_hundred_rows():
 
 @pytest.mark.parametrize("M,N,K_", [(129, 2048, 2048), (200, 4096, 4096), (256, 3072, 2112)])
 def test_products_that_no_norm_follows_are_added_by_the_library(M, N, K_):
-    """Where short tiles would leave parts for a norm to add and none follows, the library's product adds itself to the stream: the
+    """Where the tiled product would leave parts for a norm to add and none follows, the library's product adds itself to the stream: the
     float32 product added to x, bit for bit; with a norm behind it, and up to 128 rows, it does not and x stays as it was."""
     base = importlib.import_module("daisi-llogos_amd.parts.base")
     parts = importlib.import_module("daisi-llogos_amd.parts")
