@@ -517,3 +517,28 @@ def test_the_command_line_on_a_model_of_the_design(tmp_path):
     p = run("--model", str(out), "--bench", "--batch", "2", "-n", "8", "--prompt-len", "20", "--max-context", "64")
     assert p.returncode == 0, p.stderr[-2000:]
     assert "decode" in (p.stdout + p.stderr)
+
+
+def test_engines_with_some_experts_packed(monkeypatch):
+    """Memory for the copies of none, the first and all experts' matrices: a prompt and single tokens behind it give the plain logits, whichever copy
+    a layer's products read."""
+    moe = importlib.import_module("daisi-llogos_amd.parts.moe")
+    pack, name = moe._packed, "zog_c"
+    toks = H.tokens(name, 90, 11)
+    want = H.plain_logits(name, toks)
+    counts = []
+    for most in (0, 1, 2, 100):
+        held = []
+
+        def some(w, rt):
+            copy = pack(w, rt) if len(held) < most else None
+            held.extend([copy] if copy is not None else [])
+            return copy
+        monkeypatch.setattr(moe, "_packed", some)
+        eng = H.engine(name, "bfloat16")
+        counts.append(len(held))
+        slot = eng.alloc_slot()
+        H.close(_np(eng.step([(slot, list(toks[:80]))], want="all")), want[:80], "bfloat16", f"{len(held)} copies, prompt")
+        for i in range(80, 90):
+            H.close(_np(eng.step([(slot, [toks[i]])], want="last"))[0], want[i], "bfloat16", f"{len(held)} copies, token {i}")
+    assert counts == [0, 1, 2, 3]
