@@ -113,7 +113,19 @@ __global__ __launch_bounds__(WAVES * kWave) void gemm_residual_kernel(
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
     };
+    // What the sums are added to: asked for behind the first weights, there long before it is needed.
+    constexpr int kCols = HALF ? 8 : 16;                 // columns of x a strip of this block
+    const int m = threadIdx.x / kCols, c = threadIdx.x % kCols;
+    float x_old[RB], b_old[RB], nw[RB];
     if (s_begin < s_end) fetch(0, s_begin);
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+        const int n = HALF ? blockIdx.x * 8 + c : (strip0 + rb) * 16 + c;
+        const bool in = m < M && n < N;
+        x_old[rb] = in ? x[(size_t)m * ldx + n] : 0.f;
+        b_old[rb] = in && bias ? bias[n] : 0.f;
+        nw[rb] = in && unscaled ? norm_w[n] : 0.f;
+    }
     for (int s = s_begin; s < s_end; s += 2 * AHEAD) {
         if (s + AHEAD < s_end) fetch(1, s + AHEAD);
         multiply(0);
@@ -128,9 +140,7 @@ __global__ __launch_bounds__(WAVES * kWave) void gemm_residual_kernel(
 #pragma unroll
         for (int i = 0; i < 4; ++i) red[wave][rb][i][lane] = acc[rb][i];
     __syncthreads();
-    constexpr int kCols = HALF ? 8 : 16;                 // columns of x a strip of this block
     if (threadIdx.x >= kResidualRows * kCols) return;
-    const int m = threadIdx.x / kCols, c = threadIdx.x % kCols;
     const int src_lane = (c >> 2) * 16 + m, i = c & 3;
     float sq = 0.f;                                      // of this thread's row over the block's columns
 #pragma unroll
@@ -145,11 +155,10 @@ __global__ __launch_bounds__(WAVES * kWave) void gemm_residual_kernel(
         if (HALF) v += w2;
         const int n = HALF ? blockIdx.x * 8 + c : (strip0 + rb) * 16 + c;
         if (m < M && n < N) {
-            float* xp = x + (size_t)m * ldx + n;
-            const float y = *xp + (v + (bias ? bias[n] : 0.f));
-            *xp = y;
+            const float y = x_old[rb] + (v + b_old[rb]);
+            x[(size_t)m * ldx + n] = y;
             sq += y * y;
-            if (unscaled) unscaled[(size_t)m * ldu + n] = f32_to_bf16(y * norm_w[n]);
+            if (unscaled) unscaled[(size_t)m * ldu + n] = f32_to_bf16(y * nw[rb]);
         }
     }
     // the lanes of a row are neighbours: a fixed tree of additions
