@@ -115,14 +115,17 @@ struct PenaltyParams {
 // The tokens of the window h[0 .. n) that lie in first .. first + count - 1 are made again from the logits, penalty first,
 // then the scale, and put to w[token - first].  A round's threads look at a position of the window each and list those
 // that name such a token; a wave takes a listed position and reads the window 64 tokens at a time: a token's first occurrence
-// does the work.  (One thread a position, reading the window token by token, made this 11 us of a slice's 16.)
+// does the work.  (One thread a position, reading the window token by token, made this 11 us of a slice's 16.)  put(q, place, value) takes
+// the new value of a round's listed position q (place -1: an earlier position names the token), round() ends a round.
 struct WindowLds {
     int n;
     int at[kSampleThreads];
 };
 
-__device__ __forceinline__ void apply_penalties(float* w, const float* __restrict__ row, int first, int count, int V,
-                                                const int* __restrict__ h, int n, const PenaltyParams& pp, WindowLds& lds) {
+// near: h as far as it is kept nearer (LDS), or h itself.
+template <typename Near, typename Put, typename Round>
+__device__ __forceinline__ void apply_penalties(const float* __restrict__ row, int first, int count, int V, const int* __restrict__ h, Near near, int n,
+                                                const PenaltyParams& pp, WindowLds& lds, Put put, Round round) {
     const float inv_t = pp.inv_temperature;
     const bool scaled = inv_t != 1.0f;
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave, waves = blockDim.x / kWave;
@@ -131,21 +134,22 @@ __device__ __forceinline__ void apply_penalties(float* w, const float* __restric
         if (threadIdx.x == 0) lds.n = 0;
         __syncthreads();
         if (i0 + (int)threadIdx.x < n) {
-            const int tok = h[i0 + threadIdx.x];
+            const int tok = near(i0 + threadIdx.x);
             if (tok >= first && tok - first < count && tok < V && (pp.penalize_newline || (tok != 10 && tok != 13)))
                 lds.at[atomicAdd(&lds.n, 1)] = i0 + threadIdx.x;
         }
         __syncthreads();
         for (int q = wave; q < lds.n; q += waves) {
-            const int i = lds.at[q], tok = h[i];
+            const int i = lds.at[q], tok = near(i);
             int times = 0;
             for (int j0 = 0; j0 < n; j0 += kWave) {
-                const uint64_t same = __ballot(j0 + lane < n && h[j0 + lane] == tok);
+                const uint64_t same = __ballot(j0 + lane < n && near(j0 + lane) == tok);
                 const uint64_t later = j0 >= i ? ~(uint64_t)0 : i - j0 >= kWave ? 0 : ~(uint64_t)0 << (i - j0);
                 if (same & ~later) { times = 0; break; }             // an earlier position names it too
                 times += (int)__popcll(same & later);
             }
-            if (lane != 0 || times == 0) continue;
+            if (lane != 0) continue;
+            if (times == 0) { put(q, -1, 0.f); continue; }
             float l = row[tok];
             if (pp.repetition != 1.0f)
                 for (int c = 0; c < times; ++c) l = l > 0.f ? l / pp.repetition : l * pp.repetition;
@@ -153,8 +157,9 @@ __device__ __forceinline__ void apply_penalties(float* w, const float* __restric
                 l -= pp.frequency * (float)times;
                 l -= pp.presence;
             }
-            w[tok - first] = scaled ? l * inv_t : l;
+            put(q, tok - first, scaled ? l * inv_t : l);
         }
+        round();
     }
 }
 
@@ -170,7 +175,7 @@ __device__ void prepare_row(float* w, const float* __restrict__ row, int V, cons
     for_each_value(row, V, [&](int i, float x) { w[i] = scaled ? x * inv_t : x; });
     __syncthreads();
     if (has_penalties(pp) && h) {
-        apply_penalties(w, row, 0, V, V, h, n, pp, lds);
+        apply_penalties(row, 0, V, V, h, [&](int i) { return h[i]; }, n, pp, lds, [&](int, int place, float x) { if (place >= 0) w[place] = x; }, [] {});
         __syncthreads();
     }
     if (threadIdx.x < pp.n_banned) {
@@ -520,14 +525,12 @@ __global__ __launch_bounds__(kSampleThreads) void sample_pipeline_kernel(
 //
 // One block a row (the kernels above: a pass that prepares the row, then three that look for its head) left three quarters of
 // the compute units idle at 64 rows and moved each row five times.  Here a block takes a slice of a row, prepares it in
-// registers (the tokens that penalties touch are patched through LDS) and keeps what may be among the row's first top-k:
-// every value in the slice's first bins, by the same histogram of the distance to the largest that sorted_head uses, but the
-// slice's own largest.  A second kernel, one block a row, cuts the slices' lists (some tens of keys each) the same way against
+// registers and keeps what may be among the row's first top-k (sample_slices_kernel).  A second kernel, one block a row, cuts the slices' lists (some tens of keys each) the same way against
 // the row's largest, sorts what is left and draws.  Up to 64 candidates one wave does steps 2 to 6 without a barrier; its sums
 // are the additions of the block's in the same order.  Whatever these lists cannot decide (an infinite value, thousands of
 // values within a bin) is done again by the row's block in the general way.
-// 64 rows of 128,256 logits, top-k 40, penalties: 76 us in the two kernels above, 31 here (one row: 65 and 18;
-// top-k 256: 87 and 39).  Twice or four times as many, shorter slices at 64 rows: 35 and 42 us.
+// 64 rows of 128,256 logits, top-k 40, penalties: 76 us in the two kernels above, 22 here (14.3 + 7.6).  Twice or four times as many,
+// shorter slices at 64 rows took 4 and 11 us more.
 constexpr int kFewCandidates = 256;      // largest top-k served
 constexpr int kSliceThreads = 512;
 constexpr int kSliceCap = 1024;          // keys a slice can hand on
@@ -577,21 +580,31 @@ __device__ int cut_bin(const int* bins, int want, int* part, int* cut, int* tota
 
 // grid (slices, rows).  VPT values a thread.  counts, tops: [rows][slices]; keys: [rows][slices][kSliceCap].  count -1: more
 // than kSliceCap keys, or a largest value that is not finite.  hist_at (or null): row r's window is hist[hist_at[r] .. hist_at[r + 1]).
+//
+// A block is a chain of short steps that wait, so all of a launch's blocks are to be on the units at once: 64 registers let 4 in.  A
+// slice's list is cut without bins: a wave sorts its threads' own largest values and offers the (top_k / 8)-th (rounded up); the largest of
+// the eight that top_k threads' values reach (the least one in any case) cuts the list, which a tenth to a half more than top_k values pass.  64 rows of 128,256 logits 14.3 us.  (22.5 with the slice's values patched in LDS, 97
+// registers, two rounds of blocks and the top_k-th of all threads' largest values found by counting them in bins: the additions to the few
+// bins that they share, 1.9 us alone, took 5.3 with four blocks on a unit, and a bin for each value before it is listed 4.3.)
 template <int VPT>
-__global__ __launch_bounds__(kSliceThreads) void sample_slices_kernel(
+__global__ __launch_bounds__(kSliceThreads) __attribute__((amdgpu_waves_per_eu(8)))
+void sample_slices_kernel(
         uint64_t* __restrict__ keys, int* __restrict__ counts, float* __restrict__ tops, const float* __restrict__ logits, int V,
         const int* __restrict__ hist, const int* __restrict__ hist_at, PenaltyParams pp, int top_k) {
-    constexpr int kSlice = VPT * kSliceThreads;
-    constexpr int kLds = kSlice > kHeadBins ? kSlice : kHeadBins;
-    __shared__ __attribute__((aligned(16))) int lds[kLds];        // the slice's values while they are patched, then the bins
-    __shared__ float red[16];
-    __shared__ int part[16], cut[2], counter;
+    constexpr int kSlice = VPT * kSliceThreads, kWaves = kSliceThreads / kWave;
+    __shared__ int lds[kHeadBins];                                // the window's tokens, then (where all values are counted) bins
+    __shared__ int reached[kWaves][kWaves];
+    __shared__ float wave_top[kWaves], wave_least[kWaves], patch[kSliceThreads];
+    __shared__ int part[16], cut[2], counter, patch_at[kSliceThreads];
     __shared__ WindowLds window;
     const int s = blockIdx.x, r = blockIdx.y, at = r * gridDim.x + s;
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const float* row = logits + (size_t)r * V;
     const int first = s * kSlice, count = min(kSlice, V - first);
     const float inv_t = pp.inv_temperature;
-    const bool scaled = inv_t != 1.0f;
+    const bool scaled = inv_t != 1.0f, penalties = has_penalties(pp) && hist_at != nullptr;
+    const int* h = penalties ? hist + hist_at[r] : nullptr;
+    const int n_hist = penalties ? hist_at[r + 1] - hist_at[r] : 0;
     const bool wide = (V & 3) == 0 && ((uintptr_t)logits & 15) == 0;   // then four neighbours a load, else threads side by side
     auto place = [&](int j) { return wide ? ((j >> 2) * kSliceThreads + threadIdx.x) * 4 + (j & 3) : j * kSliceThreads + (int)threadIdx.x; };
     float v[VPT];
@@ -607,82 +620,110 @@ __global__ __launch_bounds__(kSliceThreads) void sample_slices_kernel(
 #pragma unroll
         for (int j = 0; j < VPT; ++j) v[j] = place(j) < count ? row[first + place(j)] : -INFINITY;
     }
+    for (int i = threadIdx.x; i < min(n_hist, kHeadBins); i += kSliceThreads) lds[i] = h[i];
+    if (threadIdx.x == 0) counter = 0;
 #pragma unroll
     for (int j = 0; j < VPT; ++j) v[j] = scaled ? v[j] * inv_t : v[j];
-    const bool penalties = has_penalties(pp) && hist_at != nullptr;
-    if (penalties || pp.n_banned > 0) {
-        float* vals = reinterpret_cast<float*>(lds);
-        if (wide) {
+    // a new value for the slice's value i: the thread that holds it takes it
+    auto take = [&](int i, float x) {
+        const int n = wide ? i >> 2 : i;
+        if (n % kSliceThreads != (int)threadIdx.x) return;
+        const int mine = wide ? n / kSliceThreads * 4 + (i & 3) : n / kSliceThreads;
 #pragma unroll
-            for (int j = 0; j < VPT; j += 4) *reinterpret_cast<float4*>(vals + place(j)) = make_float4(v[j], v[j + 1], v[j + 2], v[j + 3]);
-        } else {
-#pragma unroll
-            for (int j = 0; j < VPT; ++j) vals[place(j)] = v[j];
-        }
-        if (penalties) {
-            apply_penalties(vals, row, first, count, V, hist + hist_at[r], hist_at[r + 1] - hist_at[r], pp, window);
-        }
-        __syncthreads();
-        if (threadIdx.x < pp.n_banned) {
-            const int tok = pp.banned[threadIdx.x] - first;
-            if (tok >= 0 && tok < count) vals[tok] = -INFINITY;
-        }
-        __syncthreads();
-        if (wide) {
-#pragma unroll
-            for (int j = 0; j < VPT; j += 4) {
-                const float4 t = *reinterpret_cast<const float4*>(vals + place(j));
-                v[j] = t.x; v[j + 1] = t.y; v[j + 2] = t.z; v[j + 3] = t.w;
-            }
-        } else {
-#pragma unroll
-            for (int j = 0; j < VPT; ++j) v[j] = vals[place(j)];
-        }
+        for (int j = 0; j < VPT; ++j) v[j] = j == mine ? x : v[j];
+    };
+    if (penalties) {
+        apply_penalties(row, first, count, V, h, [&](int i) { return i < kHeadBins ? lds[i] : h[i]; }, n_hist, pp, window,
+                        [&](int q, int i, float x) { patch_at[q] = i; patch[q] = x; },
+                        [&] {
+                            __syncthreads();
+                            for (int q = 0; q < window.n; ++q)
+                                if (patch_at[q] >= 0) take(patch_at[q], patch[q]);
+                        });
+    }
+    for (int i = 0; i < pp.n_banned; ++i) {
+        const int tok = pp.banned[i] - first;
+        if (tok >= 0 && tok < count) take(tok, -INFINITY);
     }
     float m = -INFINITY;
 #pragma unroll
     for (int j = 0; j < VPT; ++j) m = fmaxf(m, v[j]);              // (places past the slice hold -inf)
-    const float top = block_max(m, red);
+    // the wave's 64 largest values of a thread in falling order (bitonic): lane l has the l-th
+    float sorted = m;
+#pragma unroll
+    for (int size = 2; size <= kWave; size <<= 1)
+#pragma unroll
+        for (int o = size >> 1; o > 0; o >>= 1) {
+            const float other = __shfl_xor(sorted, o, kWave);
+            const bool larger = ((lane & o) == 0) == ((lane & size) == 0);
+            sorted = larger ? fmaxf(sorted, other) : fminf(sorted, other);
+        }
+    // (waves whose threads all have values; the others' values are listed like any)
+    const int full = min(kWaves, (wide ? count >> 2 : count) / kWave), share = full > 0 ? (top_k + full - 1) / full : kWave + 1;
+    if (lane == 0) wave_top[wave] = sorted;
+    if (lane == min(share, kWave) - 1) wave_least[wave] = wave < full && share <= kWave ? sorted : -INFINITY;
+    __syncthreads();
+    float top = wave_top[0];
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) top = fmaxf(top, wave_top[w]);
+    // the largest of the waves' that top_k threads' largest values reach: their least one in any case
+    {
+        int reach = 0;                                            // lane w: how many of this wave's reach wave w's
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) {
+            const int n = (int)__popcll(__ballot(m >= wave_least[w]));
+            reach = lane == w ? n : reach;
+        }
+        if (lane < kWaves) reached[wave][lane] = reach;
+    }
+    __syncthreads();
+    float least = -INFINITY;
+    if (lane < kWaves) {
+        int n = 0;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) n += reached[w][lane];
+        if (n >= top_k) least = wave_least[lane];
+    }
+    least = wave_max(least);
     if (!(top > -INFINITY && top < INFINITY)) {
         if (threadIdx.x == 0) { counts[at] = top < INFINITY ? 0 : -1; tops[at] = top; }
         return;
     }
-    // The top_k largest of the threads' own largest values bound the slice's top_k from below: counting those alone (a
-    // sixteenth of the values) cuts the slice nearly as short.  Where fewer than top_k threads hold a value that counts, or the
-    // list would overflow, all values are counted.
-    bool fits = false;
-    int total = 0;
-#pragma unroll 1
-    for (int all = 0; all < 2 && !fits; ++all) {
-        __syncthreads();
-        for (int i = threadIdx.x; i < kHeadBins; i += kSliceThreads) lds[i] = 0;
-        if (threadIdx.x == 0) counter = 0;
-        __syncthreads();
-        if (all) {
-#pragma unroll
-            for (int j = 0; j < VPT; ++j) {
-                const int b = head_bin(top, v[j]);
-                if (b < kHeadBins - 1) atomicAdd(&lds[b], 1);
-            }
-        } else {
-            const int b = head_bin(top, m);
-            if (b < kHeadBins - 1) atomicAdd(&lds[b], 1);
-        }
-        __syncthreads();
-        int outside;
-        const int last = cut_bin<kSliceThreads>(lds, top_k, part, cut, &total, &outside);
-        if (all ? total > kSliceCap : outside < top_k) continue;
+    auto list = [&](int j) {
+        const int slot = atomicAdd(&counter, 1);
+        if (slot < kSliceCap) keys[(size_t)at * kSliceCap + slot] = desc_key(v[j], first + place(j));
+    };
+    if (least > -INFINITY) {
 #pragma unroll
         for (int j = 0; j < VPT; ++j)
-            if (head_bin(top, v[j]) <= last) {
-                const int slot = atomicAdd(&counter, 1);
-                if (slot < kSliceCap) keys[(size_t)at * kSliceCap + slot] = desc_key(v[j], first + place(j));
-            }
+            if (v[j] >= least) list(j);
         __syncthreads();
-        total = counter;
-        fits = total <= kSliceCap;
+        if (counter <= kSliceCap) {
+            if (threadIdx.x == 0) { counts[at] = counter; tops[at] = top; }
+            return;
+        }
     }
-    if (threadIdx.x == 0) { counts[at] = fits ? total : -1; tops[at] = top; }
+    // Where a wave has fewer threads with a value than that, or the list would overflow: all values by the distance to the largest.
+    __syncthreads();
+    for (int i = threadIdx.x; i < kHeadBins; i += kSliceThreads) lds[i] = 0;
+    if (threadIdx.x == 0) counter = 0;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) {
+        const int b = head_bin(top, v[j]);
+        if (b < kHeadBins - 1) atomicAdd(&lds[b], 1);
+    }
+    __syncthreads();
+    int total, outside;
+    const int last = cut_bin<kSliceThreads>(lds, top_k, part, cut, &total, &outside);
+    const bool fits = total <= kSliceCap;
+    if (fits) {
+#pragma unroll
+        for (int j = 0; j < VPT; ++j)
+            if (head_bin(top, v[j]) <= last) list(j);
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) { counts[at] = fits ? counter : -1; tops[at] = top; }
 }
 
 __device__ __forceinline__ float key_value(uint64_t k) {            // of a desc_key (-0 comes back as 0)

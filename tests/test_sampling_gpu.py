@@ -415,3 +415,28 @@ def test_few_candidates_draw_what_the_general_way_draws(R, V, opts):
                                     p.penalize_newline, stop)
             want = K.sample_pipeline(work, us, p.top_k, p.top_p, p.min_p, p.typical_p, p.min_keep)
             assert got.cpu().tolist() == want.cpu().tolist(), (at, step)
+
+
+@pytest.mark.parametrize("n", [511, 513, 2047, 2049, 5000])
+def test_few_candidates_with_windows_of_every_length(n):
+    """A slice's block holds a window's first 2,048 tokens itself and lists the positions of 512 at a time: windows around both, with
+    tokens that come back on either side, draw what the general way draws."""
+    K = importlib.import_module("daisi-llogos_amd.ops.kernels")
+    R, V = 3, 32000
+    rng = np.random.default_rng(n)
+    p = S.GenerationParams(seed=9, temperature=0.9, top_k=40, top_p=1.0, repetition_penalty=1.3, frequency_penalty=0.2, presence_penalty=0.1, penalty_count=0)
+    x = rng.standard_normal((R, V)).astype(np.float32)
+    top = np.argsort(-x, axis=1)[:, :30]
+    histories = [rng.integers(0, V, size=n).tolist() for _ in range(R)]
+    for r in range(R):                                     # the likeliest tokens, at the window's two ends and in its middle
+        for i, tok in enumerate(top[r]):
+            for at in (i, n // 2 + i, n - 1 - i):
+                histories[r][at] = int(tok)
+    logits = torch.tensor(x, device=DEV)
+    padded = torch.tensor(np.array(histories, np.int32), device=DEV)
+    work = K.sample_prepare(logits, padded, torch.full((R,), n, dtype=torch.int32, device=DEV), p.repetition_penalty, p.frequency_penalty,
+                            p.presence_penalty, p.temperature, p.penalize_newline, ())
+    for step in range(4):
+        us = torch.tensor(S.Sampler(p).uniforms(list(range(R)), [step] * R), dtype=torch.float32, device=DEV)
+        want = K.sample_pipeline(work, us, p.top_k, p.top_p, p.min_p, p.typical_p, p.min_keep)
+        assert S.Sampler(p).sample(logits, list(range(R)), [step] * R, histories).cpu().tolist() == want.cpu().tolist()
