@@ -1044,3 +1044,46 @@ LLOGOS_EXPORT int llogos_sample_few(int* out, const float* logits, int R, int V,
                                                         work, prob, (uint64_t*)list, n_pad, uniforms, sp);
     return LLOGOS_LAUNCH_CHECK();
 }
+
+// A sampler's settings, as its calls share them.
+struct SampleSettings {
+    float repetition, frequency, presence, inv_temperature, top_p, min_p, typical_p;
+    int penalize_newline, top_k, min_keep, n_banned;
+    int banned[kMaxBanned];
+};
+
+// 8-byte words of scratch memory for llogos_sample_few_staged beside the staged numbers; 0 where it does not serve
+LLOGOS_EXPORT long long llogos_sample_few_words(int R, int V, int top_k) {
+    const long long slices = llogos_sample_few_slices(R, V, top_k);
+    if (slices == 0) return 0;
+    long long n_pad = 1;
+    while (n_pad < V) n_pad *= 2;
+    return R * slices * kSliceCap + R * n_pad + (long long)R * V + R * slices;
+}
+
+// llogos_sample_few from what the host has packed into pinned memory: R uniform numbers (float32) and, with `windows`, the R + 1 places of the
+// rows' windows and the windows, `staged` 32-bit numbers in all.  They are copied behind the scratch (16-byte aligned: llogos_sample_few_words words, then
+// `staged` numbers), `copied` (an event or null) is recorded behind the copy, and the two kernels follow: one call for what a step of
+// the sampler queues.
+LLOGOS_EXPORT int llogos_sample_few_staged(int* out, const float* logits, int R, int V, const void* host, long long staged, int windows,
+                                           const void* settings, void* scratch, void* copied, hipStream_t stream) {
+    const SampleSettings* s = (const SampleSettings*)settings;
+    if (s == nullptr || host == nullptr || scratch == nullptr || staged < R + (windows ? R + 1 : 0)) return LLOGOS_BAD_ARGUMENT;
+    const long long slices = llogos_sample_few_slices(R, V, s->top_k), words = llogos_sample_few_words(R, V, s->top_k);
+    if (words == 0) return LLOGOS_BAD_ARGUMENT;
+    long long n_pad = 1;
+    while (n_pad < V) n_pad *= 2;
+    uint64_t* keys = (uint64_t*)scratch;
+    uint64_t* list = keys + R * slices * kSliceCap;
+    float* work = (float*)(list + R * n_pad);
+    float* prob = work + (size_t)R * V;
+    int* counts = (int*)(prob + (size_t)R * V);
+    float* tops = (float*)(counts + R * slices);
+    int* numbers = (int*)(keys + words);
+    hipError_t e = hipMemcpyAsync(numbers, host, (size_t)staged * 4, hipMemcpyHostToDevice, stream);
+    if (e == hipSuccess && copied != nullptr) e = hipEventRecord((hipEvent_t)copied, stream);
+    if (e != hipSuccess) return (int)e;
+    return llogos_sample_few(out, logits, R, V, windows ? numbers + 2 * R + 1 : nullptr, windows ? numbers + R : nullptr, s->repetition, s->frequency,
+                             s->presence, s->inv_temperature, s->penalize_newline, s->banned, s->n_banned, keys, counts, tops, work, prob, list,
+                             (int)n_pad, (const float*)numbers, s->top_k, s->top_p, s->min_p, s->typical_p, s->min_keep, stream);
+}

@@ -2812,7 +2812,40 @@ def sample_pipeline(work: torch.Tensor, uniforms: torch.Tensor, top_k: int, top_
 
 def sample_few_serves(R: int, V: int, top_k: int) -> bool:
     """Whether sample_few takes rows of V logits of which at most top_k tokens can be drawn."""
-    return _lib().llogos_sample_few_slices(R, V, int(top_k)) > 0
+    return _sample_few_words(R, V, int(top_k)) > 0
+
+
+@functools.lru_cache(maxsize=256)
+def _sample_few_words(R: int, V: int, top_k: int) -> int:
+    return _lib().llogos_sample_few_words(R, V, top_k)
+
+
+class SampleSettings(ctypes.Structure):
+    """A sampler's settings as sample_few_staged takes them."""
+    _fields_ = [(n, ctypes.c_float) for n in ("repetition", "frequency", "presence", "inv_temperature", "top_p", "min_p", "typical_p")] + \
+               [(n, ctypes.c_int) for n in ("penalize_newline", "top_k", "min_keep", "n_banned")] + [("banned", ctypes.c_int * MAX_BANNED)]
+
+
+def sample_settings(repetition: float, frequency: float, presence: float, temperature: float, penalize_newline: bool, banned: Sequence[int],
+                    top_k: int, top_p: float, min_p: float, typical_p: float, min_keep: int) -> SampleSettings:
+    _need(len(banned) <= MAX_BANNED, f"sample_few: at most {MAX_BANNED} banned ids, got {len(banned)}")
+    return SampleSettings(repetition, frequency, presence, 1.0 / temperature if temperature > 0 else 1.0, top_p, min_p, typical_p,
+                          int(penalize_newline), int(top_k), int(min_keep), len(banned), (ctypes.c_int * MAX_BANNED)(*banned))
+
+
+def sample_few_staged(logits: torch.Tensor, host: int, staged: int, windows: bool, settings: SampleSettings, copied: int) -> torch.Tensor:
+    """sample_few on numbers in pinned host memory at the address `host`: the rows' uniform numbers and, with `windows`, the places of
+    their windows and the windows, `staged` 32-bit numbers in all.  The event `copied` (its handle) is recorded behind their copy."""
+    _dev(logits)
+    _need(logits.dtype == torch.float32 and logits.dim() == 2, "sample_few: logits must be contiguous float32 [R, V]")
+    R, V = logits.shape
+    words = _sample_few_words(R, V, settings.top_k)
+    _need(words > 0, f"sample_few: top_k {settings.top_k} of {V} is not served")
+    scratch = torch.empty(words + (staged + 1) // 2, dtype=torch.int64, device=logits.device)
+    out = torch.empty((R,), dtype=torch.int32, device=logits.device)
+    _check(_lib().llogos_sample_few_staged(out.data_ptr(), logits.data_ptr(), R, V, host, staged, windows, ctypes.addressof(settings),
+                                           scratch.data_ptr(), copied, _stream()), "sample_few")
+    return out
 
 
 def sample_few(logits: torch.Tensor, history: Optional[torch.Tensor], history_at: Optional[torch.Tensor], repetition: float,

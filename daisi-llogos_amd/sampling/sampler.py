@@ -5,6 +5,7 @@ penalties, temperature, top-k, min-p, softmax over candidates, typical-p, top-p,
 from __future__ import annotations
 
 import struct
+import weakref
 from typing import List, Optional, Sequence
 
 import numpy as np
@@ -15,7 +16,19 @@ from .params import GenerationParams
 from .rng import uniforms
 
 
+# Staging buffers that nobody fills any more, until their last copies have run: those are queued by the kernel library, so that torch
+# would hand freed pinned memory out again while one still reads it.
+_retired: List[tuple] = []
+
+
+def _retire(places: dict) -> None:
+    _retired[:] = [p for p in _retired + list(places.values()) if not p[1].query()]
+
+
 class Sampler:
+    _settings = _settings_of = None         # as the kernels take them, and of which parameters and banned tokens they were made
+    _staging, _staging_next = None, 0       # number -> staging buffer, its event, its bytes and its address; the number used last
+
     def __init__(self, params: GenerationParams, stop_tokens: Sequence[int] = ()):
         self.params = params
         self.stop_tokens = tuple(stop_tokens)
@@ -66,6 +79,14 @@ class Sampler:
         R = logits.shape[0]
         # one copy: uniform numbers, then each window's place and the windows, packed straight into the staging buffer
         starts, n, host, copied = self._pack(R, requests, indices, histories) or self._pack_in_python(requests, indices, histories)
+        if logits.device.index == torch.cuda.current_device() and starts == (R, 2 * R + 1 if p.has_penalties else R + 1):
+            banned = self.stop_tokens if p.prevent_eos else ()
+            key = (p, banned)
+            if self._settings_of != key:
+                self._settings = K.sample_settings(p.repetition_penalty, p.frequency_penalty, p.presence_penalty, p.temperature, p.penalize_newline,
+                                                   banned, p.top_k, p.top_p, p.min_p, p.typical_p, p.min_keep)
+                self._settings_of = key
+            return K.sample_few_staged(logits, host.data_ptr(), n, p.has_penalties, self._settings, copied.cuda_event)
         dev = torch.empty(n, dtype=torch.int32, device=logits.device)
         dev.copy_(host[:n], non_blocking=True)
         copied.record(torch.cuda.current_stream(logits.device.index))    # (named by its number, which is quicker than finding the current device)
@@ -118,13 +139,18 @@ class Sampler:
     def _staging_buffer(self, n: int):
         """A pinned buffer of at least n 32-bit numbers, the event to record behind its copy, its memory as bytes and its address: one of a
         few, each free again once its last copy has run."""
-        ring = getattr(self, "_staging", None)
-        if ring is None or ring[0][0].numel() < n:
-            hosts = [torch.empty(max(1024, 2 * n), dtype=torch.int32, pin_memory=True) for _ in range(4)]
-            ring = self._staging = [(h, torch.cuda.Event(), memoryview(h.numpy()).cast("B"), h.data_ptr()) for h in hosts]
-            self._staging_next = 0
-        place = ring[self._staging_next]
-        self._staging_next = (self._staging_next + 1) % len(ring)
+        at = self._staging_next = (self._staging_next + 1) % 4
+        place = self._staging.get(at) if self._staging is not None else None
+        if place is None or place[0].numel() < n:
+            if self._staging is None:
+                self._staging = {}
+                weakref.finalize(self, _retire, self._staging)
+            elif place is not None:
+                _retire({at: place})
+            host = torch.empty(max(1024, 2 * n), dtype=torch.int32, pin_memory=True)
+            place = self._staging[at] = (host, torch.cuda.Event(), memoryview(host.numpy()).cast("B"), host.data_ptr())
+            place[1].record()                                    # (an event has no handle before it is recorded once)
+            return place
         place[1].synchronize()
         return place
 

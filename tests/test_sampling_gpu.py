@@ -440,3 +440,26 @@ def test_few_candidates_with_windows_of_every_length(n):
         us = torch.tensor(S.Sampler(p).uniforms(list(range(R)), [step] * R), dtype=torch.float32, device=DEV)
         want = K.sample_pipeline(work, us, p.top_k, p.top_p, p.min_p, p.typical_p, p.min_keep)
         assert S.Sampler(p).sample(logits, list(range(R)), [step] * R, histories).cpu().tolist() == want.cpu().tolist()
+
+
+def test_samplers_that_end_before_their_copies():
+    """Numbers are staged in pinned memory and copied by the kernel library; a sampler that is dropped, or that needs longer buffers, while
+    the stream is still busy leaves them to the copies that are queued."""
+    R, V = 5, 5000
+    rng = np.random.default_rng(4)
+    logits = torch.tensor(rng.standard_normal((R, V)).astype(np.float32), device=DEV)
+    p = S.GenerationParams(seed=2, temperature=1.0, top_k=50, top_p=1.0, repetition_penalty=1.5, penalty_count=0)
+    long = [rng.integers(0, V, size=4000).tolist() for _ in range(R)]
+    calls = [(step, long if step % 3 == 2 else [h[:50 + step] for h in long]) for step in range(24)]
+    want = [S.Sampler(p).sample(logits, list(range(R)), [s] * R, h).cpu().tolist() for s, h in calls]
+    busy = torch.randn(4096, 4096, device=DEV)
+    one = S.Sampler(p)
+    for keep in (True, False):
+        torch.cuda.synchronize()
+        for _ in range(20):
+            busy = torch.tanh(busy @ busy)                 # the stream is behind
+        got = []
+        for s, h in calls:
+            got.append((one if keep else S.Sampler(p)).sample(logits, list(range(R)), [s] * R, h))
+            torch.full((12000,), 7, dtype=torch.int32, pin_memory=True)        # (would land in memory that was given back too early)
+        assert [t.cpu().tolist() for t in got] == want
