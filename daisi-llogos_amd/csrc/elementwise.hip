@@ -326,6 +326,78 @@ LLOGOS_EXPORT int llogos_rope_table(void* cs, const int* pos, const double* inv_
     return LLOGOS_LAUNCH_CHECK();
 }
 
+// ---------------------------------------------------------------- a step's opening: embedding, first norm, rotary table
+// Three kernels that nothing but their launches kept apart, in one: blocks 0 .. T - 1 take a token each, whose embedding row they
+// write to the stream x (times scale) and, normed, to out; the blocks behind them make the rotary table (half > 0).  A block's row is
+// laid out over its threads as rmsnorm_vec_kernel's is, so the rows have that kernel's bits.  What bounds it in a step of few rows is
+// the chain id, row, sum, and beside it the table's double sines.
+template <typename TO, typename TT, int ITEMS>
+__global__ __launch_bounds__(1024) void step_open_kernel(float* __restrict__ x, TO* __restrict__ out, const TT* __restrict__ table,
+                                                         const int* __restrict__ ids, const float* __restrict__ w, float scale, float eps,
+                                                         int T, int H, float2* __restrict__ cs, const int* __restrict__ pos,
+                                                         const double* __restrict__ inv_freq, int half, double amplitude) {
+    __shared__ float red[16];
+    const int r = blockIdx.x;
+    if (r >= T) {
+        const long long idx = (long long)(r - T) * blockDim.x + threadIdx.x;
+        if (idx >= (long long)T * half) return;
+        const double a = (double)pos[idx / half] * inv_freq[idx % half];
+        cs[idx] = make_float2((float)(cos(a) * amplitude), (float)(sin(a) * amplitude));
+        return;
+    }
+    const TT* row = table + (size_t)ids[r] * H;
+    float4 v[ITEMS], wv[ITEMS];
+    float ss = 0.f;
+#pragma unroll
+    for (int it = 0; it < ITEMS; ++it) {
+        const int i = 4 * (it * blockDim.x + threadIdx.x);
+        v[it] = i < H ? load4_f32(row + i) : make_float4(0.f, 0.f, 0.f, 0.f);
+        wv[it] = i < H ? load4_f32(w + i) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+#pragma unroll
+    for (int it = 0; it < ITEMS; ++it) {
+        const int i = 4 * (it * blockDim.x + threadIdx.x);
+        if (scale != 1.0f) { v[it].x *= scale; v[it].y *= scale; v[it].z *= scale; v[it].w *= scale; }
+        if (i < H) store4_f32(x + (size_t)r * H + i, v[it]);
+        ss += v[it].x * v[it].x + v[it].y * v[it].y + v[it].z * v[it].z + v[it].w * v[it].w;
+    }
+    const float total = block_sum(ss, red);
+    const float inv = 1.0f / sqrtf(total / (float)H + eps);
+#pragma unroll
+    for (int it = 0; it < ITEMS; ++it) {
+        const int i = 4 * (it * blockDim.x + threadIdx.x);
+        if (i < H)
+            store4_f32(out + (size_t)r * H + i, make_float4(v[it].x * inv * wv[it].x, v[it].y * inv * wv[it].y,
+                                                            v[it].z * inv * wv[it].z, v[it].w * inv * wv[it].w));
+    }
+}
+
+// x [T, H] = table[ids] * scale and out [T, H] = the rmsnorm of x with weight w; with half > 0 also cs [T, half] as llogos_rope_table.
+// Widths that are no multiple of 4 or above 16,384, and memory that is not aligned to 16 bytes, are left to the kernels apart.
+LLOGOS_EXPORT int llogos_step_open(float* x, void* out, int out_dtype, const void* table, int table_dtype, const int* ids, const float* w,
+                                   float scale, float eps, int T, int H, void* cs, const int* pos, const double* inv_freq, int half,
+                                   double amplitude, hipStream_t stream) {
+    if (T <= 0 || H <= 0 || half < 0 || (half > 0 && (cs == nullptr || pos == nullptr || inv_freq == nullptr))) return LLOGOS_BAD_ARGUMENT;
+    if (H % 4 || H > 16384 || (uintptr_t)x % 16 || (uintptr_t)out % 16 || (uintptr_t)table % 16 || (uintptr_t)w % 16) return LLOGOS_UNSUPPORTED;
+    const int groups = H / 4;
+    int items = groups <= 1024 ? 1 : (groups <= 2048 ? 2 : 4);
+    if (T >= 256 && groups >= 256) items = 4;                            // (rmsnorm's layout, as llogos_rmsnorm chooses it)
+    const int threads = ((groups + items - 1) / items + kWave - 1) / kWave * kWave;
+    const long long blocks = T + ((long long)T * half + threads - 1) / threads;
+    if (blocks > 0x7fffffffll) return LLOGOS_UNSUPPORTED;
+#define GO(TO, TT, IT) step_open_kernel<TO, TT, IT><<<(unsigned)blocks, threads, 0, stream>>>( \
+        x, (TO*)out, (const TT*)table, ids, w, scale, eps, T, H, (float2*)cs, pos, inv_freq, half, amplitude)
+#define PICK(TO, TT) do { if (items == 1) GO(TO, TT, 1); else if (items == 2) GO(TO, TT, 2); else GO(TO, TT, 4); } while (0)
+    if (out_dtype == DT_F32 && table_dtype == DT_F32) PICK(float, float);
+    else if (out_dtype == DT_BF16 && table_dtype == DT_BF16) PICK(bf16_t, bf16_t);
+    else if (out_dtype == DT_F32 && table_dtype == DT_BF16) PICK(float, bf16_t);
+    else if (out_dtype == DT_BF16 && table_dtype == DT_F32) PICK(bf16_t, float);
+    else return LLOGOS_BAD_ARGUMENT;
+#undef PICK
+#undef GO
+    return LLOGOS_LAUNCH_CHECK();
+}
+
 // ---------------------------------------------------------------- per-head norm + rotation + cache write
 // One wave per (token, head) of the fused projection row [q heads | k heads | v heads]:
 //   q, k heads: optional RMSNorm over head_dim with a shared weight, then rotation of the

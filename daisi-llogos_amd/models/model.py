@@ -11,6 +11,8 @@ from ..ops import kernels as K
 from ..parts.base import (BLOCKS, FEED_FORWARDS, MIXERS, NORMS, OTHER_PARTS, KVSpec, LayerCache, Mixer, Part, Runtime, StateSpec,
                           StepContext, TensorSpec, make)
 from ..parts.linear import Linear, _to_device
+from ..parts.norm import RMSNorm
+from ..parts.rope import Rotary
 
 
 @dataclass
@@ -109,6 +111,8 @@ class Model:
             self.entry_units.append(list(range(len(self.unit_mixers), len(self.unit_mixers) + len(mixers))))
             self.unit_mixers += mixers
         self._check_schedule()
+        # the rotation whose table every step needs (the first that a scheduled mixer names)
+        self._rotary = next((m.position for m in self.unit_mixers if type(getattr(m, "position", None)) is Rotary), None)
         self.head = Linear([spec.head_name], spec.hidden_size, [spec.vocab_size], suffix=spec.head_suffix)
         self.embed_table: Optional[torch.Tensor] = None
         self.rt: Optional[Runtime] = None
@@ -232,17 +236,31 @@ class Model:
         return total + 2.0 * wanted_rows * self.head.matrix_elements()
 
     # ---- one step ---------------------------------------------------------------
+    def _open(self, ctx: StepContext, first) -> Tuple[torch.Tensor, Optional[K.Opening]]:
+        """The stream at the first layer.  Where that layer's first norm can make it from the embedding, beside the first rotary table of the
+        step, it is still to be written, and an Opening stands for the delta."""
+        s, T = self.spec, ctx.n_tokens
+        # (a stream part reads the embedding itself, which is kept before the first norm runs)
+        norm = first.entry_norm() if first is not None and first.opens and all(e.enter is None for e in self.schedule) else None
+        if type(norm) is RMSNorm and s.position_vector <= 0.0 and K.step_opens(self.embed_table, norm.weight):
+            table = None
+            if self._rotary is not None:
+                table = ctx.shared[self._rotary.table_key] = torch.empty((T, self._rotary.rot // 2, 2), dtype=torch.float32, device=self.rt.device)
+            x = torch.empty((T, s.hidden_size), dtype=torch.float32, device=self.rt.device)
+            return x, K.Opening(self.embed_table, ctx.ids, s.embed_scale, ctx.tok_pos, self._rotary, table)
+        x = K.embed(self.embed_table, ctx.ids, s.embed_scale)
+        if s.position_vector > 0.0:
+            K.add_sinusoid(x, ctx.tok_pos, s.position_vector)
+        return x, None
+
     def forward(self, ctx: StepContext, caches: List[LayerCache], want_rows: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
         """Runs the step's tokens through the scheduled layers; `caches` holds one LayerCache for
         each unit.  Returns float32 logits [len(want_rows), vocab] for the wanted token rows, or
         None when nothing is wanted."""
         s = self.spec
-        x = K.embed(self.embed_table, ctx.ids, s.embed_scale)
-        if s.position_vector > 0.0:
-            K.add_sinusoid(x, ctx.tok_pos, s.position_vector)
-        ctx.mark("embed")
-        pending = None
         blocks = [self.layers[entry.layer] for entry in self.schedule]
+        x, pending = self._open(ctx, blocks[0] if blocks else None)
+        ctx.mark("embed")
         # the embedding output, for stream parts that read it again; the stream itself is changed in place
         x0 = x.clone() if any(e.enter is not None for e in self.schedule[1:]) else x
         for i, (block, units) in enumerate(zip(blocks, self.entry_units)):

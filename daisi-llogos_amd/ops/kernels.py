@@ -132,12 +132,53 @@ def gather_i32(dst: torch.Tensor, src: torch.Tensor, rows: torch.Tensor) -> None
     _check(_lib().llogos_gather_i32(_p(dst), _p(src), _p(rows), dst.numel(), src.numel(), _stream()), "gather_i32")
 
 
+@dataclass
+class Opening:
+    """What a step's first norm makes the stream from, in the kernel that norms it (rmsnorm's `opening`): the rows of `table` at `ids` times
+    `scale`; with a `rotary` part also its `rotary_table` of `positions` ([T, half, 2], as rope_table makes it)."""
+    table: torch.Tensor
+    ids: torch.Tensor
+    scale: float = 1.0
+    positions: Optional[torch.Tensor] = None
+    rotary: Optional[object] = None                     # inv_freq, amplitude
+    rotary_table: Optional[torch.Tensor] = None
+
+
+def step_opens(table: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether rmsnorm takes an Opening of this table: widths in groups of 4 up to 16,384, memory aligned to 16 bytes."""
+    H = table.shape[1]
+    return H % 4 == 0 and H <= 16384 and table.is_contiguous() and table.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
+
+
+def _step_open(x: torch.Tensor, weight: torch.Tensor, eps: float, out_dtype: torch.dtype, o: Opening) -> torch.Tensor:
+    _dev(x, weight, o.table, o.ids, o.positions, o.rotary_table)
+    _i32(o.ids, "ids"); _i32(o.positions, "positions")
+    T, H = x.shape
+    _need(x.dtype == torch.float32 and x.is_contiguous() and o.ids.shape == (T,) and o.table.dim() == 2 and o.table.shape[1] == H
+          and o.table.is_contiguous(), "rmsnorm: an opening's ids [T] name rows of table [V, H] for x [T, H]")
+    _need(weight.dtype == torch.float32 and weight.shape == (H,) and weight.is_contiguous(), "rmsnorm: weight must be float32 [H]")
+    half, freqs, amplitude = 0, None, 1.0
+    if o.rotary_table is not None:
+        freqs, amplitude, half = o.rotary.inv_freq, o.rotary.amplitude, o.rotary.inv_freq.numel()
+        _dev(freqs)
+        _need(freqs.dtype == torch.float64 and o.positions.shape == (T,) and o.rotary_table.shape == (T, half, 2)
+              and o.rotary_table.dtype == torch.float32 and o.rotary_table.is_contiguous(), "rmsnorm: an opening's rotary table is float32 [T, half, 2]")
+    out = torch.empty((T, H), dtype=out_dtype, device=x.device)
+    _check(_lib().llogos_step_open(_p(x), _p(out), _DT[out_dtype], _p(o.table), _dt(o.table), _p(o.ids), _p(weight), ctypes.c_float(o.scale),
+                                   ctypes.c_float(eps), T, H, _p(o.rotary_table), _p(o.positions), _p(freqs), half,
+                                   ctypes.c_double(amplitude), _stream()), "rmsnorm of an opening")
+    return out
+
+
 def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float, out_dtype: torch.dtype,
             delta: Optional[torch.Tensor] = None, rows: Optional[torch.Tensor] = None,
-            write_back: bool = True) -> torch.Tensor:
+            write_back: bool = True, opening: Optional[Opening] = None) -> torch.Tensor:
     """RMSNorm of the float32 residual stream `x` [T, H] with the pending `delta` ([T, H] or
     partial sums [parts, T, H]) added first (and written back to `x` when `write_back`).
-    With `rows` only those rows are normed, into a compact output."""
+    With `rows` only those rows are normed, into a compact output.  With `opening` x is written first, whole, from the embedding."""
+    if opening is not None:
+        _need(delta is None and rows is None, "rmsnorm: an opening's stream has no delta yet and is normed whole")
+        return _step_open(x, weight, eps, out_dtype, opening)
     _dev(x, weight, delta, rows)
     _i32(rows, "rows")
     _need(x.dtype == torch.float32 and x.dim() == 2, "rmsnorm: x must be float32 [T, H]")

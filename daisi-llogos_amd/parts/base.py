@@ -315,6 +315,7 @@ class Block(Part):
     this block (entry_norm() of the block that runs next), for parts that prepare its rows."""
 
     takes_next_norm = False
+    opens = False              # whether `pending` may be an ops.kernels.Opening: entry_norm() is then the first to touch the stream
 
     def entry_norm(self) -> Optional["Norm"]:
         """The norm that takes `pending` (None if the block has no such norm)."""

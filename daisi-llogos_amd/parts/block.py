@@ -41,6 +41,7 @@ class PreNormBlock(Block):
         return [p for p in (self.mixer_norm, self.mixer, self.ffn_norm, self.ffn, self.tail) if p is not None]
 
     takes_next_norm = True
+    opens = True
 
     def entry_norm(self) -> Optional[Norm]:
         return self.mixer_norm
@@ -113,6 +114,7 @@ class SandwichBlock(Block):
         return self.mixer_norm
 
     takes_next_norm = True
+    opens = True
 
     def _read(self, ctx, norm: Norm, conv, x, delta, cache, want_f32: bool):
         """What a sublayer reads: norm(x + delta), through the convolution when there is one."""

@@ -59,6 +59,8 @@ class RMSNorm(Norm):
             if delta.norm is self and rows is None and delta.rows.dtype == want:
                 return delta.rows
             delta = None
+        if isinstance(delta, K.Opening):
+            return K.rmsnorm(x, self.weight, self.eps, out_dtype or self.rt.dtype, rows=rows, opening=delta)
         if isinstance(delta, K.RowSquares):
             # the product before has added itself to x; if it also left this norm's rows without their
             # scale, a consumer that takes them needs no kernel here

@@ -4,6 +4,7 @@ are no power of two, many heads and groups)."""
 import ctypes
 import importlib
 import math
+from types import SimpleNamespace
 
 import numpy as np
 import pytest
@@ -40,6 +41,30 @@ def test_embed(dtype):
     ids = _t([0, 330, 7, 7, 129], torch.int32)
     out = K.embed(table, ids)
     assert out.dtype == torch.float32 and torch.equal(out, table.float()[ids.long()])
+
+
+@pytest.mark.parametrize("table_dtype,dtype", [("bfloat16", "bfloat16"), ("float32", "float32"), ("bfloat16", "float32")])
+@pytest.mark.parametrize("T,H,half,scale", [(1, 2048, 32, 1.0), (5, 200, 7, 1.5), (64, 4100, 64, 1.0), (300, 1028, 16, 0.5), (3, 8200, 0, 1.0), (2, 16384, 1, 1.0)])
+def test_step_open_is_embedding_norm_and_rotary_table(table_dtype, dtype, T, H, half, scale):
+    """The bits of the three kernels, whose layout of a row it keeps."""
+    rng = np.random.default_rng(T + H)
+    table, w = _t(rng.standard_normal((97, H)), DT[table_dtype]), _t(1 + 0.1 * rng.standard_normal(H))
+    ids, pos = _t(rng.integers(0, 97, T), torch.int32), _t(rng.integers(0, 100000, T), torch.int32)
+    freqs = _t(rng.random(half), torch.float64) if half else None
+    cs = torch.full((T, half, 2), float("nan"), device=DEV) if half else None
+    x = torch.full((T, H), float("nan"), device=DEV)
+    assert K.step_opens(table, w)
+    rows = K.rmsnorm(x, w, 1e-5, DT[dtype], opening=K.Opening(table, ids, scale, pos, SimpleNamespace(inv_freq=freqs, amplitude=1.25), cs))
+    want = K.embed(table, ids, scale)
+    assert torch.equal(x, want) and torch.equal(rows, K.rmsnorm(want, w, 1e-5, DT[dtype]))
+    assert not half or torch.equal(cs, K.rope_table(pos, freqs, 1.25))
+
+
+@pytest.mark.parametrize("H", [30, 16388])
+def test_step_open_leaves_other_widths_to_the_kernels_apart(H):
+    assert not K.step_opens(_t(np.ones((3, H))), _t(np.ones(H)))
+    with pytest.raises(K.KernelError):
+        K.rmsnorm(torch.empty(1, H, device=DEV), _t(np.ones(H)), 1e-5, torch.float32, opening=K.Opening(_t(np.ones((3, H))), _t([1], torch.int32)))
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
