@@ -44,11 +44,14 @@ def bucket_batch(batch: int) -> int:
 
 
 class DecodeGraph:
-    def __init__(self, engine, batch: int, widths: Tuple[int, ...]):
+    def __init__(self, engine, batch: int, widths: Tuple[int, ...], lent: bool = False):
+        """lent: the head is part of the captured step, whose output the next replay overwrites; otherwise the step is captured up to the
+        head's input, and the head is queued behind each replay into memory of the caller's own (as many launches as a copy of the
+        logits took, without the copy: 4.7 us for one row of 128,256, 9.8 for 64)."""
         # no strong reference back to the engine: a graph must die with its engine at once and
         # not later in a collection of reference cycles, which could fall into another capture
         self._engine = weakref.ref(engine)
-        self.batch, self.widths = batch, widths
+        self.batch, self.widths, self.lent = batch, widths, lent
         rt = engine.rt
         B = batch
         # ids, seq, pos, slots, rows, tables, rows of another step's ids to take the ids from
@@ -62,7 +65,7 @@ class DecodeGraph:
             self.views.append(self.dev[o:o + n])
             o += n
         self.graph: Optional[torch.cuda.CUDAGraph] = None
-        self.logits: Optional[torch.Tensor] = None
+        self.out = None                            # the step's logits (lent), or the head's input
         self.copied = torch.cuda.Event()
 
     def _fill(self, ids, tok_pos, slot_ids, tables: List[np.ndarray], id_rows=None) -> None:
@@ -84,13 +87,14 @@ class DecodeGraph:
         self.dev.copy_(self.host, non_blocking=True)
         self.copied.record()
 
-    def _forward(self, max_context: int) -> Optional[torch.Tensor]:
+    def _forward(self, max_context: int):
         eng, v, B = self._engine(), self.views, self.batch
         ctx = StepContext(runtime=eng.rt, n_tokens=B, batch=B, ids=v[0], tok_seq=v[1], tok_pos=v[2], slots=v[3],
                           cu_seqlens=list(range(B + 1)), starts=[], slot_ids=[], is_decode=True,
                           max_context=max_context, in_graph=True)
         tables = [t.view(B, w) for t, w in zip(v[5:5 + len(self.widths)], self.widths)]
-        return eng.model.forward(ctx, eng.cache.layer_caches(tables), v[4])
+        run = eng.model.forward if self.lent else eng.model.rows
+        return run(ctx, eng.cache.layer_caches(tables), v[4])
 
     def run(self, ids, tok_pos, slot_ids, tables: List[np.ndarray], device_ids=None) -> torch.Tensor:
         """device_ids: (int32 device vector, rows): the step's ids are that vector's values at
@@ -121,18 +125,18 @@ class DecodeGraph:
             gc.disable()
             try:
                 with torch.cuda.graph(graph):
-                    self.logits = self._forward(cap)
+                    self.out = self._forward(cap)
             finally:
                 if gc_was_on:
                     gc.enable()
             self.graph = graph
         self.graph.replay()
-        return self.logits
+        return self.out if self.lent else self._engine().model.logits(None, self.out)
 
 
 class GraphCache:
-    """Captured decode steps by (batch size, page-table widths); the least recently used
-    graph is dropped when there are too many."""
+    """Captured decode steps by (batch size, page-table widths), those that lend their logits by themselves; the least
+    recently used graph is dropped when there are too many."""
 
     def __init__(self, engine):
         self._engine = weakref.ref(engine)
@@ -141,7 +145,7 @@ class GraphCache:
     def clear(self) -> None:
         self.graphs.clear()
 
-    def step(self, ids, tok_pos, slot_ids, tables: List[np.ndarray], device_ids=None) -> torch.Tensor:
+    def step(self, ids, tok_pos, slot_ids, tables: List[np.ndarray], device_ids=None, lent: bool = False) -> torch.Tensor:
         B = len(slot_ids)
         pad = bucket_batch(B) - B
         if pad:
@@ -153,12 +157,12 @@ class GraphCache:
             tables = [np.concatenate([t, np.pad(rows, ((0, 0), (0, t.shape[1] - 1)), constant_values=-1)]) for t in tables]
             if device_ids is not None:
                 device_ids = (device_ids[0], list(device_ids[1]) + [0] * pad)
-        key = (B + pad, tuple(bucket_width(t.shape[1]) for t in tables))
+        key = (B + pad, tuple(bucket_width(t.shape[1]) for t in tables)) + (("lent",) if lent else ())
         g = self.graphs.get(key)
         if g is None:
             while len(self.graphs) >= MAX_GRAPHS:
                 self.graphs.popitem(last=False)
-            g = DecodeGraph(self._engine(), key[0], key[1])
+            g = DecodeGraph(self._engine(), key[0], key[1], lent)
             self.graphs[key] = g
         else:
             self.graphs.move_to_end(key)

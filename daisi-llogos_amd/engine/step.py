@@ -215,7 +215,7 @@ class Engine:
 
         borrow: the caller is done with the logits (on the device, in stream order) before it
         asks for the next step, so a replayed step may hand out its own output buffer, which the
-        next replay overwrites, instead of a copy (33 MB a step at batch 64 and 128,256 tokens).
+        next replay overwrites.
 
         probe: a callable that the model's parts call with their name when their kernels are
         queued (engine/probe.py: StepProbe times the step part by part); such a step is launched
@@ -268,9 +268,7 @@ class Engine:
             with torch.cuda.device(self.rt.device):
                 logits = self.graphs.step(ids.astype(np.int32), np.asarray(starts, dtype=np.int32),
                                           np.asarray(slot_ids, dtype=np.int32), self.cache.step_tables(slot_ids),
-                                          device_ids)
-                if not borrow:
-                    logits = logits.clone()      # the graph's own buffer is overwritten by its next replay
+                                          device_ids, borrow)
             return logits
         tok_seq = np.repeat(np.arange(B, dtype=np.int32), counts)
         tok_pos = np.concatenate([np.arange(s, s + c, dtype=np.int32) for s, c in zip(starts, counts)])

@@ -9,7 +9,7 @@ import torch
 
 from ..ops import kernels as K
 from ..parts.base import (BLOCKS, FEED_FORWARDS, MIXERS, NORMS, OTHER_PARTS, KVSpec, LayerCache, Mixer, Part, Runtime, StateSpec,
-                          StepContext, TensorSpec, make)
+                          StepContext, TensorSpec, make, mark)
 from ..parts.linear import Linear, _to_device
 from ..parts.norm import RMSNorm
 from ..parts.rope import Rotary
@@ -257,6 +257,11 @@ class Model:
         """Runs the step's tokens through the scheduled layers; `caches` holds one LayerCache for
         each unit.  Returns float32 logits [len(want_rows), vocab] for the wanted token rows, or
         None when nothing is wanted."""
+        rows = self.rows(ctx, caches, want_rows)
+        return None if rows is None else self.logits(ctx, rows)
+
+    def rows(self, ctx: StepContext, caches: List[LayerCache], want_rows: Optional[torch.Tensor]):
+        """forward() up to the final norm: what logits() takes."""
         s = self.spec
         blocks = [self.layers[entry.layer] for entry in self.schedule]
         x, pending = self._open(ctx, blocks[0] if blocks else None)
@@ -281,8 +286,13 @@ class Model:
             return None
         n = self.final_norm.forward(x, pending, rows=want_rows, write_back=False)
         ctx.mark("norm")
-        logits = self.head.forward(n, out_dtype=torch.float32)
-        ctx.mark("head")
+        return n
+
+    def logits(self, ctx: Optional[StepContext], rows) -> torch.Tensor:
+        """The head on the rows that rows() returned."""
+        s = self.spec
+        logits = self.head.forward(rows, out_dtype=torch.float32)
+        mark(ctx, "head")
         if s.logit_scale != 1.0 or s.logit_softcap > 0.0:
             K.scale_softcap(logits, s.logit_scale, s.logit_softcap)
         return logits
