@@ -118,6 +118,13 @@ __device__ __forceinline__ float gated_value(float gate, float up, int bounded, 
     return gate * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * gate)) * up;
 }
 
+// Four values side by side, in one store where they are aligned.
+__device__ __forceinline__ void store_quad(float* p, const float (&v)[4]) { *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]); }
+__device__ __forceinline__ void store_quad(bf16_t* p, const float (&v)[4]) {
+    *reinterpret_cast<uint2*>(p) = make_uint2((uint32_t)f32_to_bf16(v[0]) | (uint32_t)f32_to_bf16(v[1]) << 16,
+                                              (uint32_t)f32_to_bf16(v[2]) | (uint32_t)f32_to_bf16(v[3]) << 16);
+}
+
 template <int RB, int MB, int MODE, typename TO, int CHUNK, int WAVES = kLdsWaves, bool PACKED = false, bool GATED = false, int RING = 0>
 __global__ __launch_bounds__(WAVES * kWave) void gemm_skinny_lds_kernel(
         TO* __restrict__ out, ActSource src, const bf16_t* __restrict__ w, const float* __restrict__ bias,
@@ -356,6 +363,8 @@ __global__ __launch_bounds__(WAVES * kWave) void gemm_skinny_lds_kernel(
         }
         __syncthreads();
     }
+    // (the launch's rows begin at multiples of four values)
+    const bool quads = ldo % 4 == 0 && part_stride % 4 == 0 && (uintptr_t)out % (4 * sizeof(TO)) == 0;
     if (GATED) {
         // The packed strips alternate between 16 gate rows and the 16 up rows of the same columns
         // (llogos_pack_weights with gate_rows): waves 0 and 2 hold gate values, waves 1 and 3 the up
@@ -382,12 +391,20 @@ __global__ __launch_bounds__(WAVES * kWave) void gemm_skinny_lds_kernel(
                 const int m = mb * 16 + r;
                 if (m >= M) continue;
                 const float row_scale = MODE == PRODUCE_UNSCALED ? inv_rms[m] : 1.0f;
+                float y[4];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const float gate = acc[rb][mb][i] * row_scale;
                     const float up = xch[((((wave >> 1) * RB + rb) * MB + mb) * 4 + i) * kWave + lane] * row_scale;
-                    const float y = gated_value(gate, up, src.bounded, src.limit);
-                    if (col0 + i < N / 2) store_f32(out + (size_t)m * ldo + col0 + i, y);
+                    y[i] = gated_value(gate, up, src.bounded, src.limit);
+                }
+                TO* at = out + (size_t)m * ldo + col0;
+                if (quads && col0 + 3 < N / 2) {
+                    store_quad(at, y);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        if (col0 + i < N / 2) store_f32(at + i, y[i]);
                 }
             }
         }
@@ -402,10 +419,17 @@ __global__ __launch_bounds__(WAVES * kWave) void gemm_skinny_lds_kernel(
             const int m = mb * 16 + r;
             if (m >= M) continue;
             const float row_scale = MODE == PRODUCE_UNSCALED ? inv_rms[m] : 1.0f;
+            const int n = (PACKED ? ((n_block * RB + rb) * WAVES + wave) * 16 : n0 + rb * 16) + 4 * g;
+            TO* at = dst + (size_t)m * ldo + n;
+            float y[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int n = (PACKED ? ((n_block * RB + rb) * WAVES + wave) * 16 : n0 + rb * 16) + 4 * g + i;
-                if (n < N) store_f32(dst + (size_t)m * ldo + n, acc[rb][mb][i] * row_scale + (bias ? bias[n] : 0.f));
+            for (int i = 0; i < 4; ++i) y[i] = acc[rb][mb][i] * row_scale + (bias && n + i < N ? bias[n + i] : 0.f);
+            if (quads && n + 3 < N) {
+                store_quad(at, y);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (n + i < N) store_f32(at + i, y[i]);
             }
         }
 }

@@ -1487,6 +1487,21 @@ def test_products_that_no_norm_follows_are_added_by_the_library(M, N, K_):
     assert lin.add_to(a, base.Residual(x, norm)) is None and torch.equal(x, x0)
 
 
+@pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("M", [1, 16, 33, 64])
+@pytest.mark.parametrize("N", [65, 66, 67, 1087])
+def test_few_row_results_stored_by_fours_and_one_by_one(N, M, out_dtype):
+    """Rows of a multiple of four values are stored four at a time, others (and a row's last few) value by value: the same bits, bias and all."""
+    rng = np.random.default_rng(N + M)
+    a, w = _t(rng.standard_normal((M, 520)), torch.bfloat16), _t(rng.standard_normal((N + 3, 520)) * 0.05, torch.bfloat16)
+    b = _t(rng.standard_normal(N + 3))
+    few = K.gemm_packed_bf16(a, K.pack_weights(w[:N].contiguous()), b[:N].contiguous(), out_dtype)
+    whole = N + -N % 4
+    more = K.gemm_packed_bf16(a, K.pack_weights(w[:whole].contiguous()), b[:whole].contiguous(), out_dtype)
+    assert few.shape == (1, M, N) and torch.equal(few, more[:, :, :N])
+    _close(few[0], _np(a) @ _np(w[:N]).T + _np(b[:N]), "float32" if out_dtype == torch.float32 else "bfloat16")
+
+
 @pytest.mark.parametrize("G,M,N,K_", [(4, 1, 64, 8), (4, 8, 256, 1024), (3, 17, 192, 520), (2, 33, 4096, 2048), (4, 64, 128, 4096), (4, 8, 4096, 4096)])
 def test_products_of_one_shape_in_one_launch(G, M, N, K_):
     """Each of the group is the product by itself, in the parts that its own plan gives it, bit for bit; the single copies still serve alone."""
