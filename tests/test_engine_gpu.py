@@ -34,6 +34,30 @@ def test_whole_requests(name, dtype):
         H.close(got, H.plain_logits(name, toks), dtype, f"{name} whole n={n}", config=name)
 
 
+def test_prompts_are_queued_behind_work_that_still_runs():
+    """A step's integers reach the GPU without the host waiting for what is queued before them; steps queued one behind the other, whose pinned
+    memory goes back and comes out again, give what each gives alone."""
+    eng = H.engine("tiny_a", "float32", max_tokens=64 * 40, n_slots=8)
+    prompts = [H.tokens("tiny_a", 20 + 3 * i, 50 + i) for i in range(6)]
+
+    def run(p):
+        s = eng.alloc_slot()
+        out = eng.step([(s, p)], want="last")
+        eng.free_slot(s)
+        return out
+    alone = []
+    for p in prompts:
+        alone.append(run(p))
+        torch.cuda.synchronize()
+    done = torch.cuda.Event()
+    torch.cuda._sleep(40_000_000)                    # (tens of milliseconds at the least)
+    done.record()
+    behind = [run(p) for p in prompts]
+    assert not done.query()
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(alone, behind))
+
+
 @pytest.mark.parametrize("dtype", H.DTYPES)
 @pytest.mark.parametrize("name", CONFIGS)
 def test_last_32_tokens_one_by_one(name, dtype):
