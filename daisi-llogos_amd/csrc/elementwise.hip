@@ -113,6 +113,27 @@ LLOGOS_EXPORT int llogos_scale_softcap(float* x, long long n, float scale, float
     return LLOGOS_LAUNCH_CHECK();
 }
 
+// A few thousand integers from pinned host memory, which the GPU reads where it lies: bound by one trip to the host.  In front of the
+// sampler's two kernels it is 1.4 us shorter than the runtime's copy (64 rows, 40 KB: 30.0 -> 28.5 us a step); in front of a replayed
+// step, whose copy it would be too, 1 us of 700, and the buffer's life would be the caller's to watch.
+__global__ void copy_words_kernel(uint32_t* __restrict__ dst, const uint32_t* __restrict__ src, long long n, int quads) {
+    const long long i = ((long long)blockIdx.x * blockDim.x + threadIdx.x) * 4;
+    if (quads && i + 3 < n) {
+        *reinterpret_cast<uint4*>(dst + i) = *reinterpret_cast<const uint4*>(src + i);
+        return;
+    }
+    for (long long e = i; e < min(i + 4, n); ++e) dst[e] = src[e];
+}
+
+// dst[0 .. n) = src[0 .. n), 32-bit words; src: pinned host memory (hipHostMalloc) or device memory
+LLOGOS_EXPORT int llogos_copy_words(void* dst, const void* src, long long n, hipStream_t stream) {
+    if (n <= 0 || dst == nullptr || src == nullptr || (uintptr_t)dst % 4 || (uintptr_t)src % 4) return LLOGOS_BAD_ARGUMENT;
+    const long long blocks = (n + 1023) / 1024;
+    if (blocks > 0x7fffffffll) return LLOGOS_UNSUPPORTED;
+    copy_words_kernel<<<(unsigned)blocks, 256, 0, stream>>>((uint32_t*)dst, (const uint32_t*)src, n, (uintptr_t)dst % 16 == 0 && (uintptr_t)src % 16 == 0);
+    return LLOGOS_LAUNCH_CHECK();
+}
+
 // dst[i] = src[rows[i]] for int32 values: a step's token ids picked from the ids another
 // step's sampler left on the device.  rows outside 0..n_src-1 give 0.
 __global__ void gather_i32_kernel(int* __restrict__ dst, const int* __restrict__ src,

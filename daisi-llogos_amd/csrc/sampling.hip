@@ -1061,6 +1061,8 @@ LLOGOS_EXPORT long long llogos_sample_few_words(int R, int V, int top_k) {
     return R * slices * kSliceCap + R * n_pad + (long long)R * V + R * slices;
 }
 
+LLOGOS_EXPORT int llogos_copy_words(void* dst, const void* src, long long n, hipStream_t stream);     // (elementwise.hip)
+
 // llogos_sample_few from what the host has packed into pinned memory: R uniform numbers (float32) and, with `windows`, the R + 1 places of the
 // rows' windows and the windows, `staged` 32-bit numbers in all.  They are copied behind the scratch (16-byte aligned: llogos_sample_few_words words, then
 // `staged` numbers), `copied` (an event or null) is recorded behind the copy, and the two kernels follow: one call for what a step of
@@ -1080,9 +1082,12 @@ LLOGOS_EXPORT int llogos_sample_few_staged(int* out, const float* logits, int R,
     int* counts = (int*)(prob + (size_t)R * V);
     float* tops = (float*)(counts + R * slices);
     int* numbers = (int*)(keys + words);
-    hipError_t e = hipMemcpyAsync(numbers, host, (size_t)staged * 4, hipMemcpyHostToDevice, stream);
-    if (e == hipSuccess && copied != nullptr) e = hipEventRecord((hipEvent_t)copied, stream);
-    if (e != hipSuccess) return (int)e;
+    const int code = llogos_copy_words(numbers, host, staged, stream);
+    if (code != 0) return code;
+    if (copied != nullptr) {
+        const hipError_t e = hipEventRecord((hipEvent_t)copied, stream);
+        if (e != hipSuccess) return (int)e;
+    }
     return llogos_sample_few(out, logits, R, V, windows ? numbers + 2 * R + 1 : nullptr, windows ? numbers + R : nullptr, s->repetition, s->frequency,
                              s->presence, s->inv_temperature, s->penalize_newline, s->banned, s->n_banned, keys, counts, tops, work, prob, list,
                              (int)n_pad, (const float*)numbers, s->top_k, s->top_p, s->min_p, s->typical_p, s->min_keep, stream);

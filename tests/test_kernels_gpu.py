@@ -60,6 +60,18 @@ def test_step_open_is_embedding_norm_and_rotary_table(table_dtype, dtype, T, H, 
     assert not half or torch.equal(cs, K.rope_table(pos, freqs, 1.25))
 
 
+@pytest.mark.parametrize("n", [1, 3, 4, 1023, 1024, 1029, 20000])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_words_from_pinned_memory(n, shift):
+    """By fours where both sides are aligned to 16 bytes, one by one elsewhere and at the end; nothing behind the last word is touched."""
+    host = torch.randint(-2 ** 31, 2 ** 31 - 1, (n + shift,), dtype=torch.int32).pin_memory()
+    dst = torch.full((n + 9,), 7, dtype=torch.int32, device=DEV)
+    code = K._lib().llogos_copy_words(ctypes.c_void_p(dst.data_ptr()), ctypes.c_void_p(host.data_ptr() + 4 * shift), n, K._stream())
+    torch.cuda.synchronize()
+    assert code == 0 and torch.equal(dst[:n].cpu(), host[shift:]) and (dst[n:] == 7).all()
+    assert K._lib().llogos_copy_words(ctypes.c_void_p(dst.data_ptr()), ctypes.c_void_p(host.data_ptr()), 0, K._stream()) == -1
+
+
 @pytest.mark.parametrize("H", [30, 16388])
 def test_step_open_leaves_other_widths_to_the_kernels_apart(H):
     assert not K.step_opens(_t(np.ones((3, H))), _t(np.ones(H)))
