@@ -58,6 +58,23 @@ __device__ __forceinline__ float wave_sum(float v) {
     return v;
 }
 
+// wave_sum of a wave whose lanes all take part: the same additions, partners 32, 16, 8, 4, 2 and 1 lanes away.  (Rotating a row of 16 by
+// 8 brings lane i ^ 8; by 4, where lanes 8 apart hold the same by then, what lane i ^ 4 holds.)
+__device__ __forceinline__ float whole_wave_sum(float v) {
+    typedef unsigned u32x2_t __attribute__((ext_vector_type(2)));
+    u32x2_t r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+#define LLOGOS_ADD_DPP(CTRL) v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true))
+    LLOGOS_ADD_DPP(0x128);                                  // row_ror:8
+    LLOGOS_ADD_DPP(0x124);                                  // row_ror:4
+    LLOGOS_ADD_DPP(0x4e);                                   // quad_perm:[2,3,0,1]
+    LLOGOS_ADD_DPP(0xb1);                                   // quad_perm:[1,0,3,2]
+#undef LLOGOS_ADD_DPP
+    return v;
+}
+
 __device__ __forceinline__ float wave_max(float v) {
 #pragma unroll
     for (int o = kWave / 2; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, kWave));
@@ -67,15 +84,21 @@ __device__ __forceinline__ float wave_max(float v) {
 // Sum over a block of up to 1024 threads; `red` holds at least 16 floats of LDS.
 // Every thread gets the result.  The order of the additions is fixed by the block
 // shape alone, so a row gives the same sum whatever else is in the batch.
+// Row-wise kernels of a single-token step are a few dependent steps long, and this sum is one or two of them: the lanes' values go
+// from neighbour to neighbour inside the vector unit where every wave is whole, and the waves' are read from LDS together (a shuffle or a
+// read that is waited for each time is some hundred clocks).
 __device__ __forceinline__ float block_sum(float v, float* red) {
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const int nwaves = (blockDim.x + kWave - 1) / kWave;
-    v = wave_sum(v);
+    v = blockDim.x % kWave == 0 ? whole_wave_sum(v) : wave_sum(v);
     __syncthreads();
     if (lane == 0) red[wave] = v;
     __syncthreads();
-    float t = 0.f;
-    for (int i = 0; i < nwaves; ++i) t += red[i];
+    float r[16], t = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) r[i] = red[i];             // (what lies behind the last wave's is not used)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) t = i < nwaves ? t + r[i] : t;
     return t;
 }
 
