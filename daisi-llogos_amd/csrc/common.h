@@ -86,7 +86,8 @@ __device__ __forceinline__ float wave_max(float v) {
 // shape alone, so a row gives the same sum whatever else is in the batch.
 // Row-wise kernels of a single-token step are a few dependent steps long, and this sum is one or two of them: the lanes' values go
 // from neighbour to neighbour inside the vector unit where every wave is whole, and the waves' are read from LDS together (a shuffle or a
-// read that is waited for each time is some hundred clocks).
+// read that is waited for each time is some hundred clocks).  Steps of the designs whose norms follow one another: 8 sequences, three
+// wkv layers and one of latent attention, 0.5 % shorter; parallel blocks of 8 layers 0.3 %.
 __device__ __forceinline__ float block_sum(float v, float* red) {
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const int nwaves = (blockDim.x + kWave - 1) / kWave;

@@ -351,7 +351,8 @@ LLOGOS_EXPORT int llogos_rope_table(void* cs, const int* pos, const double* inv_
 // Three kernels that nothing but their launches kept apart, in one: blocks 0 .. T - 1 take a token each, whose embedding row they
 // write to the stream x (times scale) and, normed, to out; the blocks behind them make the rotary table (half > 0).  A block's row is
 // laid out over its threads as rmsnorm_vec_kernel's is, so the rows have that kernel's bits.  What bounds it in a step of few rows is
-// the chain id, row, sum, and beside it the table's double sines.
+// the chain id, row, sum, and beside it the table's double sines: 4.2 us for one row of 2,048 where the three kernels took 3.7, 4.5 and
+// 3.5 one after the other, 4.2 for 8 rows of 4,096 (7.1, 4.5, 5.0: the embedding read two bytes a load).
 template <typename TO, typename TT, int ITEMS>
 __global__ __launch_bounds__(1024) void step_open_kernel(float* __restrict__ x, TO* __restrict__ out, const TT* __restrict__ table,
                                                          const int* __restrict__ ids, const float* __restrict__ w, float scale, float eps,
