@@ -60,11 +60,9 @@ __device__ __forceinline__ float wave_sum(float v) {
 
 // wave_sum of a wave whose lanes all take part: the same additions, partners 32, 16, 8, 4, 2 and 1 lanes away.  (Rotating a row of 16 by
 // 8 brings lane i ^ 8; by 4, where lanes 8 apart hold the same by then, what lane i ^ 4 holds.)
-__device__ __forceinline__ float whole_wave_sum(float v) {
-    typedef unsigned u32x2_t __attribute__((ext_vector_type(2)));
-    u32x2_t r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-    r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+typedef unsigned u32x2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ float half_waves_sum(float v) {      // the additions behind the first
+    const u32x2_t r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
 #define LLOGOS_ADD_DPP(CTRL) v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true))
     LLOGOS_ADD_DPP(0x128);                                  // row_ror:8
@@ -73,6 +71,24 @@ __device__ __forceinline__ float whole_wave_sum(float v) {
     LLOGOS_ADD_DPP(0xb1);                                   // quad_perm:[1,0,3,2]
 #undef LLOGOS_ADD_DPP
     return v;
+}
+
+__device__ __forceinline__ float whole_wave_sum(float v) {
+    const u32x2_t r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return half_waves_sum(__uint_as_float(r[0]) + __uint_as_float(r[1]));
+}
+
+// The sum of v * v over the wave, lane 0's: its half's squares go into the first addition unrounded, the other half's are rounded.
+__device__ __forceinline__ float whole_wave_sum_of_squares(float v) {
+    const unsigned sq = __float_as_uint(v * v);
+    const u32x2_t r = __builtin_amdgcn_permlane32_swap(sq, sq, false, false);          // (r[1]: the upper half's, in both halves)
+    return half_waves_sum(fmaf(v, v, __uint_as_float(r[1])));
+}
+__device__ __forceinline__ float wave_sum_of_squares(float v) {
+    float s = fmaf(v, v, __shfl_xor(v * v, kWave / 2, kWave));
+#pragma unroll
+    for (int o = kWave / 4; o > 0; o >>= 1) s += __shfl_xor(s, o, kWave);
+    return s;
 }
 
 __device__ __forceinline__ float wave_max(float v) {
@@ -88,10 +104,9 @@ __device__ __forceinline__ float wave_max(float v) {
 // from neighbour to neighbour inside the vector unit where every wave is whole, and the waves' are read from LDS together (a shuffle or a
 // read that is waited for each time is some hundred clocks).  Steps of the designs whose norms follow one another: 8 sequences, three
 // wkv layers and one of latent attention, 0.5 % shorter; parallel blocks of 8 layers 0.3 %.
-__device__ __forceinline__ float block_sum(float v, float* red) {
+__device__ __forceinline__ float block_sum_of_waves(float v, float* red) {      // v: lane 0's is its wave's sum
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const int nwaves = (blockDim.x + kWave - 1) / kWave;
-    v = blockDim.x % kWave == 0 ? whole_wave_sum(v) : wave_sum(v);
     __syncthreads();
     if (lane == 0) red[wave] = v;
     __syncthreads();
@@ -101,6 +116,16 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) t = i < nwaves ? t + r[i] : t;
     return t;
+}
+
+__device__ __forceinline__ float block_sum(float v, float* red) {
+    return block_sum_of_waves(blockDim.x % kWave == 0 ? whole_wave_sum(v) : wave_sum(v), red);
+}
+
+// block_sum of v * v, whose additions say themselves which squares are rounded (written as a sum of products, that was the compiler's
+// choice, and another one where the lanes' values went another way).
+__device__ __forceinline__ float block_sum_of_squares(float v, float* red) {
+    return block_sum_of_waves(blockDim.x % kWave == 0 ? whole_wave_sum_of_squares(v) : wave_sum_of_squares(v), red);
 }
 
 __device__ __forceinline__ float block_max(float v, float* red) {

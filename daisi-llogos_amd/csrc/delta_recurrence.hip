@@ -252,7 +252,7 @@ __global__ __launch_bounds__(NT) void delta_step_kernel(TO* __restrict__ y, Delt
         su[tid] = ks * u;
         o = fmaf(kq, u, qs * rq);
     }
-    const float inv = 1.0f / sqrtf(block_sum(o * o, red[0]) / (float)V + eps);      // (its barriers also publish su)
+    const float inv = 1.0f / sqrtf(block_sum_of_squares(o, red[0]) / (float)V + eps);      // (its barriers also publish su)
     if (tid < V)
         store_f32(y + ((size_t)seq * H + head) * V + tid, o * inv * norm_w[tid] * (gate_silu ? delta_silu(sz[tid]) : delta_sigmoid(sz[tid])));
     // the token's projected channels join the ring (those of a key head once)

@@ -129,7 +129,7 @@ __global__ __launch_bounds__(16 * VB) void diff_merge_kernel(bf16_t* __restrict_
     merge_blocks<2, VP>(partial + ((size_t)b * n_heads + h) * 2 * n_z * (VP + 2), n_z, used, d, m, l, sums);
     const float a[2] = {l[0] > 0.f ? sums[0] / l[0] : 0.f, l[1] > 0.f ? sums[1] / l[1] : 0.f};
     const float o = a[0] - lambda * a[1];
-    const float total = block_sum(o * o, red);
+    const float total = block_sum_of_squares(o, red);
     out[((size_t)b * n_heads + h) * VP + d] = f32_to_bf16(o * (out_scale / sqrtf(total / (float)VP + eps)));
 }
 
@@ -143,7 +143,7 @@ __global__ __launch_bounds__(16 * VB) void diff_combine_kernel(bf16_t* __restric
     const int t = blockIdx.x, h = blockIdx.y, d = threadIdx.x;
     const float* src = maps + ((size_t)t * n_heads + h) * 2 * VP;
     const float o = src[d] - lambda * src[VP + d];
-    const float total = block_sum(o * o, red);
+    const float total = block_sum_of_squares(o, red);
     out[((size_t)t * n_heads + h) * VP + d] = f32_to_bf16(o * (out_scale / sqrtf(total / (float)VP + eps)));
 }
 

@@ -64,7 +64,7 @@ __global__ __launch_bounds__(1024) void post_norm_kernel(float* __restrict__ x, 
         v[it] = a;
         ss += a * a;
     }
-    const float total = block_sum(ss, red);
+    const float total = ITEMS == 1 ? block_sum_of_squares(v[0], red) : block_sum(ss, red);
     const float inv = 1.0f / sqrtf(total / (float)H + eps);
 #pragma unroll
     for (int it = 0; it < ITEMS; ++it) {

@@ -638,3 +638,57 @@ def test_blocks_along_a_long_context_are_merged_whole(lens, monkeypatch):
     want = run()
     # (weights rounded to bfloat16, 2^-9 each, in sums that a norm brings to size one; the result is rounded once more)
     assert np.abs(got - want).max() <= PART_TOL["bfloat16"] * np.abs(want).max()
+
+
+def _sum_of_squares(o, fused=True):
+    """The float32 sum of o * o over a row in the order of a block's sum (waves of 64, partners 32, 16, ... lanes away, the waves in ascending
+    order): the first addition takes the lower half's squares unrounded, or (not fused) rounded like the upper half's."""
+    f = np.float32
+    total = np.zeros(o.shape[0], f)
+    for wave in np.split(o, o.shape[1] // 64, axis=1):
+        low, high = wave[:, :32], (wave[:, 32:] * wave[:, 32:]).astype(np.longdouble)
+        squares = low.astype(np.longdouble) ** 2 if fused else (low * low).astype(np.longdouble)
+        s = (squares + high).astype(f)
+        while s.shape[1] > 1:
+            s = s[:, :s.shape[1] // 2] + s[:, s.shape[1] // 2:]
+        total = total + s[:, 0]
+    return total
+
+
+@pytest.mark.parametrize("dv", [64, 128])
+@pytest.mark.parametrize("decode", [True, False])
+def test_the_bits_of_differential_attentions_norm(dv, decode):
+    """Behind one key both maps are that key's value, so that every bit of the difference's norm is known: the additions of its sum
+    of squares are the written ones and no choice of the compiler's."""
+    rng = np.random.default_rng(dv)
+    B, heads, d, f = 512, 8, 64, np.float32
+    kp = torch.from_numpy(rng.standard_normal((B, heads, 64 * 2 * d), dtype=f)).to(DEV).bfloat16()
+    vp = torch.from_numpy(rng.standard_normal((B, heads, 64 * dv), dtype=f)).to(DEV).bfloat16()
+    q = torch.zeros(B, heads * 2 * d, dtype=torch.bfloat16, device=DEV)                  # (scores of 0, whose weight is 1 to the last bit)
+    ctx = type("Ctx", (), dict(n_tokens=B, batch=B, is_decode=decode, tok_seq=_i32(range(B)), tok_pos=_i32(np.zeros(B)), cu_dev=_i32(range(B + 1)),
+                               cu_seqlens=list(range(B + 1)), starts=[0] * B))()
+    lam, eps, table = 0.3, 1e-5, _i32(np.arange(B).reshape(B, 1))
+    place = [((i >> 4) * 128 + (i & 15)) * 8 for i in range(dv)]                # (of a page's first value)
+    v = vp.double().cpu().numpy()[:, :, place].reshape(-1, dv)
+    o = (v - np.float64(f(lam)) * v).astype(f)
+    root = {fused: np.sqrt(_sum_of_squares(o, fused) / f(dv) + f(eps)) for fused in (True, False)}
+    others = 0
+    for scale in np.linspace(0.5, 1.0, 48).astype(f):                           # (bfloat16 results show a sum's last bit once in 10^5)
+        got = K.diff_attention(ctx, q, kp, vp, table, heads, heads, d, dv, 0.3, lam, float(scale), eps).float().cpu().reshape(-1, dv)
+        want, other = (torch.from_numpy(o * (scale / root[fused])[:, None]).bfloat16().float() for fused in (True, False))
+        assert torch.equal(got, want), (int((got != want).sum()), int((got != other).sum()))
+        others += int((want != other).sum())
+    assert others > 0
+
+
+@pytest.mark.parametrize("H_", [50, 64])
+def test_the_bits_of_a_narrow_norm_behind_the_scaled_sum(H_):
+    """A row of one wave: its additions are the written ones too."""
+    f, eps = np.float32, 1e-5
+    x = np.random.default_rng(H_).standard_normal((300, H_)).astype(f)
+    xs = torch.tensor(x, device=DEV)
+    K.post_norm(xs, None, 1.0, torch.ones(H_, device=DEV), eps, torch.float32)
+    wide = np.pad(x, ((0, 0), (0, 64 - H_)))
+    rows = {fused: x * (f(1) / np.sqrt(_sum_of_squares(wide, fused) / f(H_) + f(eps)))[:, None] for fused in (True, False)}
+    assert not np.array_equal(rows[True], rows[False])
+    assert np.array_equal(xs.cpu().numpy(), rows[True])
