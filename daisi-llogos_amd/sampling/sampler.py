@@ -6,6 +6,7 @@ from __future__ import annotations
 
 import struct
 import weakref
+from collections import deque
 from typing import List, Optional, Sequence
 
 import numpy as np
@@ -17,12 +18,29 @@ from .rng import uniforms
 
 
 # Staging buffers that nobody fills any more, until their last copies have run: those are queued by the kernel library, so that torch
-# would hand freed pinned memory out again while one still reads it.
-_retired: List[tuple] = []
+# would hand freed pinned memory out again while one still reads it.  Samplers end on any thread, in the middle of anything (a collection of
+# cycles): what ends only appends, and one buffer at a time is taken out, looked at and, if still needed, put back.
+_retired: deque = deque()
 
 
 def _retire(places: dict) -> None:
-    _retired[:] = [p for p in _retired + list(places.values()) if not p[1].query()]
+    for place in list(places.values()):
+        _retired.append(place)
+
+
+def _give_back() -> None:
+    """Lets go of the retired buffers whose last copies have run."""
+    for _ in range(len(_retired)):
+        try:
+            place = _retired.popleft()
+        except IndexError:                          # (another thread was quicker)
+            return
+        done = False
+        try:
+            done = place[1].query()
+        finally:
+            if not done:
+                _retired.append(place)
 
 
 class Sampler:
@@ -139,6 +157,8 @@ class Sampler:
     def _staging_buffer(self, n: int):
         """A pinned buffer of at least n 32-bit numbers, the event to record behind its copy, its memory as bytes and its address: one of a
         few, each free again once its last copy has run."""
+        if _retired:
+            _give_back()
         at = self._staging_next = (self._staging_next + 1) % 4
         place = self._staging.get(at) if self._staging is not None else None
         if place is None or place[0].numel() < n:
