@@ -65,6 +65,9 @@ class Sampler:
         """int32 token ids [R] for float32 logits [R, V].  requests/indices: which request each
         row belongs to and which of its generated tokens this is (for the random stream);
         histories: each row's prompt + generated tokens (for penalties)."""
+        if logits.is_cuda and logits.device.index != torch.cuda.current_device():
+            with torch.cuda.device(logits.device):          # (kernels, copies and the staging buffers' events are all that device's)
+                return self.sample(logits, requests, indices, histories)
         p = self.params
         if p.is_greedy:
             return K.argmax(logits)

@@ -124,3 +124,49 @@ def test_an_event_that_can_not_be_asked_keeps_its_buffer():
         rest._staging_buffer(10)
     gc.collect()
     assert kept() is not None
+
+
+@pytest.mark.parametrize("current", [0, 1])
+def test_logits_on_a_device_that_is_not_the_current_one(current, monkeypatch):
+    """Everything that a draw queues is the logits' device's: an event is its first record's device's, and refuses another one's stream."""
+    import contextlib
+    from types import SimpleNamespace
+    now = [current]
+
+    class OnDevice(Event):
+        device, cuda_event = None, 0
+
+        def record(self, stream=None):
+            at = now[0] if stream is None else stream
+            self.device = at if self.device is None else self.device
+            assert self.device == at, "the event's device is not the stream's"
+
+    @contextlib.contextmanager
+    def device(d):
+        before, now[0] = now[0], d.index
+        yield
+        now[0] = before
+    monkeypatch.setattr(torch.cuda, "Event", OnDevice)
+    monkeypatch.setattr(torch.cuda, "device", device)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: now[0])
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda d=None: now[0] if d is None else d)
+    drawn = []
+
+    def draw(logits, host, staged, windows, settings, copied):
+        drawn.append(now[0])
+        return "ids"
+    monkeypatch.setattr(staging, "K", SimpleNamespace(**{**vars(staging.K), "sample_few_serves": lambda *a: True, "sample_few": lambda logits, *a: draw(logits, 0, 0, 0, 0, 0),
+                                                         "sample_few_staged": draw}))
+
+    class Logits:
+        device, shape, is_cuda = SimpleNamespace(index=1, type="cuda"), (2, 100), True
+        dim = staticmethod(lambda: 2)
+        is_contiguous = staticmethod(lambda: True)
+    if current == 0:                                          # (the general way's copy, which this stand-in for logits has no device for)
+        empty = torch.empty
+        monkeypatch.setattr(torch, "empty", lambda *a, device=None, **kw: empty(*a, **kw))
+    s = S.Sampler(S.GenerationParams(seed=1, repetition_penalty=1.0))
+    for step in range(6):
+        assert s.sample(Logits(), [0, 1], [step, step]) == "ids"
+    assert drawn == [1] * 6 and now == [current]
+    assert all(p[1].device == 1 for p in s._staging.values())
