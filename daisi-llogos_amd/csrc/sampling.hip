@@ -1013,24 +1013,21 @@ static int slice_values(int R, int V, int top_k) {
     return vpt * kSliceThreads;
 }
 
-// slices a row for sample_few, 0: not served (the entry below then refuses too): among others more rows than a grid is high
-LLOGOS_EXPORT int llogos_sample_few_slices(int R, int V, int top_k) {
+// slices a row, 0: not served: among others more rows than a grid is high
+static int few_slices(int R, int V, int top_k) {
     if (R <= 0 || R > 65535 || V <= 0 || top_k <= 0 || top_k > kFewCandidates || top_k >= V) return 0;
     const int values = slice_values(R, V, top_k), slices = (V + values - 1) / values;
     return slices <= kWave ? slices : 0;
 }
 
-LLOGOS_EXPORT int llogos_sample_few_cap(void) { return kSliceCap; }
-
 // Preparation and pipeline of rows of which at most top_k <= kFewCandidates tokens can be drawn: the tokens that llogos_sample_prepare
 // and llogos_sample_pipeline give.  keys [R][slices][cap] uint64, counts [R][slices], tops [R][slices]: scratch; work, prob [R][V] and
 // list [R][n_pad]: scratch of the rows that need the general way.  hist_at (or null): offsets [R + 1] of the rows' windows in hist.
-LLOGOS_EXPORT int llogos_sample_few(int* out, const float* logits, int R, int V, const int* hist, const int* hist_at,
-                                    float repetition, float frequency, float presence, float inv_temperature,
-                                    int penalize_newline, const int* banned, int n_banned, void* keys, int* counts, float* tops,
-                                    float* work, float* prob, void* list, int n_pad, const float* uniforms, int top_k, float top_p,
-                                    float min_p, float typical_p, int min_keep, hipStream_t stream) {
-    const int slices = llogos_sample_few_slices(R, V, top_k);
+static int sample_few(int* out, const float* logits, int R, int V, const int* hist, const int* hist_at, float repetition, float frequency,
+                      float presence, float inv_temperature, int penalize_newline, const int* banned, int n_banned, void* keys, int* counts,
+                      float* tops, float* work, float* prob, void* list, int n_pad, const float* uniforms, int top_k, float top_p,
+                      float min_p, float typical_p, int min_keep, hipStream_t stream) {
+    const int slices = few_slices(R, V, top_k);
     if (slices == 0 || n_banned < 0 || n_banned > kMaxBanned || n_pad < V || (n_pad & (n_pad - 1))) return LLOGOS_BAD_ARGUMENT;
     PenaltyParams pp{repetition, frequency, presence, inv_temperature, penalize_newline, n_banned, {}};
     for (int i = 0; i < n_banned; ++i) pp.banned[i] = banned[i];
@@ -1054,7 +1051,7 @@ struct SampleSettings {
 
 // 8-byte words of scratch memory for llogos_sample_few_staged beside the staged numbers; 0 where it does not serve
 LLOGOS_EXPORT long long llogos_sample_few_words(int R, int V, int top_k) {
-    const long long slices = llogos_sample_few_slices(R, V, top_k);
+    const long long slices = few_slices(R, V, top_k);
     if (slices == 0) return 0;
     long long n_pad = 1;
     while (n_pad < V) n_pad *= 2;
@@ -1063,7 +1060,7 @@ LLOGOS_EXPORT long long llogos_sample_few_words(int R, int V, int top_k) {
 
 LLOGOS_EXPORT int llogos_copy_words(void* dst, const void* src, long long n, hipStream_t stream);     // (elementwise.hip)
 
-// llogos_sample_few from what the host has packed into pinned memory: R uniform numbers (float32) and, with `windows`, the R + 1 places of the
+// sample_few from what the host has packed into pinned memory: R uniform numbers (float32) and, with `windows`, the R + 1 places of the
 // rows' windows and the windows, `staged` 32-bit numbers in all.  They are copied behind the scratch (16-byte aligned: llogos_sample_few_words words, then
 // `staged` numbers), `copied` (an event or null) is recorded behind the copy, and the two kernels follow: one call for what a step of
 // the sampler queues.
@@ -1071,7 +1068,7 @@ LLOGOS_EXPORT int llogos_sample_few_staged(int* out, const float* logits, int R,
                                            const void* settings, void* scratch, void* copied, hipStream_t stream) {
     const SampleSettings* s = (const SampleSettings*)settings;
     if (s == nullptr || host == nullptr || scratch == nullptr || staged < R + (windows ? R + 1 : 0)) return LLOGOS_BAD_ARGUMENT;
-    const long long slices = llogos_sample_few_slices(R, V, s->top_k), words = llogos_sample_few_words(R, V, s->top_k);
+    const long long slices = few_slices(R, V, s->top_k), words = llogos_sample_few_words(R, V, s->top_k);
     if (words == 0) return LLOGOS_BAD_ARGUMENT;
     long long n_pad = 1;
     while (n_pad < V) n_pad *= 2;
@@ -1088,7 +1085,7 @@ LLOGOS_EXPORT int llogos_sample_few_staged(int* out, const float* logits, int R,
         const hipError_t e = hipEventRecord((hipEvent_t)copied, stream);
         if (e != hipSuccess) return (int)e;
     }
-    return llogos_sample_few(out, logits, R, V, windows ? numbers + 2 * R + 1 : nullptr, windows ? numbers + R : nullptr, s->repetition, s->frequency,
+    return sample_few(out, logits, R, V, windows ? numbers + 2 * R + 1 : nullptr, windows ? numbers + R : nullptr, s->repetition, s->frequency,
                              s->presence, s->inv_temperature, s->penalize_newline, s->banned, s->n_banned, keys, counts, tops, work, prob, list,
                              (int)n_pad, (const float*)numbers, s->top_k, s->top_p, s->min_p, s->typical_p, s->min_keep, stream);
 }

@@ -2852,7 +2852,7 @@ def sample_pipeline(work: torch.Tensor, uniforms: torch.Tensor, top_k: int, top_
 
 
 def sample_few_serves(R: int, V: int, top_k: int) -> bool:
-    """Whether sample_few takes rows of V logits of which at most top_k tokens can be drawn."""
+    """Whether sample_few_staged takes rows of V logits of which at most top_k tokens can be drawn."""
     return _sample_few_words(R, V, int(top_k)) > 0
 
 
@@ -2875,8 +2875,9 @@ def sample_settings(repetition: float, frequency: float, presence: float, temper
 
 
 def sample_few_staged(logits: torch.Tensor, host: int, staged: int, windows: bool, settings: SampleSettings, copied: int) -> torch.Tensor:
-    """sample_few on numbers in pinned host memory at the address `host`: the rows' uniform numbers and, with `windows`, the places of
-    their windows and the windows, `staged` 32-bit numbers in all.  The event `copied` (its handle) is recorded behind their copy."""
+    """sample_prepare and sample_pipeline in one, for a small top-k: the same token ids int32 [R].  On numbers in pinned host memory at
+    the address `host`: the rows' uniform numbers and, with `windows`, the R + 1 places of their windows and the windows of recent tokens,
+    one after the other, `staged` 32-bit numbers in all.  The event `copied` (its handle) is recorded behind their copy."""
     _dev(logits)
     _need(logits.dtype == torch.float32 and logits.dim() == 2, "sample_few: logits must be contiguous float32 [R, V]")
     R, V = logits.shape
@@ -2886,36 +2887,6 @@ def sample_few_staged(logits: torch.Tensor, host: int, staged: int, windows: boo
     out = torch.empty((R,), dtype=torch.int32, device=logits.device)
     _check(_lib().llogos_sample_few_staged(out.data_ptr(), logits.data_ptr(), R, V, host, staged, windows, ctypes.addressof(settings),
                                            scratch.data_ptr(), copied, _stream()), "sample_few")
-    return out
-
-
-def sample_few(logits: torch.Tensor, history: Optional[torch.Tensor], history_at: Optional[torch.Tensor], repetition: float,
-               frequency: float, presence: float, temperature: float, penalize_newline: bool, banned: Sequence[int],
-               uniforms: torch.Tensor, top_k: int, top_p: float, min_p: float, typical_p: float, min_keep: int) -> torch.Tensor:
-    """sample_prepare and sample_pipeline in one, for a small top-k: the same token ids int32 [R].  The rows' windows of recent
-    tokens come one after the other: row r's are history[history_at[r] .. history_at[r + 1]) (int32, [R + 1] offsets)."""
-    _dev(logits, history, history_at, uniforms)
-    _i32(history, "history"); _i32(history_at, "history_at")
-    _need(logits.dtype == torch.float32 and logits.dim() == 2 and logits.is_contiguous(), "sample_few: logits must be contiguous float32 [R, V]")
-    _need(len(banned) <= MAX_BANNED, f"sample_few: at most {MAX_BANNED} banned ids, got {len(banned)}")
-    R, V = logits.shape
-    _need(uniforms.dtype == torch.float32 and uniforms.numel() == R, "sample_few: one float32 uniform per row")
-    _need((history is None) == (history_at is None) and (history_at is None or history_at.numel() == R + 1), "sample_few: history with R + 1 offsets")
-    lib = _lib()
-    slices = lib.llogos_sample_few_slices(R, V, int(top_k))
-    _need(slices > 0, f"sample_few: top_k {top_k} of {V} is not served")
-    n_pad = 1 << (V - 1).bit_length()
-    # one piece: the slices' keys, the rows' lists (8 bytes each), work and probabilities, the slices' counts and largest values
-    n_keys = R * slices * lib.llogos_sample_few_cap()
-    scratch = torch.empty(n_keys + R * n_pad + R * V + R * slices, dtype=torch.int64, device=logits.device)
-    keys, base = scratch.data_ptr(), scratch.data_ptr() + 8 * (n_keys + R * n_pad)
-    out = torch.empty((R,), dtype=torch.int32, device=logits.device)
-    ban = (ctypes.c_int * MAX_BANNED)(*list(banned))
-    inv_t = 1.0 / temperature if temperature > 0 else 1.0
-    _check(lib.llogos_sample_few(
-        _p(out), _p(logits), R, V, _p(history), _p(history_at), repetition, frequency, presence, inv_t, int(penalize_newline),
-        ban, len(banned), keys, base + 8 * R * V, base + 8 * R * V + 4 * R * slices, base, base + 4 * R * V, keys + 8 * n_keys, n_pad,
-        _p(uniforms), int(top_k), top_p, min_p, typical_p, int(min_keep), _stream()), "sample_few")
     return out
 
 

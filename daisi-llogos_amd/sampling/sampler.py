@@ -100,21 +100,15 @@ class Sampler:
         R = logits.shape[0]
         # one copy: uniform numbers, then each window's place and the windows, packed straight into the staging buffer
         starts, n, host, copied = self._pack(R, requests, indices, histories) or self._pack_in_python(requests, indices, histories)
-        if logits.device.index == torch.cuda.current_device() and starts == (R, 2 * R + 1 if p.has_penalties else R + 1):
-            banned = self.stop_tokens if p.prevent_eos else ()
-            key = (p, banned)
-            if self._settings_of != key:
-                self._settings = K.sample_settings(p.repetition_penalty, p.frequency_penalty, p.presence_penalty, p.temperature, p.penalize_newline,
-                                                   banned, p.top_k, p.top_p, p.min_p, p.typical_p, p.min_keep)
-                self._settings_of = key
-            return K.sample_few_staged(logits, host.data_ptr(), n, p.has_penalties, self._settings, copied.cuda_event)
-        dev = torch.empty(n, dtype=torch.int32, device=logits.device)
-        dev.copy_(host[:n], non_blocking=True)
-        copied.record(torch.cuda.current_stream(logits.device.index))    # (named by its number, which is quicker than finding the current device)
-        us = dev[:starts[0]].view(torch.float32)
-        hist, hist_at = (dev[starts[1]:], dev[starts[0]:starts[1]]) if p.has_penalties else (None, None)
-        return K.sample_few(logits, hist, hist_at, p.repetition_penalty, p.frequency_penalty, p.presence_penalty, p.temperature,
-                            p.penalize_newline, self.stop_tokens if p.prevent_eos else (), us, p.top_k, p.top_p, p.min_p, p.typical_p, p.min_keep)
+        if starts != (R, 2 * R + 1 if p.has_penalties else R + 1):
+            raise K.KernelError(f"sample: {R} rows of logits need a uniform number and, with penalties, a token history each")
+        banned = self.stop_tokens if p.prevent_eos else ()
+        key = (p, banned)
+        if self._settings_of != key:
+            self._settings = K.sample_settings(p.repetition_penalty, p.frequency_penalty, p.presence_penalty, p.temperature, p.penalize_newline,
+                                               banned, p.top_k, p.top_p, p.min_p, p.typical_p, p.min_keep)
+            self._settings_of = key
+        return K.sample_few_staged(logits, host.data_ptr(), n, p.has_penalties, self._settings, copied.cuda_event)
 
     def _pack(self, R: int, requests, indices, histories):
         """((where the windows' places begin, where the windows do), 32-bit numbers in all, staging buffer, its event) with R rows' uniform numbers and

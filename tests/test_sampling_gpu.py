@@ -442,6 +442,20 @@ def test_few_candidates_with_windows_of_every_length(n):
         assert S.Sampler(p).sample(logits, list(range(R)), [step] * R, histories).cpu().tolist() == want.cpu().tolist()
 
 
+def test_rows_without_a_number_or_a_window_are_refused():
+    K = importlib.import_module("daisi-llogos_amd.ops.kernels")
+    logits = torch.zeros(3, 500, device=DEV)
+    plain, penalties = (S.Sampler(S.GenerationParams(seed=2, repetition_penalty=r)) for r in (1.0, 1.2))
+    for rows in (2, 4):
+        with pytest.raises(K.KernelError, match="3 rows"):
+            plain.sample(logits, list(range(rows)), [0] * rows)
+        with pytest.raises(K.KernelError, match="3 rows"):
+            penalties.sample(logits, [0, 1, 2], [0, 0, 0], [[1]] * rows)
+    with pytest.raises(K.KernelError):
+        plain.sample(logits.cpu(), [0, 1, 2], [0, 0, 0])
+    assert plain.sample(logits, [0, 1, 2], [0, 0, 0]).shape == penalties.sample(logits, [0, 1, 2], [0, 0, 0], [[1]] * 3).shape == (3,)
+
+
 def test_samplers_that_end_before_their_copies():
     """Numbers are staged in pinned memory and copied by the kernel library; a sampler that is dropped, or that needs longer buffers, while
     the stream is still busy leaves them to the copies that are queued."""

@@ -152,19 +152,15 @@ def test_logits_on_a_device_that_is_not_the_current_one(current, monkeypatch):
     monkeypatch.setattr(torch.cuda, "current_stream", lambda d=None: now[0] if d is None else d)
     drawn = []
 
-    def draw(logits, host, staged, windows, settings, copied):
+    def draw(*a):
         drawn.append(now[0])
         return "ids"
-    monkeypatch.setattr(staging, "K", SimpleNamespace(**{**vars(staging.K), "sample_few_serves": lambda *a: True, "sample_few": lambda logits, *a: draw(logits, 0, 0, 0, 0, 0),
-                                                         "sample_few_staged": draw}))
+    monkeypatch.setattr(staging, "K", SimpleNamespace(**{**vars(staging.K), "sample_few_serves": lambda *a: True, "sample_few_staged": draw}))
 
     class Logits:
         device, shape, is_cuda = SimpleNamespace(index=1, type="cuda"), (2, 100), True
         dim = staticmethod(lambda: 2)
         is_contiguous = staticmethod(lambda: True)
-    if current == 0:                                          # (the general way's copy, which this stand-in for logits has no device for)
-        empty = torch.empty
-        monkeypatch.setattr(torch, "empty", lambda *a, device=None, **kw: empty(*a, **kw))
     s = S.Sampler(S.GenerationParams(seed=1, repetition_penalty=1.0))
     for step in range(6):
         assert s.sample(Logits(), [0, 1], [step, step]) == "ids"
