@@ -167,7 +167,7 @@ __global__ __launch_bounds__(WAVES * kWave) void gemm_residual_kernel(
     if (c == 0) sums[(size_t)blockIdx.x * kResidualRows + m] = sq;
 }
 
-// strips_per_block: 1 or 2 strips of 16 rows of w a block (two share a wave's copy of the activations and halve
+// strips_per_block: 1 or 2 strips of 16 rows of w a block (two, of 4 or 8 waves, share a wave's copy of the activations and halve
 // the number of blocks), or 0: half a strip.  sums: float32 [blocks][16], blocks = ceil(ceil(N / 16) / strips_per_block)
 // or 2 ceil(N / 16), written whole (rows from M on hold 0): a block's sum of squares of each row of x over its 8, 16 or 32
 // columns.  unscaled (optional, with norm_w [N]): bfloat16 [M][ldu] = x * norm_w of the new x, the rows of an rmsnorm that
@@ -189,7 +189,6 @@ LLOGOS_EXPORT int llogos_gemm_residual_bf16(float* x, int ldx, float* sums, void
     else if (strips_per_block == 1 && waves == 16) GO(16, 1, false, 4);
     else if (strips_per_block == 2 && waves == 4) GO(4, 2, false, 4);
     else if (strips_per_block == 2 && waves == 8) GO(8, 2, false, 4);
-    else if (strips_per_block == 2 && waves == 16) GO(16, 2, false, 4);
     else if (strips_per_block == 0 && waves == 8) GO(8, 1, true, 8);
     else if (strips_per_block == 0 && waves == 16) GO(16, 1, true, 4);
     else return LLOGOS_BAD_ARGUMENT;

@@ -1031,7 +1031,9 @@ def test_product_that_adds_itself_to_the_residual_stream(M, N, K_, waves, strips
     alone = x0[:1].clone()
     K.gemm_residual_bf16(alone, a[:1].contiguous(), pw, None, waves, strips=strips)
     assert torch.equal(alone, x1[:1])
-    # refused: more than 16 rows, a packed gate/up matrix
+    # refused: two strips a block of 16 waves, whose registers do not fit; more than 16 rows
+    with pytest.raises(K.KernelError):
+        K.gemm_residual_bf16(x1, a, pw, None, 16, strips=2)
     assert K.gemm_residual_bf16(torch.zeros(17, N, device=DEV), torch.zeros(17, K_, device=DEV, dtype=torch.bfloat16), pw, None, waves) is None
 
 
