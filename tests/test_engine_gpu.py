@@ -508,6 +508,44 @@ def test_replayed_steps_of_twenty_sequences():
     assert len(engines[0].graphs.graphs) >= 1
 
 
+@pytest.mark.parametrize("order", ["keep first", "lend first"])
+@pytest.mark.parametrize("design", ["tiny_b", "nip_a"])
+def test_logits_that_are_kept_and_logits_that_are_lent(design, order, monkeypatch):
+    """Logits of replayed steps belong to the caller, also when the batch is padded, the head has a scale, or the shape's logits are lent in
+    between: later replays leave them alone, and all are those of uncaptured steps.  Keeping and lending share a shape's one graph,
+    which is captured again at most once, and take its place among those that are kept."""
+    import nipulorn_helpers
+    graph_mod = importlib.import_module("daisi-llogos_amd.engine.graph")
+    monkeypatch.setattr(graph_mod, "MAX_GRAPHS", 2)
+    captures, capture = [], torch.cuda.graph
+    monkeypatch.setattr(torch.cuda, "graph", lambda g: (captures.append(g), capture(g))[1])
+    helper = H if design == "tiny_b" else nipulorn_helpers
+    engines = [helper.engine(design, "bfloat16", max_tokens=64 * 24, n_slots=12, use_graphs=g) for g in (True, False)]
+    slots = [[eng.alloc_slot() for _ in range(9)] for eng in engines]
+    for eng, sl in zip(engines, slots):
+        eng.step([(s, list(helper.tokens(design, 3 + i, 40 + i))) for i, s in enumerate(sl)], want=None)
+    kept, lent, want = [], [], []
+    for t in range(12):
+        n, borrow = (2, 9)[t % 2], (t // 2 % 3 == 1) if order == "keep first" else (t // 2 % 3 == 0)
+        toks = helper.tokens(design, n, 90 + t)
+        out = engines[0].step([(s, [int(k)]) for s, k in zip(slots[0], toks)], want="last", borrow=borrow)
+        if borrow:
+            lent.append((t, out.clone()))                    # (in stream order, before the next step)
+        else:
+            kept.append((t, out))
+        want.append(engines[1].step([(s, [int(k)]) for s, k in zip(slots[1], toks)], want="last"))
+    assert len(kept) == 8 and len(lent) == 4
+    assert len({out.data_ptr() for _, out in kept}) == len(kept)
+    for t, out in kept + lent:
+        assert torch.equal(out, want[t]), t
+    assert len(engines[0].graphs.graphs) == 2
+    assert len(captures) == (4 if order == "keep first" else 2)
+    # (a third shape takes the place of the one used longest ago, not of both)
+    two = list(engines[0].graphs.graphs)
+    engines[0].step([(slots[0][0], [1])], want="last")
+    assert list(engines[0].graphs.graphs)[0] == two[1]
+
+
 def test_captured_steps_are_dropped_and_made_again(monkeypatch):
     """More batch shapes than captured steps are kept: the least recently used one goes, and
     a shape that comes back is captured again; results stay those of uncaptured steps."""
