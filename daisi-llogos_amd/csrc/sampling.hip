@@ -112,20 +112,29 @@ struct PenaltyParams {
     int banned[kMaxBanned];
 };
 
-// The tokens of the window h[0 .. n) that lie in first .. first + count - 1 are made again from the logits, penalty first,
-// then the scale, and put to w[token - first].  A round's threads look at a position of the window each and list those
+// The tokens of a window of n that lie in first .. first + count - 1 are made again from the logits, penalty first, then the scale.  A round's threads look at a position of the window each and list those
 // that name such a token; a wave takes a listed position and reads the window 64 tokens at a time: a token's first occurrence
 // does the work.  (One thread a position, reading the window token by token, made this 11 us of a slice's 16.)  put(q, place, value) takes
-// the new value of a round's listed position q (place -1: an earlier position names the token), round() ends a round.
+// the new value for first + place of a round's listed position q (place -1: an earlier position names the token), round() ends a round.
 struct WindowLds {
     int n;
     int at[kSampleThreads];
 };
 
-// near: h as far as it is kept nearer (LDS), or h itself.
-template <typename Near, typename Put, typename Round>
-__device__ __forceinline__ void apply_penalties(const float* __restrict__ row, int first, int count, int V, const int* __restrict__ h, Near near, int n,
-                                                const PenaltyParams& pp, WindowLds& lds, Put put, Round round) {
+// Adds to `times` how often a wave (lane) finds position i's token tok at positions BEGIN .. END - 1; where a position before i names it too, times is 0
+// and LAST is done.  (As a loop each for LDS and memory: choosing for each position where to read, 64 windows of 8,000 tokens took 8 % longer.)
+#define LLOGOS_COUNT_TOKEN(TOKEN, BEGIN, END, LAST) \
+    for (int j0 = (BEGIN); j0 < (END); j0 += kWave) { \
+        const uint64_t same = __ballot(j0 + lane < (END) && TOKEN(j0 + lane) == tok); \
+        const uint64_t later = j0 >= i ? ~(uint64_t)0 : i - j0 >= kWave ? 0 : ~(uint64_t)0 << (i - j0); \
+        if (same & ~later) { times = 0; LAST; break; } \
+        times += (int)__popcll(same & later); \
+    }
+
+// token(i): the window's token at a position; times_of(i, tok): how often the window names position i's token, 0 where an earlier one does.
+template <typename Token, typename Times, typename Put, typename Round>
+__device__ __forceinline__ void apply_penalties(const float* __restrict__ row, int first, int count, int V, int n, const PenaltyParams& pp,
+                                                WindowLds& lds, Token token, Times times_of, Put put, Round round) {
     const float inv_t = pp.inv_temperature;
     const bool scaled = inv_t != 1.0f;
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave, waves = blockDim.x / kWave;
@@ -134,20 +143,13 @@ __device__ __forceinline__ void apply_penalties(const float* __restrict__ row, i
         if (threadIdx.x == 0) lds.n = 0;
         __syncthreads();
         if (i0 + (int)threadIdx.x < n) {
-            const int tok = near(i0 + threadIdx.x);
+            const int i = i0 + threadIdx.x, tok = token(i);
             if (tok >= first && tok - first < count && tok < V && (pp.penalize_newline || (tok != 10 && tok != 13)))
-                lds.at[atomicAdd(&lds.n, 1)] = i0 + threadIdx.x;
+                lds.at[atomicAdd(&lds.n, 1)] = i;
         }
         __syncthreads();
         for (int q = wave; q < lds.n; q += waves) {
-            const int i = lds.at[q], tok = near(i);
-            int times = 0;
-            for (int j0 = 0; j0 < n; j0 += kWave) {
-                const uint64_t same = __ballot(j0 + lane < n && near(j0 + lane) == tok);
-                const uint64_t later = j0 >= i ? ~(uint64_t)0 : i - j0 >= kWave ? 0 : ~(uint64_t)0 << (i - j0);
-                if (same & ~later) { times = 0; break; }             // an earlier position names it too
-                times += (int)__popcll(same & later);
-            }
+            const int i = lds.at[q], tok = token(i), times = times_of(i, tok);
             if (lane != 0) continue;
             if (times == 0) { put(q, -1, 0.f); continue; }
             float l = row[tok];
@@ -175,7 +177,10 @@ __device__ void prepare_row(float* w, const float* __restrict__ row, int V, cons
     for_each_value(row, V, [&](int i, float x) { w[i] = scaled ? x * inv_t : x; });
     __syncthreads();
     if (has_penalties(pp) && h) {
-        apply_penalties(row, 0, V, V, h, [&](int i) { return h[i]; }, n, pp, lds, [&](int, int place, float x) { if (place >= 0) w[place] = x; }, [] {});
+        const int lane = threadIdx.x & (kWave - 1);
+        auto token = [&](int i) { return h[i]; };
+        apply_penalties(row, 0, V, V, n, pp, lds, token, [&](int i, int tok) { int times = 0; LLOGOS_COUNT_TOKEN(token, 0, n, ) return times; },
+                        [&](int, int place, float x) { if (place >= 0) w[place] = x; }, [] {});
         __syncthreads();
     }
     if (threadIdx.x < pp.n_banned) {
@@ -624,26 +629,44 @@ void sample_slices_kernel(
     if (threadIdx.x == 0) counter = 0;
 #pragma unroll
     for (int j = 0; j < VPT; ++j) v[j] = scaled ? v[j] * inv_t : v[j];
-    // a new value for the slice's value i: the thread that holds it takes it
-    auto take = [&](int i, float x) {
-        const int n = wide ? i >> 2 : i;
-        if (n % kSliceThreads != (int)threadIdx.x) return;
-        const int mine = wide ? n / kSliceThreads * 4 + (i & 3) : n / kSliceThreads;
-#pragma unroll
-        for (int j = 0; j < VPT; ++j) v[j] = j == mine ? x : v[j];
+    // the thread that holds the slice's value i, and in which of its places (above 16 bits); it takes a new value for it (`at` the same for all)
+    auto holder = [&](unsigned i) {
+        const unsigned n = wide ? i >> 2 : i;
+        return n % kSliceThreads | (wide ? n / kSliceThreads * 4 + (i & 3) : n / kSliceThreads) << 16;
+    };
+    auto take = [&](unsigned at, float x) {
+        if ((at & 0xffff) == threadIdx.x) v[at >> 16] = x;
     };
     if (penalties) {
-        apply_penalties(row, first, count, V, h, [&](int i) { return i < kHeadBins ? lds[i] : h[i]; }, n_hist, pp, window,
-                        [&](int q, int i, float x) { patch_at[q] = i; patch[q] = x; },
-                        [&] {
-                            __syncthreads();
-                            for (int q = 0; q < window.n; ++q)
-                                if (patch_at[q] >= 0) take(patch_at[q], patch[q]);
-                        });
+        // A round's new values, 64 at a time: a wave passes over those that others hold.  (One after the other, each waited for in LDS by all
+        // waves, they were 40 us of a draw's 144 where 512 tokens of a window lie in one slice; so it takes 111.)
+        auto put = [&](int q, int i, float x) { patch_at[q] = i; patch[q] = x; };
+        auto round = [&] {
+            __syncthreads();
+            for (int q0 = 0; q0 < window.n; q0 += kWave) {
+                const int i = q0 + lane < window.n ? patch_at[q0 + lane] : -1;
+                const int x = __float_as_int(patch[q0 + lane]);                // (of those behind the last nothing is used)
+                const unsigned at = holder(i);
+                for (uint64_t mine = __ballot(i >= 0 && (at & 0xffff) / kWave == wave); mine; mine &= mine - 1) {
+                    const int l = __builtin_ctzll(mine);
+                    take(__builtin_amdgcn_readlane(at, l), __int_as_float(__builtin_amdgcn_readlane(x, l)));
+                }
+            }
+        };
+        auto near = [&](int i) { return lds[i]; };
+        auto far = [&](int i) { return h[i]; };
+        const int n_near = min(n_hist, kHeadBins);
+        apply_penalties(row, first, count, V, n_hist, pp, window, [&](int i) { return i < n_near ? near(i) : far(i); }, [&](int i, int tok) {
+            int times = 0;
+            bool more = n_near < n_hist;
+            LLOGOS_COUNT_TOKEN(near, 0, n_near, more = false)
+            if (more) { LLOGOS_COUNT_TOKEN(far, n_near, n_hist, ) }
+            return times;
+        }, put, round);
     }
     for (int i = 0; i < pp.n_banned; ++i) {
         const int tok = pp.banned[i] - first;
-        if (tok >= 0 && tok < count) take(tok, -INFINITY);
+        if (tok >= 0 && tok < count) take(holder(tok), -INFINITY);
     }
     float m = -INFINITY;
 #pragma unroll

@@ -442,6 +442,29 @@ def test_few_candidates_with_windows_of_every_length(n):
         assert S.Sampler(p).sample(logits, list(range(R)), [step] * R, histories).cpu().tolist() == want.cpu().tolist()
 
 
+@pytest.mark.parametrize("V", [32000, 32002, 128256])
+@pytest.mark.parametrize("n,distinct", [(64, 64), (65, 500), (600, 500), (2100, 700)])
+def test_few_candidates_with_a_window_crowded_into_one_slice(n, distinct, V):
+    """Tokens that lie next to one another are held by a few waves of one block, several by one thread: each gets its new value, once."""
+    K = importlib.import_module("daisi-llogos_amd.ops.kernels")
+    R, first = 3, (0, 5, V - 1000)
+    rng = np.random.default_rng(n + V)
+    p = S.GenerationParams(seed=9, temperature=0.9, top_k=100, top_p=1.0, repetition_penalty=1.2, frequency_penalty=0.05, presence_penalty=0.1, penalty_count=0)
+    x = rng.standard_normal((R, V)).astype(np.float32)
+    for r in range(R):                                     # (what the window names is what may be drawn)
+        x[r, first[r]:first[r] + distinct] += 4.0
+    histories = [(first[r] + rng.integers(0, distinct, size=n)).tolist() for r in range(R)]
+    logits = torch.tensor(x, device=DEV)
+    padded = torch.tensor(np.array(histories, np.int32), device=DEV)
+    work = K.sample_prepare(logits, padded, torch.full((R,), n, dtype=torch.int32, device=DEV), p.repetition_penalty, p.frequency_penalty,
+                            p.presence_penalty, p.temperature, p.penalize_newline, ())
+    sampler = S.Sampler(p)
+    for step in range(40):
+        us = torch.tensor(sampler.uniforms(list(range(R)), [step] * R), dtype=torch.float32, device=DEV)
+        want = K.sample_pipeline(work, us, p.top_k, p.top_p, p.min_p, p.typical_p, p.min_keep)
+        assert sampler.sample(logits, list(range(R)), [step] * R, histories).cpu().tolist() == want.cpu().tolist()
+
+
 def test_rows_without_a_number_or_a_window_are_refused():
     K = importlib.import_module("daisi-llogos_amd.ops.kernels")
     logits = torch.zeros(3, 500, device=DEV)
