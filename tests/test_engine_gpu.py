@@ -49,13 +49,17 @@ def test_prompts_are_queued_behind_work_that_still_runs():
     for p in prompts:
         alone.append(run(p))
         torch.cuda.synchronize()
-    done = torch.cuda.Event()
-    torch.cuda._sleep(40_000_000)                    # (tens of milliseconds at the least)
-    done.record()
-    behind = [run(p) for p in prompts]
-    assert not done.query()
-    torch.cuda.synchronize()
-    assert all(torch.equal(a, b) for a, b in zip(alone, behind))
+    for milliseconds in (50.0, 200.0, 800.0):        # (a host that waits outlasts every spin, a slow one the short ones)
+        done = torch.cuda.Event()
+        H.llogos.StepProbe().hold(milliseconds)
+        done.record()
+        behind = [run(p) for p in prompts]
+        queued = not done.query()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(alone, behind))
+        if queued:
+            break
+    assert queued
 
 
 @pytest.mark.parametrize("dtype", H.DTYPES)

@@ -479,24 +479,41 @@ def test_rows_without_a_number_or_a_window_are_refused():
     assert plain.sample(logits, [0, 1, 2], [0, 0, 0]).shape == penalties.sample(logits, [0, 1, 2], [0, 0, 0], [[1]] * 3).shape == (3,)
 
 
-def test_samplers_that_end_before_their_copies():
-    """Numbers are staged in pinned memory and copied by the kernel library; a sampler that is dropped, or that needs longer buffers, while
-    the stream is still busy leaves them to the copies that are queued."""
+@pytest.mark.parametrize("keep", [True, False])
+def test_samplers_that_end_before_their_copies(keep):
+    """Numbers are staged in pinned memory and copied by the kernel library; a sampler that needs longer buffers (keep), or that is dropped,
+    while the stream is still busy leaves them to the copies that are queued.  What torch would hand out again of such memory (it keeps
+    freed blocks by powers of two of their size) is filled with other numbers at once."""
+    staging = importlib.import_module("daisi-llogos_amd.sampling.sampler")
     R, V = 5, 5000
     rng = np.random.default_rng(4)
     logits = torch.tensor(rng.standard_normal((R, V)).astype(np.float32), device=DEV)
     p = S.GenerationParams(seed=2, temperature=1.0, top_k=50, top_p=1.0, repetition_penalty=1.5, penalty_count=0)
     long = [rng.integers(0, V, size=4000).tolist() for _ in range(R)]
-    calls = [(step, long if step % 3 == 2 else [h[:50 + step] for h in long]) for step in range(24)]
-    want = [S.Sampler(p).sample(logits, list(range(R)), [s] * R, h).cpu().tolist() for s, h in calls]
-    busy = torch.randn(4096, 4096, device=DEV)
-    one = S.Sampler(p)
-    for keep in (True, False):
+    # a kept sampler fills its four places with short buffers, and replaces each by a long one without waiting for its copy
+    calls = [(step, long if step >= 4 else [h[:50 + step] for h in long]) for step in range(8)]
+    draw = lambda sampler, s, h: sampler.sample(logits, list(range(R)), [s] * R, h)
+    want = [draw(S.Sampler(p), s, h).cpu().tolist() for s, h in calls]
+    numbers = {1024, 2 * (R + R + 1 + 4000 * R)}                            # (of a short and of a long buffer)
+    for milliseconds in (100.0, 400.0, 1600.0):                             # (a spin that the host's eight calls outlast shows nothing)
         torch.cuda.synchronize()
-        for _ in range(20):
-            busy = torch.tanh(busy @ busy)                 # the stream is behind
-        got = []
+        one, done = S.Sampler(p), torch.cuda.Event()
+        H.llogos.StepProbe().hold(milliseconds)
+        done.record()
+        got, places, again = [], set(), set()
         for s, h in calls:
-            got.append((one if keep else S.Sampler(p)).sample(logits, list(range(R)), [s] * R, h))
-            torch.full((12000,), 7, dtype=torch.int32, pin_memory=True)        # (would land in memory that was given back too early)
+            sampler = one if keep else S.Sampler(p)
+            got.append(draw(sampler, s, h))
+            places |= {place[0].data_ptr() for place in sampler._staging.values()}
+            del sampler
+            again |= places & {f.data_ptr() for f in [torch.full((n,), 7, dtype=torch.int32, pin_memory=True) for n in numbers]}
+        kept = {place[0].numel() for place in staging._retired}
+        behind = not done.query()
         assert [t.cpu().tolist() for t in got] == want
+        if behind:
+            break
+    assert behind and kept == ({1024} if keep else numbers) and not again
+    torch.cuda.synchronize()
+    last = S.Sampler(p)
+    draw(last, 0, long)
+    assert not [place for place in staging._retired if place[0].data_ptr() in places]
