@@ -15,7 +15,8 @@ import torch
 
 class StepProbe:
     """Collects marks of one or several steps; `totals()` gives, per name, how many intervals ended at a
-    mark of that name and how many milliseconds they took together.
+    mark of that name and how many milliseconds they took together.  (Where a step's first norm makes the stream from the
+    embedding, and the rotary table beside it, in one kernel, "embed" ends before it: its time is the first "norm"'s.)
 
     The host queues a step's kernels more slowly than the GPU runs the short ones, and an interval would
     then hold the GPU's waiting.  `hold(ms)` queues a spin of that length first, so that the host gets

@@ -265,7 +265,7 @@ class Model:
         s = self.spec
         blocks = [self.layers[entry.layer] for entry in self.schedule]
         x, pending = self._open(ctx, blocks[0] if blocks else None)
-        ctx.mark("embed")
+        ctx.mark("embed")                       # (nothing is queued yet where the first norm opens the step: that norm's mark holds its time)
         # the embedding output, for stream parts that read it again; the stream itself is changed in place
         x0 = x.clone() if any(e.enter is not None for e in self.schedule[1:]) else x
         for i, (block, units) in enumerate(zip(blocks, self.entry_units)):
