@@ -114,8 +114,8 @@ LLOGOS_EXPORT int llogos_scale_softcap(float* x, long long n, float scale, float
 }
 
 // A few thousand integers from pinned host memory, which the GPU reads where it lies: bound by one trip to the host.  In front of the
-// sampler's two kernels it is 1.4 us shorter than the runtime's copy (64 rows, 40 KB: 30.0 -> 28.5 us a step); in front of a replayed
-// step, whose copy it would be too, 1 us of 700, and the buffer's life would be the caller's to watch.
+// sampler's two kernels a step is 1.4 us shorter with it than with the runtime's copy (64 rows, 40 KB: 2.9 us for 3.5, and no gap of the
+// copy's own); in front of a replayed step, whose copy it would be too, 1 us of 700, and the buffer's life would be the caller's to watch.
 __global__ void copy_words_kernel(uint32_t* __restrict__ dst, const uint32_t* __restrict__ src, long long n, int quads) {
     const long long i = ((long long)blockIdx.x * blockDim.x + threadIdx.x) * 4;
     if (quads && i + 3 < n) {

@@ -534,7 +534,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_pipeline_kernel(
 // the row's largest, sorts what is left and draws.  Up to 64 candidates one wave does steps 2 to 6 without a barrier; its sums
 // are the additions of the block's in the same order.  Whatever these lists cannot decide (an infinite value, thousands of
 // values within a bin) is done again by the row's block in the general way.
-// 64 rows of 128,256 logits, top-k 40, penalties: 76 us in the two kernels above, 22 here (14.3 + 7.6).  Twice or four times as many,
+// 64 rows of 128,256 logits, top-k 40, penalties: 76 us in the two kernels above, 20 here (13.0 + 6.8; one row 65 and 14).  Twice or four times as many,
 // shorter slices at 64 rows took 4 and 11 us more.
 constexpr int kFewCandidates = 256;      // largest top-k served
 constexpr int kSliceThreads = 512;
@@ -588,9 +588,10 @@ __device__ int cut_bin(const int* bins, int want, int* part, int* cut, int* tota
 //
 // A block is a chain of short steps that wait, so all of a launch's blocks are to be on the units at once: 64 registers let 4 in.  A
 // slice's list is cut without bins: a wave sorts its threads' own largest values and offers the (top_k / 8)-th (rounded up); the largest of
-// the eight that top_k threads' values reach (the least one in any case) cuts the list, which a tenth to a half more than top_k values pass.  64 rows of 128,256 logits 14.3 us.  (22.5 with the slice's values patched in LDS, 97
-// registers, two rounds of blocks and the top_k-th of all threads' largest values found by counting them in bins: the additions to the few
-// bins that they share, 1.9 us alone, took 5.3 with four blocks on a unit, and a bin for each value before it is listed 4.3.)
+// the eight that top_k threads' values reach (the least one in any case) cuts the list, which a tenth to a half more than top_k values pass.
+// 64 rows of 128,256 logits 13.0 us.  (19.3 with the slice's values patched in LDS, 97 registers, two rounds of blocks and the top_k-th of all
+// threads' largest values found by counting them in bins: the additions to the few bins that they share, 1.9 us alone, took 5.3 with four
+// blocks on a unit, and a bin for each value before it is listed 4.3.)
 template <int VPT>
 __global__ __launch_bounds__(kSliceThreads) __attribute__((amdgpu_waves_per_eu(8)))
 void sample_slices_kernel(
